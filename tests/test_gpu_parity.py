@@ -416,3 +416,27 @@ def test_fp32_fits_against_fp64(ctx, kind):
         assert ang.max() < 1e-3
     if kind == "lines":
         assert fb.sum() > 0.9 * live.sum()
+
+
+@pytest.mark.parametrize("slope,min_hs", [(1.0, 0.1), (4.0, 0.0)])
+def test_classify_long_leaf_lists_match_oracle(ctx, slope, min_hs):
+    # outliers far above a cloud of more than 256 leaves: waves whose walk
+    # takes more leaves than a list's own place (64) and than a list (256)
+    # holds; a steep slope reaches few of them and leaves most points open
+    cloud = synth.generate(seed=91, extent=46.0, density=24.0, buildings=60, trees=200,
+                           outliers=0.02, outlier_low=0.0)
+    center, side = W.Octree.size_fit(cloud["bbmin"], cloud["bbmax"])
+    tree = W.Octree.build(ctx, cloud["xi"], cloud["yi"], cloud["zi"], cloud["scale"],
+                          cloud["offset"], center, side)
+    try:
+        assert tree.info()["nleaves"] > 256
+        got, _, st = W.classify(tree, cloud["bbmin"], cloud["bbmax"],
+                                W.default_params(max_slope=slope, min_hs=min_hs),
+                                want_tiles=False)
+        op = O.default_params()
+        op.max_slope, op.min_hs = slope, min_hs
+        want, _, _ = O.run(cloud, op)
+        print("leaves", tree.info()["nleaves"], "heavy", st["heavy_points"])
+        assert np.array_equal(got, want)
+    finally:
+        tree.free()

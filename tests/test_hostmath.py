@@ -506,3 +506,92 @@ def test_membership_candidates_cover_every_tile_within_reach():
                 cx, cy = centre(a, b)
                 if (cx - x) ** 2 + (cy - y) ** 2 <= lim * lim:
                     assert (a, b) in seven, (x, y, a, b)
+
+
+def test_lane_wedges_keep_every_care_direction(hm):
+    # a lane's two-wedge forms: a box, or a direction, they refuse holds no
+    # direction in an empty run of 24 bins or more
+    hm.wbh_lane_wedges.argtypes = [C.c_uint64] + [C.c_double] * 6
+    hm.wbh_dir_bin.argtypes = [C.c_double, C.c_double]
+    rng = np.random.default_rng(31)
+    refused = [0, 0]
+    for it in range(20000):
+        nb = int(rng.integers(1, 7))
+        occ = 0
+        base = int(rng.integers(0, 64))
+        for _ in range(nb):
+            occ |= 1 << ((base + int(rng.integers(0, 40))) % 64)
+        care = care_bins(occ)
+        w, h = rng.uniform(0, 3, 2) if it % 3 else (0.0, 0.0)
+        x0, y0 = rng.normal(size=2) * 3
+        if it % 2:  # a corner within 0.01 rad of a bin's edge
+            th = -math.pi + int(rng.integers(0, 64)) * math.pi / 32 + rng.uniform(-0.01, 0.01)
+            d = rng.uniform(0.1, 20)
+            x0, y0 = d * math.cos(th), d * math.sin(th)
+        got = hm.wbh_lane_wedges(occ, 0.0, 0.0, x0, x0 + w, y0, y0 + h)
+        first = hm.wbh_dir_bin(y0, x0)
+        if not got & 2:
+            refused[1] += 1
+            assert first not in care, (occ, x0, y0)
+        if not got & 1:
+            refused[0] += 1
+            for u in np.linspace(0, 1, 5):
+                for v in np.linspace(0, 1, 5):
+                    assert hm.wbh_dir_bin(y0 + v * h, x0 + u * w) not in care, (occ, x0, y0, w, h)
+    assert min(refused) > 500
+
+
+def test_hyp_near_covers_hyp_in(hm):
+    # every point hyp_in takes reaches hyp_near's threshold: random points, and
+    # points within a few roundings of the surface at map coordinates
+    hm.wbh_hyp_near.argtypes = [D, D]
+    rng = np.random.default_rng(32)
+    seen = 0
+    for it in range(60000):
+        c = np.array([5e5, 4.4e6, 100.0]) * (it % 2) + rng.normal(size=3) * 10
+        hs, sl = rng.choice([0.0, 0.1, 0.3, 2.0]), rng.choice([0.02, 0.5, 1.0, 3.0])
+        p = np.array([c[0], c[1], c[2], hs, sl])
+        d, th = abs(rng.normal()) * rng.choice([1e-3, 1.0, 40.0]), rng.uniform(0, 2 * np.pi)
+        por = hs * (sl * sl)
+        drop = math.sqrt(por * por + (sl * d) ** 2) - por
+        q = np.array([c[0] + d * math.cos(th), c[1] + d * math.sin(th),
+                      c[2] - drop + rng.choice([0.0, 1.0]) * rng.normal() * 2.0 ** rng.integers(-45, 2)])
+        got = hm.wbh_hyp_near(p.ctypes.data_as(D), q.ctypes.data_as(D))
+        seen += got & 1
+        assert got != 1, (p, q)
+    assert seen > 10000
+
+
+def test_direction_position_within_margin(hm):
+    # where the float path is sure, its position lies within 2^-14 bins of
+    # atan2i's (the gap pass looks 2^-13 either side)
+    hm.wbh_dir_est.argtypes = [C.c_double, C.c_double, C.POINTER(C.c_float), D]
+    rng = np.random.default_rng(33)
+    pos, exact = C.c_float(), C.c_double()
+    sure = 0
+    for it in range(60000):
+        dx, dy = rng.integers(-4000, 4000, 2) * 0.001 if it % 2 else rng.normal(size=2)
+        b = hm.wbh_dir_est(dy, dx, C.byref(pos), C.byref(exact))
+        if b < 0:
+            continue
+        sure += 1
+        assert b == int(exact.value)
+        assert abs(pos.value - exact.value) < 2.0 ** -14, (dy, dx)
+    assert sure > 50000
+
+
+def test_octet_bounds_round_outwards(hm):
+    # rel_down and rel_up hold the difference with room for the rounding of
+    # any other difference from the origin
+    for f in ("wbh_rel_down", "wbh_rel_up"):
+        getattr(hm, f).restype = C.c_float
+        getattr(hm, f).argtypes = [C.c_double] * 3
+    rng = np.random.default_rng(34)
+    for it in range(20000):
+        side = 2.0 ** rng.integers(-3, 14)
+        o = rng.normal() * 4e6
+        v = o + rng.uniform(-1, 1) * side * (100 if it % 5 == 0 else 0.5)
+        d, slack = v - o, side * 2.0 ** -41
+        assert hm.wbh_rel_down(v, o, side) <= d - slack
+        assert hm.wbh_rel_up(v, o, side) >= d + slack
+    assert hm.wbh_rel_down(1e300, 0.0, 1.0) <= 3.1e38 and hm.wbh_rel_up(-1e300, 0.0, 1.0) >= -3.1e38

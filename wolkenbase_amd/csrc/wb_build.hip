@@ -752,7 +752,8 @@ __global__ void k_fill_pt_leaf(const uint32_t *leaf_start, uint32_t nl, uint32_t
 // level above splits), so a node's depth follows from its side.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_leaf_zlow(const uint32_t *leaf_start, uint32_t nl,
-                                                   const double *pz, double *leaf_zlow)
+                                                   const double *pz, double *leaf_zlow,
+                                                   float *leaf_low)
 {
   const uint32_t l = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   if (l >= nl) return;
@@ -760,7 +761,10 @@ __global__ void __launch_bounds__(256) k_leaf_zlow(const uint32_t *leaf_start, u
   double m = __builtin_inf();
   for (uint32_t j = b + lane; j < e; j += WAVE) m = fmin(m, pz[j]);
   for (int d = 1; d < WAVE; d <<= 1) m = fmin(m, __shfl_xor(m, d, WAVE));
-  if (lane == 0) leaf_zlow[l] = m;
+  if (lane == 0) {
+    leaf_zlow[l] = m;
+    leaf_low[l] = (float)(m - fabs(m) * 0x1p-22);
+  }
 }
 
 __global__ void k_node_zlow(const int32_t *node_child, const double *node_cube, uint32_t nn,
@@ -786,7 +790,7 @@ __global__ void k_node_zlow(const int32_t *node_child, const double *node_cube, 
 template <bool F64>
 __global__ void k_permute(Src src, const uint32_t *sidx, uint64_t n, Xform f, double *px,
                           double *py, double *pz, double *box, uint32_t *low, double *lowx,
-                          double *lowy, double *lowz)
+                          double *lowy, double *lowz, float4 *oct_xy, float *oct_z)
 {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool ok = i < n;
@@ -821,6 +825,14 @@ __global__ void k_permute(Src src, const uint32_t *sidx, uint64_t n, Xform f, do
     y1 = fmax(y1, __shfl_xor(y1, d, WAVE));
     z0 = fmin(z0, __shfl_xor(z0, d, WAVE));
     z1 = fmax(z1, __shfl_xor(z1, d, WAVE));
+    if (2 * d == WB_OCT && (i % WB_OCT) == 0 && i < (n + WB_CHUNK - 1) / WB_CHUNK * WB_CHUNK) {
+      // the octet's box, relative to the root's centre
+      const double side = f.cell * (double)(1 << WB_MAX_LEVEL), h = side / 2;
+      oct_xy[i / WB_OCT] =
+          make_float4(wb::rel_down(x0, f.lox + h, side), wb::rel_up(x1, f.lox + h, side),
+                      wb::rel_down(y0, f.loy + h, side), wb::rel_up(y1, f.loy + h, side));
+      oct_z[i / WB_OCT] = wb::rel_down(z0, f.loz + h, side);
+    }
   }
   const uint64_t chunk = i / WB_CHUNK;
   if ((i % WB_CHUNK) == 0 && chunk < (n + WB_CHUNK - 1) / WB_CHUNK) {
@@ -1199,9 +1211,10 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
   wb_free(c, lt, sizeof(LeafTmp) * leaf_cap);
 
   t->pt_leaf = wb_talloc<uint32_t>(t, n);
-  t->px = wb_talloc<double>(t, n);
-  t->py = wb_talloc<double>(t, n);
-  t->pz = wb_talloc<double>(t, n);
+  // (whole groups: the ground test reads the last one past its end)
+  t->px = wb_talloc<double>(t, n + WB_CHUNK);
+  t->py = wb_talloc<double>(t, n + WB_CHUNK);
+  t->pz = wb_talloc<double>(t, n + WB_CHUNK);
   t->canon = wb_talloc<uint32_t>(t, n);
   t->crank = wb_talloc<uint32_t>(t, n);
   uint64_t nchunks = (n + WB_CHUNK - 1) / WB_CHUNK;
@@ -1210,17 +1223,19 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
   t->chunk_sx = wb_talloc<double>(t, nchunks + 1);
   t->chunk_sy = wb_talloc<double>(t, nchunks + 1);
   t->chunk_sz = wb_talloc<double>(t, nchunks + 1);
+  t->oct_xy = wb_talloc<float4>(t, (WB_CHUNK / WB_OCT) * nchunks + 1);
+  t->oct_z = wb_talloc<float>(t, (WB_CHUNK / WB_OCT) * nchunks + 1);
   if (n > 0) {
     hipLaunchKernelGGL(k_fill_pt_leaf, dim3(nl), dim3(256), 0, c->stream, t->leaf_start, nl,
                        t->pt_leaf);
     if (f64)
       hipLaunchKernelGGL(k_permute<true>, dim3(wb_blocks(nchunks * WB_CHUNK, 256)), dim3(256), 0,
                          c->stream, src, t->sidx, n, f, t->px, t->py, t->pz, t->chunk_box,
-                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz);
+                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz, t->oct_xy, t->oct_z);
     else
       hipLaunchKernelGGL(k_permute<false>, dim3(wb_blocks(nchunks * WB_CHUNK, 256)), dim3(256), 0,
                          c->stream, src, t->sidx, n, f, t->px, t->py, t->pz, t->chunk_box,
-                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz);
+                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz, t->oct_xy, t->oct_z);
     wb_free(c, src.packed, pk_bytes);
     src.packed = nullptr;
     {
@@ -1241,8 +1256,9 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
       double *leaf_zlow = (double *)wb_alloc(c, 8 * (size_t)nl);
       double *node_zlow = (double *)wb_alloc(c, 8 * (size_t)t->nnodes);
       t->child_zlow = wb_talloc<double>(t, 8 * (size_t)t->nnodes);
+      t->leaf_low = wb_talloc<float>(t, nl);
       hipLaunchKernelGGL(k_leaf_zlow, dim3(wb_blocks(nl, 4)), dim3(256), 0, c->stream,
-                         t->leaf_start, nl, t->pz, leaf_zlow);
+                         t->leaf_start, nl, t->pz, leaf_zlow, t->leaf_low);
       for (int d = t->maxdepth - 1; d >= 0; d--)
         hipLaunchKernelGGL(k_node_zlow, dim3(wb_blocks(t->nnodes, 256)), dim3(256), 0, c->stream,
                            t->node_child, t->node_cube, t->nnodes, d, leaf_zlow, node_zlow,

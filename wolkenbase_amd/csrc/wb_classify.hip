@@ -39,7 +39,7 @@
 #define WAVE 64
 // waves per SIMD the ground-test kernel is compiled for
 #ifndef WB_GROUND_MINW
-#define WB_GROUND_MINW 6
+#define WB_GROUND_MINW 5
 #endif
 constexpr double kSqrt34 = 0.86602540378443864676372317;  // eisenstein.h:33
 constexpr double kSqrt7 = 2.6457513110645905905016;       // scan.h:23
@@ -76,6 +76,9 @@ struct TreeView {
   const double *chunk_box;
   const uint32_t *chunk_low;
   const double *chunk_sx, *chunk_sy, *chunk_sz;
+  const float4 *oct_xy;
+  const float *oct_z, *leaf_low;
+  double ox, oy, oz, side;  // the root cube
   const uint2 *node_crange;
   const double *child_zlow;
   const uint32_t *pt_leaf, *canon, *crank, *sidx;
@@ -90,6 +93,8 @@ static TreeView view(const wb_tree *t)
   v.leaf_start = t->leaf_start; v.leaf_cube = t->leaf_cube; v.leaf_parent = t->leaf_parent;
   v.node_cube = t->node_cube; v.node_child = t->node_child; v.node_parent = t->node_parent;
   v.chunk_box = t->chunk_box; v.chunk_low = t->chunk_low;
+  v.oct_xy = t->oct_xy; v.oct_z = t->oct_z; v.leaf_low = t->leaf_low;
+  v.ox = t->center[0]; v.oy = t->center[1]; v.oz = t->center[2]; v.side = t->side;
   v.chunk_sx = t->chunk_sx; v.chunk_sy = t->chunk_sy; v.chunk_sz = t->chunk_sz; v.node_crange = t->node_crange;
   v.child_zlow = t->child_zlow;
   v.pt_leaf = t->pt_leaf; v.canon = t->canon; v.crank = t->crank;
@@ -1731,9 +1736,24 @@ struct ClassifyArgs {
   uint8_t *cls_in;       // per input index (the caller's class bytes)
   uint32_t *nslow;       // points decided by the exact gap pass
   HeavyRec *heavy;       // points handed to the wave-per-point kernel
-  uint32_t *nheavy;
+  uint32_t *nheavy, *heavy_next;
   unsigned long long *atan_exact;
-  unsigned long long *counters;  // 16 work counters (only with the counting kernel)
+  // What walk A leaves to walk B: per wave with open lanes units of up to
+  // open_per of them: the place in pool (and upper 16 bits of y) and length
+  // of its leaf list, its records and the first one.  Records lie at the
+  // wave's own place; a list of up to OPEN_LIST leaves does too, a longer one
+  // past pool_shared (npool: entries taken).
+  // open_classes: the units of class k lie from unit_cap * k on (nopen: of
+  // each class; open_next: units the resident kernel has taken); else unit w is wave w's, with no
+  // records when it left no lane open.
+  HeavyRec *open;
+  uint4 *open_unit;
+  uint32_t *pool;
+  uint64_t pool_shared, pool_cap;
+  uint32_t unit_cap, open_per;
+  int open_classes;
+  uint32_t *nopen, *open_next;
+  unsigned long long *npool;
   // work items in place of the points (nullptr: work index k is sorted slot
   // k with the hyperboloid size of its deciding tile): item k is (slot,
   // tile record index), and its verdict goes to item_cls[k] only
@@ -1772,45 +1792,6 @@ __device__ inline void work_verdict(const ClassifyArgs &A, uint64_t k, uint32_t 
 }
 
 __device__ inline uint64_t rotr64(uint64_t x, int a) { return (x >> a) | (x << (64 - a)); }
-
-// Per-lane care wedges of k_ground: the wedges of wb::care_wedges for each
-// lane, at most two, kept in LDS; a lane with more than two wedges (two runs,
-// one of them 32 bins or more) is not pruned (n < 0).
-struct LaneWedges {
-  float ax[2][256], ay[2][256], bx[2][256], by[2][256];
-  int n[256];
-};
-
-__device__ inline void lane_wedges_update(uint64_t occ, const float *edges, LaneWedges &W, int t)
-{
-  wb::Wedges w;
-  wb::care_wedges(occ, w, edges);
-  // live is 1, 3 (one run, split) or 5 (two runs) when at most two are in use;
-  // the second kept wedge is slot 1 or slot 2
-  const int n = w.live < 0 ? -1 : __builtin_popcount(w.live);
-  if (n >= 0 && n <= 2) {
-    const bool s1 = (w.live & 2) != 0;
-    W.ax[0][t] = w.ax[0]; W.ay[0][t] = w.ay[0];
-    W.bx[0][t] = w.bx[0]; W.by[0][t] = w.by[0];
-    W.ax[1][t] = s1 ? w.ax[1] : w.ax[2]; W.ay[1][t] = s1 ? w.ay[1] : w.ay[2];
-    W.bx[1][t] = s1 ? w.bx[1] : w.bx[2]; W.by[1][t] = s1 ? w.by[1] : w.by[2];
-    W.n[t] = n;
-  } else {
-    W.n[t] = -1;
-  }
-}
-
-// wb::wedge_hit against thread t's wedges (at most two)
-__device__ inline bool lane_hit(const LaneWedges &W, int t, double px, double py, double x0,
-                                double x1, double y0, double y1)
-{
-  const int n = W.n[t];
-  if (n < 0) return true;
-  const float ax[2] = {W.ax[0][t], W.ax[1][t]}, ay[2] = {W.ay[0][t], W.ay[1][t]};
-  const float bx[2] = {W.bx[0][t], W.bx[1][t]}, by[2] = {W.by[0][t], W.by[1][t]};
-  return wb::wedge_hit2(n, ax, ay, bx, by, (float)(x0 - px), (float)(x1 - px), (float)(y0 - py),
-                        (float)(y1 - py));
-}
 
 // classification of the empty-bin mask: 1 pass, 2 fail, 0 undecided
 __device__ inline int gap_verdict(uint64_t occupied)
@@ -1888,175 +1869,209 @@ __device__ inline void half_or(uint64_t v, uint64_t &h0, uint64_t &h1)
 // on a subset of D is a pass on D, and a fail or an exact gap needs all of D.
 // ---------------------------------------------------------------------------
 // Entries pending at one time: at most 7 siblings per level on the path
-// (internal nodes sit at levels 0..WB_MAX_LEVEL) plus 8 children.
+// (internal nodes sit at levels 0..WB_MAX_LEVEL) plus 8 children.  All
+// entries of one level are children of one node (a node is expanded when it
+// is popped, and its children are taken before its siblings), so the lanes
+// that reach them are kept per level.
 #define WB_STK (7 * (WB_MAX_LEVEL + 1) + 8 + 2)
+// leaves walk A takes before it hands its open lanes to k_ground_heavy,
+// or, of all entries it takes from its stack
+#define GROUND_LEAVES 256
+#define GROUND_STEPS 1024
 struct WaveStack {
-  int code[WB_STK];
-  uint32_t lo[WB_STK], hi[WB_STK];
-  uint32_t b[WB_STK], e[WB_STK];  // slot range of a leaf entry
+  // x: node or leaf code; y: level, and the point count of a leaf << 8; z: a
+  // leaf's first slot; w: (float) at most the lowest z stored under the entry
+  uint4 ent[WB_STK];
+  uint2 mask[WB_MAX_LEVEL + 2];  // lanes whose walk reached the parent
+  uint32_t leaf[GROUND_LEAVES];  // the leaves walk A took, in its order
 };
 
-// rank of child k in the visiting order for quadrant o and lower-first flag
-__device__ inline int child_rank(int k, int o, int zf) { return ((k ^ o) & 3) | ((k ^ zf) & 4); }
-
-// Pushes the children of internal node `code` that intersect the
-// hyperboloid of a lane in `m` (this lane takes part iff `on`), in reverse
-// visiting order.  Returns the new stack depth.
-// Each child's test is wb::hyp_intersect on the child cube of Octree::cube
-// (wb::hyp_intersect_low with the lowest point stored under the child when
-// every point lies in its leaf's cube) and the lane's care wedges on the
-// child's xy square, with the shared parts computed once: the clamped
-// coordinate of the closest point takes one of two values per axis (x from
-// bit 0 of the child index, y from bit 1, z from bit 2) and the two children
-// of one xy square (bit 2 differs) share the wedge test.  Every value is the
-// same double operation on the same operands as in the per-child form.
-__device__ inline int expand_node(const TreeView &T, WaveStack &S, int sp, int code, bool on,
-                                  const wb::Shape &H, double rx, double ry, int zf,
-                                  const LaneWedges &LW, bool cube_wedges)
+// A value every lane of the wave reads from the same address, fetched by the
+// scalar unit into scalar registers (i wave-uniform; nothing writes the
+// tree's arrays while a ground kernel runs).
+__device__ inline double uload(const double *p, size_t i)
 {
-  const double *nc = T.node_cube + 4 * (size_t)code;
-  const double cx = nc[0], cy = nc[1], cz = nc[2], side = nc[3];
-  const int *chp = T.node_child + 8 * (size_t)code;
-  const int o = rfl((rx >= cx ? 1 : 0) | (ry >= cy ? 2 : 0));
-  int ck[8];
-  uint32_t pushed = 0;  // bit t: the child of rank t is pushed
-  uint64_t mk[8];       // lanes for which child k is pushed
-#pragma unroll
-  for (int k = 0; k < 8; k++) ck[k] = rfl(chp[k]);
-  // lane k < 8 holds child k's slot range (leaf children), pushed with it
-  const uint2 cr = __lane_id() < 8 ? T.node_crange[8 * (size_t)code + __lane_id()]
-                                   : make_uint2(0u, 0u);
-  // lane k < 8 holds the lowest z under child k
-  const double zl = cube_wedges && __lane_id() < 8 ? T.child_zlow[8 * (size_t)code + __lane_id()]
-                                                   : -__builtin_inf();
-  // Octree::cube (octree.cpp:349-358) per axis bit, and the closest point of
-  // wb::hyp_intersect: clamp_axis on x and y, the bottom (top for a negative
-  // slope) face on z
-  const double cs = side / 2;
-  double ncx[2], ncy[2], qx[2], qy[2], qz[2];
-#pragma unroll
-  for (int b = 0; b < 2; b++) {
-    ncx[b] = cx + (double)(2 * b - 1) * side / 4;
-    ncy[b] = cy + (double)(2 * b - 1) * side / 4;
-    const double ncz = cz + (double)(2 * b - 1) * side / 4;
-    qx[b] = wb::clamp_axis(H.cx, ncx[b], cs);
-    qy[b] = wb::clamp_axis(H.cy, ncy[b], cs);
-    qz[b] = ncz;
-    if (H.slope > 0) qz[b] -= cs / 2;
-    if (H.slope < 0) qz[b] += cs / 2;
-  }
-  // the lane's wedges (at most two), read from LDS once; one test per xy
-  // square, on the three x and three y edges of the four squares as offsets
-  // from the point (the middle edge ncx[0] + side/4 = ncx[1] - side/4: cube
-  // centres and sides are exact dyadics)
-  bool wq[4] = {true, true, true, true};
-  const int nw = cube_wedges ? LW.n[threadIdx.x] : -1;
-  if (nw >= 0) {
-    const int t = threadIdx.x;
-    const float ax[2] = {LW.ax[0][t], LW.ax[1][t]}, ay[2] = {LW.ay[0][t], LW.ay[1][t]};
-    const float bx[2] = {LW.bx[0][t], LW.bx[1][t]}, by[2] = {LW.by[0][t], LW.by[1][t]};
-    const float ux[3] = {(float)((ncx[0] - side / 4) - H.cx), (float)((ncx[0] + side / 4) - H.cx),
-                         (float)((ncx[1] + side / 4) - H.cx)};
-    const float vy[3] = {(float)((ncy[0] - side / 4) - H.cy), (float)((ncy[0] + side / 4) - H.cy),
-                         (float)((ncy[1] + side / 4) - H.cy)};
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-      if ((ck[q] != -1) | (ck[q + 4] != -1))
-        wq[q] = wb::wedge_hit2(nw, ax, ay, bx, by, ux[q & 1], ux[(q & 1) + 1], vy[q >> 1],
-                               vy[(q >> 1) + 1]);
-  }
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    mk[k] = 0;
-    if (ck[k] != -1) {
-      const double zlk = rdl(zl, k);
-      const double qzk = H.slope > 0 && zlk > qz[k >> 2] ? zlk : qz[k >> 2];
-      const bool h = on & wq[k & 3] & wb::hyp_in(H, qx[k & 1], qy[(k >> 1) & 1], qzk);
-      mk[k] = __ballot(h);
-      if (mk[k]) pushed |= 1u << child_rank(k, o, zf);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    if (mk[k]) {
-      const int pos = sp + __popc(pushed >> (child_rank(k, o, zf) + 1));
-      S.code[pos] = ck[k];
-      S.lo[pos] = (uint32_t)mk[k];
-      S.hi[pos] = (uint32_t)(mk[k] >> 32);
-      S.b[pos] = (uint32_t)__builtin_amdgcn_readlane((int)cr.x, k);
-      S.e[pos] = (uint32_t)__builtin_amdgcn_readlane((int)cr.y, k);
-    }
-  }
-  return sp + __popc(pushed);
+  return ((const __attribute__((address_space(4))) double *)p)[i];
 }
 
-// per-wave work counters of the instrumented kernel
-enum {
-  CT_LANES_A, CT_LANES_B, CT_LANES_C, CT_LEAF_A, CT_GROUP_A, CT_DIR_A, CT_LEAF_B, CT_POINT_B,
-  CT_DIR_B, CT_EXP_A, CT_WLEAF_A, CT_EXP_B, CT_WLEAF_B, CT_HEAVY, CT_WAVES,
-  CT_TSUM, CT_TMAX, CT_THIST, CT_TSUMS = CT_THIST + 5,
-  // shader cycles per wave in: walk A expansions, walk A leaves, walk B
-  // expansions, walk B leaves, wedge refreshes; wave-level sample and slot
-  // iterations of walks A and B
-  CT_CYC = CT_TSUMS + 5, CT_ITER_A = CT_CYC + 8, CT_ITER_B, CT_N,
-  // the counting kernels add into 64 copies (block index mod 64) so their
-  // own atomics do not slow the memory system they measure
-  CT_STRIDE = CT_N + 24, CT_COPIES = 64
+// A lane's hyperboloid as hyp_near reads it
+struct Near {
+  double x, y, cz, por2, thr;  // thr = por2 * wb::kNearShrink
 };
 
-// a lane whose sampled pass enters leaves with more than HEAVY_B_GROUPS
-// 32-point groups, or whose sampled pass alone passes HEAVY_A_GROUPS, is
-// finished by k_ground_heavy
-#ifndef HEAVY_A_GROUPS
-#define HEAVY_A_GROUPS 2048u
+__device__ inline double near_t(const Near &P, double s2, double qx, double qy, double qz)
+{
+  return wb::hyp_near(s2, qx - P.x, qy - P.y, P.cz - qz);
+}
+
+// What holds every hyperboloid of the wave's open lanes: the box of their
+// axes, the highest centre and the lowest threshold (wave-uniform).  A box
+// that fails union_hits meets none of them: its distance from the axes' box
+// is at most its distance from any lane's axis (each difference rounds
+// monotonically), so near_t's bound holds for the union too.
+struct Union {
+  double x0, x1, y0, y1, cz, thr;
+};
+
+__device__ inline Union wave_union(const Near &P, bool open)
+{
+  const double inf = __builtin_inf();
+  Union U;
+  U.x0 = wave_dmin(open ? P.x : inf);
+  U.x1 = wave_dmax(open ? P.x : -inf);
+  U.y0 = wave_dmin(open ? P.y : inf);
+  U.y1 = wave_dmax(open ? P.y : -inf);
+  U.cz = wave_dmax(open ? P.cz : -inf);
+  U.thr = wave_dmin(open ? P.thr : inf);
+  return U;
+}
+
+__device__ inline bool union_hits(const Union &U, double s2, double x0, double x1, double y0,
+                                  double y1, double z0)
+{
+  const double dx = fmax(fmax(x0 - U.x1, U.x0 - x1), 0.0);
+  const double dy = fmax(fmax(y0 - U.y1, U.y0 - y1), 0.0);
+  const double dz = U.cz - z0;
+  return wb::hyp_near(s2, dx, dy, dz) >= U.thr;
+}
+
+// bit k of the result is bit k ^ r of the 8-bit mask m (r < 8)
+__device__ inline uint32_t xor_bits8(uint32_t m, int r)
+{
+  if (r & 1) m = ((m & 0x55) << 1) | ((m >> 1) & 0x55);
+  if (r & 2) m = ((m & 0x33) << 2) | ((m >> 2) & 0x33);
+  if (r & 4) m = ((m & 0x0f) << 4) | (m >> 4);
+  return m;
+}
+
+// visiting order: child k has rank k ^ o (o: the xy quadrant taken first;
+// for a downward hyperboloid the lower half, bit 2 clear, comes first)
+__device__ inline int child_rank(int k, int o, int zf) { return ((k ^ o) & 3) | ((k ^ zf) & 4); }
+
+// Pushes the children of node `code` (cube cx, cy, cz, side at level lvl)
+// that may meet the hyperboloid of an open lane, in reverse visiting order:
+// lane k < 8 tests child k (its cube by Octree::cube, octree.cpp:349-358,
+// the operations of the build; its bottom face raised to the lowest point
+// stored under it when every point lies in its leaf's cube) against the
+// wave's union.  The lanes' own tests follow when a child is popped.
+// Returns the new stack depth.
+template <bool IN>
+__device__ inline int push_children(const TreeView &T, WaveStack &S, int sp, int code, int lvl,
+                                    double cx, double cy, double cz, double side, uint64_t mk,
+                                    const Union &U, double s2, double rx, double ry)
+{
+  const uint32_t lane = __lane_id();
+  const int o = rfl((rx >= cx ? 1 : 0) | (ry >= cy ? 2 : 0));
+  int ck = -1;
+  uint2 cr = make_uint2(0u, 0u);
+  double zl = -__builtin_inf();
+  if (lane < 8) {
+    const size_t at = 8 * (size_t)code + lane;
+    ck = T.node_child[at];
+    cr = T.node_crange[at];
+    if (IN) zl = T.child_zlow[at];
+  }
+  const double h = side / 4;
+  const double x = cx + ((lane & 1) ? h : -h), y = cy + ((lane & 2) ? h : -h);
+  const double z = cz + ((lane & 4) ? h : -h);
+  const bool hit = ck != -1 && union_hits(U, s2, x - h, x + h, y - h, y + h, fmax(z - h, zl));
+  const uint32_t pm = (uint32_t)__ballot(hit);
+  if (hit) {
+    const uint32_t above = xor_bits8(pm, o) >> (((int)lane ^ o) + 1);  // taken after this one
+    S.ent[sp + __popc(above)] =
+        make_uint4((uint32_t)ck, (uint32_t)(lvl + 1) | ((cr.y - cr.x) << 8), cr.x,
+                   __float_as_uint((float)(zl - __builtin_fabs(zl) * 0x1p-22)));
+  }
+  S.mask[lvl + 1] = make_uint2((uint32_t)mk, (uint32_t)(mk >> 32));
+  return sp + __popc(pm);
+}
+
+// classes of walk B's units by the length of their leaf lists
+#define OPEN_CLASSES 4
+// leaf list entries kept at a wave's own place
+#define OPEN_LIST 64
+#ifndef OPEN_P1
+#define OPEN_P1 16
 #endif
+#ifndef OPEN_P2
+#define OPEN_P2 32
+#endif
+// candidates of one 32-point group from which on a lane's care wedges are
+// taken anew before the next group
+#ifndef OPEN_REFRESH
+#define OPEN_REFRESH 4
+#endif
+// lanes that need a 32-point group up to which it is tested two lanes at a
+// time, half a wave of slots each
+#ifndef OPEN_PAIR
+#define OPEN_PAIR 12
+#endif
+// a lane whose walk A entered leaves with more groups than this is finished
+// by k_ground_heavy, a wave to the point
+#define HEAVY_B_GROUPS 1024u
 // blocks of the heavy kernel at most: 4 waves on each SIMD of 256 CUs
 #define HEAVY_GRID 4096u
-#ifndef HEAVY_B_GROUPS
-#define HEAVY_B_GROUPS 1024u
-#endif
 
-// The ground test of classify.cpp:128-165 for one point per lane, in two
-// walks over the octree:
-//   A  the lowest point of each 32-point group of every leaf (a subset of D;
-//      only a pass is decided here),
-//   B  every point, for lanes A left open.
-// Lanes whose walks would be long, and lanes whose directions leave a
-// longest empty run of 24 or 25 bins (decided by the exact directions in
-// the two bins bordering the run), go to k_ground_heavy with the directions
-// found so far.
-// The hyperboloid is Hyperboloid(p - (0,0,thickness), hs, slope)
-// (shape.cpp:119-125) with its axis at x, y instead of x + 0, y + 0: the
-// two differ only in the sign of a zero, which no test below can see (every
-// use is a difference that is squared, compared or passed to hypot).
-// unit: the index of the wave's 64 work items (items 64*unit ..); stacks,
-// LW, edges: the block's shared arrays (edges: the bin-edge table, read by
-// wedge refreshes, loaded by ground_setup).  No barrier: the waves of a
-// block run their units independently.
+// the lanes' hyperboloids: Hyperboloid(p - (0,0,thickness), hs, slope)
+// (shape.cpp:119-125) with its axis at x, y instead of x + 0, y + 0: the two
+// differ only in the sign of a zero, which no test can see (every use is a
+// difference that is squared, compared or passed to hypot)
+__device__ inline Near make_near(const ClassifyArgs &A, double x, double y, double z, double hs)
+{
+  const double sl = A.max_slope, por = hs * (sl * sl);
+  Near P;
+  P.x = x;
+  P.y = y;
+  P.cz = (z - A.thickness) + por;
+  P.por2 = por * por;
+  P.thr = P.por2 * wb::kNearShrink;
+  return P;
+}
+
+// A point this far inside (near_t less 2^-39 of a reaches por2 + sure_slack)
+// is in, and findBlocks reaches its leaf, whatever the roundings: a cube that
+// holds the point lies no farther from the axis than the point but for the
+// rounding of clamp_axis's difference (2^-53 of the root's side), and 2^-39
+// of a covers those of the products.
+__device__ inline double sure_slack(const ClassifyArgs &A)
+{
+  const double d = A.max_slope * (A.T.side * 0x1p-52);
+  return 2 * d * d;
+}
+
 __device__ __forceinline__ void ground_setup(const ClassifyArgs &A, float *edges)
 {
   for (int k = threadIdx.x; k < 3 * 128; k += blockDim.x) edges[k] = A.edges[k];
   __syncthreads();
 }
 
-template <bool COUNT>
-__device__ __forceinline__ void ground_body(const ClassifyArgs &A, uint64_t unit,
-                                            WaveStack *stacks, LaneWedges &LW, const float *edges)
+// Walk A for 64 points, one per lane: the lowest point of each 32-point group
+// of every leaf findBlocks returns (a subset of D, so only a pass is decided
+// here).  The lanes left open go to walk B (k_ground_open) in units of
+// at most 64 with the directions found and the list of the leaves taken here,
+// which holds every leaf B needs: what A left out by a hyperboloid or by care
+// wedges (which only shrink) no open lane needs.  A wave that fills its list
+// and a lane with many groups go to k_ground_heavy.
+//
+// What bounds it: VALU issue (the tests of boxes and samples), and the wait
+// for a popped cube.  So a node's children are tested by eight lanes at once
+// against the wave's union instead of by every lane in turn, the lanes' own
+// test of a cube is the eight-operation near_t, and walk B, whose work per
+// point varies most, is a kernel of its own.
+// IN: every point lies in its leaf's cube (the build flags the other case),
+// so the care wedges may skip a node or leaf by its cube and a cube's bottom
+// face may be raised to the lowest point stored under it.
+template <bool IN>
+__device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, WaveStack &S,
+                                          const float *edges)
 {
-  WaveStack &S = stacks[threadIdx.x / WAVE];
-  LW.n[threadIdx.x] = -1;
-  const uint32_t blk = (uint32_t)unit;  // spreads the instrumented counters
   const TreeView &T = A.T;
   const uint32_t lane = __lane_id();
   // work index: a sorted slot, or a work item
   const uint64_t i = unit * WAVE + lane;
   const bool inrange = i < (A.items ? A.n_items : T.n);
-  const double *ttan = A.tab, *tcos = A.tab + 511, *tsin = A.tab + 1023;
-  const uint64_t t_start = COUNT ? wall_clock64() : 0;
-  uint32_t cnt[CT_WAVES] = {};
-  uint64_t cyc[8] = {}, iter_a = 0, iter_b = 0;
-  // lane state: 0 undecided, 1 not ground, 2 ground, 3 no tile; handed to
-  // k_ground_heavy: 5 walk A cut short, 6 after walk A, 7 after walk B
+  // lane state: 0 undecided, 1 not ground, 3 no tile; handed on: 5 to the
+  // heavy kernel, walk A cut short
   int state = 3;
   double x = 0, y = 0, z = 0, hs = 0;
   uint32_t slot = 0;
@@ -2064,307 +2079,589 @@ __device__ __forceinline__ void ground_body(const ClassifyArgs &A, uint64_t unit
     x = T.px[slot]; y = T.py[slot]; z = T.pz[slot];
     state = 0;
   }
-  wb::Shape H;
-  {
-    const double sl = A.max_slope, por = hs * (sl * sl);
-    H.kind = wb::SHAPE_HYPERBOLOID;
-    H.cx = x;
-    H.cy = y;
-    H.cz = (z - A.thickness) + por;
-    H.r = 0;
-    H.por2 = por * por;
-    H.slope = sl;
-  }
-  const int zf = A.max_slope > 0 ? 0 : 4;
+  const double sl = A.max_slope, s2 = (sl * sl) * wb::kNearShrink;
+  const Near P = make_near(A, x, y, z, hs);
+  // a subset of D will do here, so a sample that rounding might put either
+  // side of the surface, or of a bin's edge, is left to walk B
+  const double sure = P.por2 + sure_slack(A);
+  wb::LaneWedges W;
+  W.n = -1;
   uint64_t occ = 0, checked = 0;
-  int nexact = 0;
-  uint32_t groups_a = 0;
-  for (int phase = 0; phase < 2; phase++) {
-    if (phase == 1 && state == 0 && groups_a > HEAVY_B_GROUPS) state = 6;
-    const bool act = state == 0;
-    uint64_t alive = __ballot(act);
-    if (alive == 0) break;
-    if (COUNT && act) {
-      if (phase == 0) cnt[CT_LANES_A]++;
-      else cnt[CT_LANES_B]++;
-    }
+  uint32_t groups_a = 0, nleaf = 0;
+  uint64_t alive = __ballot(state == 0);
+  if (alive) {
+    Union U = wave_union(P, state == 0);
+    int ualive = __popcll(alive);
     // the wave's first point orders the children
     const int ld = __ffsll((long long)alive) - 1;
-    const double rx = __shfl(x, ld, 64), ry = __shfl(y, ld, 64);
-    int sp = 0;
-    {
-      const double *rc = T.node_cube;
-      const uint64_t m = __ballot(act && wb::hyp_intersect(H, rc[0], rc[1], rc[2], rc[3]));
-      if (m) {
-        S.code[0] = 0;
-        S.lo[0] = (uint32_t)m;
-        S.hi[0] = (uint32_t)(m >> 32);
-        sp = 1;
+    const double rx = rdl(x, ld), ry = rdl(y, ld);
+    int sp = 1;
+    S.ent[0] = make_uint4(0u, 0u, 0u, __float_as_uint(-__builtin_inff()));
+    S.mask[0] = make_uint2((uint32_t)alive, (uint32_t)(alive >> 32));
+    for (uint32_t steps = 0; sp > 0; steps++) {
+      if (steps == GROUND_STEPS) {
+        if (state == 0) state = 5;
+        break;
       }
-    }
-    while (sp > 0) {
-      sp--;
-      const int code = rfl(S.code[sp]);
-      const uint64_t m = (((uint64_t)(uint32_t)rfl((int)S.hi[sp]) << 32) |
-                          (uint32_t)rfl((int)S.lo[sp])) & alive;
+      const uint4 en = S.ent[--sp];
+      const int code = rfl((int)en.x), lvl = rfl((int)(en.y & 255u));
+      const uint2 mw = S.mask[lvl];
+      uint64_t m = (((uint64_t)(uint32_t)rfl((int)mw.y) << 32) | (uint32_t)rfl((int)mw.x)) & alive;
       if (m == 0) continue;
-      const bool on = (m >> lane) & 1;
-      const uint64_t c0t = COUNT ? clock64() : 0;
+      const double *cb = code >= 0 ? T.node_cube + 4 * (size_t)code
+                                   : T.leaf_cube + 4 * (size_t)(-2 - code);
+      const double cx = uload(cb, 0), cy = uload(cb, 1), cz = uload(cb, 2), side = uload(cb, 3);
+      // the lanes' own tests: whether the cube, its bottom face raised, may
+      // meet the lane's hyperboloid and care wedges
+      bool on = (m >> lane) & 1;
+      const bool anyw = IN && __ballot(on && W.n >= 0) != 0;
+      const double hh = side / 2, x0 = cx - hh, x1 = cx + hh, y0 = cy - hh, y1 = cy + hh;
+      if (!IN) {
+        // a point may lie outside its leaf's cube, so reaching the leaf does
+        // not follow from the point: findBlocks' own test, cube by cube
+        wb::Shape H = wb::make_cylinder(x, y, 0);
+        H.kind = wb::SHAPE_HYPERBOLOID;
+        H.cz = P.cz;
+        H.por2 = P.por2;
+        H.slope = sl;
+        on = on && wb::hyp_intersect(H, cx, cy, cz, side);
+        m = __ballot(on);
+      } else if (code < 0 || anyw) {
+        const double zb = fmax(cz - hh, (double)__uint_as_float((uint32_t)rfl((int)en.w)));
+        on = on && near_t(P, s2, fmin(fmax(x, x0), x1), fmin(fmax(y, y0), y1), zb) >= P.thr;
+        if (anyw) on = on && wb::lane_hit(W, x, y, x0, x1, y0, y1);
+        m = __ballot(on);
+      }
+      if (m == 0) continue;
       if (code >= 0) {
-        if (COUNT) {
-          if (phase == 0) cnt[CT_EXP_A]++;
-          else cnt[CT_EXP_B]++;
-        }
-        sp = expand_node(T, S, sp, code, on, H, rx, ry, zf, LW, A.cube_wedges != 0);
-        if (COUNT) cyc[phase == 0 ? 0 : 2] += clock64() - c0t;
+        sp = push_children<IN>(T, S, sp, code, lvl, cx, cy, cz, side, m, U, s2, rx, ry);
         continue;
       }
-      const int leaf = -2 - code;
-      const uint32_t b = (uint32_t)rfl((int)S.b[sp]);
-      const uint32_t e = (uint32_t)rfl((int)S.e[sp]);
-      // the lane skips a leaf outside its care wedges
-      const double *lc = T.leaf_cube + 4 * (size_t)leaf;
-      const double lh = lc[3] / 2;
-      const bool onl = on && (!A.cube_wedges || lane_hit(LW, threadIdx.x, x, y, lc[0] - lh,
-                                                         lc[0] + lh, lc[1] - lh, lc[1] + lh));
-      uint64_t c2t = 0;
-      if (COUNT && phase == 0) {
-        __builtin_amdgcn_s_waitcnt(0);
-        c2t = clock64();
-        cyc[5] += c2t - c0t;
+      if (nleaf == GROUND_LEAVES) {
+        if (state == 0) state = 5;
+        break;
       }
-      if (phase == 0) {
-        if (COUNT) {
-          cnt[CT_WLEAF_A]++;
-          if (onl) cnt[CT_LEAF_A]++;
-        }
-        const uint32_t g0 = b / WB_CHUNK, ng = (e - 1) / WB_CHUNK - g0 + 1;
-        if (onl) groups_a += ng;
-        if (COUNT && onl) cnt[CT_GROUP_A] += ng;
-        // the lowest point of each group (the likeliest to lie in a downward
-        // hyperboloid), or the group's first slot in the leaf when the
-        // lowest one belongs to the neighbouring leaf; lane g fetches the
-        // sample of group g, then every lane tests every sample
-        for (uint32_t gb = 0; gb < ng; gb += WAVE) {
-          const uint32_t g = gb + lane;
-          double sx = 0, sy = 0, sz = 0;
-          if (g < ng) {
-            // the group's lowest point from the per-group copy (consecutive
-            // lanes, consecutive words); a group that starts or ends in
-            // another leaf takes its first slot in this leaf instead
-            const uint32_t j = T.chunk_low[g0 + g];
-            if (j < b || j >= e) {
-              const uint32_t jf = g == 0 ? b : (g0 + g) * WB_CHUNK;
-              sx = T.px[jf]; sy = T.py[jf]; sz = T.pz[jf];
-            } else {
-              sx = T.chunk_sx[g0 + g]; sy = T.chunk_sy[g0 + g]; sz = T.chunk_sz[g0 + g];
-            }
-          }
-          if (COUNT) {
-            __builtin_amdgcn_s_waitcnt(0);
-            const uint64_t c3t = clock64();
-            cyc[6] += c3t - c2t;
-            c2t = c3t;
-          }
-          const uint32_t ns = min((uint32_t)WAVE, ng - gb);
-          if (COUNT && __ballot(onl)) iter_a += ns;
-          for (uint32_t s = 0; s < ns; s++) {
-            const double qx = rdl(sx, s), qy = rdl(sy, s), qz = rdl(sz, s);
-            if (onl & wb::hyp_in(H, qx, qy, qz) & ((qx != x) | (qy != y))) {
-              if (COUNT) cnt[CT_DIR_A]++;
-              occ |= 1ull << wb::dir_bin(qy - y, qx - x, ttan, tcos, tsin, A.K, &nexact);
-            }
-          }
-          if (COUNT) {
-            const uint64_t c3t = clock64();
-            cyc[7] += c3t - c2t;
-            c2t = c3t;
+      const uint32_t b = (uint32_t)rfl((int)en.z), e = b + ((uint32_t)rfl((int)en.y) >> 8);
+      S.leaf[nleaf++] = (uint32_t)(-2 - code);
+      // the lowest point of each group (the likeliest to lie in a downward
+      // hyperboloid), or the group's first slot in the leaf when the lowest
+      // one belongs to the neighbouring leaf: lane g fetches the sample of
+      // group g and tests it against the wave's union, and the samples that
+      // pass are tested by every lane
+      const uint32_t g0 = b / WB_CHUNK, ng = (e - 1) / WB_CHUNK - g0 + 1;
+      if (on) groups_a += ng;
+      for (uint32_t gb = 0; gb < ng; gb += WAVE) {
+        const uint32_t g = gb + lane;
+        double sx = 0, sy = 0, sz = 0;
+        if (g < ng) {
+          // the group's lowest point from the per-group copy (consecutive
+          // lanes, consecutive words)
+          const uint32_t j = T.chunk_low[g0 + g];
+          if (j < b || j >= e) {
+            const uint32_t jf = g == 0 ? b : (g0 + g) * WB_CHUNK;
+            sx = T.px[jf]; sy = T.py[jf]; sz = T.pz[jf];
+          } else {
+            sx = T.chunk_sx[g0 + g]; sy = T.chunk_sy[g0 + g]; sz = T.chunk_sz[g0 + g];
           }
         }
-      } else {
-        if (COUNT) {
-          cnt[CT_WLEAF_B]++;
-          if (onl) cnt[CT_LEAF_B]++;
-        }
-        const bool all = onl && wb::hyp_in_cube(H, lc[0], lc[1], lc[2], lc[3]);
-        const uint64_t allm = __ballot(all);
-        const uint32_t js = lane & (WB_CHUNK - 1);
-        for (uint32_t c0 = b; c0 < e;) {
-          const uint32_t chk = c0 / WB_CHUNK;
-          const uint32_t ce = min(e, (chk + 1) * WB_CHUNK);
-          // lanes j and j + 32 fetch slot c0 + j while the group's box is tested
-          double sx = 0, sy = 0, sz = 0;
-          if (js < ce - c0) {
-            sx = T.px[c0 + js]; sy = T.py[c0 + js]; sz = T.pz[c0 + js];
-          }
-          bool chit = onl;
-          if (chit) {
-            const double *bx = T.chunk_box + 6 * (uint64_t)chk;
-            if (!all) chit = wb::hyp_may_hit_box(H, bx[0], bx[1], bx[2], bx[3], bx[4], bx[5]);
-            if (chit) chit = lane_hit(LW, threadIdx.x, x, y, bx[0], bx[1], bx[2], bx[3]);
-          }
-          // The lanes that need the group ("owners"), two per step: lanes
-          // 0-31 test its slots against the first owner's hyperboloid, lanes
-          // 32-63 against the second's, and each half's direction bits are
-          // ORed into its owner's occupancy.
-          uint64_t own = __ballot(chit);
-          if (COUNT && chit) cnt[CT_POINT_B] += ce - c0;
-          while (own) {
-            const int o1 = __ffsll((long long)own) - 1;
-            own &= own - 1;
-            const int o2 = own ? __ffsll((long long)own) - 1 : o1;
-            const bool two = own != 0;
-            own &= own - 1;
-            if (COUNT) iter_b++;
-            const bool hi_half = lane >= WAVE / 2;
-            const int o = hi_half ? o2 : o1;
-            // the owner's hyperboloid, fetched across lanes by the LDS unit
-            wb::Shape Ho = H;
-            Ho.cx = __shfl(x, o, WAVE);
-            Ho.cy = __shfl(y, o, WAVE);
-            Ho.cz = __shfl(H.cz, o, WAVE);
-            Ho.por2 = __shfl(H.por2, o, WAVE);
-            const bool valid = js < ce - c0 && (!hi_half || two);
-            bool in = valid & ((((allm >> o) & 1) != 0) | wb::hyp_in(Ho, sx, sy, sz)) &
-                      ((sx != Ho.cx) | (sy != Ho.cy));
-            // A direction outside the owner's care wedges is not binned: its
-            // bin is occupied or in an empty run of fewer than 24 bins, runs
-            // only shrink, so it never lies in a run of 24 or more, and the
-            // runs of 24 or more (the verdict, and the occupied bins that
-            // border them) come out the same without it.
-            if (in) {
-              const int ot = (int)(threadIdx.x & ~(WAVE - 1)) + o;
-              const int nw = LW.n[ot];
-              if (nw >= 0) {
-                const float ax[2] = {LW.ax[0][ot], LW.ax[1][ot]}, ay[2] = {LW.ay[0][ot], LW.ay[1][ot]};
-                const float bx[2] = {LW.bx[0][ot], LW.bx[1][ot]}, by[2] = {LW.by[0][ot], LW.by[1][ot]};
-                const float u = (float)(sx - Ho.cx), v = (float)(sy - Ho.cy);
-                in = wb::wedge_hit2(nw, ax, ay, bx, by, u, u, v, v);
-              }
-            }
-            uint64_t bit = 0;
-            if (in) {
-              if (COUNT) cnt[CT_DIR_B]++;
-              bit = 1ull << wb::dir_bin(sy - Ho.cy, sx - Ho.cx, ttan, tcos, tsin, A.K, &nexact);
-            }
-            if (__ballot(bit != 0)) {
-              uint64_t r1, r2;
-              half_or(bit, r1, r2);
-              if ((int)lane == o1) occ |= r1;
-              if ((int)lane == o2 && two) occ |= r2;
-            }
-          }
-          c0 = ce;
+        uint64_t todo = __ballot(g < ng && union_hits(U, s2, sx, sx, sy, sy, sz));
+        while (todo) {
+          const uint32_t s = (uint32_t)__ffsll((long long)todo) - 1;
+          todo &= todo - 1;
+          const double qx = rdl(sx, s), qy = rdl(sy, s), qz = rdl(sz, s);
+          const double dx = qx - x, dy = qy - y, dz = P.cz - qz;
+          const double t = wb::hyp_near(s2, dx, dy, dz), a = dz * __builtin_fabs(dz);
+          const bool in = on & ((qx != x) | (qy != y)) & (__builtin_fma(-0x1p-39, a, t) >= sure);
+          if (!__ballot(in)) continue;
+          bool ok;
+          const int bin = wb::dir_bin_est(dy, dx, &ok);
+          if (in & ok) occ |= 1ull << bin;
         }
       }
-      const uint64_t c1t = COUNT ? clock64() : 0;
-      if (COUNT) cyc[phase == 0 ? 1 : 3] += c1t - c0t;
       if (state == 0 && occ != checked) {
         checked = occ;
         if (gap_verdict(occ) == 1) state = 1;
-        else lane_wedges_update(occ, edges, LW, threadIdx.x);
+        else if (IN) wb::lane_wedges_update(occ, edges, W);
       }
-      if (COUNT) cyc[4] += clock64() - c1t;
-      if (phase == 0 && state == 0 && groups_a > HEAVY_A_GROUPS) state = 5;
       alive = __ballot(state == 0);
       if (alive == 0) break;
+      // the union shrinks with the open lanes: taken again once a quarter of
+      // them are decided
+      const int na = __popcll(alive);
+      if (4 * na <= 3 * ualive) {
+        U = wave_union(P, state == 0);
+        ualive = na;
+      }
     }
   }
-  if (state == 0) {
-    const int v = gap_verdict(occ);
-    state = v == 0 ? 7 : v;
-  }
+  if (state == 0 && groups_a > HEAVY_B_GROUPS) state = 6;
   // hand the open lanes over, with the directions found so far
-  const uint64_t hb = __ballot(state >= 5);
-  if (hb) {
-    const int leader = __ffsll((long long)hb) - 1;
-    uint32_t base = 0;
-    if ((int)lane == leader) base = atomicAdd(A.nheavy, (uint32_t)__popcll(hb));
-    base = __shfl(base, leader, 64);
+  const uint64_t hb = __ballot(state >= 5), ob = __ballot(state == 0);
+  const uint64_t lt = (1ull << lane) - 1;
+  if (!ob && !A.open_classes && lane == 0) A.open_unit[unit] = make_uint4(0u, 0u, 0u, 0u);
+  if (hb | ob) {
+    // where units are few, those with the longest leaf lists come first
+    // (class 0), so that the longest ones don't start last
+    const uint32_t no = (uint32_t)__popcll(ob), wave = (uint32_t)unit;
+    const uint32_t cls = nleaf >= 64 ? 0 : nleaf >= 32 ? 1 : nleaf >= 16 ? 2 : 3;
+    const uint32_t per = A.open_per, nu = (no + per - 1) / per;
+    uint32_t hbase = 0, uat = wave;
+    uint64_t pbase = (uint64_t)wave * OPEN_LIST;
+    if (lane == 0) {
+      if (hb) hbase = atomicAdd(A.nheavy, (uint32_t)__popcll(hb));
+      if (ob && A.open_classes) uat = atomicAdd(A.nopen + cls, nu) + cls * A.unit_cap;
+      // a longer list takes its place from the pool's shared end
+      if (ob && nleaf > OPEN_LIST) pbase = A.pool_shared + atomicAdd(A.npool, (unsigned long long)nleaf);
+    }
+    hbase = (uint32_t)rfl((int)hbase);
+    uat = (uint32_t)rfl((int)uat);
+    pbase = rdl64(pbase, 0);
+    HeavyRec r;
+    r.occ = occ;
+    r.i = (uint32_t)i;
+    r.start = 0;
     if (state >= 5) {
-      HeavyRec r;
-      r.occ = occ;
-      r.i = (uint32_t)i;
       r.start = (uint32_t)(state - 5);
-      A.heavy[base + __popcll(hb & ((1ull << lane) - 1))] = r;
+      A.heavy[hbase + __popcll(hb & lt)] = r;
+    }
+    if (ob) {
+      const uint32_t rec = wave * WAVE + lane * per;
+      uint4 desc = make_uint4((uint32_t)pbase, nleaf | (uint32_t)(pbase >> 32) << 16,
+                              min(per, no - min(no, lane * per)), rec);
+      if (pbase + nleaf > A.pool_cap) {
+        // the shared end is full: the wave-per-point kernel takes the lanes
+        if (lane == 0) hbase = atomicAdd(A.nheavy, no);
+        hbase = (uint32_t)rfl((int)hbase);
+        r.start = 1;
+        if (state == 0) A.heavy[hbase + __popcll(ob & lt)] = r;
+        desc = make_uint4(0u, 0u, 0u, 0u);
+      } else {
+        for (uint32_t k = lane; k < nleaf; k += WAVE) A.pool[pbase + k] = S.leaf[k];
+        if (state == 0) A.open[(size_t)wave * WAVE + __popcll(ob & lt)] = r;
+      }
+      if (lane < nu) A.open_unit[uat + lane] = desc;
+    }
+  }
+  if (inrange && (state == 1 || state == 3)) work_verdict(A, i, slot, state == 1 ? 1 : 0);
+}
+
+// Walk B for a unit of up to 64 points, a lane each: every point of D that
+// can change the verdict, from the leaves walk A listed.  64 leaves at a time
+// are tested against the unit's union, a lane each; in a leaf that passes,
+// its octets (8 slots), a lane each; then every lane tests the 32-point group
+// of an octet that passed (its box against the lane's hyperboloid and care
+// wedges), the octet's box, and the octet's points one after the other, a
+// point in scalar registers, into a mask of its candidates; last each lane
+// takes its own candidates, so lanes with different ones work together.
+// A point left with a longest empty run of 24 or 25 bins takes the leaves
+// once more (GAP) for the exact extreme directions in the two bins bordering
+// the run.  A point that meets a neighbour so near its surface that rounding
+// decides goes to the heavy kernel, which tests as the reference does.
+// What bounds it: VALU issue (the points' tests, 45k instructions per unit of
+// the 23.7M-point tile with all outliers above the surface).  Walks A and B
+// and the gap pass in one kernel, with every lane testing every child, sample
+// and box by hyp_in and the gap pass left to the heavy kernel, took 41.5 and
+// 12.7 ms on that tile against 9 + 20 and 0.25 ms now, 4.9 and 0.32 against
+// 3.7 and 0.08 ms on the one with low outliers, 2.7 and 0.67 against 2.0 and
+// 0.08 ms on 1.17M points, 0.46 and 0.04 against 0.28 and 0.01 ms on 18.5k.
+struct OpenPoint {
+  int state;  // 0 undecided, 1 not ground, 2 ground, 3 none, 4 the exact gap
+              // decides; to the heavy kernel: 6 walk B, 7 the exact gap
+  uint64_t occ;
+  wb::LaneWedges W;
+  // of the gap pass: the bins bordering the runs (8 bits each: before and
+  // after the first, the second), the largest position in a bin before a run
+  // and the smallest in a bin after it
+  uint32_t border;
+  int hi[2], lo[2];
+};
+
+// a value every lane reads from the same address, as uload
+__device__ inline float uloadf(const float *p, size_t i)
+{
+  return ((const __attribute__((address_space(4))) float *)p)[i];
+}
+__device__ inline uint32_t uloadu(const uint32_t *p, size_t i)
+{
+  return ((const __attribute__((address_space(4))) uint32_t *)p)[i];
+}
+
+template <bool IN, bool GAP>
+__device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t *pool, uint32_t nleaf,
+                                          const Near &P, OpenPoint &O, const float *edges,
+                                          double2 *edge, int &nexact)
+{
+  const TreeView &T = A.T;
+  const uint32_t lane = __lane_id();
+  const double sl = A.max_slope, s2 = (sl * sl) * wb::kNearShrink, x = P.x, y = P.y;
+  const double slack = sure_slack(A);
+  const int want = GAP ? 4 : 0;
+  bool pend = false;
+  uint64_t checked = O.occ;
+  uint64_t alive = __ballot(O.state == want);
+  if (alive == 0) return;
+  Union U = wave_union(P, O.state == want);
+  int ualive = __popcll(alive);
+  for (uint32_t lb = 0; lb < nleaf && alive; lb += WAVE) {
+    uint32_t leaf_l = 0;
+    bool lh = lb + lane < nleaf;
+    if (lh) {
+      leaf_l = pool[lb + lane];
+      const double *c = T.leaf_cube + 4 * (size_t)leaf_l;
+      const double h = c[3] / 2;
+      lh = union_hits(U, s2, c[0] - h, c[0] + h, c[1] - h, c[1] + h,
+                      IN ? fmax(c[2] - h, (double)T.leaf_low[leaf_l]) : c[2] - h);
+    }
+    uint64_t ltodo = __ballot(lh);
+    while (ltodo) {
+      const uint32_t ls = (uint32_t)__ffsll((long long)ltodo) - 1;
+      ltodo &= ltodo - 1;
+      const uint32_t leaf = (uint32_t)__builtin_amdgcn_readlane((int)leaf_l, (int)ls);
+      const uint32_t b = uloadu(T.leaf_start, leaf), e = uloadu(T.leaf_start, leaf + 1);
+      bool on = O.state == want, all = false;
+      bool anyw = IN && __ballot(on && O.W.n >= 0) != 0;
+      {
+        const double *c = T.leaf_cube + 4 * (size_t)leaf;
+        const double cx = uload(c, 0), cy = uload(c, 1), cz = uload(c, 2), hh = uload(c, 3) / 2;
+        if (IN) {
+          const double x0 = cx - hh, x1 = cx + hh, y0 = cy - hh, y1 = cy + hh;
+          on = on && near_t(P, s2, fmin(fmax(x, x0), x1), fmin(fmax(y, y0), y1),
+                            fmax(cz - hh, (double)uloadf(T.leaf_low, leaf))) >= P.thr;
+          if (anyw && __ballot(on))
+            on = on & wb::wedge_hit2(min(O.W.n, 2), O.W.ax, O.W.ay, O.W.bx, O.W.by, (float)(x0 - x),
+                                     (float)(x1 - x), (float)(y0 - y), (float)(y1 - y));
+        } else {
+          // points outside their leaf's cube: findBlocks' own tests, and the
+          // leaf whose eight corners are all in
+          wb::Shape H = wb::make_cylinder(x, y, 0);
+          H.kind = wb::SHAPE_HYPERBOLOID;
+          H.cz = P.cz;
+          H.por2 = P.por2;
+          H.slope = sl;
+          on = on && wb::hyp_intersect(H, cx, cy, cz, 2 * hh);
+          all = on && wb::hyp_in_cube(H, cx, cy, cz, 2 * hh);
+          for (int nd = T.leaf_parent[leaf]; nd >= 0; nd = T.node_parent[nd]) {
+            const double *q = T.node_cube + 4 * (size_t)nd;
+            on = on && wb::hyp_intersect(H, q[0], q[1], q[2], q[3]);
+          }
+          all = all && on;
+        }
+      }
+      if (!__ballot(on)) continue;
+      const uint32_t q0 = b / WB_OCT, nq = (e - 1) / WB_OCT - q0 + 1;
+      for (uint32_t qb = 0; qb < nq; qb += WAVE) {
+        bool h = qb + lane < nq;
+        if (IN && h) {
+          const Union R = {U.x0 - T.ox, U.x1 - T.ox, U.y0 - T.oy, U.y1 - T.oy, U.cz - T.oz, U.thr};
+          const float4 bx = T.oct_xy[q0 + qb + lane];
+          h = union_hits(R, s2, bx.x, bx.y, bx.z, bx.w, T.oct_z[q0 + qb + lane]);
+        }
+        uint64_t todo = __ballot(h);
+        while (todo) {
+          // the group of the next octet, and its octets that passed
+          const uint32_t qf = q0 + qb + (uint32_t)__ffsll((long long)todo) - 1;
+          const uint32_t chk = qf / (WB_CHUNK / WB_OCT);
+          bool hit = on;
+          {
+            const double *bx = T.chunk_box + 6 * (size_t)chk;
+            const double x0 = uload(bx, 0), x1 = uload(bx, 1), y0 = uload(bx, 2), y1 = uload(bx, 3),
+                         z0 = uload(bx, 4);
+            hit = on & (all | (near_t(P, s2, fmin(fmax(x, x0), x1), fmin(fmax(y, y0), y1), z0) >=
+                               P.thr));
+            if (anyw && __ballot(hit))
+              hit = hit & wb::wedge_hit2(min(O.W.n, 2), O.W.ax, O.W.ay, O.W.bx, O.W.by,
+                                         (float)(x0 - x), (float)(x1 - x), (float)(y0 - y),
+                                         (float)(y1 - y));
+          }
+          const uint64_t hb = __ballot(hit);
+          // lanes j and j + 32 fetch slot j of the group (the arrays are padded
+          // to whole groups)
+          double gx = 0, gy = 0, gz = 0;
+          if (hb) {
+            const uint32_t j = chk * WB_CHUNK + (lane & (WB_CHUNK - 1));
+            gx = T.px[j]; gy = T.py[j]; gz = T.pz[j];
+          }
+          uint32_t cand = 0;  // this lane's candidates among the group's slots
+          if (hb && __popcll(hb) <= OPEN_PAIR) {
+            // few lanes need the group: two at a time, lanes 0-31 test its
+            // slots against the first one's hyperboloid and care run, lanes
+            // 32-63 against the second's
+            uint64_t own = hb;
+            while (own) {
+              const uint32_t o1 = (uint32_t)__ffsll((long long)own) - 1;
+              own &= own - 1;
+              const uint32_t o2 = own ? (uint32_t)__ffsll((long long)own) - 1 : o1;
+              own &= own - 1;
+              const bool up = lane >= WAVE / 2;
+              const double ox = rdl(x, o1), oy = rdl(y, o1), oz = rdl(P.cz, o1), ot = rdl(P.thr, o1);
+              const double qx = rdl(x, o2), qy = rdl(y, o2), qz = rdl(P.cz, o2), qt = rdl(P.thr, o2);
+              const double dx = gx - (up ? qx : ox), dy = gy - (up ? qy : oy);
+              const double dz = (up ? qz : oz) - gz;
+              bool c = wb::hyp_near(s2, dx, dy, dz) >= (up ? qt : ot);
+              if (anyw && __ballot(c)) {
+                wb::LaneWedges V;
+                const int o = (int)(up ? o2 : o1);
+                V.ax[0] = __shfl(O.W.ax[0], o, WAVE); V.ay[0] = __shfl(O.W.ay[0], o, WAVE);
+                V.bx[0] = __shfl(O.W.bx[0], o, WAVE); V.by[0] = __shfl(O.W.by[0], o, WAVE);
+                V.bx[1] = __shfl(O.W.bx[1], o, WAVE); V.by[1] = __shfl(O.W.by[1], o, WAVE);
+                V.n = __shfl(O.W.n, o, WAVE);
+                c = c & wb::lane_dir(V, (float)dx, (float)dy);
+              }
+              const uint64_t cm = __ballot(c);
+              if (lane == o1) cand = (uint32_t)cm;
+              if (lane == o2 && o2 != o1) cand = (uint32_t)(cm >> 32);
+            }
+            if (!IN && all) cand = 0xffffffffu;
+            // the group's slots inside the leaf
+            const uint32_t s0 = chk * WB_CHUNK;
+            if (b > s0) cand &= ~0u << (b - s0);
+            if (e < s0 + WB_CHUNK) cand &= (1u << (e - s0)) - 1;
+            const uint32_t past = (chk + 1) * (WB_CHUNK / WB_OCT) - (q0 + qb);
+            todo = past < WAVE ? (todo >> past) << past : 0;
+          }
+          // otherwise octet by octet, every lane tests a point at a time
+          for (uint32_t q = qf; todo && q0 + qb + (uint32_t)__ffsll((long long)todo) - 1 <
+                                            (chk + 1) * (WB_CHUNK / WB_OCT);) {
+            q = q0 + qb + (uint32_t)__ffsll((long long)todo) - 1;
+            todo &= todo - 1;
+            if (!hb) continue;
+            uint32_t c8 = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < WB_OCT; k++) {
+              const uint32_t j = WB_OCT * (q % (WB_CHUNK / WB_OCT)) + k;
+              const double dx = rdl(gx, j) - x, dy = rdl(gy, j) - y, dz = P.cz - rdl(gz, j);
+              bool c = hit & (wb::hyp_near(s2, dx, dy, dz) >= P.thr);
+              if (!__ballot(c)) continue;
+              if (anyw) c = c & wb::lane_dir(O.W, (float)dx, (float)dy);
+              c8 |= c ? 1u << k : 0u;
+            }
+            // the octet's slots inside the leaf
+            const uint32_t k0 = b > q * WB_OCT ? b - q * WB_OCT : 0;
+            const uint32_t k1 = e < (q + 1) * WB_OCT ? e - q * WB_OCT : WB_OCT;
+            const uint32_t in8 = ((1u << k1) - 1) & ~((1u << k0) - 1);
+            cand |= ((!IN && all ? 0xffu : c8) & in8) << (WB_OCT * (q % (WB_CHUNK / WB_OCT)));
+          }
+          if (!hit) cand = 0;
+          uint32_t taken = 0;
+          while (__ballot(cand != 0)) {
+            taken++;
+            const bool has = cand != 0;
+            const uint32_t j = chk * WB_CHUNK + (has ? (uint32_t)__ffs((int)cand) - 1 : 0u);
+            cand &= cand - 1;
+            double dx = 0, dy = 0, dz = 0;
+            if (has) {
+              dx = T.px[j] - x;
+              dy = T.py[j] - y;
+              dz = P.cz - T.pz[j];
+            }
+            // (a difference is zero only between equal coordinates)
+            const bool c = has & ((dx != 0) | (dy != 0));
+            if (!__ballot(c)) continue;
+            const double t = wb::hyp_near(s2, dx, dy, dz), a = dz * __builtin_fabs(dz);
+            const bool in = c & (all | (__builtin_fma(-0x1p-39, a, t) >= P.por2 + slack));
+            if (c & !in) O.state = GAP ? 7 : 6;
+            if (!GAP) {
+              // a direction near a bin's edge waits for the leaf's end (the
+              // call of the exact form would cost every lane registers in
+              // this loop); a second one in the same leaf is left to the
+              // heavy kernel
+              bool ok;
+              const int bin = wb::dir_bin_est(dy, dx, &ok);
+              if (in & ok) O.occ |= 1ull << bin;
+              if (in & !ok) {
+                if (pend) O.state = 6;
+                pend = true;
+                edge[lane] = make_double2(dx, dy);
+              }
+            } else {
+              // only a direction that may be a border bin's extreme one is
+              // taken exactly: by the float position, within 2^11 units of the
+              // exact one
+              bool ok;
+              float q;
+              const uint32_t bin = (uint32_t)wb::dir_bin_est(dy, dx, &ok, &q), bd = O.border;
+              const int est = (int)(q * 0x1p25f);
+              const bool b0 = bin == (bd & 255u), a0 = bin == ((bd >> 8) & 255u);
+              const bool b1 = bin == ((bd >> 16) & 255u), a1 = bin == (bd >> 24);
+              const bool may = (b0 & (est > O.hi[0] - 4096)) | (a0 & (est - 4096 < O.lo[0])) |
+                               (b1 & (est > O.hi[1] - 4096)) | (a1 & (est - 4096 < O.lo[1]));
+              if (__builtin_expect(in & (!ok | may), 0)) {
+                const double *ttan = A.tab, *tcos = A.tab + 511, *tsin = A.tab + 1023;
+                const int p = dir_bin_pos(wb::atan2i_ext(dy, dx, ttan, tcos, tsin, A.K, &nexact));
+                const uint32_t xb = (uint32_t)p >> 25;
+                if (xb == (bd & 255u)) O.hi[0] = max(O.hi[0], p);
+                if (xb == ((bd >> 16) & 255u)) O.hi[1] = max(O.hi[1], p);
+                if (xb == ((bd >> 8) & 255u)) O.lo[0] = min(O.lo[0], p);
+                if (xb == (bd >> 24)) O.lo[1] = min(O.lo[1], p);
+              }
+            }
+          }
+          // many candidates: the directions just found may leave out the next
+          // group's
+          if (IN && !GAP && taken >= OPEN_REFRESH && O.occ != checked && O.state == 0) {
+            checked = O.occ;
+            if (gap_verdict(O.occ) == 1) {
+              O.state = 1;
+              on = false;
+            } else {
+              wb::lane_wedges_update(O.occ, edges, O.W);
+            }
+          }
+          if (IN && !GAP && taken >= OPEN_REFRESH) anyw = __ballot(on && O.W.n >= 0) != 0;
+        }
+      }
+      if (!GAP) {
+        if (__builtin_expect(__ballot(pend) != 0, 0)) {
+          const double *ttan = A.tab, *tcos = A.tab + 511, *tsin = A.tab + 1023;
+          if (pend) {
+            const double2 d = edge[lane];
+            O.occ |= 1ull << wb::dir_bin(d.y, d.x, ttan, tcos, tsin, A.K, &nexact);
+          }
+          pend = false;
+        }
+        if (O.state == 0 && O.occ != checked) {
+          checked = O.occ;
+          if (gap_verdict(O.occ) == 1) O.state = 1;
+          else if (IN) wb::lane_wedges_update(O.occ, edges, O.W);
+        }
+      }
+      alive = __ballot(O.state == want);
+      if (alive == 0) break;
+      const int na = __popcll(alive);
+      if (4 * na <= 3 * ualive) {
+        U = wave_union(P, O.state == want);
+        ualive = na;
+      }
+    }
+  }
+}
+
+template <bool IN>
+__device__ __forceinline__ void open_body(const ClassifyArgs &A, uint32_t u, const float *edges,
+                                          double2 *edge)
+{
+  const TreeView &T = A.T;
+  const uint32_t lane = __lane_id();
+  const uint4 un = A.open_unit[u];
+  const uint32_t *pool = A.pool + (((uint64_t)((uint32_t)rfl((int)un.y) >> 16) << 32) |
+                                   (uint32_t)rfl((int)un.x));
+  const uint32_t nleaf = (uint32_t)rfl((int)un.y) & 0xffffu;
+  const uint32_t npt = (uint32_t)rfl((int)un.z);
+  if (npt == 0) return;
+  const bool live = lane < npt;
+  const size_t at = (size_t)un.w + lane;
+  OpenPoint O;
+  O.state = live ? 0 : 3;
+  O.occ = 0;
+  double x = 0, y = 0, z = 0, hs = 0;
+  if (live) {
+    const HeavyRec r = A.open[at];
+    uint32_t slot = 0;
+    work_point(A, r.i, slot, hs);
+    x = T.px[slot]; y = T.py[slot]; z = T.pz[slot];
+    O.occ = r.occ;
+  }
+  const Near P = make_near(A, x, y, z, hs);
+  int nexact = 0;
+  wb::lane_wedges_update(O.occ, edges, O.W);
+  if (!IN) O.W.n = -1;
+  open_pass<IN, false>(A, pool, nleaf, P, O, edges, edge, nexact);
+  if (O.state == 0) {
+    O.state = gap_verdict(O.occ);
+    if (O.state == 0) O.state = 4;
+  }
+  if (__ballot(O.state == 4)) {
+    int before[2] = {255, 255}, after[2] = {255, 255}, nr = 0;
+    if (O.state == 4) {
+      for (int st = 0; st < 64; st++) {
+        if ((O.occ >> st) & 1) continue;
+        if (!((O.occ >> ((st + 63) & 63)) & 1)) continue;
+        int len = 0;
+        while (len < 64 && !((O.occ >> ((st + len) & 63)) & 1)) len++;
+        if (len >= 24 && nr < 2) {
+          const int bf = (st + 63) & 63, af = (st + len) & 63;
+          if (nr == 0) { before[0] = bf; after[0] = af; }
+          else { before[1] = bf; after[1] = af; }
+          nr++;
+        }
+      }
+      // the border wedges span at most 27 bins: each one wedge
+      wb::Wedges w;
+      wb::border_wedges(before, after, nr, w, edges);
+      O.W.ax[0] = w.ax[0]; O.W.ay[0] = w.ay[0]; O.W.bx[0] = w.bx[0]; O.W.by[0] = w.by[0];
+      O.W.ax[1] = w.ax[2]; O.W.ay[1] = w.ay[2]; O.W.bx[1] = w.bx[2]; O.W.by[1] = w.by[2];
+      O.W.n = IN && nr ? nr == 2 ? 3 : 1 : -1;
+    }
+    O.border = (uint32_t)before[0] | (uint32_t)after[0] << 8 | (uint32_t)before[1] << 16 |
+               (uint32_t)after[1] << 24;
+    O.hi[0] = O.hi[1] = -1;
+    O.lo[0] = O.lo[1] = 0x7fffffff;
+    open_pass<IN, true>(A, pool, nleaf, P, O, edges, edge, nexact);
+    if (O.state == 4) {
+      const int g0 = (int)(((uint32_t)O.lo[0] - (uint32_t)O.hi[0]) & 0x7fffffffu);
+      const int g1 = (int)(((uint32_t)O.lo[1] - (uint32_t)O.hi[1]) & 0x7fffffffu);
+      O.state = (g0 >= wb::DEG144) | ((nr > 1) & (g1 >= wb::DEG144)) ? 2 : 1;
+      atomicAdd(A.nslow, 1u);
     }
   }
   if (nexact) atomicAdd(A.atan_exact, (unsigned long long)nexact);
-  if (inrange && state < 5) work_verdict(A, i, slot, state == 1 ? 1 : (state == 2 ? 2 : 0));
-  if (COUNT) {
-    if (state == 7) cnt[CT_LANES_C]++;
-    if (state >= 5) cnt[CT_HEAVY]++;
-    uint64_t v[CT_WAVES];
-    for (int k = 0; k < CT_WAVES; k++) {
-      uint64_t t = cnt[k];
-      // wave-level counters are the same in every lane
-      if (k != CT_EXP_A && k != CT_WLEAF_A && k != CT_EXP_B && k != CT_WLEAF_B)
-        for (int sft = 1; sft < 64; sft <<= 1) t += __shfl_xor(t, sft, 64);
-      v[k] = t;
-    }
-    if (lane == 0) {
-      unsigned long long *ctr = A.counters + (blk % CT_COPIES) * CT_STRIDE;
-      for (int k = 0; k < CT_WAVES; k++) atomicAdd(&ctr[k], (unsigned long long)v[k]);
-      atomicAdd(&ctr[CT_WAVES], 1ull);
-      const uint64_t dt = wall_clock64() - t_start;
-      atomicAdd(&ctr[CT_TSUM], (unsigned long long)dt);
-      atomicMax(&ctr[CT_TMAX], (unsigned long long)dt);
-      // wave times in ticks: <1e3, <1e4, <1e5, <1e6, >=1e6
-      const int hb = dt < 1000 ? 0 : dt < 10000 ? 1 : dt < 100000 ? 2 : dt < 1000000 ? 3 : 4;
-      atomicAdd(&ctr[CT_THIST + hb], 1ull);
-      atomicAdd(&ctr[CT_TSUMS + hb], (unsigned long long)dt);
-      for (int k = 0; k < 8; k++) atomicAdd(&ctr[CT_CYC + k], (unsigned long long)cyc[k]);
-      atomicAdd(&ctr[CT_ITER_A], (unsigned long long)iter_a);
-      atomicAdd(&ctr[CT_ITER_B], (unsigned long long)iter_b);
+  if (live) {
+    HeavyRec r = A.open[at];
+    if (O.state >= 6) {
+      r.occ = O.occ;
+      r.start = (uint32_t)(O.state - 5);
+      A.heavy[atomicAdd(A.nheavy, 1u)] = r;
+    } else {
+      uint32_t slot = 0;
+      work_point(A, r.i, slot, hs);
+      work_verdict(A, r.i, slot, (uint8_t)O.state);
     }
   }
 }
 
+#ifndef WB_OPEN_MINW
+#define WB_OPEN_MINW 5
+#endif
 
-template <bool COUNT, int MINW>
-__global__ void __launch_bounds__(256, MINW) k_ground(ClassifyArgs A)
+template <bool IN, int MINW>
+__global__ void __launch_bounds__(WAVE, MINW) k_ground(ClassifyArgs A)
 {
-  __shared__ WaveStack stacks[256 / WAVE];
-  __shared__ LaneWedges LW;
+  __shared__ WaveStack S;
   __shared__ float edges[3 * 128];
   ground_setup(A, edges);
-  ground_body<COUNT>(A, (uint64_t)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE, stacks, LW,
-                     edges);
+  walk_body<IN>(A, blockIdx.x, S, edges);
 }
 
-// The same test on a grid that stays resident: each wave takes its first
+// The same walk on a grid that stays resident: each wave takes its first
 // unit of 64 items by its place in the grid, then the next unit no wave has
 // taken (*next counts the units taken beyond the grid's; zero before the
 // launch), until none is left.  Launched with fewer blocks than fit on the
 // device, it leaves room on every CU for the kernels of other streams,
 // which a kernel of many short blocks does not: each freed slot goes to its
 // next block.
-template <int MINW>
-__global__ void __launch_bounds__(256, MINW) k_ground_resident(ClassifyArgs A, uint32_t *next)
+template <bool IN, int MINW>
+__global__ void __launch_bounds__(WAVE, MINW) k_ground_resident(ClassifyArgs A, uint32_t *next)
 {
-  __shared__ WaveStack stacks[256 / WAVE];
-  __shared__ LaneWedges LW;
+  __shared__ WaveStack S;
   __shared__ float edges[3 * 128];
   ground_setup(A, edges);
   const uint64_t nunits = ((A.items ? A.n_items : A.T.n) + WAVE - 1) / WAVE;
-  const uint32_t waves = gridDim.x * (256 / WAVE);
-  uint64_t unit = (uint64_t)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
+  uint64_t unit = blockIdx.x;
   while (unit < nunits) {
-    ground_body<false>(A, unit, stacks, LW, edges);
+    walk_body<IN>(A, unit, S, edges);
     uint32_t u = 0;
     if (__lane_id() == 0) u = atomicAdd(next, 1u);
-    unit = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)u) + waves;
+    unit = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)u) + gridDim.x;
   }
 }
 
-// The ground tests of several trees in one launch: blocks boff[k] ..
-// boff[k+1]-1 take tree k, whose arguments are AA[k].
-template <int MINW>
-__global__ void __launch_bounds__(256, MINW) k_ground_batch(const ClassifyArgs *AA,
-                                                            const uint32_t *boff, int ntrees)
+// Walk A of several trees in one launch: blocks boff[k] .. boff[k+1]-1 take
+// tree k, whose arguments are AA[k].
+template <bool IN, int MINW>
+__global__ void __launch_bounds__(WAVE, MINW) k_ground_batch(const ClassifyArgs *AA,
+                                                             const uint32_t *boff, int ntrees)
 {
-  __shared__ WaveStack stacks[256 / WAVE];
-  __shared__ LaneWedges LW;
+  __shared__ WaveStack S;
   __shared__ float edges[3 * 128];
   int lo = 0, hi = ntrees;  // boff[lo] <= blockIdx.x < boff[hi]
   while (hi - lo > 1) {
@@ -2373,8 +2670,108 @@ __global__ void __launch_bounds__(256, MINW) k_ground_batch(const ClassifyArgs *
     else hi = mid;
   }
   ground_setup(AA[lo], edges);
-  ground_body<false>(AA[lo], (uint64_t)(blockIdx.x - boff[lo]) * (256 / WAVE) + threadIdx.x / WAVE,
-                     stacks, LW, edges);
+  walk_body<IN>(AA[lo], blockIdx.x - boff[lo], S, edges);
+}
+
+// Unit u of walk B in the order of the classes (those with the longest leaf
+// lists first); false past the last.
+template <bool IN>
+__device__ __forceinline__ bool open_unit(const ClassifyArgs &A, uint32_t u, const float *edges,
+                                          double2 *edge)
+{
+  uint32_t cls = 0;
+#pragma unroll
+  for (int k = 0; k < OPEN_CLASSES; k++) {
+    const uint32_t nk = (uint32_t)rfl((int)A.nopen[k]);
+    if (cls == (uint32_t)k && u >= nk) {
+      u -= nk;
+      cls++;
+    }
+  }
+  if (cls == OPEN_CLASSES) return false;
+  open_body<IN>(A, cls * A.unit_cap + u, edges, edge);
+  return true;
+}
+
+// Walk B over the units walk A left, a block per unit there can be: with
+// classes block u takes unit u of their order, else wave u's.  (A resident
+// grid that takes the units by a counter was 3 to 7% slower on 40k to 300k
+// points: every claim waits for the counter's word.)
+template <bool IN>
+__global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open(ClassifyArgs A)
+{
+  __shared__ float edges[3 * 128];
+  __shared__ double2 edge[WAVE];
+  ground_setup(A, edges);
+  if (A.open_classes) open_unit<IN>(A, blockIdx.x, edges, edge);
+  else if (blockIdx.x < A.unit_cap) open_body<IN>(A, blockIdx.x, edges, edge);
+}
+
+// The same as a grid that stays resident and takes the units by a counter
+// (A.open_next, zero before the launch): with the context's sharing switch.
+template <bool IN>
+__global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open_resident(ClassifyArgs A)
+{
+  __shared__ float edges[3 * 128];
+  __shared__ double2 edge[WAVE];
+  ground_setup(A, edges);
+  for (;;) {
+    uint32_t u = 0;
+    if (threadIdx.x == 0) u = atomicAdd(A.open_next, 1u);
+    if (!open_unit<IN>(A, (uint32_t)rfl((int)u), edges, edge)) return;
+  }
+}
+
+// The entry of off[0..m] (ascending) that holds u: off[e] <= u < off[e+1]; m
+// past the last.
+__device__ __forceinline__ int batch_find(const uint32_t *off, int m, uint32_t u)
+{
+  for (int b = 0; b < m; b += WAVE) {
+    const int k = b + (int)threadIdx.x;
+    const uint64_t past = __ballot(k < m && off[k + 1] > u);
+    if (past) return b + __builtin_ctzll(past);
+  }
+  return m;
+}
+
+// off[0..m]: the running sums of what the batch's trees counted: units of
+// walk B by class and then tree (open), or heavy points by tree.
+__global__ void __launch_bounds__(WAVE) k_batch_sums(const ClassifyArgs *AA, int ntrees, int open,
+                                                     uint32_t *off)
+{
+  const int m = open ? ntrees * OPEN_CLASSES : ntrees;
+  const int lane = threadIdx.x;
+  uint32_t sum = 0;
+  if (lane == 0) off[0] = 0;
+  for (int b = 0; b < m; b += WAVE) {
+    const int k = b + lane;
+    uint32_t v = 0;
+    if (k < m) v = open ? AA[k % ntrees].nopen[k / ntrees] : *AA[k].nheavy;
+    for (int d = 1; d < WAVE; d <<= 1) {
+      const uint32_t w = __shfl_up(v, d, WAVE);
+      if (lane >= d) v += w;
+    }
+    if (k < m) off[k + 1] = sum + v;
+    sum += (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+  }
+}
+
+// Walk B over several trees: block u takes unit u of the batch, those with
+// the longest lists of every tree first (uoff: k_batch_sums).  A grid of as
+// many blocks as there can be units needs no counter: taking the units tree by
+// tree, each wave by each tree's counter, took 12 trees of 150k points 4.4 ms.
+template <bool IN>
+__global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open_batch(const ClassifyArgs *AA,
+                                                                          const uint32_t *uoff,
+                                                                          int ntrees)
+{
+  __shared__ float edges[3 * 128];
+  __shared__ double2 edge[WAVE];
+  const int e = batch_find(uoff, ntrees * OPEN_CLASSES, blockIdx.x);
+  if (e == ntrees * OPEN_CLASSES) return;
+  const ClassifyArgs &A = AA[e % ntrees];
+  ground_setup(A, edges);
+  open_body<IN>(A, (uint32_t)(e / ntrees) * A.unit_cap + blockIdx.x - uoff[e], edges, edge);
 }
 
 // One heavy point per 64-lane block.  The shape is the same in every lane,
@@ -2413,15 +2810,12 @@ struct HeavyShared {
   wb::Wedges wg;
 };
 
-template <bool COUNT>
-__device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec hr, uint32_t blk,
+__device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec hr,
                                            HeavyShared &SH)
 {
   int *stk = SH.stk;
   uint32_t *lq = SH.lq, *lb = SH.lb, *le = SH.le, *lmask = SH.lmask, *lpre = SH.lpre;
   wb::Wedges &wg = SH.wg;
-  const uint64_t t_start = COUNT ? wall_clock64() : 0;
-  uint64_t c_leaf = 0, c_pts = 0, c_exp = 0, c_test = 0, c_in = 0;
   const TreeView &T = A.T;
   const uint32_t i = hr.i;  // work index (k_ground hands over only lanes with a tile)
   const uint32_t lane = threadIdx.x;
@@ -2483,7 +2877,6 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
         const int gi = (int)(lane >> 3), k = (int)(lane & 7);
         const int code = gi < P ? stk[sp - 1 - gi] : 0;
         __syncthreads();
-        if (COUNT) c_exp += P;
         bool h = false;
         int ck = -1, t = 0;
         if (gi < P) {
@@ -2531,7 +2924,6 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
       }
       if (nq == 0) break;
       lim = min(4 * lim, (uint32_t)HB_LEAVES);
-      if (COUNT) c_leaf += nq;
       // per-leaf bounds, inside flag (bit 31 of lmask) and group mask, and
       // the prefix of the leaves' sample counts (walk A) or selected-group
       // counts (walks B and C)
@@ -2578,7 +2970,6 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
       if (lane == 0) lpre[0] = 0;
       __syncthreads();
       const uint32_t S = carry;
-      if (COUNT) c_pts += phase == 0 ? S : WB_CHUNK * S;
       uint32_t kc = 0;  // this lane's leaf in the batch
       // walk A: a sample per lane; walks B and C: two selected groups per
       // step, lanes 0-31 the slots of the first, 32-63 of the second
@@ -2612,10 +3003,6 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
           if (test) {
             const double qx = T.px[j], qy = T.py[j], qz = T.pz[j];
             const bool in = (phase != 0 && (mask >> 31)) || wb::hyp_in(H, qx, qy, qz);
-            if (COUNT) {
-              c_test++;
-              if (in) c_in++;
-            }
             if (in && (qx != x || qy != y)) {
               const int bin = wb::dir_bin(qy - y, qx - x, ttan, tcos, tsin, A.K, &nexact);
               if (phase < 2) {
@@ -2665,28 +3052,9 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
     if (lane == 0) atomicAdd(A.nslow, 1u);
   }
   for (int s = 1; s < 64; s <<= 1) nexact += __shfl_xor(nexact, s, 64);
-  if (COUNT)
-    for (int s = 1; s < 64; s <<= 1) {
-      c_test += __shfl_xor(c_test, s, 64);
-      c_in += __shfl_xor(c_in, s, 64);
-    }
   if (lane == 0) {
     work_verdict(A, i, slot, (uint8_t)verdict);
     if (nexact) atomicAdd(A.atan_exact, (unsigned long long)nexact);
-    if (COUNT) {
-      // per start walk: points, passes, leaves, slots, expansions, ticks,
-      // slots tested, slots inside the shape
-      unsigned long long *h =
-          A.counters + (blk % CT_COPIES) * CT_STRIDE + CT_N + 8 * hr.start;
-      atomicAdd(&h[0], 1ull);
-      if (verdict == 1) atomicAdd(&h[1], 1ull);
-      atomicAdd(&h[2], (unsigned long long)c_leaf);
-      atomicAdd(&h[3], (unsigned long long)c_pts);
-      atomicAdd(&h[4], (unsigned long long)c_exp);
-      atomicAdd(&h[5], (unsigned long long)(wall_clock64() - t_start));
-      atomicAdd(&h[6], (unsigned long long)c_test);
-      atomicAdd(&h[7], (unsigned long long)c_in);
-    }
   }
 }
 
@@ -2695,7 +3063,6 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
 // read on the device, so the host does not wait for the count): block b
 // takes record b, then the next record not yet taken (*next counts the
 // records taken beyond the first gridDim.x; zero before the launch).
-template <bool COUNT>
 __global__ void __launch_bounds__(64, WB_HEAVY_MINW) k_ground_heavy(ClassifyArgs A, const HeavyRec *heavy,
                                                                     const uint32_t *nheavy,
                                                                     uint32_t *next)
@@ -2705,7 +3072,7 @@ __global__ void __launch_bounds__(64, WB_HEAVY_MINW) k_ground_heavy(ClassifyArgs
   const uint32_t nh = *nheavy;
   uint32_t r = blockIdx.x;
   while (r < nh) {
-    heavy_body<COUNT>(A, heavy[r], r, SH);
+    heavy_body(A, heavy[r], SH);
     __syncthreads();
     if (threadIdx.x == 0) take = atomicAdd(next, 1u) + gridDim.x;
     __syncthreads();
@@ -2713,22 +3080,24 @@ __global__ void __launch_bounds__(64, WB_HEAVY_MINW) k_ground_heavy(ClassifyArgs
   }
 }
 
-// The heavy points of several trees in one launch: blocks hoff[k] ..
-// hoff[k+1]-1 take the heavy records of tree k (AA[k].heavy).
+// the same over several trees (hoff: k_batch_sums; the first tree's counter
+// counts the records taken)
 __global__ void __launch_bounds__(64, WB_HEAVY_MINW) k_ground_heavy_batch(const ClassifyArgs *AA,
                                                                           const uint32_t *hoff,
                                                                           int ntrees)
 {
   __shared__ HeavyShared SH;
-  if (blockIdx.x >= hoff[ntrees]) return;
-  int lo = 0, hi = ntrees;  // hoff[lo] <= blockIdx.x < hoff[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) / 2;
-    if (hoff[mid] <= blockIdx.x) lo = mid;
-    else hi = mid;
+  __shared__ uint32_t take;
+  uint32_t r = blockIdx.x;
+  for (;;) {
+    const int k = batch_find(hoff, ntrees, r);
+    if (k == ntrees) return;
+    heavy_body(AA[k], AA[k].heavy[r - hoff[k]], SH);
+    __syncthreads();
+    if (threadIdx.x == 0) take = atomicAdd(AA[0].heavy_next, 1u) + gridDim.x;
+    __syncthreads();
+    r = take;
   }
-  const ClassifyArgs &A = AA[lo];
-  heavy_body<false>(A, A.heavy[blockIdx.x - hoff[lo]], blockIdx.x, SH);
 }
 
 // an input merged into an earlier point at its location gets that point's class
@@ -2881,6 +3250,17 @@ void wb_run_points(wb_tree *t, int kind, const double *dparams, uint64_t ns, con
                        order, ns, doffs, dout);
 }
 
+// Room for what walk A of n work indices leaves to walk B: units of every
+// wave (in each class), and leaf lists of OPEN_LIST entries a wave, with a
+// shared end for the longer ones (a list that finds no room there sends its
+// lanes to the heavy kernel).
+struct OpenBuffers {
+  HeavyRec *open;
+  uint4 *unit;
+  uint32_t *pool;
+  size_t nrec, nunit, npool;
+};
+
 // The state of one tree's classification pass between its phases:
 // classify_prepare (tile geometry, membership, SCAN, POSTSCAN, the ground
 // test's arguments), the ground test (one tree, or several in one launch),
@@ -2899,10 +3279,11 @@ struct ClassifyRun {
   int32_t *tex, *tey, *memb, *grid;
   uint32_t *tile_cnt, *tile_fill, *nmemb, *err, *nslow, *tile_off, *lists;
   TileRec *rec;
-  unsigned long long *ctr, *dcount;
+  unsigned long long *ctr;
   uint64_t gcells, total;
   uint8_t *cls;
   HeavyRec *heavy;
+  OpenBuffers open;
   ClassifyArgs A;
   uint32_t h_nheavy, h_nslow;
   uint32_t *heavy_next;  // records the heavy kernel has taken beyond its grid
@@ -2955,19 +3336,50 @@ static const wb_ctx::TileGeoCache &tile_geometry(wb_ctx *c, const TileGeo &g0)
   return c->geo.back();
 }
 
-static bool classify_count_work()
+static void open_buffers(wb_ctx *c, ClassifyArgs &A, uint64_t n, uint64_t nbatch, OpenBuffers &B)
 {
-  static const bool on = getenv("WB_CLASSIFY_COUNTERS") != nullptr;
-  return on;
+  const uint64_t waves = (n + WAVE - 1) / WAVE;
+  B.nrec = (size_t)waves * WAVE;
+  const uint32_t ucap = (uint32_t)std::min<uint64_t>(waves * 4, 0x3fffffffull);
+  A.pool_shared = waves * OPEN_LIST;
+  B.npool = (size_t)(waves * (OPEN_LIST + 16) + 65536);
+  A.pool_cap = B.npool;
+  A.unit_cap = (uint32_t)waves;
+  A.open_per = WAVE;
+  // The longest first while a long one is a large part of the whole (1.17M
+  // points 3.07 to 2.49 ms); with more points neighbours in space stay
+  // neighbours in time, which the caches gain from, and no place in a class is
+  // claimed (23.7M points, mostly ground: 31.8 to 29.8 ms).
+  const uint64_t resident = 20 * (uint64_t)c->ncu;
+  A.open_classes = nbatch || c->sharing || waves < 20 * resident;
+  if (A.open_classes) {
+    A.unit_cap = ucap;
+    // Lanes of a unit.  A unit of 16 takes more than a quarter of the time of
+    // one of 64 (lanes that need the same points share their tests), but with
+    // few units the longest one is the kernel.
+    const uint64_t all = nbatch ? nbatch / WAVE : waves;
+    A.open_per = 2 * all < resident ? OPEN_P1 : 3 * all < 4 * resident ? OPEN_P2 : WAVE;
+  }
+  B.nunit = (size_t)A.unit_cap * (A.open_classes ? OPEN_CLASSES : 1);
+  A.open = B.open = (HeavyRec *)wb_alloc(c, sizeof(HeavyRec) * B.nrec + 16);
+  A.open_unit = B.unit = (uint4 *)wb_alloc(c, sizeof(uint4) * B.nunit + 16);
+  A.pool = B.pool = (uint32_t *)wb_alloc(c, 4 * B.npool);
+}
+
+static void open_release(wb_ctx *c, OpenBuffers &B)
+{
+  wb_free(c, B.open, sizeof(HeavyRec) * B.nrec + 16);
+  wb_free(c, B.unit, sizeof(uint4) * B.nunit + 16);
+  wb_free(c, B.pool, 4 * B.npool);
 }
 
 static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double *corners,
                              int ncorners, const wb_classify_params *p, uint8_t *d_class_out,
-                             bool want_tiles, bool scan_only, ClassifyOut *out, bool counters)
+                             bool want_tiles, bool scan_only, uint64_t nbatch, ClassifyOut *out)
 {
   R.t = t; R.c = c; R.st = c->stream; R.p = p; R.d_class_out = d_class_out;
   R.want_tiles = want_tiles; R.scan_only = scan_only; R.out = out;
-  R.cls = nullptr; R.heavy = nullptr; R.dcount = nullptr; R.h_nheavy = 0; R.h_nslow = 0;
+  R.cls = nullptr; R.heavy = nullptr; R.h_nheavy = 0; R.h_nslow = 0;
   hipStream_t st = R.st;
   const uint64_t n = R.n = t->n;
   wb::SnakeSetup ss = wb::snake_setup_corners(corners, ncorners, p->tile_size);
@@ -2989,12 +3401,14 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
   // err[0] error flags; then u64 counters: 0 sector borderline, 1 exact atan2i
   // steps, 2-4 class histogram, 5 non-empty tiles, 6 (two u32) exact gap
   // points and heavy points, 7 FP64 fit fallbacks; u32 18-19 work counters of
-  // the heavy and resident ground kernels, 20-25 the scan's class list lengths
-  uint32_t *err = R.err = (uint32_t *)wb_alloc(c, 128);
+  // the heavy and resident ground kernels, 20-25 the scan's class list lengths;
+  // past the words the host reads: 32-37 walk B's units of each class, records
+  // and units taken, u64 at 38 its leaf list entries
+  uint32_t *err = R.err = (uint32_t *)wb_alloc(c, 256);
   unsigned long long *ctr = R.ctr = (unsigned long long *)err + 1;
   uint32_t *nslow = R.nslow = (uint32_t *)(ctr + 6);
   R.heavy_next = err + 18;
-  WB_CHECK(hipMemsetAsync(err, 0, 128, st));
+  WB_CHECK(hipMemsetAsync(err, 0, 256, st));
   WB_CHECK(hipMemsetAsync(tile_cnt, 0, 4ull * g.ntiles, st));
   WB_CHECK(hipMemsetAsync(tile_fill, 0, 4ull * g.ntiles, st));
   TreeView T = view(t);
@@ -3079,53 +3493,74 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
   A.items = nullptr;
   A.n_items = 0;
   A.item_cls = nullptr;
-  if (counters) {
-    R.dcount = (unsigned long long *)wb_alloc(c, CT_STRIDE * CT_COPIES * 8);
-    WB_CHECK(hipMemsetAsync(R.dcount, 0, CT_STRIDE * CT_COPIES * 8, st));
-  }
-  A.counters = R.dcount;
   R.heavy = (HeavyRec *)wb_alloc(c, sizeof(HeavyRec) * (n + 1));
   A.heavy = R.heavy;
+  open_buffers(c, A, n, nbatch, R.open);
+  A.nopen = err + 32;
+  A.open_next = err + 37;
+  A.npool = (unsigned long long *)(err + 38);
+  A.heavy_next = R.heavy_next;
   A.nheavy = nslow + 1;
 }
 
-// the ground test of one tree: the main kernel, then the heavy kernel for
-// the points it hands over
-static void classify_ground_single(ClassifyRun &R)
+// walk A, walk B and the heavy kernel over n work indices of A; ev (may be
+// null): events around the first two and around the heavy kernel
+static void launch_ground(wb_ctx *c, const ClassifyArgs &A, uint64_t n, uint32_t *resident_next,
+                          hipEvent_t *ev)
 {
-  hipStream_t st = R.st;
-  ClassifyArgs &A = R.A;
-  const bool count_work = R.dcount != nullptr;
-  WB_CHECK(hipEventRecord(R.ev[4], st));
-  if (R.n > 0) {
-    const uint32_t nb = wb_blocks(R.n, 256);
-    if (count_work)
-      hipLaunchKernelGGL((k_ground<true, WB_GROUND_MINW>), dim3(nb), dim3(256), 0, st, A);
-    else if (R.c->sharing)
-      // 4 of the 6 blocks a CU holds: a wave slot with 192 VGPRs and 2
-      // blocks' LDS stay free on every SIMD for other contexts' kernels
-      hipLaunchKernelGGL((k_ground_resident<WB_GROUND_MINW>),
-                         dim3(std::min<uint32_t>(nb, 4u * (uint32_t)R.c->ncu)), dim3(256), 0, st,
-                         A, R.err + 19);
-    else
-      hipLaunchKernelGGL((k_ground<false, WB_GROUND_MINW>), dim3(nb), dim3(256), 0, st, A);
+  hipStream_t st = c->stream;
+  const uint32_t ncu = (uint32_t)c->ncu;
+  if (ev) WB_CHECK(hipEventRecord(ev[0], st));
+  if (n > 0) {
+    const uint32_t nb = wb_blocks(n, WAVE);
+    const dim3 one(WAVE);
+    // sharing: 16 of the 20 waves a CU holds: a wave slot and LDS stay free on
+    // every SIMD for other contexts' kernels
+    const bool res = c->sharing && resident_next;
+    const dim3 rgrid(std::min<uint32_t>(nb, 16u * ncu));
+    if (A.cube_wedges) {
+      if (res)
+        hipLaunchKernelGGL((k_ground_resident<true, WB_GROUND_MINW>), rgrid, one, 0, st, A,
+                           resident_next);
+      else
+        hipLaunchKernelGGL((k_ground<true, WB_GROUND_MINW>), dim3(nb), one, 0, st, A);
+    } else {
+      if (res)
+        hipLaunchKernelGGL((k_ground_resident<false, WB_GROUND_MINW>), rgrid, one, 0, st, A,
+                           resident_next);
+      else
+        hipLaunchKernelGGL((k_ground<false, WB_GROUND_MINW>), dim3(nb), one, 0, st, A);
+    }
+    if (c->sharing) {  // 12 of the 20 waves a CU holds
+      const dim3 ogrid(std::min<uint32_t>(nb, 12u * ncu));
+      if (A.cube_wedges) hipLaunchKernelGGL(k_ground_open_resident<true>, ogrid, one, 0, st, A);
+      else hipLaunchKernelGGL(k_ground_open_resident<false>, ogrid, one, 0, st, A);
+    } else {
+      const dim3 ogrid(nb * (WAVE / A.open_per));
+      if (A.cube_wedges) hipLaunchKernelGGL(k_ground_open<true>, ogrid, one, 0, st, A);
+      else hipLaunchKernelGGL(k_ground_open<false>, ogrid, one, 0, st, A);
+    }
   }
-  WB_CHECK(hipEventRecord(R.ev[5], st));
-  WB_CHECK(hipEventRecord(R.ev[6], st));
-  if (R.n > 0) {
+  if (ev) {
+    WB_CHECK(hipEventRecord(ev[1], st));
+    WB_CHECK(hipEventRecord(ev[2], st));
+  }
+  if (n > 0) {
     // at most one block per handed-over point, and no more than fit on the
     // device at once; the count is read on the device
     // sharing: 8 blocks per CU, about half the LDS the kernel could hold
-    const unsigned nb = (unsigned)std::min<uint64_t>(
-        R.n, R.c->sharing ? 8ull * (uint64_t)R.c->ncu : (uint64_t)HEAVY_GRID);
-    if (count_work)
-      hipLaunchKernelGGL(k_ground_heavy<true>, dim3(nb), dim3(64), 0, st, A, R.heavy, A.nheavy,
-                         R.heavy_next);
-    else
-      hipLaunchKernelGGL(k_ground_heavy<false>, dim3(nb), dim3(64), 0, st, A, R.heavy, A.nheavy,
-                         R.heavy_next);
+    const unsigned nb =
+        (unsigned)std::min<uint64_t>(n, c->sharing ? 8ull * ncu : (uint64_t)HEAVY_GRID);
+    hipLaunchKernelGGL(k_ground_heavy, dim3(nb), dim3(64), 0, st, A, A.heavy, A.nheavy,
+                       A.heavy_next);
   }
-  WB_CHECK(hipEventRecord(R.ev[7], st));
+  if (ev) WB_CHECK(hipEventRecord(ev[3], st));
+}
+
+// the ground test of one tree
+static void classify_ground_single(ClassifyRun &R)
+{
+  launch_ground(R.c, R.A, R.n, R.err + 19, R.ev + 4);
 }
 
 static void classify_finish(ClassifyRun &R)
@@ -3141,7 +3576,7 @@ static void classify_finish(ClassifyRun &R)
   int32_t *memb = R.memb;
   uint32_t *nmemb = R.nmemb, *nslow = R.nslow, *err = R.err;
   TileRec *rec = R.rec;
-  unsigned long long *ctr = R.ctr, *dcount = R.dcount;
+  unsigned long long *ctr = R.ctr;
   uint8_t *cls = R.cls, *d_class_out = R.d_class_out;
   const ClassifyArgs &A = R.A;
   int32_t *nground = (int32_t *)R.tile_fill;  // reused once the lists are built
@@ -3177,8 +3612,8 @@ static void classify_finish(ClassifyRun &R)
         HeavyRec *iheavy = (HeavyRec *)wb_alloc(c, sizeof(HeavyRec) * (nitems + 1));
         // the pass's own counters: exact gap points, handed-over items,
         // emulated atan2i steps (the statistics keep the main pass's)
-        unsigned long long *ict = (unsigned long long *)wb_alloc(c, 32);
-        WB_CHECK(hipMemsetAsync(ict, 0, 32, st));
+        unsigned long long *ict = (unsigned long long *)wb_alloc(c, 64);
+        WB_CHECK(hipMemsetAsync(ict, 0, 64, st));
         hipLaunchKernelGGL(k_overlap_items, dim3(wb_blocks(n, 256)), dim3(256), 0, st, n, memb,
                            nmemb, rec, g.lo, off, items);
         ClassifyArgs B = A;
@@ -3189,19 +3624,21 @@ static void classify_finish(ClassifyRun &R)
         B.nslow = (uint32_t *)ict;
         B.nheavy = (uint32_t *)ict + 1;
         B.atan_exact = ict + 1;
-        B.counters = nullptr;
-        hipLaunchKernelGGL((k_ground<false, WB_GROUND_MINW>), dim3(wb_blocks(nitems, 256)),
-                           dim3(256), 0, st, B);
-        hipLaunchKernelGGL(k_ground_heavy<false>,
-                           dim3((unsigned)std::min<uint64_t>(nitems, HEAVY_GRID)), dim3(64), 0, st,
-                           B, iheavy, B.nheavy, (uint32_t *)ict + 4);
+        B.heavy_next = (uint32_t *)ict + 4;
+        B.nopen = (uint32_t *)ict + 5;
+        B.open_next = (uint32_t *)ict + 10;
+        B.npool = ict + 6;
+        OpenBuffers ib;
+        open_buffers(c, B, nitems, 0, ib);
+        launch_ground(c, B, nitems, nullptr, nullptr);
         hipLaunchKernelGGL(k_item_ground, dim3(wb_blocks(nitems, 256)), dim3(256), 0, st, nitems,
                            items, icls, nground);
         WB_CHECK(hipStreamSynchronize(st));
         wb_free(c, items, 8 * nitems);
         wb_free(c, icls, nitems + 16);
         wb_free(c, iheavy, sizeof(HeavyRec) * (nitems + 1));
-        wb_free(c, ict, 32);
+        wb_free(c, ict, 64);
+        open_release(c, ib);
       }
       wb_free(c, off, 4 * n + 4);
     }
@@ -3246,45 +3683,6 @@ static void classify_finish(ClassifyRun &R)
   out->nonempty = hc[5];
   out->fallbacks = hc[7];
   out->nslow = R.h_nslow;
-  if (dcount) {
-    std::vector<unsigned long long> hc((size_t)CT_STRIDE * CT_COPIES);
-    WB_CHECK(hipMemcpy(hc.data(), dcount, hc.size() * 8, hipMemcpyDeviceToHost));
-    unsigned long long h[CT_STRIDE] = {};
-    for (int k = 0; k < CT_STRIDE; k++)
-      for (int r = 0; r < CT_COPIES; r++) {
-        const unsigned long long v = hc[(size_t)r * CT_STRIDE + k];
-        h[k] = k == CT_TMAX ? std::max(h[k], v) : h[k] + v;
-      }
-    for (int s = 0; s < 3; s++)
-      fprintf(stderr,
-              "[wb counters] heavy from walk %c: points %llu passed %llu leaves %llu slots %llu "
-              "expansions %llu ticks %llu tested %llu inside %llu\n",
-              "ABC"[s], h[CT_N + 8 * s], h[CT_N + 8 * s + 1], h[CT_N + 8 * s + 2],
-              h[CT_N + 8 * s + 3], h[CT_N + 8 * s + 4], h[CT_N + 8 * s + 5],
-              h[CT_N + 8 * s + 6], h[CT_N + 8 * s + 7]);
-    fprintf(stderr,
-            "[wb counters] lanes A %llu B %llu open after B %llu heavy %llu | A: leaf-lanes %llu "
-            "group-lanes %llu dirs %llu | B: leaf-lanes %llu point-lanes %llu dirs %llu | per "
-            "wave: expansions A %llu leaves A %llu expansions B %llu leaves B %llu | waves %llu\n",
-            h[CT_LANES_A], h[CT_LANES_B], h[CT_LANES_C], h[CT_HEAVY], h[CT_LEAF_A], h[CT_GROUP_A],
-            h[CT_DIR_A], h[CT_LEAF_B], h[CT_POINT_B], h[CT_DIR_B], h[CT_EXP_A], h[CT_WLEAF_A],
-            h[CT_EXP_B], h[CT_WLEAF_B], h[CT_WAVES]);
-    fprintf(stderr,
-            "[wb counters] cycles: expansions A %llu leaves A %llu expansions B %llu leaves B "
-            "%llu wedge refresh %llu | leaves A: to bounds %llu to samples %llu loop %llu | wave "
-            "iterations: samples A %llu slots B %llu\n",
-            h[CT_CYC], h[CT_CYC + 1], h[CT_CYC + 2], h[CT_CYC + 3], h[CT_CYC + 4], h[CT_CYC + 5],
-            h[CT_CYC + 6], h[CT_CYC + 7], h[CT_ITER_A], h[CT_ITER_B]);
-    int rate = 0;
-    hipDeviceGetAttribute(&rate, hipDeviceAttributeWallClockRate, c->device);
-    fprintf(stderr,
-            "[wb counters] wave time: sum %llu max %llu ticks (rate %d kHz); hist counts %llu "
-            "%llu %llu %llu %llu ; hist tick sums %llu %llu %llu %llu %llu\n",
-            h[CT_TSUM], h[CT_TMAX], rate, h[CT_THIST], h[CT_THIST + 1], h[CT_THIST + 2],
-            h[CT_THIST + 3], h[CT_THIST + 4], h[CT_TSUMS], h[CT_TSUMS + 1], h[CT_TSUMS + 2],
-            h[CT_TSUMS + 3], h[CT_TSUMS + 4]);
-    wb_free(c, dcount, CT_STRIDE * CT_COPIES * 8);
-  }
   out->ms_tiles = ms1; out->ms_scan = ms2; out->ms_classify = ms3;
   wb_free(c, R.tile_cnt, 4ull * g.ntiles + 4);
   wb_free(c, R.tile_fill, 4ull * g.ntiles + 4);
@@ -3294,11 +3692,14 @@ static void classify_finish(ClassifyRun &R)
   wb_free(c, R.tile_off, 4ull * g.ntiles + 4);
   wb_free(c, R.lists, 4 * R.total + 4);
   if (cls) wb_free(c, cls, n + 16);
-  if (R.heavy) wb_free(c, R.heavy, sizeof(HeavyRec) * (n + 1));
+  if (R.heavy) {
+    wb_free(c, R.heavy, sizeof(HeavyRec) * (n + 1));
+    open_release(c, R.open);
+  }
   out->nheavy = R.h_nheavy;
-  if (h_err[0] & 1u) { wb_free(c, err, 128); throw std::string("a point lies in more than 4 tile cylinders"); }
-  if (h_err[0] & 2u) { wb_free(c, err, 128); throw std::string("a tile cylinder holds more than 1024 points"); }
-  wb_free(c, err, 128);
+  if (h_err[0] & 1u) { wb_free(c, err, 256); throw std::string("a point lies in more than 4 tile cylinders"); }
+  if (h_err[0] & 2u) { wb_free(c, err, 256); throw std::string("a tile cylinder holds more than 1024 points"); }
+  wb_free(c, err, 256);
 }
 
 void wb_run_classify(wb_tree *t, const double *corners, int ncorners,
@@ -3306,8 +3707,7 @@ void wb_run_classify(wb_tree *t, const double *corners, int ncorners,
                      bool scan_only, ClassifyOut *out)
 {
   ClassifyRun R;
-  classify_prepare(R, t, t->ctx, corners, ncorners, p, d_class_out, want_tiles, scan_only, out,
-                   !scan_only && classify_count_work());
+  classify_prepare(R, t, t->ctx, corners, ncorners, p, d_class_out, want_tiles, scan_only, 0, out);
   if (!scan_only) classify_ground_single(R);
   classify_finish(R);
 }
@@ -3318,45 +3718,60 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
 {
   hipStream_t st = c->stream;
   std::vector<ClassifyRun> R(ntrees);
+  uint64_t nbatch = 0;
+  for (int k = 0; k < ntrees; k++) nbatch += trees[k]->n;
   for (int k = 0; k < ntrees; k++)
     classify_prepare(R[k], trees[k], c, corners + 6 * k, 2, p, d_class_out[k], false, false,
-                     &outs[k], false);
-  // one launch of the ground kernel over every tree's points, then one of
-  // the heavy kernel over every tree's handed-over points
+                     nbatch, &outs[k]);
+  // one launch of walk A over every tree's points, one of walk B and one of
+  // the heavy kernel over what the trees' walks left; the counts stay on the
+  // device
   std::vector<ClassifyArgs> AA(ntrees);
-  std::vector<uint32_t> boff(ntrees + 1, 0), hoff(ntrees + 1, 0);
+  std::vector<uint32_t> boff(ntrees + 1, 0);
+  bool inside = true;  // every tree's points lie in their leaves' cubes
   for (int k = 0; k < ntrees; k++) {
     AA[k] = R[k].A;
-    const uint64_t nb = boff[k] + (uint64_t)wb_blocks(R[k].n, 256);
+    inside = inside && AA[k].cube_wedges;
+    const uint64_t nb = boff[k] + (uint64_t)wb_blocks(R[k].n, WAVE);
     if (nb > 0xffffffffull) throw std::string("too many points in one batch");
     boff[k + 1] = (uint32_t)nb;
   }
   ClassifyArgs *dAA = (ClassifyArgs *)wb_alloc(c, sizeof(ClassifyArgs) * ntrees);
-  uint32_t *doff = (uint32_t *)wb_alloc(c, 8 * (ntrees + 1));
+  uint32_t *doff = (uint32_t *)wb_alloc(c, 4 * (ntrees + 1));
+  const size_t nsum = (size_t)ntrees * OPEN_CLASSES + 1;
+  uint32_t *dsum = (uint32_t *)wb_alloc(c, 4 * nsum);
   WB_CHECK(hipMemcpyAsync(dAA, AA.data(), sizeof(ClassifyArgs) * ntrees, hipMemcpyHostToDevice, st));
   WB_CHECK(hipMemcpyAsync(doff, boff.data(), 4 * (ntrees + 1), hipMemcpyHostToDevice, st));
   for (int k = 0; k < ntrees; k++) WB_CHECK(hipEventRecord(R[k].ev[4], st));
-  if (boff[ntrees])
-    hipLaunchKernelGGL((k_ground_batch<WB_GROUND_MINW>), dim3(boff[ntrees]), dim3(256), 0, st, dAA,
-                       doff, ntrees);
+  if (boff[ntrees]) {
+    const dim3 one(WAVE), ogrid(boff[ntrees] * (WAVE / AA[0].open_per));
+    if (inside) {
+      hipLaunchKernelGGL((k_ground_batch<true, WB_GROUND_MINW>), dim3(boff[ntrees]), one, 0, st, dAA,
+                         doff, ntrees);
+      hipLaunchKernelGGL(k_batch_sums, dim3(1), one, 0, st, dAA, ntrees, 1, dsum);
+      hipLaunchKernelGGL(k_ground_open_batch<true>, ogrid, one, 0, st, dAA, dsum, ntrees);
+    } else {
+      hipLaunchKernelGGL((k_ground_batch<false, WB_GROUND_MINW>), dim3(boff[ntrees]), one, 0, st,
+                         dAA, doff, ntrees);
+      hipLaunchKernelGGL(k_batch_sums, dim3(1), one, 0, st, dAA, ntrees, 1, dsum);
+      hipLaunchKernelGGL(k_ground_open_batch<false>, ogrid, one, 0, st, dAA, dsum, ntrees);
+    }
+  }
   for (int k = 0; k < ntrees; k++) {
     WB_CHECK(hipEventRecord(R[k].ev[5], st));
-    WB_CHECK(hipMemcpyAsync(&R[k].h_nheavy, R[k].nslow + 1, 4, hipMemcpyDeviceToHost, st));
-  }
-  WB_CHECK(hipStreamSynchronize(st));
-  for (int k = 0; k < ntrees; k++) {
     WB_CHECK(hipEventRecord(R[k].ev[6], st));
-    hoff[k + 1] = hoff[k] + R[k].h_nheavy;
   }
-  if (hoff[ntrees]) {
-    uint32_t *dh = doff + ntrees + 1;
-    WB_CHECK(hipMemcpyAsync(dh, hoff.data(), 4 * (ntrees + 1), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_ground_heavy_batch, dim3(hoff[ntrees]), dim3(64), 0, st, dAA, dh,
-                       ntrees);
+  if (boff[ntrees]) {
+    hipLaunchKernelGGL(k_batch_sums, dim3(1), dim3(WAVE), 0, st, dAA, ntrees, 0, dsum);
+    hipLaunchKernelGGL(k_ground_heavy_batch,
+                       dim3((uint32_t)std::min<uint64_t>((uint64_t)boff[ntrees] * WAVE, HEAVY_GRID)),
+                       dim3(64), 0, st, dAA, dsum, ntrees);
   }
   for (int k = 0; k < ntrees; k++) WB_CHECK(hipEventRecord(R[k].ev[7], st));
+  // (the arguments' host copy is read until here)
   WB_CHECK(hipStreamSynchronize(st));
   wb_free(c, dAA, sizeof(ClassifyArgs) * ntrees);
-  wb_free(c, doff, 8 * (ntrees + 1));
+  wb_free(c, doff, 4 * (ntrees + 1));
+  wb_free(c, dsum, 4 * nsum);
   for (int k = 0; k < ntrees; k++) classify_finish(R[k]);
 }

@@ -64,6 +64,46 @@ int wbh_wedge_hit(uint64_t occ, double px, double py, double x0, double x1, doub
   return wb::wedge_hit(w, px, py, x0, x1, y0, y1) ? 1 : 0;
 }
 
+// a lane's wedges (at most two) of a direction mask: bit 0 the box test, bit 1
+// the test of the direction of the box's first corner
+int wbh_lane_wedges(uint64_t occ, double px, double py, double x0, double x1, double y0, double y1)
+{
+  static float tab[3 * 128];
+  static int filled;
+  if (!filled) {
+    wb::fill_edge_table(tab);
+    filled = 1;
+  }
+  wb::LaneWedges w;
+  wb::lane_wedges_update(occ, tab, w);
+  return (wb::lane_hit(w, px, py, x0, x1, y0, y1) ? 1 : 0) |
+         (wb::lane_dir(w, (float)(x0 - px), (float)(y0 - py)) ? 2 : 0);
+}
+
+// bit 0: hyp_in; bit 1: hyp_near reaches its threshold
+int wbh_hyp_near(const double *p, const double *q)
+{
+  const wb::Shape s = wb::make_hyperboloid(p[0], p[1], p[2], p[3], p[4]);
+  const double s2 = (s.slope * s.slope) * wb::kNearShrink;
+  const double t = wb::hyp_near(s2, q[0] - s.cx, q[1] - s.cy, s.cz - q[2]);
+  return (wb::hyp_in(s, q[0], q[1], q[2]) ? 1 : 0) | (t >= s.por2 * wb::kNearShrink ? 2 : 0);
+}
+
+// the float path's bin and position, and atan2i's position
+int wbh_dir_est(double dy, double dx, float *pos, double *exact)
+{
+  ready();
+  bool sure;
+  const int b = wb::dir_bin_est(dy, dx, &sure, pos);
+  const int a = wb::atan2i(dy, dx, (const double *)g_tan, (const double *)g_cos,
+                           (const double *)g_sin, g_k);
+  *exact = (double)(((uint32_t)a + 0x40000000u) & 0x7fffffffu) * 0x1p-25;
+  return sure ? b : -1;
+}
+
+float wbh_rel_down(double v, double o, double side) { return wb::rel_down(v, o, side); }
+float wbh_rel_up(double v, double o, double side) { return wb::rel_up(v, o, side); }
+
 // the border wedges of the runs of >= 24 bins of occ (before/after as the
 // exact pass finds them) and the box test against them
 int wbh_border_wedge_hit(uint64_t occ, double px, double py, double x0, double x1, double y0,

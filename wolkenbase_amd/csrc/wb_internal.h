@@ -13,6 +13,9 @@
 //                                 equal z)
 //   chunk_sx/sy/sz[ceil(n/32)] f64 that point's coordinates (the ground
 //                                 test's samples, read coalesced per leaf)
+//   oct_xy[4*ceil(n/32)] f32x4, oct_z f32  x0, x1, y0, y1 and lowest z of each
+//                                 8-slot octet from the root cube's centre,
+//                                 rounded outwards
 //   leaf_start[nl+1] u32, leaf_cube[nl] f64x4 (cx,cy,cz,side), leaf_parent[nl]
 //   node_cube[nn] f64x4, node_child[8*nn] i32 (>=0 node, -2-l leaf, -1 empty),
 //   node_crange[8*nn] u32x2 (slot range of each leaf child; 0,0 otherwise),
@@ -34,6 +37,7 @@
 #define WB_RECORDS 537  // octree.h:40-41: a leaf holds at most 537 locations
 #define WB_MAX_LEVEL 21
 #define WB_CHUNK 32
+#define WB_OCT 8  // slots per octet box (the ground test's walk B)
 #define WB_HBOX_WORDS 1024
 // word offsets of the pinned host words of each use
 #define WB_HBOX_SCAN 0     // wb_exclusive_scan_u32: total (2 words)
@@ -118,6 +122,9 @@ struct wb_tree {
   double *chunk_box;
   uint32_t *chunk_low;
   double *chunk_sx, *chunk_sy, *chunk_sz;
+  float4 *oct_xy;
+  float *oct_z;
+  float *leaf_low;  // per leaf, at most the lowest z stored in it
   uint32_t *leaf_start;
   double *leaf_cube;
   int32_t *leaf_parent;

@@ -425,40 +425,51 @@ WB_HD int atan2i_ext(double y, double x, const double *tab_tan, const double *ta
   return (int)(uint32_t)r;
 }
 
+// the float path: the bin, where *sure is set; *pos is then within
+// DIR_MARGIN of atan2i's position on the circle, in bins
+WB_HD int dir_bin_est(double dy, double dx, bool *sure, float *pos = nullptr)
+{
+  const float fx = (float)dx, fy = (float)dy;
+  const float ax = fabsf(fx), ay = fabsf(fy);
+  const float mx = fmaxf(ax, ay), mn = fminf(ax, ay);
+#ifdef __HIP_DEVICE_COMPILE__
+  const float t = mn * __builtin_amdgcn_rcpf(mx);
+#else
+  const float t = mn / mx;
+#endif
+  const float u = t * t;
+  float p = 0.006811794359236956f;
+  p = fmaf(p, u, -0.033604223281145096f);
+  p = fmaf(p, u, 0.07962367683649063f);
+  p = fmaf(p, u, -0.1323334276676178f);
+  p = fmaf(p, u, 0.19807815551757812f);
+  p = fmaf(p, u, -0.3331736922264099f);
+  p = fmaf(p, u, 0.9999961256980896f);
+  const float s = (p * t) * 10.185916357881302f;  // 32/pi
+  const float fl = floorf(s);
+  const float fr = s - fl;  // exact
+  // mx in [2^-100, 2^100]: both conversions normal or t below the margin
+  // (a NaN fails a compare and takes atan2i)
+  *sure = (fr > DIR_MARGIN) & (fr < 1.0f - DIR_MARGIN) & (s < 8.0f) & (mx >= 0x1p-100f) &
+          (mx <= 0x1p100f);
+  const uint32_t ux = __builtin_bit_cast(uint32_t, fx), uy = __builtin_bit_cast(uint32_t, fy);
+  int b = (int)fl;
+  if (ay > ax) b ^= 15;
+  if ((ux ^ uy) >> 31) b ^= 31;
+  if (pos) {
+    float q = ay > ax ? 16.0f - s : s;
+    if ((ux ^ uy) >> 31) q = 32.0f - q;
+    *pos = q + (fy > 0 ? 32.0f : 0.0f);
+  }
+  return b + (fy > 0 ? 32 : 0);
+}
+
 WB_HD int dir_bin(double dy, double dx, const double *tab_tan, const double *tab_cos,
                   const double *tab_sin, const AtanConst &K, int *exact_used = nullptr)
 {
-  {
-    const float fx = (float)dx, fy = (float)dy;
-    const float ax = fabsf(fx), ay = fabsf(fy);
-    const float mx = fmaxf(ax, ay), mn = fminf(ax, ay);
-#ifdef __HIP_DEVICE_COMPILE__
-    const float t = mn * __builtin_amdgcn_rcpf(mx);
-#else
-    const float t = mn / mx;
-#endif
-    const float u = t * t;
-    float p = 0.006811794359236956f;
-    p = fmaf(p, u, -0.033604223281145096f);
-    p = fmaf(p, u, 0.07962367683649063f);
-    p = fmaf(p, u, -0.1323334276676178f);
-    p = fmaf(p, u, 0.19807815551757812f);
-    p = fmaf(p, u, -0.3331736922264099f);
-    p = fmaf(p, u, 0.9999961256980896f);
-    const float s = (p * t) * 10.185916357881302f;  // 32/pi
-    const float fl = floorf(s);
-    const float fr = s - fl;  // exact
-    // mx in [2^-100, 2^100]: both conversions normal or t below the margin
-    // (a NaN fails a compare and takes atan2i)
-    if (fr > DIR_MARGIN && fr < 1.0f - DIR_MARGIN && s < 8.0f && mx >= 0x1p-100f &&
-        mx <= 0x1p100f) {
-      const uint32_t ux = __builtin_bit_cast(uint32_t, fx), uy = __builtin_bit_cast(uint32_t, fy);
-      int b = (int)fl;
-      if (ay > ax) b ^= 15;
-      if ((ux ^ uy) >> 31) b ^= 31;
-      return b + (fy > 0 ? 32 : 0);
-    }
-  }
+  bool sure;
+  const int b = dir_bin_est(dy, dx, &sure);
+  if (__builtin_expect(sure, 1)) return b;
   const int a = atan2i_ext(dy, dx, tab_tan, tab_cos, tab_sin, K, exact_used);
   return (int)((((uint32_t)a + 0x40000000u) & 0x7fffffffu) >> 25);
 }
@@ -497,7 +508,7 @@ WB_HD int scan_sector(double vx, double vy, double r, int *edge)
   const double rr = r / kScanSqrt7;
   const double a = kScanSqrt3 * dabs(vy), b = dabs(vx), m = 1e-9 * (a + b);
   const double q2 = vx * vx + vy * vy, t2 = rr * rr;
-  if ((dabs(a - b) > m) & (b > m) & (dabs(q2 - t2) > 1e-12 * t2)) {
+  if (__builtin_expect((dabs(a - b) > m) & (b > m) & (dabs(q2 - t2) > 1e-12 * t2), 1)) {
     *edge = 0;
     if (q2 < t2) return 0;
     if (a < b) return vx > 0 ? 1 : 4;
@@ -600,7 +611,7 @@ WB_HD bool hyp_in(const Shape &s, double qx, double qy, double qz)
   const double d = (a - b) - s.por2;
   const double m = 0x1p-44 * (a + b);
   bool in = side & (d > m);
-  if (side & !(d > m) & !(d < -m)) in = hyp_in_tail(dx, dy, a, s.slope, s.por2);
+  if (__builtin_expect(side & !(d > m) & !(d < -m), 0)) in = hyp_in_tail(dx, dy, a, s.slope, s.por2);
   return in;
 }
 
@@ -659,6 +670,34 @@ WB_HD bool shape_may_hit_box(const Shape &s, double x0, double x1, double y0, do
   else if (s.kind == SHAPE_HYPERBOLOID) qz = s.slope > 0 ? z0 : z1;
   else qz = z0;
   return shape_in(s, qx, qy, qz);
+}
+
+// v - o as a float at most (rel_down) or at least (rel_up) the exact
+// difference, by a slack above the rounding of any other difference from o
+// that is taken in double (|v - o| up to a few times `side`): the octet boxes,
+// which only prune.
+WB_HD float rel_down(double v, double o, double side)
+{
+  const double d = v - o;
+  const double r = d - dabs(d) * 0x1p-22 - side * 0x1p-40;
+  return r > 3e38 ? 3e38f : r < -3e38 ? -__builtin_inff() : (float)r;
+}
+WB_HD float rel_up(double v, double o, double side) { return -rel_down(-v, -o, side); }
+
+// The conservative form of hyp_in (slope > 0): with s2 = slope^2 * kNearShrink
+// and dx, dy the differences to the axis and dz = cz - qz, hyp_near is at
+// least por2 * kNearShrink at every point hyp_in takes.  hyp_in takes q only
+// when dz > 0 and, up to 2^-43 of a + b in rounding (hypot's tail included),
+// a - b >= por2, where a = dz^2 and b = slope^2 (dx^2 + dy^2).  With
+// e = 2^-40, a - b(1 - e) then reaches por2(1 - e) whatever the roundings of
+// hyp_near's own products (2^-50 of a + b): b <= a there, so the slack needed
+// is at most 2^-41 a, and either por2 or b is at least a/4 (e times it covers
+// the slack) or a - b is above twice por2.  Five FP64 operations and a
+// compare on the differences, against about seventeen for hyp_in.
+constexpr double kNearShrink = 1.0 - 0x1p-40;
+WB_HD double hyp_near(double s2, double dx, double dy, double dz)
+{
+  return __builtin_fma(-s2, __builtin_fma(dy, dy, dx * dx), dz * __builtin_fabs(dz));
 }
 
 // The three tests above for a shape known to be a hyperboloid (the same
@@ -876,15 +915,63 @@ WB_HD bool wedge_hit2(int n, const float ax[2], const float ay[2], const float b
 {
   if (n < 0) return true;
   bool hit = false;
+  // the largest value of each cross product over the box: at its middle, plus
+  // the half widths times the edge's components (rounding within 10^-6 of
+  // the offsets, against the wedges' 10^-3 rad)
+  const float uc = 0.5f * (u0 + u1), vc = 0.5f * (v0 + v1), uh = 0.5f * (u1 - u0),
+              vh = 0.5f * (v1 - v0);
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const float ra = ax[k] * (ax[k] > 0 ? v1 : v0) - ay[k] * (ay[k] > 0 ? u0 : u1);
-    const float lb = (by[k] > 0 ? u1 : u0) * by[k] - (bx[k] > 0 ? v0 : v1) * bx[k];
+    const float ra = fmaf(ax[k], vc, fmaf(-ay[k], uc, fmaf(fabsf(ax[k]), vh, fabsf(ay[k]) * uh)));
+    const float lb = fmaf(uc, by[k], fmaf(-vc, bx[k], fmaf(fabsf(by[k]), uh, fabsf(bx[k]) * vh)));
     const bool in_k = !(ra < 0) & !(lb < 0);
     hit |= k < n ? in_k : false;
   }
   return hit;
 }
 
+// A lane's care wedges: those of care_wedges, at most two; a lane with
+// more (two runs, one of them 32 bins or more) is not pruned (n < 0).  n: 0
+// none, 1 one run, 2 one run split in two, 3 two runs (two wedges).
+struct LaneWedges {
+  float ax[2], ay[2], bx[2], by[2];
+  int n;
+};
+
+WB_HD void lane_wedges_update(uint64_t occ, const float *edges, LaneWedges &W)
+{
+  Wedges w;
+  care_wedges(occ, w, edges);
+  // live is 1, 3 (one run, split) or 5 (two runs) when at most two are in use;
+  // the second kept wedge is slot 1 or slot 2
+  const int n = w.live < 0 ? -1 : __builtin_popcount(w.live);
+  const bool s1 = (w.live & 2) != 0;
+  W.ax[0] = w.ax[0]; W.ay[0] = w.ay[0];
+  W.bx[0] = w.bx[0]; W.by[0] = w.by[0];
+  W.ax[1] = s1 ? w.ax[1] : w.ax[2]; W.ay[1] = s1 ? w.ay[1] : w.ay[2];
+  W.bx[1] = s1 ? w.bx[1] : w.bx[2]; W.by[1] = s1 ? w.by[1] : w.by[2];
+  W.n = n < 0 || n > 2 ? -1 : n == 2 && !s1 ? 3 : n;
+}
+
+// wedge_hit against the lane's wedges
+WB_HD bool lane_hit(const LaneWedges &W, double px, double py, double x0, double x1,
+                                double y0, double y1)
+{
+  return wedge_hit2(W.n, W.ax, W.ay, W.bx, W.by, (float)(x0 - px), (float)(x1 - px),
+                        (float)(y0 - py), (float)(y1 - py));
+}
+
+// false only if the direction (u, v) lies outside the lane's care run: its
+// bin is then occupied or in an empty run of fewer than 24 bins, and the runs
+// of 24 or more come out the same without it.  One run is tested whole, from
+// its first edge to its last, narrower or wider than pi; a lane without
+// wedges or with two runs takes every direction.
+WB_HD bool lane_dir(const LaneWedges &W, float u, float v)
+{
+  const bool wide = W.n == 2;
+  const float bx = wide ? W.bx[1] : W.bx[0], by = wide ? W.by[1] : W.by[0];
+  const bool ra = !(W.ax[0] * v - W.ay[0] * u < 0), lb = !(u * by - v * bx < 0);
+  return (W.n < 0) | (W.n == 3) | (wide & (ra | lb)) | ((W.n == 1) & ra & lb);
+}
 
 }  // namespace wb
