@@ -440,3 +440,40 @@ def test_classify_long_leaf_lists_match_oracle(ctx, slope, min_hs):
         assert np.array_equal(got, want)
     finally:
         tree.free()
+
+
+@pytest.mark.parametrize("kind", [W.WB_SHAPE_CYLINDER, W.WB_SHAPE_SPHERE, W.WB_SHAPE_HYPERBOLOID])
+def test_queries_of_few_and_many_leaves_match_oracle(ctx, kind):
+    # shapes cutting from one leaf to all of a tree of uneven depth (a cluster
+    # of 1500 points in a few millimetres): a walk's stack past its wide part,
+    # leaf batches of under, over and about 64; a batch of a wave per shape and
+    # the same shapes in one large enough for a lane each
+    cloud = synth.generate(seed=51, extent=60.0, density=25.0, outliers=0.02)
+    rng = np.random.default_rng(51 + kind)
+    n = len(cloud["xi"])
+    for k, r in (("xi", 4), ("yi", 4), ("zi", 1)):
+        v = cloud[k].copy()
+        v[n // 2:n // 2 + 1500] = v[n // 2] + rng.integers(-r, r + 1, 1500)
+        cloud[k] = v
+    tree, ref, (x, y, z) = build_both(ctx, cloud)
+    P = random_shapes(rng, x, y, z, kind, 90)
+    at = {W.WB_SHAPE_CYLINDER: 2, W.WB_SHAPE_SPHERE: 3, W.WB_SHAPE_HYPERBOLOID: 3}[kind]
+    i = n // 2
+    for k, r in enumerate(np.geomspace(0.001, 60.0, 40)):
+        P[k, :2] = x[i] + r * 0.3, y[i]
+        if kind != W.WB_SHAPE_CYLINDER:
+            P[k, 2] = z[i] + (0.1 * r if kind == W.WB_SHAPE_SPHERE else r)
+        P[k, at] = r if kind != W.WB_SHAPE_HYPERBOLOID else 0.001
+    counts = tree.count_points_in((kind, P))
+    lists = tree.points_in((kind, P))
+    for s in range(len(P)):
+        assert counts[s] == ref.count_points_in(kind, P[s]), (s, P[s])
+        assert np.array_equal(lists[s].astype(np.int64), ref.points_in(kind, P[s])), (s, P[s])
+    few = np.flatnonzero(counts < 40)
+    assert len(few) > 0 and counts.max() > n // 2
+    many = np.tile(P[few], (200000 // len(few), 1))
+    got = tree.points_in((kind, many))
+    for s in list(range(len(few))) + list(rng.integers(0, len(many), 200)):
+        assert np.array_equal(got[s], lists[few[s % len(few)]])
+    many = np.tile(P, (400000 // len(P), 1))
+    assert np.array_equal(tree.count_points_in((kind, many)), np.tile(counts, 400000 // len(P)))

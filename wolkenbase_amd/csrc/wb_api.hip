@@ -473,10 +473,17 @@ int wb_tree_order(wb_tree *t, uint32_t *order)
 
 static int check_kind(int kind) { return kind == WB_SHAPE_CYLINDER || kind == WB_SHAPE_SPHERE || kind == WB_SHAPE_HYPERBOLOID; }
 
-// Batches of up to this many shapes take a wave per shape in the caller's
-// order: one wave would hold them all in the lane-per-shape kernel, and
-// ordering them first would cost more launches than the query.
-#define WB_QUERY_SORT_MIN 65
+// Batches of fewer shapes take a wave per shape in the caller's order; the
+// others a lane per shape, sorted so that the 64 of a wave share one walk.
+// The sort and the longest of those walks (each as long as 64 shapes') cost
+// about 0.4 to 1 ms whatever the number, a wave per shape 2.4 to 3.6 ns a
+// shape counted and 4 to 7 ns listed.  1 m spheres at points of 1.15M and 20M
+// points, wave and lane per shape, ms: counted, 65k 0.17 and 0.42, 0.22 and
+// 1.09; 262k 0.64 and 0.69, 0.84 and 1.06; 1M 2.4 and 1.1, 3.2 and 1.5.
+// Counted and listed: 65k 0.46 and 0.91, 0.59 and 2.3; 262k 1.7 and 1.3, 2.3
+// and 2.0.  Small batches gain most: 4096 cylinders of 0.877 m 0.035 and 1.5.
+#define WB_QUERY_SORT_MIN 393216
+#define WB_QUERY_SORT_MIN_LIST 196608
 
 // Events around a query's kernels on the context stream; ms() after the
 // stream has passed the second one.
@@ -504,6 +511,23 @@ int wb_count_points_in(wb_tree *t, int kind, const double *params, uint64_t ns, 
   if (ns == 0) return WB_OK;
   API_TRY(c)
   size_t pb = sizeof(double) * WB_SHAPE_NPARAMS * ns;
+  if (ns <= WB_HBOX_SHAPES) {
+    // the kernel reads the shapes from pinned host memory and writes the
+    // counts there: two copies fewer (the whole call on
+    // 16 spheres of 1 m 85 to 28 us, of which the walk gives about 45)
+    double *hp = (double *)(c->hbox + WB_HBOX_QUERY);
+    uint64_t *hc = (uint64_t *)(hp + WB_SHAPE_NPARAMS * WB_HBOX_SHAPES);
+    memcpy(hp, params, pb);
+    QueryTimer qt(c);
+    qt.start();
+    wb_run_count(t, kind, hp, ns, hc, nullptr);
+    qt.stop();
+    WB_CHECK(hipStreamSynchronize(c->stream));
+    memcpy(counts, hc, 8 * ns);
+    t->ms_query_count = qt.ms();
+    t->ms_query_points = 0;
+    return WB_OK;
+  }
   double *dp = (double *)wb_alloc(c, pb);
   uint64_t *dc = (uint64_t *)wb_alloc(c, 8 * ns);
   WB_CHECK(hipMemcpyAsync(dp, params, pb, hipMemcpyHostToDevice, c->stream));
@@ -567,7 +591,7 @@ int wb_points_in(wb_tree *t, int kind, const double *params, uint64_t ns, uint64
   WB_CHECK(hipMemcpyAsync(dp, params, pb, hipMemcpyHostToDevice, c->stream));
   QueryTimer qt(c);
   qt.start();
-  uint32_t *order = ns >= WB_QUERY_SORT_MIN ? wb_query_order(t, kind, dp, ns) : nullptr;
+  uint32_t *order = ns >= (idx ? WB_QUERY_SORT_MIN_LIST : WB_QUERY_SORT_MIN) ? wb_query_order(t, kind, dp, ns) : nullptr;
   wb_run_count(t, kind, dp, ns, dc, order);
   qt.stop();
   std::vector<uint64_t> cnt(ns);

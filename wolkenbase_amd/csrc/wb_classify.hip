@@ -103,115 +103,304 @@ static TreeView view(const wb_tree *t)
 }
 
 // ---------------------------------------------------------------------------
-// Octree::findBlocks (octree.cpp:234-251) without a stack: the next child
-// to visit at each depth is kept in 4-bit fields of two registers and the
-// walk goes back up through parent links.  Leaves are visited in DFS order.
-// f(leaf) returns true to stop the walk.
+// Batched countPointsIn / pointsIn: one wave per shape.  The walk expands up
+// to eight nodes of its stack per round, lane 8i+k testing child k of the
+// i-th node from the top; the children that pass take the nodes' places in
+// the order of the lanes, so the stack holds leaves and nodes in DFS order
+// (octree.cpp:234-251) from its top down, and leaves come off it in that
+// order.  They are served in batches of up to 64.
+// What bounds it: the latency of a round's loads (child links and the nodes'
+// cubes, read together) and of a batch's, at about 20 waves per CU.
 // ---------------------------------------------------------------------------
-struct Iter {
-  uint64_t lo, hi;
-  __device__ int get(int d) const { return d < 16 ? (int)((lo >> (4 * d)) & 15) : (int)((hi >> (4 * (d - 16))) & 15); }
-  __device__ void set(int d, int v)
-  {
-    if (d < 16) lo = (lo & ~(15ull << (4 * d))) | ((uint64_t)v << (4 * d));
-    else hi = (hi & ~(15ull << (4 * (d - 16)))) | ((uint64_t)v << (4 * (d - 16)));
-  }
+// Entries a wave's stack holds.  A round takes up to eight nodes while that
+// leaves room for what one node per round (the plain depth-first walk: at
+// most 7 waiting entries per level and 8 children) can still add.
+#define WB_WSTK 512
+#define WB_WSTK_WIDE (WB_WSTK - 8 * 8 - 7 * (WB_MAX_LEVEL + 1) - 8)
+struct ShapeWalk {
+  int stk[WB_WSTK];
+  int leaf[2 * WAVE];
+  uint32_t pre[WAVE], b[WAVE], e[WAVE], mask[WAVE];
 };
 
-template <class F>
-__device__ inline void for_leaves(const TreeView &T, const wb::Shape &S, F &&f)
+template <int KIND>
+__device__ inline wb::Shape query_shape(const double *p)
 {
-  if (T.nleaves == 0) return;
-  if (!wb::shape_intersect(S, T.node_cube[0], T.node_cube[1], T.node_cube[2], T.node_cube[3])) return;
-  int node = 0, depth = 0;
-  Iter it = {0, 0};
-  for (;;) {
-    int c = it.get(depth);
-    if (c == 8) {
-      if (depth == 0) return;
-      node = T.node_parent[node];
-      depth--;
-      continue;
-    }
-    it.set(depth, c + 1);
-    int ch = T.node_child[8 * node + c];
-    if (ch == -1) continue;
-    if (ch >= 0) {
-      const double *q = T.node_cube + 4 * ch;
-      if (wb::shape_intersect(S, q[0], q[1], q[2], q[3])) {
-        node = ch;
-        depth++;
-        it.set(depth, 0);
-      }
-      continue;
-    }
-    int leaf = -2 - ch;
-    const double *q = T.leaf_cube + 4 * leaf;
-    if (!wb::shape_intersect(S, q[0], q[1], q[2], q[3])) continue;
-    if (f(leaf)) return;
-  }
-}
-
-__device__ inline wb::Shape make_shape(int kind, const double *p)
-{
-  if (kind == wb::SHAPE_CYLINDER) return wb::make_cylinder(p[0], p[1], p[2]);
-  if (kind == wb::SHAPE_SPHERE) return wb::make_sphere(p[0], p[1], p[2], p[3]);
+  if (KIND == wb::SHAPE_CYLINDER) return wb::make_cylinder(p[0], p[1], p[2]);
+  if (KIND == wb::SHAPE_SPHERE) return wb::make_sphere(p[0], p[1], p[2], p[3]);
   return wb::make_hyperboloid(p[0], p[1], p[2], p[3], p[4]);
 }
 
-// ---------------------------------------------------------------------------
-// Batched countPointsIn / pointsIn: one wave per shape, lanes split a leaf.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_count_points_in(TreeView T, int kind, const double *params,
-                                                        uint64_t nshapes, uint64_t *counts)
+// Octree::cube (octree.cpp:349-358) of child k of the cube (cx, cy, cz, side):
+// the operations the build used for the stored cubes
+__device__ inline void child_cube(double cx, double cy, double cz, double side, int k,
+                                  double &x, double &y, double &z, double &sd)
 {
-  uint64_t s = blockIdx.x;
-  if (s >= nshapes) return;
-  wb::Shape S = make_shape(kind, params + WB_SHAPE_NPARAMS * s);
-  uint64_t cnt = 0;
-  for_leaves(T, S, [&](int leaf) {
-    const double *q = T.leaf_cube + 4 * leaf;
-    uint32_t b = T.leaf_start[leaf], e = T.leaf_start[leaf + 1];
-    if (wb::shape_in_cube(S, q[0], q[1], q[2], q[3])) {
-      cnt += e - b;
-      return false;
-    }
-    for (uint32_t j0 = b; j0 < e; j0 += WAVE) {
-      uint32_t j = j0 + threadIdx.x;
-      bool in = j < e && wb::shape_in(S, T.px[j], T.py[j], T.pz[j]);
-      cnt += __popcll(__ballot(in));
-    }
-    return false;
-  });
-  if (threadIdx.x == 0) counts[s] = cnt;
+  x = cx + (double)(2 * (k & 1) - 1) * side / 4;
+  y = cy + (double)(2 * ((k >> 1) & 1) - 1) * side / 4;
+  z = cz + (double)(2 * (k >> 2) - 1) * side / 4;
+  sd = side / 2;
 }
 
-__global__ void __launch_bounds__(64) k_points_in(TreeView T, int kind, const double *params,
+// serve(nb): the leaves K.leaf[0 .. nb) (nb <= 64), in DFS order
+template <class Serve>
+__device__ inline void shape_walk(const TreeView &T, const wb::Shape &S, ShapeWalk &K,
+                                  Serve &&serve)
+{
+  if (T.nleaves == 0) return;
+  if (!wb::shape_intersect(S, T.node_cube[0], T.node_cube[1], T.node_cube[2], T.node_cube[3]))
+    return;
+  const int lane = threadIdx.x;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  if (lane == 0) K.stk[0] = 0;
+  int sp = 1, nb = 0;
+  while (sp > 0) {
+    __syncthreads();
+    const bool have = lane < sp;
+    const int code = have ? K.stk[sp - 1 - lane] : 0;
+    const uint64_t isleaf = __ballot(have && code < 0), isnode = __ballot(have && code >= 0);
+    // the leaves above the first node
+    const int nl = isnode ? __builtin_ctzll(isnode) : __popcll(isleaf);
+    if (lane < nl) K.leaf[nb + lane] = -2 - code;
+    nb += nl;
+    sp -= nl;
+    if (isnode) {
+      // the nodes down to the next leaf
+      const uint64_t rest = ~(isnode >> nl);
+      int run = rest ? __builtin_ctzll(rest) : WAVE;
+      run = sp > WB_WSTK_WIDE ? 1 : run < 8 ? run : 8;
+      const bool on = (lane >> 3) < run;
+      int ch = -1;
+      bool hit = false;
+      if (on) {
+        const int nd = K.stk[sp - 1 - (lane >> 3)];
+        const double *nc = T.node_cube + 4 * (size_t)nd;
+        ch = T.node_child[8 * (size_t)nd + (lane & 7)];
+        double x, y, z, sd;
+        child_cube(nc[0], nc[1], nc[2], nc[3], lane & 7, x, y, z, sd);
+        hit = ch != -1 && wb::shape_intersect(S, x, y, z, sd);
+      }
+      const uint64_t hits = __ballot(hit);
+      sp += __popcll(hits) - run;
+      __syncthreads();
+      if (hit) K.stk[sp - 1 - __popcll(hits & lt)] = ch;
+    }
+    while (nb >= WAVE || (sp == 0 && nb > 0)) {
+      __syncthreads();
+      serve(nb < WAVE ? nb : WAVE);
+      nb = nb < WAVE ? 0 : nb - WAVE;
+      __syncthreads();
+      const int left = K.leaf[WAVE + lane];
+      __syncthreads();
+      K.leaf[lane] = left;
+    }
+  }
+}
+
+// exclusive running sum over the wave's lanes, and the total
+__device__ inline uint32_t wave_prefix(uint32_t v, uint32_t &total)
+{
+  const int lane = threadIdx.x;
+  uint32_t s = v;
+#pragma unroll
+  for (int d = 1; d < WAVE; d <<= 1) {
+    const uint32_t w = __shfl_up(s, d, WAVE);
+    if (lane >= d) s += w;
+  }
+  total = (uint32_t)__builtin_amdgcn_readlane((int)s, 63);
+  return s - v;
+}
+
+// the last of pre[0..nb) (ascending from 0) that is at most t
+__device__ inline int prefix_find(const uint32_t *pre, int nb, uint32_t t)
+{
+  int lo = 0;
+#pragma unroll
+  for (int d = WAVE / 2; d > 0; d >>= 1)
+    if (lo + d < nb && pre[lo + d] <= t) lo += d;
+  return lo;
+}
+
+// The 32-point groups of the leaves K.b..K.e (K.pre: running sums of their
+// numbers, tot in all), 64 at a time, a lane each: f(q, g, hit) with the leaf,
+// the group and whether the shape may reach its box.
+template <class F>
+__device__ inline void leaf_groups(const TreeView &T, const wb::Shape &S, const ShapeWalk &K,
+                                   int nb, uint32_t tot, F &&f)
+{
+  for (uint32_t t0 = 0; t0 < tot; t0 += WAVE) {
+    const uint32_t t = t0 + threadIdx.x;
+    bool hit = false;
+    int q = 0;
+    uint32_t g = 0;
+    if (t < tot) {
+      q = prefix_find(K.pre, nb, t);
+      g = K.b[q] / WB_CHUNK + (t - K.pre[q]);
+      const double *bx = T.chunk_box + 6 * (size_t)g;
+      hit = wb::shape_may_hit_box(S, bx[0], bx[1], bx[2], bx[3], bx[4], bx[5]);
+    }
+    f(q, g, hit);
+  }
+}
+
+// countPointsIn of shape blockIdx.x.  A leaf whose corners are all in the
+// shape counts whole (octree.cpp:1226-1231, 1256-1257); of the others the
+// groups whose box the shape may reach are read, four per step.
+template <int KIND>
+__global__ void __launch_bounds__(64) k_count_points_in(TreeView T, const double *params,
+                                                        uint64_t nshapes, uint64_t *counts)
+{
+  __shared__ ShapeWalk K;
+  const uint64_t s = blockIdx.x;
+  if (s >= nshapes) return;
+  const int lane = threadIdx.x;
+  const wb::Shape S = query_shape<KIND>(params + WB_SHAPE_NPARAMS * s);
+  uint64_t cnt = 0;  // this lane's share
+  shape_walk(T, S, K, [&](int nb) {
+    uint32_t b = 0, e = 0, ng = 0;
+    if (lane < nb) {
+      const int l = K.leaf[lane];
+      const double *lc = T.leaf_cube + 4 * (size_t)l;
+      b = T.leaf_start[l];
+      e = T.leaf_start[l + 1];
+      if (wb::shape_in_cube(S, lc[0], lc[1], lc[2], lc[3])) cnt += e - b;
+      else if (e > b) ng = (e - 1) / WB_CHUNK - b / WB_CHUNK + 1;
+    }
+    uint32_t tot;
+    K.pre[lane] = wave_prefix(ng, tot);
+    K.b[lane] = b;
+    K.e[lane] = e;
+    __syncthreads();
+    leaf_groups(T, S, K, nb, tot, [&](int q, uint32_t g, bool hit) {
+      const uint32_t gb = K.b[q], ge = K.e[q];
+      uint64_t own = __ballot(hit);
+      while (own) {
+        // four groups per step, two loads in flight per lane
+        uint32_t j[2];
+        bool ok[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const bool any = own != 0;
+          const int o1 = any ? __builtin_ctzll(own) : 0;
+          own &= own - 1;
+          const bool two = own != 0;
+          const int o2 = two ? __builtin_ctzll(own) : o1;
+          own &= own - 1;
+          const int o = lane < 32 ? o1 : o2;
+          const uint32_t gg = (uint32_t)__shfl((int)g, o, WAVE);
+          const uint32_t bb = (uint32_t)__shfl((int)gb, o, WAVE);
+          const uint32_t ee = (uint32_t)__shfl((int)ge, o, WAVE);
+          j[u] = gg * WB_CHUNK + (lane & 31);
+          ok[u] = (lane < 32 ? any : two) && j[u] >= bb && j[u] < ee;
+          if (!ok[u]) j[u] = bb;
+        }
+        double x[2], y[2], z[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          x[u] = T.px[j[u]];
+          y[u] = T.py[j[u]];
+          z[u] = T.pz[j[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) cnt += ok[u] && wb::shape_in(S, x[u], y[u], z[u]);
+      }
+    });
+    __syncthreads();
+  });
+  for (int d = WAVE / 2; d > 0; d >>= 1) cnt += __shfl_xor(cnt, d, WAVE);
+  if (lane == 0) counts[s] = cnt;
+}
+
+// pointsIn of shape blockIdx.x: its input indices from offs[s] on, leaf by
+// leaf in DFS order and in canonical (input) order inside a leaf.  The leaves
+// of a batch that lie whole in the shape or have a group the shape may reach
+// are read as one sequence, four points per lane and step; of a leaf not whole
+// in the shape only the points of such groups are tested.
+template <int KIND>
+__global__ void __launch_bounds__(64) k_points_in(TreeView T, const double *params,
                                                   uint64_t nshapes, const uint64_t *offs,
                                                   uint32_t *out)
 {
-  uint64_t s = blockIdx.x;
+  __shared__ ShapeWalk K;
+  const uint64_t s = blockIdx.x;
   if (s >= nshapes) return;
-  wb::Shape S = make_shape(kind, params + WB_SHAPE_NPARAMS * s);
+  const int lane = threadIdx.x;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  const wb::Shape S = query_shape<KIND>(params + WB_SHAPE_NPARAMS * s);
+  // the writes stay inside the shape's own range whatever the walk finds
   uint64_t pos = offs[s];
-  const uint64_t lanelt = (1ull << __lane_id()) - 1ull;
-  for_leaves(T, S, [&](int leaf) {
-    const double *q = T.leaf_cube + 4 * leaf;
-    uint32_t b = T.leaf_start[leaf], e = T.leaf_start[leaf + 1];
-    bool all = wb::shape_in_cube(S, q[0], q[1], q[2], q[3]);
-    for (uint32_t j0 = b; j0 < e; j0 += WAVE) {
-      uint32_t c = j0 + threadIdx.x;  // canonical position
-      bool in = false;
-      uint32_t slot = 0;
-      if (c < e) {
-        slot = T.canon[c];
-        in = all || wb::shape_in(S, T.px[slot], T.py[slot], T.pz[slot]);
-      }
-      uint64_t bal = __ballot(in);
-      if (in) out[pos + __popcll(bal & lanelt)] = T.sidx[slot];
-      pos += __popcll(bal);
+  const uint64_t lim = offs[s + 1];
+  shape_walk(T, S, K, [&](int nb) {
+    uint32_t b = 0, e = 0, ng = 0;
+    bool all = false, wide = false;
+    if (lane < nb) {
+      const int l = K.leaf[lane];
+      const double *lc = T.leaf_cube + 4 * (size_t)l;
+      b = T.leaf_start[l];
+      e = T.leaf_start[l + 1];
+      all = wb::shape_in_cube(S, lc[0], lc[1], lc[2], lc[3]);
+      if (!all && e > b) ng = (e - 1) / WB_CHUNK - b / WB_CHUNK + 1;
+      // a leaf of at most 537 points spans at most 18 groups; a longer one is
+      // not pruned
+      wide = ng > 32;
+      if (wide) ng = 0;
     }
-    return false;
+    uint32_t tot;
+    K.pre[lane] = wave_prefix(ng, tot);
+    K.b[lane] = b;
+    K.e[lane] = e;
+    K.mask[lane] = wide ? ~0u : 0u;
+    __syncthreads();
+    leaf_groups(T, S, K, nb, tot, [&](int q, uint32_t g, bool hit) {
+      if (hit) atomicOr(&K.mask[q], 1u << (g - K.b[q] / WB_CHUNK));
+    });
+    __syncthreads();
+    // K.e: first group of a leaf whose points are tested, all ones for whole
+    const uint32_t np = all || K.mask[lane] ? e - b : 0u;
+    K.pre[lane] = wave_prefix(np, tot);
+    const uint32_t g0 = all ? ~0u : wide ? ~0u - 1 : b / WB_CHUNK;
+    K.e[lane] = g0;
+    __syncthreads();
+    constexpr int U = 4;
+    for (uint32_t t0 = 0; t0 < tot; t0 += U * WAVE) {
+      uint32_t slot[U];
+      int q[U];
+      bool in[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint32_t t = t0 + u * WAVE + lane;
+        in[u] = t < tot;
+        q[u] = prefix_find(K.pre, nb, in[u] ? t : 0u);
+        slot[u] = in[u] ? T.canon[K.b[q[u]] + (t - K.pre[q[u]])] : 0u;
+      }
+      double x[U], y[U], z[U];
+      bool test[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint32_t gq = K.e[q[u]];
+        test[u] = in[u] && gq != ~0u;
+        if (test[u] && gq != ~0u - 1) test[u] = in[u] = (K.mask[q[u]] >> (slot[u] / WB_CHUNK - gq)) & 1u;
+        if (test[u]) {
+          x[u] = T.px[slot[u]];
+          y[u] = T.py[slot[u]];
+          z[u] = T.pz[slot[u]];
+        }
+      }
+      uint32_t id[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (test[u]) in[u] = wb::shape_in(S, x[u], y[u], z[u]);
+        if (in[u]) id[u] = T.sidx[slot[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint64_t bal = __ballot(in[u]);
+        const uint64_t w = pos + (uint64_t)__popcll(bal & lt);
+        if (in[u] && w < lim) out[w] = id[u];
+        pos += (uint64_t)__popcll(bal);
+      }
+    }
+    __syncthreads();
   });
 }
 
@@ -237,25 +426,6 @@ struct QueryStack {
   int code[WB_QSTK];
   uint32_t lo[WB_QSTK], hi[WB_QSTK];
 };
-
-template <int KIND>
-__device__ inline wb::Shape query_shape(const double *p)
-{
-  if (KIND == wb::SHAPE_CYLINDER) return wb::make_cylinder(p[0], p[1], p[2]);
-  if (KIND == wb::SHAPE_SPHERE) return wb::make_sphere(p[0], p[1], p[2], p[3]);
-  return wb::make_hyperboloid(p[0], p[1], p[2], p[3], p[4]);
-}
-
-// Octree::cube (octree.cpp:349-358) of child k of the cube (cx, cy, cz, side):
-// the operations the build used for the stored cubes
-__device__ inline void child_cube(double cx, double cy, double cz, double side, int k,
-                                  double &x, double &y, double &z, double &sd)
-{
-  x = cx + (double)(2 * (k & 1) - 1) * side / 4;
-  y = cy + (double)(2 * ((k >> 1) & 1) - 1) * side / 4;
-  z = cz + (double)(2 * (k >> 2) - 1) * side / 4;
-  sd = side / 2;
-}
 
 // The walk: leaf(l, on) for every leaf some lane reaches, in DFS order; `on`
 // tells whether this lane's findBlocks returns it.
@@ -3212,8 +3382,13 @@ void wb_run_count(wb_tree *t, int kind, const double *dparams, uint64_t ns, uint
   if (ns == 0) return;
   hipStream_t st = t->ctx->stream;
   if (!order) {
-    hipLaunchKernelGGL(k_count_points_in, dim3((unsigned)ns), dim3(64), 0, st, view(t), kind,
-                       dparams, ns, dcounts);
+    const dim3 grid((unsigned)ns), blk(WAVE);
+    if (kind == wb::SHAPE_CYLINDER)
+      hipLaunchKernelGGL(k_count_points_in<wb::SHAPE_CYLINDER>, grid, blk, 0, st, view(t), dparams, ns, dcounts);
+    else if (kind == wb::SHAPE_SPHERE)
+      hipLaunchKernelGGL(k_count_points_in<wb::SHAPE_SPHERE>, grid, blk, 0, st, view(t), dparams, ns, dcounts);
+    else
+      hipLaunchKernelGGL(k_count_points_in<wb::SHAPE_HYPERBOLOID>, grid, blk, 0, st, view(t), dparams, ns, dcounts);
     return;
   }
   const dim3 grid(wb_blocks(ns, 256)), blk(256);
@@ -3234,8 +3409,13 @@ void wb_run_points(wb_tree *t, int kind, const double *dparams, uint64_t ns, con
   if (ns == 0) return;
   hipStream_t st = t->ctx->stream;
   if (!order) {
-    hipLaunchKernelGGL(k_points_in, dim3((unsigned)ns), dim3(64), 0, st, view(t), kind, dparams,
-                       ns, doffs, dout);
+    const dim3 grid((unsigned)ns), blk(WAVE);
+    if (kind == wb::SHAPE_CYLINDER)
+      hipLaunchKernelGGL(k_points_in<wb::SHAPE_CYLINDER>, grid, blk, 0, st, view(t), dparams, ns, doffs, dout);
+    else if (kind == wb::SHAPE_SPHERE)
+      hipLaunchKernelGGL(k_points_in<wb::SHAPE_SPHERE>, grid, blk, 0, st, view(t), dparams, ns, doffs, dout);
+    else
+      hipLaunchKernelGGL(k_points_in<wb::SHAPE_HYPERBOLOID>, grid, blk, 0, st, view(t), dparams, ns, doffs, dout);
     return;
   }
   const dim3 grid(wb_blocks(ns, 256)), blk(256);

@@ -43,7 +43,8 @@
 #define WB_HBOX_SCAN 0     // wb_exclusive_scan_u32: total (2 words)
 #define WB_HBOX_GEO 16     // tile grid bounds (4 words)
 #define WB_HBOX_ERR 32     // classification flags and counters (32 words)
-#define WB_HBOX_BATCH 64   // batch classification: heavy counts per tree
+#define WB_HBOX_QUERY 64   // a few shapes' parameters and counts
+#define WB_HBOX_SHAPES 64  // as many
 #define WB_GEO_CACHE 4
 
 struct wb_stream_alloc;
