@@ -477,3 +477,58 @@ def test_queries_of_few_and_many_leaves_match_oracle(ctx, kind):
         assert np.array_equal(got[s], lists[few[s % len(few)]])
     many = np.tile(P, (400000 // len(P), 1))
     assert np.array_equal(tree.count_points_in((kind, many)), np.tile(counts, 400000 // len(P)))
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 1024, 4095, 4096, 4097, 65535, 65537, 70001])
+def test_build_sizes_at_block_edges_match_oracle(ctx, n):
+    # word, scan, sort and leaf-mark tile edges; a third of the points given
+    # again and merged (a scan over all inputs)
+    rng = np.random.default_rng(n)
+    cloud = synth.generate(seed=71, extent=70.0, density=25.0)
+    for k in ("xi", "yi", "zi"):
+        cloud[k] = cloud[k][:n].copy()
+    assert len(cloud["xi"]) == n
+    _, keep = np.unique(np.stack([cloud[k] for k in ("xi", "yi", "zi")], 1), axis=0,
+                        return_index=True)
+    keep = np.sort(keep)
+    for k in ("xi", "yi", "zi"):
+        cloud[k] = cloud[k][keep]
+    tree, ref, _ = build_both(ctx, cloud)
+    assert np.array_equal(tree.leaves()["count"], ref.leaves()["count"])
+    assert np.array_equal(tree.leaves()["center"], ref.leaves()["center"])
+    assert np.array_equal(tree.order().astype(np.int64), ref.order())
+    m = len(keep)
+    again = rng.permutation(m)[:n // 3]
+    xi, yi, zi = (np.concatenate([cloud[k], cloud[k][again]]) for k in ("xi", "yi", "zi"))
+    center, side = W.Octree.size_fit(cloud["bbmin"], cloud["bbmax"])
+    t2 = W.Octree.build(ctx, xi, yi, zi, cloud["scale"], cloud["offset"], center, side, dedupe=True)
+    assert t2.ndup == len(again)
+    assert np.array_equal(t2.order().astype(np.int64), ref.order())
+    pairs = t2.duplicates()
+    pairs = pairs[np.argsort(pairs[:, 0])]
+    assert np.array_equal(pairs[:, 0], m + np.arange(len(again)))
+    assert np.array_equal(pairs[:, 1], again)
+
+
+def test_merge_of_a_scan_of_many_tiles(ctx):
+    # more values than the scan's blocks add up directly (8192 tiles of 4096):
+    # 34M locations, 1000 of them given again
+    n0 = 34_000_000
+    i = np.arange(n0, dtype=np.int64)
+    xi, yi = (i % 5831).astype(np.int32), (i // 5831).astype(np.int32)
+    zi = ((i * 2654435761) >> 7 & 0xff).astype(np.int32)
+    again = (np.arange(1000, dtype=np.int64) * 33_999) % n0
+    xi, yi, zi = (np.concatenate([a, a[again]]) for a in (xi, yi, zi))
+    center, side = W.Octree.size_fit([0.0, 0.0, 0.0], [58.4, 58.4, 2.6])
+    tree = W.Octree.build(ctx, xi, yi, zi, [0.01] * 3, [0.0] * 3, center, side, dedupe=True)
+    try:
+        assert tree.ndup == 1000
+        pairs = tree.duplicates()
+        pairs = pairs[np.argsort(pairs[:, 0])]
+        assert np.array_equal(pairs[:, 0], n0 + np.arange(1000))
+        assert np.array_equal(pairs[:, 1], again)
+        leaves = tree.leaves()
+        assert leaves["count"].sum() == n0 and leaves["count"].max() <= 537
+        assert np.array_equal(leaves["first"], np.cumsum(leaves["count"]) - leaves["count"])
+    finally:
+        tree.free()

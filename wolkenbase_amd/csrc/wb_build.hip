@@ -9,7 +9,6 @@
 // z*4+y*2+x), and the DFS visits children 0..7, so DFS order is ascending
 // order of the Morton key built from those compare bits.
 #include "wb_internal.h"
-#include "wb_wave.h"
 
 #include <string.h>
 
@@ -54,110 +53,122 @@ __device__ inline uint32_t block_excl_scan256(uint32_t v, uint32_t *total)
 }
 
 // ---------------------------------------------------------------------------
-// device-wide exclusive scan (u32), 1024 elements per block
+// device-wide exclusive scan (u32), SCAN_TILE elements per block
 // ---------------------------------------------------------------------------
-__global__ void k_scan_reduce(const uint32_t *in, uint64_t n, uint32_t *bsum)
+// Two launches: the tiles' sums, then every block adds up the sums of the
+// tiles before its own (a read of at most SCAN_FLAT words from the L2) and
+// scans its tile.  A scan of the sums by one block between the two would be a
+// third dependent launch, and over all values in one block (the form for up
+// to 65536 values before) 65536 values took 110 us on one CU against 6 us.
+#define SCAN_TILE 4096
+#define SCAN_FLAT 8192
+
+// the thread's 16 consecutive values of the block's tile, 0 past n
+__device__ inline void scan_load(const uint32_t *in, uint64_t n, uint32_t (&v)[16])
 {
-  uint64_t base = (uint64_t)blockIdx.x * 1024;
-  uint32_t s = 0;
-  for (int k = 0; k < 4; k++) {
-    uint64_t i = base + threadIdx.x * 4 + k;
-    if (i < n) s += in[i];
+  const uint64_t i = (uint64_t)blockIdx.x * SCAN_TILE + threadIdx.x * 16;
+  if (i + 16 <= n && ((uintptr_t)in & 15) == 0) {
+    const uint4 *q = (const uint4 *)(in + i);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint4 w = q[k];
+      v[4 * k] = w.x;
+      v[4 * k + 1] = w.y;
+      v[4 * k + 2] = w.z;
+      v[4 * k + 3] = w.w;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 16; k++) v[k] = i + k < n ? in[i + k] : 0u;
   }
-  uint32_t tot;
+}
+
+__global__ void __launch_bounds__(256) k_scan_reduce(const uint32_t *in, uint64_t n, uint32_t *bsum)
+{
+  uint32_t v[16], s = 0, tot;
+  scan_load(in, n, v);
+#pragma unroll
+  for (int k = 0; k < 16; k++) s += v[k];
   block_excl_scan256(s, &tot);
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ void k_scan_down(uint32_t *data, uint64_t n, const uint32_t *boff)
+// boff: the tiles' sums, or with scanned their exclusive scan; total (null or
+// two host words): the sum of all values, written by the last block
+__global__ void __launch_bounds__(256) k_scan_down(uint32_t *data, uint64_t n, const uint32_t *boff,
+                                                   int scanned, uint32_t *total)
 {
-  uint64_t base = (uint64_t)blockIdx.x * 1024;
-  uint32_t v[4], s = 0;
-  for (int k = 0; k < 4; k++) {
-    uint64_t i = base + threadIdx.x * 4 + k;
-    v[k] = (i < n) ? data[i] : 0;
-    s += v[k];
+  uint32_t v[16], s = 0, tot, off = 0;
+  scan_load(data, n, v);
+#pragma unroll
+  for (int k = 0; k < 16; k++) s += v[k];
+  if (scanned) {
+    off = boff[blockIdx.x];
+  } else if (gridDim.x > 1) {
+    for (uint32_t k = threadIdx.x; k < blockIdx.x; k += 256) off += boff[k];
+    uint32_t all;
+    block_excl_scan256(off, &all);
+    off = all;
   }
-  uint32_t tot;
-  uint32_t ex = block_excl_scan256(s, &tot) + boff[blockIdx.x];
-  for (int k = 0; k < 4; k++) {
-    uint64_t i = base + threadIdx.x * 4 + k;
-    if (i < n) data[i] = ex;
-    ex += v[k];
+  uint32_t ex = block_excl_scan256(s, &tot) + off;
+  const uint64_t i = (uint64_t)blockIdx.x * SCAN_TILE + threadIdx.x * 16;
+  if (total && i < n && i + 16 >= n) {
+    uint64_t t = ex;
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (i + k + 1 < n) t = (uint32_t)(t + v[k]);
+      else if (i + k + 1 == n) t += v[k];
+    total[0] = (uint32_t)t;
+    total[1] = (uint32_t)(t >> 32);
   }
-}
-
-// exclusive scan of n <= SCAN1_MAX values by one block of 1024 threads, each
-// taking a run of consecutive values (the block sums of a larger scan)
-#define SCAN1_MAX 65536
-__global__ void __launch_bounds__(1024) k_scan_one(uint32_t *data, uint32_t n)
-{
-  __shared__ uint32_t wsum[16];
-  const uint32_t per = (n + 1023) / 1024, b = threadIdx.x * per;
-  uint32_t s = 0;
-  for (uint32_t k = 0; k < per; k++)
-    if (b + k < n) s += data[b + k];
-  uint32_t inc = s;  // inclusive scan within the wave
-  for (int d = 1; d < WAVE; d <<= 1) {
-    const uint32_t o = __shfl_up(inc, d, WAVE);
-    if ((int)lane_id() >= d) inc += o;
-  }
-  const int w = threadIdx.x / WAVE;
-  if ((int)lane_id() == WAVE - 1) wsum[w] = inc;
-  __syncthreads();
-  uint32_t off = 0;
-  for (int k = 0; k < w; k++) off += wsum[k];
-  uint32_t ex = off + inc - s;
-  for (uint32_t k = 0; k < per; k++)
-    if (b + k < n) {
-      const uint32_t v = data[b + k];
-      data[b + k] = ex;
-      ex += v;
+  if (i + 16 <= n && ((uintptr_t)data & 15) == 0) {
+    uint4 *q = (uint4 *)(data + i);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      uint4 w;
+      w.x = ex;
+      w.y = w.x + v[4 * k];
+      w.z = w.y + v[4 * k + 1];
+      w.w = w.z + v[4 * k + 2];
+      ex = w.w + v[4 * k + 3];
+      q[k] = w;
     }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      if (i + k < n) data[i + k] = ex;
+      ex += v[k];
+    }
+  }
 }
 
-static void scan_rec(wb_ctx *c, uint32_t *data, uint64_t n)
+static void scan_rec(wb_ctx *c, uint32_t *data, uint64_t n, uint32_t *total)
 {
-  if (n <= SCAN1_MAX) {
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, c->stream, data, (uint32_t)n);
-    return;
+  const unsigned nb = wb_blocks(n, SCAN_TILE);
+  uint32_t *bs = nullptr;
+  if (nb > 1) {
+    bs = (uint32_t *)wb_alloc(c, sizeof(uint32_t) * nb);
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, c->stream, data, n, bs);
+    if (nb > SCAN_FLAT) scan_rec(c, bs, nb, nullptr);
   }
-  unsigned nb = wb_blocks(n, 1024);
-  uint32_t *bs = (uint32_t *)wb_alloc(c, sizeof(uint32_t) * (nb + 1));
-  hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, c->stream, data, n, bs);
-  scan_rec(c, bs, nb);
-  hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(256), 0, c->stream, data, n, bs);
-  wb_free(c, bs, sizeof(uint32_t) * (nb + 1));
-}
-
-// total = the last element before the scan + the last after it, written by
-// the device into the context's pinned words
-__global__ void k_scan_total(const uint32_t *last_in, const uint32_t *last_out, uint32_t *host)
-{
-  if (threadIdx.x == 0) {
-    const uint64_t t = (uint64_t)*last_in + *last_out;
-    host[0] = (uint32_t)t;
-    host[1] = (uint32_t)(t >> 32);
-  }
+  hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(256), 0, c->stream, data, n, bs,
+                     nb > SCAN_FLAT ? 1 : 0, total);
+  wb_free(c, bs, sizeof(uint32_t) * nb);
 }
 
 uint64_t wb_exclusive_scan_u32(wb_ctx *c, uint32_t *data, uint64_t n)
 {
   if (n == 0) return 0;
-  uint32_t *keep = (uint32_t *)wb_alloc(c, 4);
-  WB_CHECK(hipMemcpyAsync(keep, data + n - 1, 4, hipMemcpyDeviceToDevice, c->stream));
-  scan_rec(c, data, n);
   uint32_t *h = c->hbox + WB_HBOX_SCAN;
-  hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, c->stream, keep, data + n - 1, h);
+  scan_rec(c, data, n, h);
   WB_CHECK(hipStreamSynchronize(c->stream));
-  wb_free(c, keep, 4);
   return (uint64_t)h[0] | ((uint64_t)h[1] << 32);
 }
 
 // ---------------------------------------------------------------------------
-// LSD radix sort, 8-bit digits.  Per pass: per-block digit histograms in LDS,
-// a device-wide exclusive scan of the digit-major histogram table, then a
-// stable scatter in which each wave ranks its keys with 8 ballots (peer
+// LSD radix sort, 8-bit digits.  Per pass: per-block digit histograms in LDS;
+// a block per digit scans that digit's row of the digit-major table and leaves
+// its total; then a stable scatter in which each wave ranks its keys with 8 ballots (peer
 // mask of equal digits) and one LDS atomic per distinct digit per round.
 // The block's keys are then placed in LDS in digit order, and consecutive
 // threads write each digit's run to its consecutive output slots, so every
@@ -175,6 +186,7 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const K *keys, uint64_t 
   h[threadIdx.x] = 0;
   __syncthreads();
   uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
+#pragma unroll
   for (int k = 0; k < RS_ITEMS; k++) {
     uint64_t i = base + (uint64_t)k * RS_THREADS + threadIdx.x;
     if (i < n) atomicAdd(&h[(unsigned)(keys[i] >> shift) & 255u], 1u);
@@ -183,11 +195,34 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const K *keys, uint64_t 
   hist[(uint64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
+// row d = blockIdx.x of the table: its exclusive scan, and its sum to tot[d]
+__global__ void __launch_bounds__(RS_THREADS) k_rs_rows(uint32_t *hist, unsigned nblocks,
+                                                        uint32_t *tot)
+{
+  uint32_t *row = hist + (uint64_t)blockIdx.x * nblocks;
+  uint32_t run = 0;
+  for (unsigned b = 0; b < nblocks; b += 4 * RS_THREADS) {
+    const unsigned i = b + 4 * threadIdx.x;
+    uint32_t v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = i + k < nblocks ? row[i + k] : 0u;
+    uint32_t all;
+    uint32_t ex = run + block_excl_scan256(v[0] + v[1] + v[2] + v[3], &all);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (i + k < nblocks) row[i + k] = ex;
+      ex += v[k];
+    }
+    run += all;
+  }
+  if (threadIdx.x == 0) tot[blockIdx.x] = run;
+}
+
 template <typename K>
 __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K *kin, const uint32_t *vin,
                                                              K *kout, uint32_t *vout, uint64_t n,
                                                              int shift, const uint32_t *offs,
-                                                             unsigned nblocks)
+                                                             const uint32_t *tot, unsigned nblocks)
 {
   __shared__ uint32_t wcnt[4][256];
   __shared__ uint32_t dstart[256];
@@ -197,13 +232,18 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K *kin, const u
   const int w = threadIdx.x / WAVE;
   const unsigned lane = lane_id();
   for (int d = threadIdx.x; d < 4 * 256; d += RS_THREADS) (&wcnt[0][0])[d] = 0;
-  for (int d = threadIdx.x; d < 256; d += RS_THREADS) dbase[d] = offs[(uint64_t)d * nblocks + blockIdx.x];
+  {
+    uint32_t all;
+    const uint32_t first = block_excl_scan256(tot[threadIdx.x], &all);
+    dbase[threadIdx.x] = first + offs[(uint64_t)threadIdx.x * nblocks + blockIdx.x];
+  }
   __syncthreads();
   const uint64_t base = (uint64_t)blockIdx.x * RS_TILE + (uint64_t)w * (RS_TILE / 4);
   K key[RS_ITEMS];
   uint32_t val[RS_ITEMS];
   uint32_t rank[RS_ITEMS];
   uint32_t dig[RS_ITEMS];
+#pragma unroll
   for (int r = 0; r < RS_ITEMS; r++) {
     uint64_t i = base + (uint64_t)r * WAVE + lane;
     bool ok = i < n;
@@ -249,6 +289,7 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K *kin, const u
     wcnt[3][d] = a0 + a1 + a2;
   }
   __syncthreads();
+#pragma unroll
   for (int r = 0; r < RS_ITEMS; r++) {
     uint64_t i = base + (uint64_t)r * WAVE + lane;
     if (i >= n) continue;
@@ -274,20 +315,21 @@ static void radix_sort_impl(wb_ctx *c, K *key, uint32_t *val, uint64_t n, int fi
                             int passes)
 {
   if (n <= 1 || passes <= 0) return;
-  unsigned nb = wb_blocks(n, RS_TILE);
-  uint64_t hsz = (uint64_t)nb * 256;
-  uint32_t *hist = (uint32_t *)wb_alloc(c, sizeof(uint32_t) * hsz);
+  const unsigned nb = wb_blocks(n, RS_TILE);
+  const uint64_t hsz = (uint64_t)nb * 256;
+  uint32_t *hist = (uint32_t *)wb_alloc(c, sizeof(uint32_t) * (hsz + 256));
+  uint32_t *tot = hist + hsz;
   K *k2 = (K *)wb_alloc(c, sizeof(K) * n);
   uint32_t *v2 = (uint32_t *)wb_alloc(c, sizeof(uint32_t) * n);
   K *ka = key, *kb = k2;
   uint32_t *va = val, *vb = v2;
   for (int p = 0; p < passes; p++) {
     int shift = first_shift + 8 * p;
-    hipLaunchKernelGGL(k_rs_hist<K>, dim3(nb), dim3(RS_THREADS), 0, c->stream, ka, n, shift, hist,
-                       nb);
-    scan_rec(c, hist, hsz);
-    hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nb), dim3(RS_THREADS), 0, c->stream, ka, va, kb, vb,
-                       n, shift, hist, nb);
+    hipLaunchKernelGGL(k_rs_hist<K>, dim3(nb), dim3(RS_THREADS), 0, c->stream, ka, n, shift,
+                       hist, nb);
+    hipLaunchKernelGGL(k_rs_rows, dim3(256), dim3(RS_THREADS), 0, c->stream, hist, nb, tot);
+    hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nb), dim3(RS_THREADS), 0, c->stream, ka, va, kb,
+                       vb, n, shift, hist, tot, nb);
     std::swap(ka, kb);
     std::swap(va, vb);
   }
@@ -295,7 +337,7 @@ static void radix_sort_impl(wb_ctx *c, K *key, uint32_t *val, uint64_t n, int fi
     WB_CHECK(hipMemcpyAsync(key, ka, sizeof(K) * n, hipMemcpyDeviceToDevice, c->stream));
     WB_CHECK(hipMemcpyAsync(val, va, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, c->stream));
   }
-  wb_free(c, hist, sizeof(uint32_t) * hsz);
+  wb_free(c, hist, sizeof(uint32_t) * (hsz + 256));
   wb_free(c, k2, sizeof(K) * n);
   wb_free(c, v2, sizeof(uint32_t) * n);
 }
@@ -308,11 +350,6 @@ void wb_radix_sort_pairs(wb_ctx *c, uint64_t *key, uint32_t *val, uint64_t n, in
 void wb_radix_sort_u32_prefix(wb_ctx *c, uint32_t *key, uint32_t *val, uint64_t n, int passes)
 {
   radix_sort_impl<uint32_t>(c, key, val, n, 32 - 8 * passes, passes);
-}
-
-void wb_radix_sort_u32_pairs(wb_ctx *c, uint32_t *key, uint32_t *val, uint64_t n)
-{
-  radix_sort_impl<uint32_t>(c, key, val, n, 0, 4);
 }
 
 // ---------------------------------------------------------------------------
@@ -440,8 +477,37 @@ struct LeafTmp {
 };
 
 struct SplitOut {
-  uint32_t n_next, n_leaf, n_node, overflow, maxdepth;
+  uint32_t outside, n_leaf, n_node, overflow, maxdepth;
 };
+
+// What a build attempt starts from: the root as node 0 and the only active
+// node, empty counters, and no slot marked as a leaf's first.
+__global__ void __launch_bounds__(256) k_build_init(uint32_t n, double cx, double cy, double cz,
+                                                    double side, double *node_cube,
+                                                    int32_t *node_child, int32_t *node_parent,
+                                                    SplitOut *out, Active *act, uint32_t *cnt,
+                                                    uint32_t *bits, uint32_t nwords)
+{
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < nwords) bits[i] = 0;
+  if (i < 8) node_child[i] = -1;
+  if (i < WB_MAX_LEVEL + 2) cnt[i] = i == 0 && n > 0;
+  if (i == 0) {
+    node_cube[0] = cx;
+    node_cube[1] = cy;
+    node_cube[2] = cz;
+    node_cube[3] = side;
+    node_parent[0] = -1;
+    act[0] = Active{0u, n, 0, 0};
+    *out = SplitOut{0u, 0u, 1u, 0u, 0u};
+  }
+}
+
+// slots from which a leaf starts, one bit each
+__device__ inline void mark_leaf(uint32_t *bits, uint32_t start)
+{
+  atomicOr(bits + start / 32, 1u << (start % 32));
+}
 
 // the level-`level` digit of a key whose top bit is bit 8*sizeof(K)-1
 template <typename K>
@@ -466,7 +532,8 @@ __global__ void k_split_level_t(const K *key, const Active *act, const uint32_t 
                               uint32_t act_cap, int level, int max_level, Active *next,
                               uint32_t *next_cnt, uint32_t next_cap, LeafTmp *leaves,
                               uint32_t leaf_cap, double *node_cube, int32_t *node_child,
-                              int32_t *node_parent, uint32_t node_cap, SplitOut *out)
+                              int32_t *node_parent, uint32_t node_cap, SplitOut *out,
+                              uint32_t *bits)
 {
   if (out->overflow) return;
   const uint32_t nact = min(*act_cnt, act_cap);
@@ -539,6 +606,7 @@ __global__ void k_split_level_t(const K *key, const Active *act, const uint32_t 
           L.c[3] = ns;
           leaves[ls] = L;
           code = -2 - (int32_t)ls;
+          mark_leaf(bits, L.start);
           atomicMax(&out->maxdepth, (uint32_t)lv);
         } else {
           atomicOr(&out->overflow, 4u);
@@ -559,7 +627,7 @@ __global__ void __launch_bounds__(256) k_split_level(
     const K *key, const Active *act, const uint32_t *act_cnt, uint32_t act_cap, int level,
     int max_level, Active *next, uint32_t *next_cnt, uint32_t next_cap, LeafTmp *leaves,
     uint32_t leaf_cap, double *node_cube, int32_t *node_child, int32_t *node_parent,
-    uint32_t node_cap, SplitOut *out)
+    uint32_t node_cap, SplitOut *out, uint32_t *bits)
 {
   if (out->overflow) return;
   const uint32_t nact = min(*act_cnt, act_cap);
@@ -681,6 +749,7 @@ __global__ void __launch_bounds__(256) k_split_level(
             L.c[3] = ns;
             leaves[ls] = L;
             code = -2 - (int32_t)ls;
+            mark_leaf(bits, L.start);
           } else {
             atomicOr(&out->overflow, 4u);
           }
@@ -691,17 +760,58 @@ __global__ void __launch_bounds__(256) k_split_level(
   }
 }
 
-__global__ void k_leaf_keys(const LeafTmp *lt, uint32_t nl, uint32_t *k, uint32_t *v)
+// The leaves in DFS order are the leaves in ascending order of their first
+// slot, so a leaf's number is the number of marked slots before its own: the
+// bits' running sums by word (k_bits_sums over tiles of BITS_TILE words,
+// k_bits_down within them).  A radix sort of the first slots, before, was 14
+// launches.
+#define BITS_TILE 2048
+__device__ inline uint32_t bits_load(const uint32_t *bits, uint32_t nwords, uint32_t (&v)[8])
 {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nl) return;
-  k[i] = lt[i].start;
-  v[i] = i;
+  const uint32_t i = blockIdx.x * BITS_TILE + threadIdx.x * 8;
+  uint32_t s = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    v[k] = i + k < nwords ? (uint32_t)__popc(bits[i + k]) : 0u;
+    s += v[k];
+  }
+  return s;
 }
 
-__global__ void k_leaf_final(const LeafTmp *lt, const uint32_t *perm, uint32_t nl, uint64_t n,
-                             uint32_t *leaf_start, double *leaf_cube, int32_t *leaf_parent,
-                             uint32_t *inv)
+__global__ void __launch_bounds__(256) k_bits_sums(const uint32_t *bits, uint32_t nwords,
+                                                   uint32_t *bsum)
+{
+  uint32_t v[8], tot;
+  block_excl_scan256(bits_load(bits, nwords, v), &tot);
+  if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+}
+
+// bsum: the tiles' sums (every block adds up those before its own)
+__global__ void __launch_bounds__(256) k_bits_down(const uint32_t *bits, uint32_t nwords,
+                                                   const uint32_t *bsum, uint32_t *pre)
+{
+  uint32_t off = 0, all, v[8];
+  for (uint32_t k = threadIdx.x; k < blockIdx.x; k += 256) off += bsum[k];
+  block_excl_scan256(off, &all);
+  const uint32_t s = bits_load(bits, nwords, v);
+  uint32_t tot, ex = all + block_excl_scan256(s, &tot);
+  const uint32_t i = blockIdx.x * BITS_TILE + threadIdx.x * 8;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    if (i + k < nwords) pre[i + k] = ex;
+    ex += v[k];
+  }
+}
+
+// marked slots up to and with slot i
+__device__ inline uint32_t bits_upto(const uint32_t *bits, const uint32_t *pre, uint32_t i)
+{
+  return pre[i / 32] + (uint32_t)__popc(bits[i / 32] & (0xffffffffu >> (31 - i % 32)));
+}
+
+__global__ void k_leaf_final(const LeafTmp *lt, const uint32_t *bits, const uint32_t *pre,
+                             uint32_t nl, uint64_t n, uint32_t *leaf_start, double *leaf_cube,
+                             int32_t *leaf_parent, uint32_t *inv)
 {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > nl) return;
@@ -709,19 +819,22 @@ __global__ void k_leaf_final(const LeafTmp *lt, const uint32_t *perm, uint32_t n
     leaf_start[nl] = (uint32_t)n;
     return;
   }
-  LeafTmp L = lt[perm[i]];
-  leaf_start[i] = L.start;
-  leaf_cube[4 * i] = L.c[0];
-  leaf_cube[4 * i + 1] = L.c[1];
-  leaf_cube[4 * i + 2] = L.c[2];
-  leaf_cube[4 * i + 3] = L.c[3];
-  leaf_parent[i] = L.parent;
-  inv[perm[i]] = i;
+  LeafTmp L = lt[i];
+  const uint32_t l = bits_upto(bits, pre, L.start) - 1;
+  leaf_start[l] = L.start;
+  leaf_cube[4 * (size_t)l] = L.c[0];
+  leaf_cube[4 * (size_t)l + 1] = L.c[1];
+  leaf_cube[4 * (size_t)l + 2] = L.c[2];
+  leaf_cube[4 * (size_t)l + 3] = L.c[3];
+  leaf_parent[l] = L.parent;
+  inv[i] = l;
 }
 
-// leaf children renumbered in DFS order, with the slot range of each
+// leaf children renumbered in DFS order, with the slot range of each and the
+// start of its lowest z
 __global__ void k_patch_children(int32_t *child, uint32_t nn, const uint32_t *inv,
-                                 const uint32_t *leaf_start, uint2 *crange)
+                                 const uint32_t *leaf_start, uint2 *crange,
+                                 double *child_zlow)
 {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nn * 8u) return;
@@ -733,55 +846,7 @@ __global__ void k_patch_children(int32_t *child, uint32_t nn, const uint32_t *in
     r = make_uint2(leaf_start[l], leaf_start[l + 1]);
   }
   crange[i] = r;
-}
-
-__global__ void k_fill_pt_leaf(const uint32_t *leaf_start, uint32_t nl, uint32_t *pt_leaf)
-{
-  uint32_t l = blockIdx.x;
-  if (l >= nl) return;
-  uint32_t s = leaf_start[l], e = leaf_start[l + 1];
-  for (uint32_t i = s + threadIdx.x; i < e; i += blockDim.x) pt_leaf[i] = l;
-}
-
-// ---------------------------------------------------------------------------
-// The lowest point under every child of every internal node (the ground
-// test raises a child cube's bottom face to it, wb::hyp_intersect_low): a
-// wave per leaf for the leaves' lowest z, then one launch per depth, deepest
-// first, in which each internal node of that depth takes the lowest of its
-// children's.  Node ids grow with depth (a level's nodes are made while the
-// level above splits), so a node's depth follows from its side.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_leaf_zlow(const uint32_t *leaf_start, uint32_t nl,
-                                                   const double *pz, double *leaf_zlow,
-                                                   float *leaf_low)
-{
-  const uint32_t l = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  if (l >= nl) return;
-  const uint32_t b = leaf_start[l], e = leaf_start[l + 1];
-  double m = __builtin_inf();
-  for (uint32_t j = b + lane; j < e; j += WAVE) m = fmin(m, pz[j]);
-  for (int d = 1; d < WAVE; d <<= 1) m = fmin(m, __shfl_xor(m, d, WAVE));
-  if (lane == 0) {
-    leaf_zlow[l] = m;
-    leaf_low[l] = (float)(m - fabs(m) * 0x1p-22);
-  }
-}
-
-__global__ void k_node_zlow(const int32_t *node_child, const double *node_cube, uint32_t nn,
-                            int depth, const double *leaf_zlow, double *node_zlow,
-                            double *child_zlow)
-{
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nn) return;
-  if (ilogb(node_cube[3]) - ilogb(node_cube[4 * (size_t)v + 3]) != depth) return;
-  double m = __builtin_inf();
-  for (int k = 0; k < 8; k++) {
-    const int32_t c = node_child[8 * (size_t)v + k];
-    const double zl = c <= -2 ? leaf_zlow[-2 - c] : c >= 0 ? node_zlow[c] : __builtin_inf();
-    child_zlow[8 * (size_t)v + k] = zl;
-    m = fmin(m, zl);
-  }
-  node_zlow[v] = m;
+  child_zlow[i] = __builtin_inf();  // k_leaf_finish lowers it
 }
 
 // ---------------------------------------------------------------------------
@@ -790,13 +855,15 @@ __global__ void k_node_zlow(const int32_t *node_child, const double *node_cube, 
 template <bool F64>
 __global__ void k_permute(Src src, const uint32_t *sidx, uint64_t n, Xform f, double *px,
                           double *py, double *pz, double *box, uint32_t *low, double *lowx,
-                          double *lowy, double *lowz, float4 *oct_xy, float *oct_z)
+                          double *lowy, double *lowz, float4 *oct_xy, float *oct_z,
+                          const uint32_t *bits, const uint32_t *pre, uint32_t *pt_leaf)
 {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool ok = i < n;
   double x = 0, y = 0, z = 0;
   if (ok) {
     load_packed<F64>(src, f, sidx[i], x, y, z);
+    pt_leaf[i] = bits_upto(bits, pre, (uint32_t)i) - 1;
     px[i] = x;
     py[i] = y;
     pz[i] = z;
@@ -923,36 +990,95 @@ __global__ void k_dup_compact(const uint64_t *key, const uint32_t *sidx, const u
   }
 }
 
-// Per-leaf canonical order, input order inside each leaf: a sort of the
-// leaf's input indices by a wave per leaf, in registers: leaves of
-// 64(K/2)+1 .. 64K points (K = 1: up to 64) hold K keys per lane, element
-// e = 64s + lane in slot s, sorted by the register network of wb_wave.h up
-// to the next power of two of the leaf size.  No barrier, no LDS.  Keys
-// (input indices) are distinct.
-template <int K>
-__global__ void __launch_bounds__(256) k_leaf_canon_reg(const uint32_t *leaf_start, uint32_t nl,
-                                                        const uint32_t *sidx, uint32_t *canon,
-                                                        uint32_t *crank)
+// lowers *z to v (both directions of the order of doubles by their bits: an
+// int64 minimum where v >= 0, a u64 maximum where v < 0)
+__device__ inline void lower_to(double *z, double v)
 {
-  const uint32_t lane = threadIdx.x & 63;
-  for (uint32_t l = blockIdx.x * 4 + threadIdx.x / 64; l < nl; l += gridDim.x * 4) {
-    const uint32_t b = leaf_start[l], m = leaf_start[l + 1] - b;
-    if (m <= (K == 1 ? 0u : 32u * K) || m > 64u * K) continue;
-    uint32_t key[K], val[K];
+  const long long b = __builtin_bit_cast(long long, v);
+  if (b >= 0) atomicMin((long long *)z, b);
+  else atomicMax((unsigned long long *)z, (unsigned long long)b);
+}
+
+// A block per leaf.
+// The canonical order (input order inside each leaf): a point's place is the
+// number of smaller input indices in the leaf, counted by a thread per point
+// (up to three) over the leaf's indices in LDS, four per read, the same
+// address in every lane.  At most 537^2 comparisons a leaf; a bitonic sort of
+// the leaf by one wave (55 stages for 512 keys, each waiting for the one
+// before) took 43 us of latency and one launch per size class (150k points,
+// five launches: 75 us; 23.7M points: 530 us).
+// The leaf's lowest point, and with it the lowest z under every child of every
+// internal node (the ground test raises a child cube's bottom face to it,
+// wb::hyp_intersect_low): up the parents until one is as low already (then so
+// are those above it, or its own block is on the way to them).
+#define CANON_PT 3  // 256 * 3 >= WB_RECORDS
+__global__ void __launch_bounds__(256) k_leaf_finish(const uint32_t *leaf_start,
+                                                     const uint32_t *sidx, const double *pz,
+                                                     const int32_t *leaf_parent,
+                                                     const int32_t *node_child,
+                                                     const int32_t *node_parent, uint32_t *canon,
+                                                     uint32_t *crank, float *leaf_low,
+                                                     double *child_zlow)
+{
+  static_assert(CANON_PT * 256 >= WB_RECORDS, "");
+  __shared__ __align__(16) uint32_t id[CANON_PT * 256];
+  __shared__ double wz[4];
+  const uint32_t l = blockIdx.x, t = threadIdx.x;
+  const uint32_t b = leaf_start[l], m = leaf_start[l + 1] - b;
+  double zl = __builtin_inf();
+  uint32_t my[CANON_PT], rank[CANON_PT];
 #pragma unroll
-    for (int s = 0; s < K; s++) {
-      const uint32_t e = 64u * s + lane;
-      key[s] = e < m ? sidx[b + e] : 0xffffffffu;
-      val[s] = b + e;
-    }
-    wbw::wave_sort<K, true>(key, val, wbw::pow2_ceil(m));
-#pragma unroll
-    for (int s = 0; s < K; s++) {
-      const uint32_t e = 64u * s + lane;
-      if (e < m) {
-        canon[b + e] = val[s];
-        crank[val[s]] = b + e;
+  for (int k = 0; k < CANON_PT; k++) {
+    const uint32_t e = t + 256u * k;
+    my[k] = e < m ? sidx[b + e] : 0xffffffffu;
+    rank[k] = 0;
+    id[e] = my[k];
+    if (e < m) zl = fmin(zl, pz[b + e]);
+  }
+  for (int d = 1; d < WAVE; d <<= 1) zl = fmin(zl, __shfl_xor(zl, d, WAVE));
+  if (t % WAVE == 0) wz[t / WAVE] = zl;
+  __syncthreads();
+  const uint32_t w0 = t & ~(WAVE - 1u);  // the wave's first element
+  if (w0 < m) {
+    const uint4 *q = (const uint4 *)id;
+    const uint32_t nq = (m + 3) / 4;
+    if (w0 + 256 >= m) {
+      for (uint32_t j = 0; j < nq; j++) {
+        const uint4 v = q[j];
+        rank[0] += (v.x < my[0]) + (v.y < my[0]) + (v.z < my[0]) + (v.w < my[0]);
       }
+    } else {
+      for (uint32_t j = 0; j < nq; j++) {
+        const uint4 v = q[j];
+#pragma unroll
+        for (int k = 0; k < CANON_PT; k++)
+          rank[k] += (v.x < my[k]) + (v.y < my[k]) + (v.z < my[k]) + (v.w < my[k]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < CANON_PT; k++) {
+      const uint32_t e = t + 256u * k;
+      if (e < m) {
+        canon[b + rank[k]] = b + e;
+        crank[b + e] = b + rank[k];
+      }
+    }
+  }
+  if (t == 0) {
+    zl = fmin(fmin(wz[0], wz[1]), fmin(wz[2], wz[3]));
+    leaf_low[l] = (float)(zl - fabs(zl) * 0x1p-22);
+    int32_t code = -2 - (int32_t)l;
+    for (int32_t p = leaf_parent[l]; p >= 0;) {
+      const int4 c0 = *(const int4 *)(node_child + 8 * (size_t)p);
+      const int4 c1 = *(const int4 *)(node_child + 8 * (size_t)p + 4);
+      const int32_t up = node_parent[p];
+      const int k = (c0.y == code) + 2 * (c0.z == code) + 3 * (c0.w == code) + 4 * (c1.x == code) +
+                    5 * (c1.y == code) + 6 * (c1.z == code) + 7 * (c1.w == code);
+      double *at = child_zlow + 8 * (size_t)p + k;
+      if (*at <= zl) break;
+      lower_to(at, zl);
+      code = p;
+      p = up;
     }
   }
 }
@@ -1018,9 +1144,8 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
   LeafTmp *lt = nullptr;
   SplitOut *d_out = (SplitOut *)wb_alloc(c, sizeof(SplitOut));
   uint32_t *d_cnt = (uint32_t *)wb_alloc(c, 4 * (WB_MAX_LEVEL + 2));
-  uint32_t *d_outside = (uint32_t *)wb_alloc(c, 4);
-  static const uint32_t zero_word = 0;
-  uint32_t h_outside = 0;
+  const uint32_t nwords = (uint32_t)(n_input / 32 + 1);
+  uint32_t *bits = (uint32_t *)wb_alloc(c, 4 * (size_t)nwords);
   SplitOut h_out;
   Active *act = (Active *)wb_alloc(c, sizeof(Active) * node_cap);
   Active *nxt = (Active *)wb_alloc(c, sizeof(Active) * node_cap);
@@ -1042,24 +1167,31 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
     // pairs: 8 B per point moved per pass instead of 12
     const bool narrow = !dedupe && passes <= 4;
     uint32_t *key32 = (uint32_t *)key0;
+    auto init = [&](uint64_t count) {
+      hipLaunchKernelGGL(k_build_init, dim3(wb_blocks(nwords, 256)), dim3(256), 0, c->stream,
+                         (uint32_t)count, t->center[0], t->center[1], t->center[2], t->side,
+                         t->node_cube, t->node_child, t->node_parent, d_out, act, d_cnt, bits,
+                         nwords);
+    };
+    if (n == 0) init(0);
     if (n > 0) {
       WB_CHECK(hipEventRecord(evb[0], c->stream));
-      WB_CHECK(hipMemcpyAsync(d_outside, &zero_word, 4, hipMemcpyHostToDevice, c->stream));
+      init(n);
       const dim3 kg(wb_blocks(n, 256)), kb(256);
       if (narrow) {
         if (f64)
           hipLaunchKernelGGL((k_keygen<true, uint32_t>), kg, kb, 0, c->stream, src, n, f, key32,
-                             t->sidx, d_outside);
+                             t->sidx, &d_out->outside);
         else
           hipLaunchKernelGGL((k_keygen<false, uint32_t>), kg, kb, 0, c->stream, src, n, f, key32,
-                             t->sidx, d_outside);
+                             t->sidx, &d_out->outside);
       } else {
         if (f64)
           hipLaunchKernelGGL((k_keygen<true, uint64_t>), kg, kb, 0, c->stream, src, n, f, t->key,
-                             t->sidx, d_outside);
+                             t->sidx, &d_out->outside);
         else
           hipLaunchKernelGGL((k_keygen<false, uint64_t>), kg, kb, 0, c->stream, src, n, f, t->key,
-                             t->sidx, d_outside);
+                             t->sidx, &d_out->outside);
       }
       WB_CHECK(hipEventRecord(evb[1], c->stream));
       if (narrow) wb_radix_sort_u32_prefix(c, key32, t->sidx, n, passes);
@@ -1100,57 +1232,45 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
         wb_free(c, pos, 4 * n_input);
       }
     }
-    // root node 0
-    double root[4] = {t->center[0], t->center[1], t->center[2], t->side};
-    int32_t empty8[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
-    int32_t m1 = -1;
-    WB_CHECK(hipMemcpyAsync(t->node_cube, root, sizeof root, hipMemcpyHostToDevice, c->stream));
-    WB_CHECK(hipMemcpyAsync(t->node_child, empty8, sizeof empty8, hipMemcpyHostToDevice, c->stream));
-    WB_CHECK(hipMemcpyAsync(t->node_parent, &m1, 4, hipMemcpyHostToDevice, c->stream));
-    memset(&h_out, 0, sizeof h_out);
-    h_out.n_node = 1;
-    WB_CHECK(hipMemcpyAsync(d_out, &h_out, sizeof h_out, hipMemcpyHostToDevice, c->stream));
     if (lt) wb_free(c, lt, sizeof(LeafTmp) * leaf_cap);
     lt = (LeafTmp *)wb_alloc(c, sizeof(LeafTmp) * leaf_cap);
     int max_level = std::min(WB_MAX_LEVEL, (8 * passes) / 3);
     // active nodes of one level are disjoint and hold more than 537 points
     const uint32_t act_ub = (uint32_t)std::min<uint64_t>(node_cap, n / (WB_RECORDS + 1) + 1);
-    uint32_t hcnt[WB_MAX_LEVEL + 2] = {};
-    if (n > 0) {
-      Active r0 = {0u, (uint32_t)n, 0, 0};
+    if (n < n_input) {  // (merged: the root holds fewer points)
+      const Active r0 = {0u, (uint32_t)n, 0, 0};
       WB_CHECK(hipMemcpyAsync(act, &r0, sizeof r0, hipMemcpyHostToDevice, c->stream));
-      hcnt[0] = 1;
     }
-    WB_CHECK(hipMemcpyAsync(d_cnt, hcnt, sizeof hcnt, hipMemcpyHostToDevice, c->stream));
     for (int level = 0; n > 0 && level < max_level; level++) {
       const dim3 gw(std::min<uint32_t>(wb_blocks(act_ub, 4), 512)), gt(wb_blocks(act_ub, 128));
       if (narrow) {
         hipLaunchKernelGGL(k_split_level<uint32_t>, gw, dim3(256), 0, c->stream, key32, act,
                            d_cnt + level, node_cap, level, max_level, nxt, d_cnt + level + 1,
                            node_cap, lt, leaf_cap, t->node_cube, t->node_child, t->node_parent,
-                           node_cap, d_out);
+                           node_cap, d_out, bits);
         if (act_ub > SPLIT_WAVE_MAX)
           hipLaunchKernelGGL(k_split_level_t<uint32_t>, gt, dim3(128), 0, c->stream, key32, act,
                              d_cnt + level, node_cap, level, max_level, nxt, d_cnt + level + 1,
                              node_cap, lt, leaf_cap, t->node_cube, t->node_child,
-                             t->node_parent, node_cap, d_out);
+                             t->node_parent, node_cap, d_out, bits);
       } else {
         hipLaunchKernelGGL(k_split_level<uint64_t>, gw, dim3(256), 0, c->stream, t->key, act,
                            d_cnt + level, node_cap, level, max_level, nxt, d_cnt + level + 1,
                            node_cap, lt, leaf_cap, t->node_cube, t->node_child, t->node_parent,
-                           node_cap, d_out);
+                           node_cap, d_out, bits);
         if (act_ub > SPLIT_WAVE_MAX)
           hipLaunchKernelGGL(k_split_level_t<uint64_t>, gt, dim3(128), 0, c->stream, t->key, act,
                              d_cnt + level, node_cap, level, max_level, nxt, d_cnt + level + 1,
                              node_cap, lt, leaf_cap, t->node_cube, t->node_child,
-                             t->node_parent, node_cap, d_out);
+                             t->node_parent, node_cap, d_out, bits);
       }
       std::swap(act, nxt);
     }
-    WB_CHECK(hipMemcpyAsync(&h_out, d_out, sizeof h_out, hipMemcpyDeviceToHost, c->stream));
-    WB_CHECK(hipMemcpyAsync(&h_outside, d_outside, 4, hipMemcpyDeviceToHost, c->stream));
+    uint32_t *hb = c->hbox + WB_HBOX_BUILD;
+    WB_CHECK(hipMemcpyAsync(hb, d_out, sizeof h_out, hipMemcpyDeviceToHost, c->stream));
     WB_CHECK(hipStreamSynchronize(c->stream));
-    t->outside_root = n > 0 ? h_outside : 0;
+    memcpy(&h_out, hb, sizeof h_out);
+    t->outside_root = h_out.outside;
     // the split's scratch goes back to the cache before an error leaves
     auto release = [&]() {
       wb_free(c, src.packed, pk_bytes);
@@ -1159,7 +1279,7 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
       wb_free(c, lt, sizeof(LeafTmp) * leaf_cap);
       wb_free(c, d_out, sizeof(SplitOut));
       wb_free(c, d_cnt, 4 * (WB_MAX_LEVEL + 2));
-      wb_free(c, d_outside, 4);
+      wb_free(c, bits, 4 * (size_t)nwords);
     };
     if (h_out.overflow & 1u) {
       if (passes >= 8) {
@@ -1183,26 +1303,29 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
   t->maxdepth = (int)h_out.maxdepth;
   wb_free(c, d_out, sizeof(SplitOut));
   wb_free(c, d_cnt, 4 * (WB_MAX_LEVEL + 2));
-  wb_free(c, d_outside, 4);
 
   // leaves in DFS order = ascending start
   const uint32_t nl = t->nleaves;
+  uint32_t *pre = nullptr;
   t->leaf_start = wb_talloc<uint32_t>(t, nl + 1);
   t->leaf_cube = wb_talloc<double>(t, 4 * (size_t)nl + 4);
   t->leaf_parent = wb_talloc<int32_t>(t, nl + 1);
   if (nl > 0) {
-    uint32_t *lk = (uint32_t *)wb_alloc(c, 4 * (size_t)nl), *lv = (uint32_t *)wb_alloc(c, 4 * (size_t)nl);
+    const unsigned nt = wb_blocks(nwords, BITS_TILE);
+    uint32_t *bsum = (uint32_t *)wb_alloc(c, 4 * (size_t)nt);
     uint32_t *inv = (uint32_t *)wb_alloc(c, 4 * (size_t)nl);
-    hipLaunchKernelGGL(k_leaf_keys, dim3(wb_blocks(nl, 256)), dim3(256), 0, c->stream, lt, nl, lk, lv);
-    wb_radix_sort_u32_pairs(c, lk, lv, nl);
-    hipLaunchKernelGGL(k_leaf_final, dim3(wb_blocks(nl + 1, 256)), dim3(256), 0, c->stream, lt, lv,
-                       nl, n, t->leaf_start, t->leaf_cube, t->leaf_parent, inv);
+    pre = (uint32_t *)wb_alloc(c, 4 * (size_t)nwords);
+    t->child_zlow = wb_talloc<double>(t, 8 * (size_t)t->nnodes);
+    if (nt > 1)
+      hipLaunchKernelGGL(k_bits_sums, dim3(nt), dim3(256), 0, c->stream, bits, nwords, bsum);
+    hipLaunchKernelGGL(k_bits_down, dim3(nt), dim3(256), 0, c->stream, bits, nwords, bsum, pre);
+    hipLaunchKernelGGL(k_leaf_final, dim3(wb_blocks(nl + 1, 256)), dim3(256), 0, c->stream, lt, bits,
+                       pre, nl, n, t->leaf_start, t->leaf_cube, t->leaf_parent, inv);
     t->node_crange = wb_talloc<uint2>(t, 8 * (size_t)t->nnodes);
     hipLaunchKernelGGL(k_patch_children, dim3(wb_blocks((uint64_t)t->nnodes * 8, 256)), dim3(256),
                        0, c->stream, t->node_child, t->nnodes, inv, t->leaf_start,
-                       t->node_crange);
-    wb_free(c, lk, 4 * (size_t)nl);
-    wb_free(c, lv, 4 * (size_t)nl);
+                       t->node_crange, t->child_zlow);
+    wb_free(c, bsum, 4 * (size_t)nt);
     wb_free(c, inv, 4 * (size_t)nl);
   } else {
     uint32_t zero = 0;
@@ -1226,51 +1349,29 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
   t->oct_xy = wb_talloc<float4>(t, (WB_CHUNK / WB_OCT) * nchunks + 1);
   t->oct_z = wb_talloc<float>(t, (WB_CHUNK / WB_OCT) * nchunks + 1);
   if (n > 0) {
-    hipLaunchKernelGGL(k_fill_pt_leaf, dim3(nl), dim3(256), 0, c->stream, t->leaf_start, nl,
-                       t->pt_leaf);
     if (f64)
       hipLaunchKernelGGL(k_permute<true>, dim3(wb_blocks(nchunks * WB_CHUNK, 256)), dim3(256), 0,
                          c->stream, src, t->sidx, n, f, t->px, t->py, t->pz, t->chunk_box,
-                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz, t->oct_xy, t->oct_z);
+                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz, t->oct_xy, t->oct_z, bits, pre,
+                         t->pt_leaf);
     else
       hipLaunchKernelGGL(k_permute<false>, dim3(wb_blocks(nchunks * WB_CHUNK, 256)), dim3(256), 0,
                          c->stream, src, t->sidx, n, f, t->px, t->py, t->pz, t->chunk_box,
-                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz, t->oct_xy, t->oct_z);
+                         t->chunk_low, t->chunk_sx, t->chunk_sy, t->chunk_sz, t->oct_xy, t->oct_z, bits, pre,
+                         t->pt_leaf);
     wb_free(c, src.packed, pk_bytes);
     src.packed = nullptr;
-    {
-      // a wave per leaf, by size class (every leaf holds at most 537 points)
-      const unsigned nb = std::min<unsigned>(wb_blocks(nl, 4), 4096);
-      hipLaunchKernelGGL(k_leaf_canon_reg<1>, dim3(nb), dim3(256), 0, c->stream, t->leaf_start,
-                         nl, t->sidx, t->canon, t->crank);
-      hipLaunchKernelGGL(k_leaf_canon_reg<2>, dim3(nb), dim3(256), 0, c->stream, t->leaf_start,
-                         nl, t->sidx, t->canon, t->crank);
-      hipLaunchKernelGGL(k_leaf_canon_reg<4>, dim3(nb), dim3(256), 0, c->stream, t->leaf_start,
-                         nl, t->sidx, t->canon, t->crank);
-      hipLaunchKernelGGL(k_leaf_canon_reg<8>, dim3(nb), dim3(256), 0, c->stream, t->leaf_start,
-                         nl, t->sidx, t->canon, t->crank);
-      hipLaunchKernelGGL(k_leaf_canon_reg<16>, dim3(nb), dim3(256), 0, c->stream, t->leaf_start,
-                         nl, t->sidx, t->canon, t->crank);
-    }
-    {
-      double *leaf_zlow = (double *)wb_alloc(c, 8 * (size_t)nl);
-      double *node_zlow = (double *)wb_alloc(c, 8 * (size_t)t->nnodes);
-      t->child_zlow = wb_talloc<double>(t, 8 * (size_t)t->nnodes);
-      t->leaf_low = wb_talloc<float>(t, nl);
-      hipLaunchKernelGGL(k_leaf_zlow, dim3(wb_blocks(nl, 4)), dim3(256), 0, c->stream,
-                         t->leaf_start, nl, t->pz, leaf_zlow, t->leaf_low);
-      for (int d = t->maxdepth - 1; d >= 0; d--)
-        hipLaunchKernelGGL(k_node_zlow, dim3(wb_blocks(t->nnodes, 256)), dim3(256), 0, c->stream,
-                           t->node_child, t->node_cube, t->nnodes, d, leaf_zlow, node_zlow,
-                           t->child_zlow);
-      wb_free(c, leaf_zlow, 8 * (size_t)nl);
-      wb_free(c, node_zlow, 8 * (size_t)t->nnodes);
-    }
+    t->leaf_low = wb_talloc<float>(t, nl);
+    hipLaunchKernelGGL(k_leaf_finish, dim3(nl), dim3(256), 0, c->stream, t->leaf_start, t->sidx,
+                       t->pz, t->leaf_parent, t->node_child, t->node_parent, t->canon,
+                       t->crank, t->leaf_low, t->child_zlow);
     WB_CHECK(hipEventRecord(evb[3], c->stream));
   } else {
     t->evb_read = true;
   }
   if (src.packed) wb_free(c, src.packed, pk_bytes);
+  wb_free(c, bits, 4 * (size_t)nwords);
+  if (pre) wb_free(c, pre, 4 * (size_t)nwords);
 }
 
 void wb_tree_read_timing(wb_tree *t)

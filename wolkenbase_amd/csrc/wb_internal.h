@@ -43,6 +43,7 @@
 #define WB_HBOX_SCAN 0     // wb_exclusive_scan_u32: total (2 words)
 #define WB_HBOX_GEO 16     // tile grid bounds (4 words)
 #define WB_HBOX_ERR 32     // classification flags and counters (32 words)
+#define WB_HBOX_BUILD 8    // the build's counters (5 words)
 #define WB_HBOX_QUERY 64   // a few shapes' parameters and counts
 #define WB_HBOX_SHAPES 64  // as many
 #define WB_GEO_CACHE 4
@@ -212,8 +213,6 @@ uint64_t wb_exclusive_scan_u32(wb_ctx *c, uint32_t *data, uint64_t n);
 void wb_radix_sort_pairs(wb_ctx *c, uint64_t *key, uint32_t *val, uint64_t n, int passes);
 // LSD radix sort of (u32 key, u32 val) pairs on bits [32-8*passes, 32)
 void wb_radix_sort_u32_prefix(wb_ctx *c, uint32_t *key, uint32_t *val, uint64_t n, int passes);
-// LSD radix sort of (u32 key, u32 val) pairs on all 32 bits
-void wb_radix_sort_u32_pairs(wb_ctx *c, uint32_t *key, uint32_t *val, uint64_t n);
 
 // builds the canonical octree of t->n_input points, decoded from int32 LAS
 // coordinates (dx, dy, dz with t->scale / t->offset) or given in FP64 (fx,
