@@ -1,6 +1,8 @@
 """GPU parity: the HIP path through the C ABI against the CPU oracle on the
 same seeded inputs.  Octree contents, point order, neighbour counts and class
 bytes must be bit-identical."""
+import math
+
 import numpy as np
 import pytest
 
@@ -532,3 +534,71 @@ def test_merge_of_a_scan_of_many_tiles(ctx):
         assert np.array_equal(leaves["first"], np.cumsum(leaves["count"]) - leaves["count"])
     finally:
         tree.free()
+
+
+def tile_record(vx, vy, z, r, min_hs):
+    """scanCylinder's record (scan.cpp:31-140) of points relative to the axis."""
+    sx, sy, _ = O.lls3(vx, vy, z)
+    length = float(np.hypot(sx, sy))  # (the C library's; Python's own rounds otherwise)
+    if length > 1:
+        sx, sy = sx / length, sy / length
+    if math.isnan(sx) or math.isnan(sy):
+        sx = sy = 0.0
+    u = z - (sy * vy + sx * vx)
+    first = int(np.argmin(u))
+    bottom2 = u[:first].min() if first else u[first]
+    low = u < bottom2 + 2 * r
+    sec = np.rint(np.arctan2(vy[low], vx[low]) * 3 / math.pi).astype(int)
+    sec = np.where(sec < 0, sec + 6, sec) % 6 + 1
+    sec[np.hypot(vx[low], vy[low]) < r / math.sqrt(7)] = 0
+    total = int((np.bincount(sec, minlength=7) ** 2).sum())
+    density = math.sqrt(float(total)) * 2.6457513110645905905016 / (r * r) / math.pi
+    more = len(z) > low.sum()
+    tree = (more and total < 7) or (more and density < 0.5) or u.max() - u.min() > 1.5
+    return dict(npoints=len(z), tree_flags=int(tree), density=density,
+                hs_scan=math.sqrt(1 / density + min_hs * min_hs), height=u.max() - u.min(),
+                tilt_x=sx, tilt_y=sy)
+
+
+@pytest.mark.parametrize("height", [25.0, 200.0])
+def test_scan_of_every_tile_size(ctx, height):
+    # strips of 2 to 500 points per m2 and tiles of one point to several
+    # hundred, in a cloud whose size classes share one launch (200k points) and
+    # in one where each has its own (1.6M)
+    rng = np.random.default_rng(77)
+    x, x0 = [], 0.0
+    for dens in (2, 5, 10, 20, 40, 80, 160, 500):
+        w = 1143.0 / dens
+        x.append(x0 + rng.random(int(1143 * height)) * w)
+        x0 += w
+    x = np.concatenate(x)
+    n = len(x)
+    y = rng.random(n) * height
+    z = 0.1 * x + 0.05 * y + rng.exponential(0.4, n) * (rng.random(n) < 0.5)
+    off, sc = np.array([1000.0, 2000.0, 0.0]), np.array([0.001] * 3)
+    raw = np.stack([np.round(a * 1000).astype(np.int32) for a in (x, y, z)])
+    px, py, pz = (off[k] + sc[k] * raw[k] for k in range(3))
+    mn, mx = off + sc * raw.min(1), off + sc * raw.max(1)
+    center, side = W.Octree.size_fit(mn, mx)
+    tree = W.Octree.build(ctx, raw[0], raw[1], raw[2], sc, off, center, side)
+    prm = W.default_params()
+    tiles, _ = W.scan_tiles(tree, mn, mx, prm)
+    m = tiles["npoints"]
+    sn = O.snake_setup(mn, mx)
+    pick = []
+    for lo, hi in ((1, 1), (2, 2), (3, 3), (4, 7), (8, 8), (9, 9), (10, 15), (16, 16), (17, 17),
+                   (18, 31), (32, 32), (33, 33), (34, 63), (64, 64), (65, 65), (66, 127),
+                   (128, 128), (129, 129), (130, 256), (257, 1024)):
+        at = np.flatnonzero((m >= lo) & (m <= hi))
+        assert len(at) or lo == hi, (lo, hi)
+        pick += list(rng.permutation(at)[:12])
+    addr = np.array([O.to_flowsnake(sn.lo + int(k)) for k in pick])
+    cyl = np.array([O.snake_cyl(sn, ex, ey) for ex, ey in addr])
+    P = np.zeros((len(pick), 5))
+    P[:, :3] = cyl
+    lists = tree.points_in((W.WB_SHAPE_CYLINDER, P))
+    tree.free()
+    for k, (cx, cy, r), ids in zip(pick, cyl, lists):
+        want = tile_record(px[ids] - cx, py[ids] - cy, pz[ids], r, prm.min_hs)
+        for f, v in want.items():
+            assert tiles[f][k] == v, (k, f, len(ids))

@@ -1219,34 +1219,41 @@ __device__ inline double wave_dmax(double v)
 }
 
 // wave_pairwise for m <= 64*K values held K per lane (value e in slot e/64
-// of lane e%64): the same block trees and block order.  A block of up to 64
-// values lies in one slot, aligned to its size; a larger one is the
-// balanced tree over its whole slots.
+// of lane e%64): the same block trees and block order.  The blocks of up to 64
+// values lie in the last slot that is not full, aligned to their size, so one
+// pass over that slot's levels meets them in ascending order; the larger ones
+// are balanced trees over the full slots before it.
 template <int K>
 __device__ inline double wave_pairwise_reg(uint32_t m, const double (&v)[K])
 {
   static_assert(K <= 4, "blocks of up to 256 values");
   double acc = 0;
-  for (int k = 0; k < 9; k++) {
-    if (!((m >> k) & 1u)) continue;
-    const uint32_t off = (m >> (k + 1)) << (k + 1);
-    const uint32_t sz = 1u << k;
-    double blk;
-    if (sz <= WAVE) {
-      blk = lanes_pairwise(slot_sel<K>(v, off / WAVE), sz, off & (WAVE - 1));
-    } else {
-      const uint32_t s0 = off / WAVE;
-      const double c0 = lanes_pairwise(slot_sel<K>(v, s0), WAVE, 0);
-      const double c1 = lanes_pairwise(slot_sel<K>(v, s0 + 1), WAVE, 0);
-      if (sz == 2 * WAVE) {
-        blk = c0 + c1;
-      } else {
-        const double c2 = lanes_pairwise(slot_sel<K>(v, s0 + 2), WAVE, 0);
-        const double c3 = lanes_pairwise(slot_sel<K>(v, s0 + 3), WAVE, 0);
-        blk = (c0 + c1) + (c2 + c3);
-      }
+  const uint32_t full = m / WAVE, rest = m % WAVE;
+  if (rest) {
+    double b = slot_sel<K>(v, full);
+    if (rest & 1) acc += rdl(b, rest & ~1u);
+    b = b + dpp_d<0xb1>(b);
+    if (rest & 2) acc += rdl(b, rest & ~3u);
+    b = b + dpp_d<0x4e>(b);
+    if (rest & 4) acc += rdl(b, rest & ~7u);
+    b = b + dpp_d<0x141>(b);
+    if (rest & 8) acc += rdl(b, rest & ~15u);
+    if (rest >= 16) {
+      b = b + dpp_d<0x140>(b);
+      if (rest & 16) acc += rdl(b, rest & ~31u);
+      if (rest & 32) acc += rdl(b, 0) + rdl(b, 16);
     }
-    acc += blk;
+  }
+  if (full & 1) acc += lanes_pairwise(slot_sel<K>(v, full - 1), WAVE, 0);
+  if constexpr (K >= 2) {
+    if (full & 2) {
+      acc += lanes_pairwise(v[0], WAVE, 0) + lanes_pairwise(v[1], WAVE, 0);
+    }
+  }
+  if constexpr (K >= 4) {
+    if (full & 4)
+      acc += (lanes_pairwise(v[0], WAVE, 0) + lanes_pairwise(v[1], WAVE, 0)) +
+             (lanes_pairwise(v[2], WAVE, 0) + lanes_pairwise(v[3], WAVE, 0));
   }
   return acc;
 }
@@ -1327,149 +1334,273 @@ __device__ inline bool plane_tilt_f32(uint32_t m, const double (&vx)[K], const d
   return well;
 }
 
-// The scan of a tile of at most 64*K points, K per lane (point e in slot
-// e/64 of lane e%64): the same operations and summation order as the
-// general path of k_scan, with the canonical sort done by a bitonic network
-// over lanes and slots and every point read once.
-template <int K, bool F32>
-__device__ __attribute__((always_inline)) inline void scan_reg(const TreeView &T, const TileGeo &g,
-                                                                int ex, int ey, uint32_t off,
-                         uint32_t m, const uint32_t *lists, double min_hs, int prec,
-                         TileRec *out, unsigned long long *ctr)
+// What a tile's scan ends in, one tile per lane: the sums of the normal
+// equations, the plane's tilt, the extremes of the untilted heights and the
+// bottom layer's sectors.  The solution and the record, a few hundred
+// instructions of divisions and square roots, are then done for all the
+// wave's tiles at once.
+struct TileFit {
+  double sxx, syx, syy, s1x, s1y, sxz, syz, s1z;
+  double sx, sy, bottom, top;
+  uint32_t m, nbottom, hist[7];
+};
+
+__device__ __attribute__((always_inline)) inline void fit_solve(TileFit &F)
+{
+  // (the sum of m ones is exact in any order)
+  plane_tilt(F.sxx, F.syx, F.syy, F.s1x, F.s1y, (double)F.m, F.sxz, F.syz, F.s1z, &F.sx, &F.sy);
+}
+
+__device__ __attribute__((always_inline)) inline void fit_record(const TileFit &F, double r,
+                                                                 double min_hs, int fit_fp64,
+                                                                 TileRec *out)
+{
+  double density = 0;
+  int tree = 0;
+  for (int i = 0; i < 7; i++) density += (int)F.hist[i] * (int)F.hist[i];
+  if (F.m > F.nbottom && density < 7) tree = 1;
+  density = sqrt(density) * kSqrt7 / (r * r) / M_PI;
+  if (F.m > F.nbottom && density < 0.5) tree = 1;
+  if (F.top - F.bottom > 1.5) tree = 1;
+  TileRec rr;
+  rr.npoints = (int32_t)F.m;
+  rr.nground = 0;
+  rr.tree_flags = tree;
+  rr.fit_fp64 = fit_fp64;
+  rr.density = density;
+  rr.hs_scan = sqrt(1 / density + min_hs * min_hs);
+  rr.hs = rr.hs_scan;
+  rr.height = F.top - F.bottom;
+  rr.tilt_x = F.sx;
+  rr.tilt_y = F.sy;
+  *out = rr;
+}
+
+// The scan of up to T tiles of at most 64*K points each by one wave, K points
+// per lane (point e in slot e/64 of lane e%64): the operations and summation
+// order of the general path of k_scan, with the canonical sort done by a
+// bitonic network over lanes and slots and every point read once.  Tile j's
+// fit is lane j's.  One tile at a time, every lane solving the same equations
+// and the sums' levels walked once per block, took 0.80 and 0.76 ms for the
+// tiles of up to 64 and 128 points of 23.7M points, against 0.54 and
+// 0.67 ms.
+template <int K, bool F32, int T>
+__device__ __attribute__((always_inline)) inline void scan_reg(
+    const TreeView &V, const TileGeo &g, const uint32_t (&t)[T], const uint32_t (&m)[T],
+    const int32_t *tex, const int32_t *tey, const uint32_t *tile_off, const uint32_t *lists,
+    double min_hs, int prec, TileRec *rec, unsigned long long *ctr)
 {
   const uint32_t lane = __lane_id();
-  uint32_t c[K];
+  uint32_t c[T][K];
 #pragma unroll
-  for (int s = 0; s < K; s++) {
-    const uint32_t e = s * WAVE + lane;
-    c[s] = e < m ? lists[off + e] : 0xffffffffu;
+  for (int j = 0; j < T; j++) {
+    const uint32_t off = m[j] ? tile_off[t[j]] : 0u;
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      const uint32_t e = s * WAVE + lane;
+      c[j][s] = e < m[j] ? lists[off + e] : 0xffffffffu;
+    }
   }
-  {
+#pragma unroll
+  for (int j = 0; j < T; j++) {
     // canonical order: the m ranks ascending (pads last), sorted only as far
     // as the next power of two
     uint32_t unused[K];
-    wbw::wave_sort<K, false>(c, unused, wbw::pow2_ceil(m));
+    wbw::wave_sort<K, false>(c[j], unused, wbw::pow2_ceil(m[j]));
   }
-  double cx, cy;
-  tile_center(g, ex, ey, &cx, &cy);
   const double r = g.r;
-  double vx[K], vy[K], vz[K];
-  bool mine[K];
+  double vx[T][K], vy[T][K], vz[T][K];
+  uint32_t q[T][K];
 #pragma unroll
-  for (int s = 0; s < K; s++) {
-    mine[s] = s * WAVE + lane < m;
-    vx[s] = 0; vy[s] = 0; vz[s] = 0;
-    if (mine[s]) {
-      const uint32_t q = T.canon[c[s]];
-      vx[s] = T.px[q] - cx;
-      vy[s] = T.py[q] - cy;
-      vz[s] = T.pz[q] - 0;
+  for (int j = 0; j < T; j++)
+#pragma unroll
+    for (int s = 0; s < K; s++) q[j][s] = s * WAVE + lane < m[j] ? V.canon[c[j][s]] : 0u;
+#pragma unroll
+  for (int j = 0; j < T; j++) {
+    double cx = 0, cy = 0;
+    if (m[j]) tile_center(g, tex[t[j]], tey[t[j]], &cx, &cy);
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      vx[j][s] = 0; vy[j][s] = 0; vz[j][s] = 0;
+      if (s * WAVE + lane < m[j]) {
+        vx[j][s] = V.px[q[j][s]] - cx;
+        vy[j][s] = V.py[q[j][s]] - cy;
+        vz[j][s] = V.pz[q[j][s]] - 0;
+      }
     }
   }
-  double sx = 0, sy = 0;
-  // FP32 fits are an option for the precision study; FP64 is the reference
-  bool fit64 = !F32 || prec == WB_FIT_FP64;
+  TileFit F;
+  F.m = 0;
+  F.sxx = F.syx = F.syy = F.s1x = F.s1y = F.sxz = F.syz = F.s1z = 0;
+  double px = 0, py = 0;  // lane j's tilt from FP32 moments
+  bool fit64 = true;
   int fell_back = 0;
-  if (F32 && !fit64) {
-    const bool well = plane_tilt_f32<K>(m, vx, vy, vz, mine, prec == WB_FIT_FP32_COMP, &sx, &sy);
-    if (!well && prec == WB_FIT_FP32_COMP) fit64 = true, fell_back = 1;
+#pragma unroll
+  for (int j = 0; j < T; j++) {
+    const bool me = lane == (uint32_t)j;
+    if (me) F.m = m[j];
+    // FP32 fits are an option for the precision study; FP64 is the reference
+    if (F32 && prec != WB_FIT_FP64) {
+      bool mine[K];
+#pragma unroll
+      for (int s = 0; s < K; s++) mine[s] = s * WAVE + lane < m[j];
+      double fx, fy;
+      const bool well =
+          plane_tilt_f32<K>(m[j], vx[j], vy[j], vz[j], mine, prec == WB_FIT_FP32_COMP, &fx, &fy);
+      const bool back = !well && prec == WB_FIT_FP32_COMP;
+      if (me) {
+        px = fx;
+        py = fy;
+        fit64 = back;
+        fell_back = back;
+      }
+      if (!back) continue;
+    }
+    double a[K];
+#define WB_SUM(dst, expr)                            \
+  {                                                  \
+    _Pragma("unroll") for (int s = 0; s < K; s++) {  \
+      const double x = vx[j][s], y = vy[j][s], z = vz[j][s]; \
+      (void)x, (void)y, (void)z;                     \
+      a[s] = (expr);                                 \
+    }                                                \
+    const double sum = wave_pairwise_reg<K>(m[j], a); \
+    if (me) dst = sum;                               \
   }
-  if (fit64) {
-    double t[K];
-#define WB_SUM(expr) (([&]() { _Pragma("unroll") for (int s = 0; s < K; s++) t[s] = (expr); }()), \
-                      wave_pairwise_reg<K>(m, t))
-    const double sxx = WB_SUM(vx[s] * vx[s]);
-    const double syx = WB_SUM(vy[s] * vx[s]);
-    const double syy = WB_SUM(vy[s] * vy[s]);
-    const double s1x = WB_SUM(1.0 * vx[s]);
-    const double s1y = WB_SUM(1.0 * vy[s]);
-    const double s11 = WB_SUM(1.0 * 1.0);
-    const double sxz = WB_SUM(vx[s] * vz[s]);
-    const double syz = WB_SUM(vy[s] * vz[s]);
-    const double s1z = WB_SUM(1.0 * vz[s]);
+    WB_SUM(F.sxx, x * x)
+    WB_SUM(F.syx, y * x)
+    WB_SUM(F.syy, y * y)
+    WB_SUM(F.s1x, 1.0 * x)
+    WB_SUM(F.s1y, 1.0 * y)
+    WB_SUM(F.sxz, x * z)
+    WB_SUM(F.syz, y * z)
+    WB_SUM(F.s1z, 1.0 * z)
 #undef WB_SUM
-    plane_tilt(sxx, syx, syy, s1x, s1y, s11, sxz, syz, s1z, &sx, &sy);
   }
-  double u[K];
-  double bottom = __builtin_inf(), top = -__builtin_inf();
+  fit_solve(F);
+  if (F32 && !fit64) {
+    F.sx = px;
+    F.sy = py;
+  }
+  uint32_t inexact = 0;  // points whose sector the exact form decides, bit K*j+s
 #pragma unroll
-  for (int s = 0; s < K; s++) {
-    u[s] = vz[s] - (sy * vy[s] + sx * vx[s]);
-    if (mine[s]) {
-      bottom = fmin(bottom, u[s]);
-      top = fmax(top, u[s]);
+  for (int j = 0; j < T; j++) {
+    const bool me = lane == (uint32_t)j;
+    const double sx = rdl(F.sx, j), sy = rdl(F.sy, j);
+    double u[K];
+    double bottom = __builtin_inf(), top = -__builtin_inf();
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      u[s] = vz[j][s] - (sy * vy[j][s] + sx * vx[j][s]);
+      if (s * WAVE + lane < m[j]) {
+        bottom = fmin(bottom, u[s]);
+        top = fmax(top, u[s]);
+      }
+    }
+    bottom = wave_dmin(bottom);
+    top = wave_dmax(top);
+    uint32_t first = 0xffffffffu;
+#pragma unroll
+    for (int s = K - 1; s >= 0; s--) {
+      const uint64_t atb = __ballot(s * WAVE + lane < m[j] && u[s] == bottom);
+      if (atb) first = s * WAVE + (uint32_t)(__ffsll((long long)atb) - 1);
+    }
+    double bottom2 = __builtin_inf();
+#pragma unroll
+    for (int s = 0; s < K; s++)
+      if (s * WAVE + lane < m[j] && s * WAVE + lane < first) bottom2 = fmin(bottom2, u[s]);
+    bottom2 = wave_dmin(bottom2);
+    if (wb::disinf(bottom2)) bottom2 = bottom;
+    if (me) {
+      F.bottom = bottom;
+      F.top = top;
+    }
+    // 7-sector histogram of the bottom layer
+    uint32_t nbottom = 0, hist[7] = {0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < K; s++) {
+      int sec = -1;
+      const bool low = s * WAVE + lane < m[j] && u[s] < bottom2 + 2 * r;
+      if (low) {
+        sec = wb::scan_sector_est(vx[j][s], vy[j][s], r);
+        if (sec < 0) inexact |= 1u << (K * j + s);
+      }
+      nbottom += (uint32_t)__popcll(__ballot(low));
+#pragma unroll
+      for (int k = 0; k < 7; k++) hist[k] += (uint32_t)__popcll(__ballot(sec == k));
+    }
+    if (me) {
+      F.nbottom = nbottom;
+#pragma unroll
+      for (int k = 0; k < 7; k++) F.hist[k] = hist[k];
     }
   }
-  bottom = wave_dmin(bottom);
-  top = wave_dmax(top);
-  uint32_t first = 0xffffffffu;
+  if (__ballot(inexact != 0)) {
+    uint32_t nedge = 0;
 #pragma unroll
-  for (int s = K - 1; s >= 0; s--) {
-    const uint64_t atb = __ballot(mine[s] && u[s] == bottom);
-    if (atb) first = s * WAVE + (uint32_t)(__ffsll((long long)atb) - 1);
+    for (int j = 0; j < T; j++)
+#pragma unroll
+      for (int s = 0; s < K; s++) {
+        const bool ask = (inexact >> (K * j + s)) & 1u;
+        if (!__ballot(ask)) continue;
+        int sec = -1, edge = 0;
+        if (ask) {
+          double cx, cy;
+          tile_center(g, tex[t[j]], tey[t[j]], &cx, &cy);
+          sec = wb::scan_sector_exact(V.px[q[j][s]] - cx, V.py[q[j][s]] - cy, r, &edge);
+        }
+        nedge += (uint32_t)__popcll(__ballot(edge != 0));
+#pragma unroll
+        for (int k = 0; k < 7; k++) {
+          const uint32_t h = (uint32_t)__popcll(__ballot(sec == k));
+          if (lane == (uint32_t)j) F.hist[k] += h;
+        }
+      }
+    if (nedge && lane == 0) atomicAdd(&ctr[0], (unsigned long long)nedge);
   }
-  double bottom2 = __builtin_inf();
+  uint32_t tl = 0;
 #pragma unroll
-  for (int s = 0; s < K; s++)
-    if (mine[s] && s * WAVE + lane < first) bottom2 = fmin(bottom2, u[s]);
-  bottom2 = wave_dmin(bottom2);
-  if (wb::disinf(bottom2)) bottom2 = bottom;
-  // 7-sector histogram of the bottom layer
-  uint32_t nbottom = 0, nedge = 0, hist[7] = {0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int s = 0; s < K; s++) {
-    int sec = -1;
-    bool edge = false;
-    if (mine[s] && u[s] < bottom2 + 2 * r) {
-      int e = 0;
-      sec = wb::scan_sector(vx[s], vy[s], r, &e);
-      edge = e != 0;
-    }
-    nbottom += (uint32_t)__popcll(__ballot(sec >= 0));
-    nedge += (uint32_t)__popcll(__ballot(edge));
-    for (int k = 0; k < 7; k++) hist[k] += (uint32_t)__popcll(__ballot(sec == k));
-  }
-  if (lane == 0) {
-    if (nedge) atomicAdd(&ctr[0], (unsigned long long)nedge);
-    double density = 0;
-    int tree = 0;
-    for (int i = 0; i < 7; i++) density += (int)hist[i] * (int)hist[i];
-    if (m > nbottom && density < 7) tree = 1;
-    density = sqrt(density) * kSqrt7 / (r * r) / M_PI;
-    if (m > nbottom && density < 0.5) tree = 1;
-    if (top - bottom > 1.5) tree = 1;
-    TileRec rr;
-    rr.npoints = (int32_t)m;
-    rr.nground = 0;
-    rr.tree_flags = tree;
-    rr.fit_fp64 = fell_back;
-    rr.density = density;
-    rr.hs_scan = sqrt(1 / density + min_hs * min_hs);
-    rr.hs = rr.hs_scan;
-    rr.height = top - bottom;
-    rr.tilt_x = sx;
-    rr.tilt_y = sy;
-    *out = rr;
+  for (int j = 0; j < T; j++)
+    if (lane == (uint32_t)j) tl = t[j];
+  if (lane < T && F.m) {
+    fit_record(F, r, min_hs, fell_back, rec + tl);
     if (fell_back) atomicAdd(&ctr[7], 1ull);
   }
 }
 
-// Size classes of the scan: 0 = 1..16 points, 1 = 17-32, 2 = 33-64,
-// 3 = 65-128, 4 = 129-256, 5 = more.  One thread per tile: an empty tile gets
-// its record here, every other tile goes on its class's list (classes 0 and
-// 5 from the front and the back of la, 2 and 4 of lb, 1 and 3 of lc; ncls[c]
-// the lengths), so each class kernel visits only its own tiles.  The order
-// inside a list does not matter: every tile's record depends on that tile
-// alone.
-#define SCAN_NCLS 6
-__device__ inline int scan_class(uint32_t m)
+// Size classes of the scan: 0 = 1..tiny points, 1 = up to 16, 2 = 17-32, 3 = 33-64,
+// 4 = 65-128, 5 = 129-256, 6 = more.  One thread per tile: every tile with
+// points goes on its class's list (the lists of classes 0 and 6 fill la from
+// the front and the back, 1 and 5 lb, 2 and 4 lc, 3 ld; ncls[c] the lengths),
+// so each class kernel visits only its own tiles.  The order inside a list
+// does not matter: every tile's record depends on that tile alone.  An empty
+// tile's record is written only where the caller gets the records: 64 B for
+// each of 27.8M tile numbers, most of them empty, took 0.5 ms.
+#define SCAN_NCLS 7
+// Points from which each class takes its own launch, several tiles per step
+// (and tiny tiles a lane each).  Mixed and own launches, scan and postscan in
+// ms: 300k points 0.075 and 0.17, 1.17M 0.195 and 0.22, 2.4M 0.31 and 0.28,
+// 2.4M at 8 points per m2 0.48 and 0.28, 10M 1.10 and 0.80 to 0.90.
+#define SCAN_MANY (3u << 19)
+// blocks of a scan launch (resident ones take more than one step; launching
+// 65536 empty blocks takes 15 us)
+#define SCAN_GRID 8192
+__device__ inline int scan_class(uint32_t m, uint32_t tiny)
 {
-  return m == 0 ? -1 : m <= 16 ? 0 : m <= 32 ? 1 : m <= WAVE ? 2 : m <= 2 * WAVE ? 3 : m <= 4 * WAVE ? 4 : 5;
+  return m == 0          ? -1
+         : m <= tiny     ? 0
+         : m <= 16       ? 1
+         : m <= 32       ? 2
+         : m <= WAVE     ? 3
+         : m <= 2 * WAVE ? 4
+         : m <= 4 * WAVE ? 5
+                         : 6;
 }
 
 __global__ void __launch_bounds__(1024) k_scan_classes(uint32_t ntiles, const uint32_t *tile_cnt,
                                                       uint32_t *la, uint32_t *lb, uint32_t *lc,
-                                                      uint32_t *ncls, TileRec *rec)
+                                                      uint32_t *ld, uint32_t *ncls,
+                                                      uint32_t tiny, int want_empty, TileRec *rec)
 {
   // slots are claimed per block: the waves' class counts summed in LDS, one
   // atomic per class and block (atomics on the list counters are
@@ -1478,11 +1609,11 @@ __global__ void __launch_bounds__(1024) k_scan_classes(uint32_t ntiles, const ui
   __shared__ uint32_t bbase[SCAN_NCLS];
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t m = t < ntiles ? tile_cnt[t] : 0u;
-  if (t < ntiles && m == 0) {
+  if (want_empty && t < ntiles && m == 0) {
     TileRec r = {0, 0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     rec[t] = r;
   }
-  const int c = scan_class(m);
+  const int c = scan_class(m, tiny);
   const uint32_t lane = __lane_id(), w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
   uint64_t mk[SCAN_NCLS];
 #pragma unroll
@@ -1506,10 +1637,11 @@ __global__ void __launch_bounds__(1024) k_scan_classes(uint32_t ntiles, const ui
   const uint32_t pos = bbase[c] + wcnt[c][w] + (uint32_t)__popcll(mk[c] & ((1ull << lane) - 1));
   switch (c) {
   case 0: la[pos] = t; break;
-  case 1: lc[pos] = t; break;
-  case 2: lb[pos] = t; break;
-  case 3: lc[ntiles - 1 - pos] = t; break;
-  case 4: lb[ntiles - 1 - pos] = t; break;
+  case 1: lb[pos] = t; break;
+  case 2: lc[pos] = t; break;
+  case 3: ld[pos] = t; break;
+  case 4: lc[ntiles - 1 - pos] = t; break;
+  case 5: lb[ntiles - 1 - pos] = t; break;
   default: la[ntiles - 1 - pos] = t; break;
   }
 }
@@ -1523,31 +1655,36 @@ struct ClassList {
   __device__ uint32_t at(uint32_t i) const { return list[(int64_t)step * i]; }
 };
 
-// One wave per tile, over the tiles of one size class: up to 64, 65-128 and
-// 129-256 points (K = 1, 2, 4 points per lane).  Each class has its own
-// register budget.  The next tile's number is read before this tile's scan.
-#ifndef WB_SCAN_MINW
-#define WB_SCAN_MINW 5
-#endif
+// T tiles per wave and step, over the tiles of one size class: up to 64,
+// 65-128 and 129-256 points (K = 1, 2, 4 points per lane).  Each class has its
+// own register budget.  The next tiles' numbers are read before these tiles'
+// scan.
 // F32: the kernel of the FP32 fit options (the precision study); the FP64
 // kernel does not carry their code or registers.
-template <int K, bool F32>
-__global__ void __launch_bounds__(64, WB_SCAN_MINW) k_scan_reg(TreeView T, TileGeo g, const int32_t *tex,
+template <int K, bool F32, int T, int MINW>
+__global__ void __launch_bounds__(64, MINW) k_scan_reg(TreeView V, TileGeo g, const int32_t *tex,
                                                  const int32_t *tey, const uint32_t *tile_off,
                                                  const uint32_t *tile_cnt, const uint32_t *lists,
                                                  ClassList cl, double min_hs, int prec,
                                                  TileRec *rec, unsigned long long *ctr)
 {
-  const uint32_t n = *cl.n;
-  uint32_t i = blockIdx.x;
+  const uint32_t n = (uint32_t)rfl((int)*cl.n);
+  uint32_t i = blockIdx.x * T;
   if (i >= n) return;
-  uint32_t t = cl.at(i);
-  for (; i < n; i += gridDim.x) {
-    const uint32_t inext = i + gridDim.x;
-    const uint32_t tnext = inext < n ? cl.at(inext) : 0u;
-    scan_reg<K, F32>(T, g, tex[t], tey[t], tile_off[t], tile_cnt[t], lists, min_hs, prec, rec + t,
-                     ctr);
-    t = tnext;
+  uint32_t next[T];
+#pragma unroll
+  for (int j = 0; j < T; j++) next[j] = i + j < n ? cl.at(i + j) : 0xffffffffu;
+  for (; i < n; i += gridDim.x * T) {
+    uint32_t t[T], m[T];
+#pragma unroll
+    for (int j = 0; j < T; j++) {
+      const bool live = next[j] != 0xffffffffu;
+      t[j] = live ? next[j] : 0u;
+      m[j] = live ? tile_cnt[t[j]] : 0u;
+      const uint32_t k = i + gridDim.x * T + j;
+      next[j] = k < n ? cl.at(k) : 0xffffffffu;
+    }
+    scan_reg<K, F32, T>(V, g, t, m, tex, tey, tile_off, lists, min_hs, prec, rec, ctr);
   }
 }
 
@@ -1608,106 +1745,316 @@ __device__ inline double group_dmax(double v)
   return v;
 }
 
-template <int GS>
-__device__ __attribute__((always_inline)) inline void scan_group(
-    const TreeView &T, const TileGeo &g, bool live, int ex, int ey, uint32_t off, uint32_t m,
-    const uint32_t *lists, double min_hs, TileRec *out, unsigned long long *ctr)
+// WAVE/GS tiles of the class list at a time and R rounds of them per wave and
+// step (the FP64 fit; the FP32 options take these tiles through
+// k_scan_reg<1>): entries i0 on of the n.  Lane NG*j + q takes the fit of
+// round j's group q.
+template <int GS, int R>
+__device__ __attribute__((always_inline)) inline void scan_rows(
+    const TreeView &V, const TileGeo &g, const int32_t *tex, const int32_t *tey,
+    const uint32_t *tile_off, const uint32_t *tile_cnt, const uint32_t *lists, const ClassList &cl,
+    uint32_t n, uint32_t i0, double min_hs, TileRec *rec, unsigned long long *ctr)
 {
-  const uint32_t lane = __lane_id(), gl = lane % GS, gbase = lane - gl;
-  const uint64_t gmask = (GS == 64 ? ~0ull : ((1ull << GS) - 1)) << gbase;
-  uint32_t c[1] = {live && gl < m ? lists[off + gl] : 0xffffffffu};
-  {
+  constexpr uint32_t NG = WAVE / GS;
+  const uint32_t lane = __lane_id(), grp = lane / GS, gl = lane % GS, gbase = lane - gl;
+  const uint64_t gmask = ((1ull << GS) - 1) << gbase;
+  const int src = (int)(lane % NG * GS);  // a lane of the group whose fit this one takes
+  const double r = g.r;
+  uint32_t t[R], m[R], q[R];
+  double vx[R], vy[R], vz[R];
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const uint32_t i = i0 + j * NG + grp;
+    t[j] = i < n ? cl.at(i) : 0u;
+    m[j] = i < n ? tile_cnt[t[j]] : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    uint32_t c[1] = {gl < m[j] ? lists[tile_off[t[j]] + gl] : 0xffffffffu};
     // canonical order inside each group: the network on GS lanes sorts every
     // aligned group of GS lanes on its own (pads last)
     uint32_t unused[1];
     wbw::wave_sort<1, false>(c, unused, GS);
+    q[j] = gl < m[j] ? V.canon[c[0]] : 0u;
   }
-  double cx = 0, cy = 0;
-  if (live) tile_center(g, ex, ey, &cx, &cy);
-  const double r = g.r;
-  const bool mine = live && gl < m;
-  double vx = 0, vy = 0, vz = 0;
-  if (mine) {
-    const uint32_t q = T.canon[c[0]];
-    vx = T.px[q] - cx;
-    vy = T.py[q] - cy;
-    vz = T.pz[q] - 0;
-  }
-  const double sxx = group_pairwise<GS>(vx * vx, m, gbase);
-  const double syx = group_pairwise<GS>(vy * vx, m, gbase);
-  const double syy = group_pairwise<GS>(vy * vy, m, gbase);
-  const double s1x = group_pairwise<GS>(1.0 * vx, m, gbase);
-  const double s1y = group_pairwise<GS>(1.0 * vy, m, gbase);
-  const double s11 = group_pairwise<GS>(1.0 * 1.0, m, gbase);
-  const double sxz = group_pairwise<GS>(vx * vz, m, gbase);
-  const double syz = group_pairwise<GS>(vy * vz, m, gbase);
-  const double s1z = group_pairwise<GS>(1.0 * vz, m, gbase);
-  double sx = 0, sy = 0;
-  plane_tilt(sxx, syx, syy, s1x, s1y, s11, sxz, syz, s1z, &sx, &sy);
-  const double u = vz - (sy * vy + sx * vx);
-  const double bottom = group_dmin<GS>(mine ? u : __builtin_inf());
-  const double top = group_dmax<GS>(mine ? u : -__builtin_inf());
-  const uint64_t atb = __ballot(mine && u == bottom) & gmask;
-  const uint32_t first = atb ? (uint32_t)(__ffsll((long long)atb) - 1) - gbase : 0xffffffffu;
-  double bottom2 = group_dmin<GS>(mine && gl < first ? u : __builtin_inf());
-  if (wb::disinf(bottom2)) bottom2 = bottom;
-  // 7-sector histogram of the bottom layer
-  int sec = -1;
-  bool edge = false;
-  if (mine && u < bottom2 + 2 * r) {
-    int e = 0;
-    sec = wb::scan_sector(vx, vy, r, &e);
-    edge = e != 0;
-  }
-  const uint32_t nbottom = (uint32_t)__popcll(__ballot(sec >= 0) & gmask);
-  const uint32_t nedge = (uint32_t)__popcll(__ballot(edge) & gmask);
-  uint32_t hist[7];
+  TileFit F;
+  F.m = 0;
+  F.sxx = F.syx = F.syy = F.s1x = F.s1y = F.sxz = F.syz = F.s1z = 0;
+  uint32_t tl = 0;
 #pragma unroll
-  for (int k = 0; k < 7; k++) hist[k] = (uint32_t)__popcll(__ballot(sec == k) & gmask);
-  if (live && gl == 0) {
-    if (nedge) atomicAdd(&ctr[0], (unsigned long long)nedge);
-    double density = 0;
-    int tree = 0;
-    for (int i = 0; i < 7; i++) density += (int)hist[i] * (int)hist[i];
-    if (m > nbottom && density < 7) tree = 1;
-    density = sqrt(density) * kSqrt7 / (r * r) / M_PI;
-    if (m > nbottom && density < 0.5) tree = 1;
-    if (top - bottom > 1.5) tree = 1;
-    TileRec rr;
-    rr.npoints = (int32_t)m;
-    rr.nground = 0;
-    rr.tree_flags = tree;
-    rr.fit_fp64 = 0;
-    rr.density = density;
-    rr.hs_scan = sqrt(1 / density + min_hs * min_hs);
-    rr.hs = rr.hs_scan;
-    rr.height = top - bottom;
-    rr.tilt_x = sx;
-    rr.tilt_y = sy;
-    *out = rr;
+  for (int j = 0; j < R; j++) {
+    vx[j] = vy[j] = vz[j] = 0;
+    if (gl < m[j]) {
+      double cx, cy;
+      tile_center(g, tex[t[j]], tey[t[j]], &cx, &cy);
+      vx[j] = V.px[q[j]] - cx;
+      vy[j] = V.py[q[j]] - cy;
+      vz[j] = V.pz[q[j]] - 0;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const bool me = lane / NG == (uint32_t)j;
+    const uint32_t mj = (uint32_t)__shfl((int)m[j], src, WAVE);
+    const uint32_t tj = (uint32_t)__shfl((int)t[j], src, WAVE);
+    if (me) {
+      F.m = mj;
+      tl = tj;
+    }
+#define WB_SUM(dst, expr)                                           \
+{                                                                 \
+  const double x = vx[j], y = vy[j], z = vz[j];                   \
+  (void)x, (void)y, (void)z;                                      \
+  const double sum = __shfl(group_pairwise<GS>((expr), m[j], gbase), src, WAVE); \
+  if (me) dst = sum;                                              \
+}
+    WB_SUM(F.sxx, x * x)
+    WB_SUM(F.syx, y * x)
+    WB_SUM(F.syy, y * y)
+    WB_SUM(F.s1x, 1.0 * x)
+    WB_SUM(F.s1y, 1.0 * y)
+    WB_SUM(F.sxz, x * z)
+    WB_SUM(F.syz, y * z)
+    WB_SUM(F.s1z, 1.0 * z)
+#undef WB_SUM
+  }
+  fit_solve(F);
+  uint32_t inexact = 0;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const bool me = lane / NG == (uint32_t)j;
+    const double sx = __shfl(F.sx, (int)(j * NG + grp), WAVE);
+    const double sy = __shfl(F.sy, (int)(j * NG + grp), WAVE);
+    const bool mine = gl < m[j];
+    const double u = vz[j] - (sy * vy[j] + sx * vx[j]);
+    const double bottom = group_dmin<GS>(mine ? u : __builtin_inf());
+    const double top = group_dmax<GS>(mine ? u : -__builtin_inf());
+    const uint64_t atb = __ballot(mine && u == bottom) & gmask;
+    const uint32_t first = atb ? (uint32_t)(__ffsll((long long)atb) - 1) - gbase : 0xffffffffu;
+    double bottom2 = group_dmin<GS>(mine && gl < first ? u : __builtin_inf());
+    if (wb::disinf(bottom2)) bottom2 = bottom;
+    // 7-sector histogram of the bottom layer
+    int sec = -1;
+    const bool low = mine && u < bottom2 + 2 * r;
+    if (low) {
+      sec = wb::scan_sector_est(vx[j], vy[j], r);
+      if (sec < 0) inexact |= 1u << j;
+    }
+    const double bs = __shfl(bottom, src, WAVE), ts = __shfl(top, src, WAVE);
+    const uint64_t smask = ((1ull << GS) - 1) << src;
+    const uint32_t nb = (uint32_t)__popcll(__ballot(low) & smask);
+    if (me) {
+      F.bottom = bs;
+      F.top = ts;
+      F.nbottom = nb;
+    }
+#pragma unroll
+    for (int k = 0; k < 7; k++) {
+      const uint32_t h = (uint32_t)__popcll(__ballot(sec == k) & smask);
+      if (me) F.hist[k] = h;
+    }
+  }
+  if (__ballot(inexact != 0)) {
+    uint32_t nedge = 0;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const bool ask = (inexact >> j) & 1u;
+      if (!__ballot(ask)) continue;
+      int sec = -1, edge = 0;
+      if (ask) {
+        double cx, cy;
+        tile_center(g, tex[t[j]], tey[t[j]], &cx, &cy);
+        sec = wb::scan_sector_exact(V.px[q[j]] - cx, V.py[q[j]] - cy, r, &edge);
+      }
+      nedge += (uint32_t)__popcll(__ballot(edge != 0));
+      const uint64_t smask = ((1ull << GS) - 1) << src;
+#pragma unroll
+      for (int k = 0; k < 7; k++) {
+        const uint32_t h = (uint32_t)__popcll(__ballot(sec == k) & smask);
+        if (lane / NG == (uint32_t)j) F.hist[k] += h;
+      }
+    }
+    if (nedge && lane == 0) atomicAdd(&ctr[0], (unsigned long long)nedge);
+  }
+  if (lane < NG * R && F.m) fit_record(F, r, min_hs, 0, rec + tl);
+}
+
+template <int GS, int R, int MINW>
+__global__ void __launch_bounds__(64, MINW) k_scan_row(TreeView V, TileGeo g, const int32_t *tex,
+                                                       const int32_t *tey, const uint32_t *tile_off,
+                                                       const uint32_t *tile_cnt,
+                                                       const uint32_t *lists, ClassList cl,
+                                                       double min_hs, TileRec *rec,
+                                                       unsigned long long *ctr)
+{
+  constexpr uint32_t per = WAVE / GS * R;
+  const uint32_t n = (uint32_t)rfl((int)*cl.n);
+  for (uint32_t i0 = blockIdx.x * per; i0 < n; i0 += gridDim.x * per)
+    scan_rows<GS, R>(V, g, tex, tey, tile_off, tile_cnt, lists, cl, n, i0, min_hs, rec, ctr);
+}
+
+// The classes of 1 to 256 points in one launch, for the clouds whose classes
+// do not fill the chip one by one: a step of a class per block (16-lane groups
+// for up to 16 points, 32-lane groups, then a wave per tile).  As five
+// launches the chain took the longest tile of each in turn (18.5k points 65
+// us, 300k points 126 us, scan and postscan, against 50 and 75 us).
+__global__ void __launch_bounds__(64, 4) k_scan_mixed(TreeView V, TileGeo g, const int32_t *tex,
+                                                      const int32_t *tey, const uint32_t *tile_off,
+                                                      const uint32_t *tile_cnt,
+                                                      const uint32_t *lists, ClassList c16,
+                                                      ClassList c32, ClassList c64, ClassList c128,
+                                                      ClassList c256, double min_hs, TileRec *rec,
+                                                      unsigned long long *ctr)
+{
+  const uint32_t n16 = (uint32_t)rfl((int)*c16.n), n32 = (uint32_t)rfl((int)*c32.n);
+  const uint32_t n64 = (uint32_t)rfl((int)*c64.n), n128 = (uint32_t)rfl((int)*c128.n);
+  const uint32_t n256 = (uint32_t)rfl((int)*c256.n);
+  // the longest steps first
+  const uint32_t e256 = n256, e128 = e256 + n128, e64 = e128 + n64, e32 = e64 + (n32 + 1) / 2;
+  const uint32_t end = e32 + (n16 + 3) / 4;
+  for (uint32_t u = blockIdx.x; u < end; u += gridDim.x) {
+    if (u >= e32) {
+      scan_rows<16, 1>(V, g, tex, tey, tile_off, tile_cnt, lists, c16, n16, 4 * (u - e32), min_hs,
+                       rec, ctr);
+    } else if (u >= e64) {
+      scan_rows<32, 1>(V, g, tex, tey, tile_off, tile_cnt, lists, c32, n32, 2 * (u - e64), min_hs,
+                       rec, ctr);
+    } else {
+      const uint32_t t[1] = {u >= e128 ? c64.at(u - e128) : u >= e256 ? c128.at(u - e256) : c256.at(u)};
+      const uint32_t m[1] = {tile_cnt[t[0]]};
+      if (u >= e128)
+        scan_reg<1, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, ctr);
+      else if (u >= e256)
+        scan_reg<2, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, ctr);
+      else
+        scan_reg<4, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, ctr);
+    }
   }
 }
 
-// WAVE/GS tiles of the class list per wave, grid-stride over the list (the
-// FP64 fit; the FP32 options take these tiles through k_scan_reg<1>)
-template <int GS>
-__global__ void __launch_bounds__(64, WB_SCAN_MINW) k_scan_row(TreeView T, TileGeo g,
-                                                             const int32_t *tex, const int32_t *tey,
-                                                             const uint32_t *tile_off,
-                                                             const uint32_t *tile_cnt,
-                                                             const uint32_t *lists, ClassList cl,
-                                                             double min_hs, TileRec *rec,
-                                                             unsigned long long *ctr)
+// ---------------------------------------------------------------------------
+// Tiles of at most 8 points, a lane each (the FP64 fit): the operations of
+// scan_reg<1> in the same order on one lane's registers.  Sixteen lanes per
+// tile took 1.62 ms for the 2.0M such tiles of a sparse 4M-point cloud, this
+// 0.26 ms.
+// ---------------------------------------------------------------------------
+// pairwisesum of the first m (1..8) of v
+__device__ inline double lane_pairwise(const double (&v)[8], uint32_t m)
 {
-  constexpr uint32_t NG = WAVE / GS;
+  const double p01 = v[0] + v[1], p23 = v[2] + v[3], p45 = v[4] + v[5], p67 = v[6] + v[7];
+  const double q03 = p01 + p23;
+  double acc = 0;
+  if (m & 1) acc = acc + (m == 1 ? v[0] : m == 3 ? v[2] : m == 5 ? v[4] : v[6]);
+  if (m & 2) acc = acc + (m & 4 ? p45 : p01);
+  if (m & 4) acc = acc + q03;
+  if (m & 8) acc = acc + (q03 + (p45 + p67));
+  return acc;
+}
+
+__global__ void __launch_bounds__(64) k_scan_lane(TreeView V, TileGeo g, const int32_t *tex,
+                                                  const int32_t *tey, const uint32_t *tile_off,
+                                                  const uint32_t *tile_cnt, const uint32_t *lists,
+                                                  ClassList cl, double min_hs, TileRec *rec,
+                                                  unsigned long long *ctr)
+{
   const uint32_t n = *cl.n;
-  const uint32_t grp = __lane_id() / GS;
-  for (uint32_t i0 = blockIdx.x * NG; i0 < n; i0 += gridDim.x * NG) {
-    const uint32_t i = i0 + grp;
-    const bool live = i < n;
-    const uint32_t t = live ? cl.at(i) : 0u;
-    scan_group<GS>(T, g, live, live ? tex[t] : 0, live ? tey[t] : 0, live ? tile_off[t] : 0u,
-                   live ? tile_cnt[t] : 0u, lists, min_hs, rec + t, ctr);
+  const double r = g.r;
+  for (uint32_t i = blockIdx.x * WAVE + threadIdx.x; i < n; i += gridDim.x * WAVE) {
+    const uint32_t t = cl.at(i), m = tile_cnt[t], off = tile_off[t];
+    uint32_t c[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) c[s] = (uint32_t)s < m ? lists[off + s] : 0xffffffffu;
+    // canonical order (Batcher's network for eight)
+    constexpr int net[19][2] = {{0, 1}, {2, 3}, {4, 5}, {6, 7}, {0, 2}, {1, 3}, {4, 6},
+                                {5, 7}, {1, 2}, {5, 6}, {0, 4}, {1, 5}, {2, 6}, {3, 7},
+                                {2, 4}, {3, 5}, {1, 2}, {3, 4}, {5, 6}};
+#pragma unroll
+    for (int k = 0; k < 19; k++) {
+      const uint32_t lo = min(c[net[k][0]], c[net[k][1]]), hi = max(c[net[k][0]], c[net[k][1]]);
+      c[net[k][0]] = lo;
+      c[net[k][1]] = hi;
+    }
+    double cx, cy, x[8], y[8], z[8], a[8];
+    tile_center(g, tex[t], tey[t], &cx, &cy);
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      x[s] = y[s] = z[s] = 0;
+      if ((uint32_t)s < m) {
+        const uint32_t q = V.canon[c[s]];
+        x[s] = V.px[q] - cx;
+        y[s] = V.py[q] - cy;
+        z[s] = V.pz[q] - 0;
+      }
+    }
+    TileFit F;
+    F.m = m;
+#define WB_SUM(dst, expr)                                     \
+  {                                                           \
+    _Pragma("unroll") for (int s = 0; s < 8; s++) a[s] = (expr); \
+    dst = lane_pairwise(a, m);                                \
+  }
+    WB_SUM(F.sxx, x[s] * x[s])
+    WB_SUM(F.syx, y[s] * x[s])
+    WB_SUM(F.syy, y[s] * y[s])
+    WB_SUM(F.s1x, 1.0 * x[s])
+    WB_SUM(F.s1y, 1.0 * y[s])
+    WB_SUM(F.sxz, x[s] * z[s])
+    WB_SUM(F.syz, y[s] * z[s])
+    WB_SUM(F.s1z, 1.0 * z[s])
+#undef WB_SUM
+    fit_solve(F);
+    F.bottom = __builtin_inf();
+    F.top = -__builtin_inf();
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      a[s] = z[s] - (F.sy * y[s] + F.sx * x[s]);
+      if ((uint32_t)s < m) {
+        F.bottom = fmin(F.bottom, a[s]);
+        F.top = fmax(F.top, a[s]);
+      }
+    }
+    // the lowest of the points before the first that is at the bottom
+    double bottom2 = __builtin_inf();
+    bool before = true;
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      before = before && (uint32_t)s < m && a[s] != F.bottom;
+      if (before) bottom2 = fmin(bottom2, a[s]);
+    }
+    if (wb::disinf(bottom2)) bottom2 = F.bottom;
+    // 7-sector histogram of the bottom layer, four bits a sector
+    uint32_t h = 0, inexact = 0;
+    F.nbottom = 0;
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+      if ((uint32_t)s < m && a[s] < bottom2 + 2 * r) {
+        F.nbottom++;
+        const int sec = wb::scan_sector_est(x[s], y[s], r);
+        if (sec < 0) inexact |= 1u << s;
+        else h += 1u << (4 * sec);
+      }
+    if (inexact) {
+      uint32_t nedge = 0;
+      for (int s = 0; s < 8; s++)
+        if ((inexact >> s) & 1u) {
+          const uint32_t cs = s == 0   ? c[0]
+                              : s == 1 ? c[1]
+                              : s == 2 ? c[2]
+                              : s == 3 ? c[3]
+                              : s == 4 ? c[4]
+                              : s == 5 ? c[5]
+                              : s == 6 ? c[6]
+                                       : c[7];
+          const uint32_t q = V.canon[cs];
+          int edge = 0;
+          h += 1u << (4 * wb::scan_sector_exact(V.px[q] - cx, V.py[q] - cy, r, &edge));
+          nedge += edge != 0;
+        }
+      if (nedge) atomicAdd(&ctr[0], (unsigned long long)nedge);
+    }
+#pragma unroll
+    for (int k = 0; k < 7; k++) F.hist[k] = (h >> (4 * k)) & 15u;
+    fit_record(F, r, min_hs, 0, rec + t);
   }
 }
 
@@ -1839,7 +2186,8 @@ __global__ void __launch_bounds__(64) k_scan(TreeView T, TileGeo g, const int32_
 // POSTSCAN (scan.cpp:142-179): tree tiles widen their hyperboloid by the
 // number of tree tiles met along six rays before an empty ring or a
 // non-tree tile.
-__global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey, TileRec *rec,
+__global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey,
+                           const uint32_t *tile_cnt, TileRec *rec,
                            unsigned long long *nonempty)
 {
   // the non-empty tiles counted per block (one atomic on the counter per
@@ -1848,7 +2196,7 @@ __global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey, Ti
   if (threadIdx.x == 0) bcount = 0;
   __syncthreads();
   uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = t < g.ntiles && rec[t].npoints;
+  const bool live = t < g.ntiles && tile_cnt[t];
   const uint64_t lv = __ballot(live);
   if (__lane_id() == 0 && lv) atomicAdd(&bcount, (uint32_t)__popcll(lv));
   __syncthreads();
@@ -1862,10 +2210,9 @@ __global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey, Ti
     for (int j = 0; j < 6 && (me.tree_flags & 1); j++) {
       int o;
       if (!tile_at(g, tex[t] + r1x[j] * i, tey[t] + r1y[j] * i, &o)) continue;
-      const TileRec &q = rec[o - g.lo];
-      if (q.npoints) {
+      if (tile_cnt[o - g.lo]) {
         ring++;
-        if (q.tree_flags & 1) count++;
+        if (rec[o - g.lo].tree_flags & 1) count++;
         else nontree++;
       }
     }
@@ -3581,7 +3928,7 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
   // err[0] error flags; then u64 counters: 0 sector borderline, 1 exact atan2i
   // steps, 2-4 class histogram, 5 non-empty tiles, 6 (two u32) exact gap
   // points and heavy points, 7 FP64 fit fallbacks; u32 18-19 work counters of
-  // the heavy and resident ground kernels, 20-25 the scan's class list lengths;
+  // the heavy and resident ground kernels, 20-26 the scan's class list lengths;
   // past the words the host reads: 32-37 walk B's units of each class, records
   // and units taken, u64 at 38 its leaf list entries
   uint32_t *err = R.err = (uint32_t *)wb_alloc(c, 256);
@@ -3621,44 +3968,60 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
     uint32_t *la = tile_fill;  // free until the ground counts
     uint32_t *lb = (uint32_t *)wb_alloc(c, 4ull * g.ntiles + 4);
     uint32_t *lc = (uint32_t *)wb_alloc(c, 4ull * g.ntiles + 4);
+    uint32_t *ld = (uint32_t *)wb_alloc(c, 4ull * g.ntiles + 4);
     uint32_t *ncls = err + 20;
-    const unsigned nb = (unsigned)std::min<uint64_t>(g.ntiles, 1u << 16);
+    // a wave per step of a class's kernel: no more than there can be points
+    // for, and no more than keep the chip busy
+    auto nb = [&](uint64_t least, unsigned per) {
+      const uint64_t tiles = std::min<uint64_t>(g.ntiles, MAX_MEMB * n / least + 1);
+      return dim3((unsigned)std::min<uint64_t>((tiles + per - 1) / per, SCAN_GRID));
+    };
     const int prec = p->fit_precision;
-    if (nb) {
+    const bool many = n >= SCAN_MANY && prec == WB_FIT_FP64;
+    if (g.ntiles) {
       hipLaunchKernelGGL(k_scan_classes, dim3(wb_blocks(g.ntiles, 1024)), dim3(1024), 0, st,
-                         g.ntiles, tile_cnt, la, lb, lc, ncls, rec);
+                         g.ntiles, tile_cnt, la, lb, lc, ld, ncls, many ? 8u : 0u, want_tiles ? 1 : 0,
+                         rec);
       const uint32_t e = g.ntiles - 1;
-      const ClassList c16 = {la, 1, ncls}, c32 = {lc, 1, ncls + 1}, c64 = {lb, 1, ncls + 2};
-      const ClassList c128 = {lc + e, -1, ncls + 3}, c256 = {lb + e, -1, ncls + 4};
-      const ClassList cbig = {la + e, -1, ncls + 5};
-#define WB_SCAN_REG(K, F32, CL)                                                                   \
-  hipLaunchKernelGGL((k_scan_reg<K, F32>), dim3(nb), dim3(64), 0, st, T, g, tex, tey, tile_off,   \
-                     tile_cnt, lists, CL, p->min_hs, prec, rec, ctr)
-      if (prec == WB_FIT_FP64) {
-        // tiles of up to 16 and 32 points four and two to a wave
-        hipLaunchKernelGGL(k_scan_row<16>, dim3(nb), dim3(64), 0, st, T, g, tex, tey, tile_off,
-                           tile_cnt, lists, c16, p->min_hs, rec, ctr);
-        hipLaunchKernelGGL(k_scan_row<32>, dim3(nb), dim3(64), 0, st, T, g, tex, tey, tile_off,
-                           tile_cnt, lists, c32, p->min_hs, rec, ctr);
-        WB_SCAN_REG(1, false, c64);
-        WB_SCAN_REG(2, false, c128);
-        WB_SCAN_REG(4, false, c256);
+      const ClassList c8 = {la, 1, ncls}, c16 = {lb, 1, ncls + 1}, c32 = {lc, 1, ncls + 2};
+      const ClassList c64 = {ld, 1, ncls + 3}, c128 = {lc + e, -1, ncls + 4};
+      const ClassList c256 = {lb + e, -1, ncls + 5}, cbig = {la + e, -1, ncls + 6};
+#define WB_SCAN_REG(K, F32, T, W, least, CL)                                                      \
+  hipLaunchKernelGGL((k_scan_reg<K, F32, T, W>), nb(least, T), dim3(64), 0, st, T_, g, tex, tey,  \
+                     tile_off, tile_cnt, lists, CL, p->min_hs, prec, rec, ctr)
+      const TreeView &T_ = T;
+      if (many) {
+        hipLaunchKernelGGL(k_scan_lane, nb(1, WAVE), dim3(64), 0, st, T, g, tex, tey, tile_off,
+                           tile_cnt, lists, c8, p->min_hs, rec, ctr);
+#define WB_SCAN_ROW(GS, R, W, least, CL)                                                          \
+  hipLaunchKernelGGL((k_scan_row<GS, R, W>), nb(least, WAVE / GS * R), dim3(64), 0, st, T, g, tex, \
+                     tey, tile_off, tile_cnt, lists, CL, p->min_hs, rec, ctr)
+        WB_SCAN_ROW(16, 4, 3, 9, c16);
+        WB_SCAN_ROW(32, 4, 3, 17, c32);
+        WB_SCAN_REG(1, false, 4, 4, 33, c64);
+        WB_SCAN_REG(2, false, 2, 4, 65, c128);
+#undef WB_SCAN_ROW
+        WB_SCAN_REG(4, false, 1, 4, 129, c256);
+      } else if (prec == WB_FIT_FP64) {
+        hipLaunchKernelGGL(k_scan_mixed, nb(1, 1), dim3(64), 0, st, T, g, tex, tey, tile_off, tile_cnt,
+                           lists, c16, c32, c64, c128, c256, p->min_hs, rec, ctr);
       } else {
-        WB_SCAN_REG(1, true, c16);
-        WB_SCAN_REG(1, true, c32);
-        WB_SCAN_REG(1, true, c64);
-        WB_SCAN_REG(2, true, c128);
-        WB_SCAN_REG(4, true, c256);
+        WB_SCAN_REG(1, true, 1, 4, 1, c16);
+        WB_SCAN_REG(1, true, 1, 4, 17, c32);
+        WB_SCAN_REG(1, true, 1, 4, 33, c64);
+        WB_SCAN_REG(2, true, 1, 4, 65, c128);
+        WB_SCAN_REG(4, true, 1, 4, 129, c256);
       }
 #undef WB_SCAN_REG
-      hipLaunchKernelGGL(k_scan, dim3(std::min(nb, 4096u)), dim3(64), 0, st, T, g, tex, tey,
-                         tile_off, tile_cnt, lists, cbig, p->min_hs, prec, rec, err, ctr);
+      hipLaunchKernelGGL(k_scan, dim3(std::min(nb(257, 1).x, 4096u)), dim3(64), 0, st, T, g, tex,
+                         tey, tile_off, tile_cnt, lists, cbig, p->min_hs, prec, rec, err, ctr);
     }
     wb_free(c, lb, 4ull * g.ntiles + 4);
     wb_free(c, lc, 4ull * g.ntiles + 4);
+    wb_free(c, ld, 4ull * g.ntiles + 4);
   }
-  hipLaunchKernelGGL(k_postscan, dim3(wb_blocks(g.ntiles, 256)), dim3(256), 0, st, g, tex, tey, rec,
-                     ctr + 5);
+  hipLaunchKernelGGL(k_postscan, dim3(wb_blocks(g.ntiles, 256)), dim3(256), 0, st, g, tex, tey,
+                     tile_cnt, rec, ctr + 5);
   WB_CHECK(hipEventRecord(ev[2], st));
   for (int k = 4; k < 8; k++) WB_CHECK(hipEventRecord(ev[k], st));
   if (scan_only) return;

@@ -503,18 +503,22 @@ WB_HD_COLD int scan_sector_exact(double vx, double vy, double r, int *edge)
 // the compares, and the edge test cannot fire; when vx^2 + vy^2 differs from
 // (r/sqrt(7))^2 by more than 1e-12 of it, hypot's rounding cannot change the
 // radius test.  Otherwise the exact form decides.
-WB_HD int scan_sector(double vx, double vy, double r, int *edge)
+// (scan_sector_est: -1 for the exact form.)
+WB_HD int scan_sector_est(double vx, double vy, double r)
 {
   const double rr = r / kScanSqrt7;
   const double a = kScanSqrt3 * dabs(vy), b = dabs(vx), m = 1e-9 * (a + b);
   const double q2 = vx * vx + vy * vy, t2 = rr * rr;
-  if (__builtin_expect((dabs(a - b) > m) & (b > m) & (dabs(q2 - t2) > 1e-12 * t2), 1)) {
-    *edge = 0;
-    if (q2 < t2) return 0;
-    if (a < b) return vx > 0 ? 1 : 4;
-    return vy > 0 ? (vx > 0 ? 2 : 3) : (vx > 0 ? 6 : 5);
-  }
-  return scan_sector_exact(vx, vy, r, edge);
+  if (!((dabs(a - b) > m) & (b > m) & (dabs(q2 - t2) > 1e-12 * t2))) return -1;
+  if (q2 < t2) return 0;
+  if (a < b) return vx > 0 ? 1 : 4;
+  return vy > 0 ? (vx > 0 ? 2 : 3) : (vx > 0 ? 6 : 5);
+}
+WB_HD int scan_sector(double vx, double vy, double r, int *edge)
+{
+  *edge = 0;
+  const int s = scan_sector_est(vx, vy, r);
+  return __builtin_expect(s >= 0, 1) ? s : scan_sector_exact(vx, vy, r, edge);
 }
 
 // ---------------------------------------------------------------------------
