@@ -302,12 +302,11 @@ class Context:
         L = lib()
         counts = np.zeros(max(nb, 1), dtype=np.uint32)
         n = C.c_uint64()
-        self.check(L.wb_store_read_blocks(self.h, buf.ctypes.data_as(_vp), nb, None, None, None,
-                                          None, counts.ctypes.data_as(_u32p), C.byref(n)),
-                   "wb_store_read_blocks")
-        m = max(n.value, 1)
-        x, y, z = np.zeros(m), np.zeros(m), np.zeros(m)
-        cls = np.zeros(m, dtype=np.uint16)
+        # room for full blocks (pages never written cost nothing), so the
+        # blocks go to the device once
+        m = max(nb * STORE_RECORDS, 1)
+        x, y, z = np.empty(m), np.empty(m), np.empty(m)
+        cls = np.empty(m, dtype=np.uint16)
         self.check(L.wb_store_read_blocks(self.h, buf.ctypes.data_as(_vp), nb,
                                           x.ctypes.data_as(_dp), y.ctypes.data_as(_dp),
                                           z.ctypes.data_as(_dp),
@@ -619,6 +618,10 @@ def tile_count(bbmin, bbmax, tile_size=1.0):
     return n.value
 
 
+def _tiles_ptr(a):
+    return a.ctypes.data_as(C.POINTER(TileRecord))
+
+
 def classify(tree, bbmin, bbmax, params=None, want_tiles=True, out=None):
     """SCAN + POSTSCAN + CLASSIFY of every flowsnake tile (scan.cpp:31-179,
     classify.cpp:96-173).  Returns (class bytes in input order, tile records
@@ -629,7 +632,7 @@ def classify(tree, bbmin, bbmax, params=None, want_tiles=True, out=None):
     params = params or default_params()
     a, b = _arr(bbmin, np.float64), _arr(bbmax, np.float64)
     ntiles = tile_count(a, b, params.tile_size) if want_tiles else 0
-    tiles = (TileRecord * max(ntiles, 1))() if want_tiles else None
+    tiles = np.empty(ntiles, dtype=np.dtype(TileRecord)) if want_tiles else None
     st = Stats()
     if out is not None and _on_device(out):
         cls = out
@@ -650,10 +653,9 @@ def classify(tree, bbmin, bbmax, params=None, want_tiles=True, out=None):
         cls = np.zeros(tree.n_input, dtype=np.uint8)
         ptr, flags = cls.ctypes.data, 0
     rc = lib().wb_classify(tree.h, _dptr(a), _dptr(b), C.byref(params), ptr, flags,
-                           tiles if want_tiles else None, ntiles, C.byref(st))
+                           _tiles_ptr(tiles) if want_tiles else None, ntiles, C.byref(st))
     tree.ctx.check(rc, "wb_classify")
-    tarr = np.ctypeslib.as_array(tiles)[:ntiles].copy() if want_tiles else None
-    return cls, tarr, st.as_dict()
+    return cls, tiles, st.as_dict()
 
 
 def classify_batch(trees, bbmins, bbmaxs, params=None, outs=None):
@@ -700,9 +702,9 @@ def scan_tiles(tree, bbmin, bbmax, params=None):
     params = params or default_params()
     a, b = _arr(bbmin, np.float64), _arr(bbmax, np.float64)
     ntiles = tile_count(a, b, params.tile_size)
-    tiles = (TileRecord * max(ntiles, 1))()
+    tiles = np.empty(ntiles, dtype=np.dtype(TileRecord))
     st = Stats()
-    rc = lib().wb_scan_tiles(tree.h, _dptr(a), _dptr(b), C.byref(params), tiles, ntiles,
+    rc = lib().wb_scan_tiles(tree.h, _dptr(a), _dptr(b), C.byref(params), _tiles_ptr(tiles), ntiles,
                              C.byref(st))
     tree.ctx.check(rc, "wb_scan_tiles")
-    return np.ctypeslib.as_array(tiles)[:ntiles].copy(), st.as_dict()
+    return tiles, st.as_dict()

@@ -716,7 +716,7 @@ static int run_pass(wb_tree *t, const double *corners, int ncorners,
   bool host_out = !(flags & WB_DEVICE_INPUT) && !scan_only;
   if (host_out) dcls = (uint8_t *)wb_alloc(c, t->n_input + 16);
   ClassifyOut co;
-  wb_run_classify(t, corners, ncorners, p, dcls, tiles_out != nullptr, scan_only, &co);
+  wb_run_classify(t, corners, ncorners, p, dcls, tiles_out, scan_only, &co);
   if (host_out) {
     if (t->n_input)
       WB_CHECK(hipMemcpyAsync(class_out, dcls, t->n_input, hipMemcpyDeviceToHost, c->stream));
@@ -724,24 +724,6 @@ static int run_pass(wb_tree *t, const double *corners, int ncorners,
     wb_free(c, dcls, t->n_input + 16);
   }
   auto t1 = std::chrono::steady_clock::now();
-  if (tiles_out) {
-    for (uint64_t k = 0; k < ntiles; k++) {
-      const TileRec &r = co.tiles[k];
-      wb_tile &o = tiles_out[k];
-      o.npoints = r.npoints;
-      o.nground = r.nground;
-      o.tree_flags = r.tree_flags;
-      o.flowsnake_x = co.tex[k];
-      o.flowsnake_y = co.tey[k];
-      o.fit_fp64 = r.fit_fp64;
-      o.density = r.density;
-      o.hs_scan = r.hs_scan;
-      o.hs = r.hs;
-      o.height = r.height;
-      o.tilt_x = r.tilt_x;
-      o.tilt_y = r.tilt_y;
-    }
-  }
   if (stats) fill_stats(stats, t, co, ntiles, std::chrono::duration<double, std::milli>(t1 - t0).count());
   return WB_OK;
   API_CATCH(c)

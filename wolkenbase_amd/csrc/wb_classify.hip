@@ -1574,8 +1574,8 @@ __device__ __attribute__((always_inline)) inline void scan_reg(
 // the front and the back, 1 and 5 lb, 2 and 4 lc, 3 ld; ncls[c] the lengths),
 // so each class kernel visits only its own tiles.  The order inside a list
 // does not matter: every tile's record depends on that tile alone.  An empty
-// tile's record is written only where the caller gets the records: 64 B for
-// each of 27.8M tile numbers, most of them empty, took 0.5 ms.
+// tile has no record: 64 B for each of 27.8M tile numbers, most of them empty,
+// took 0.5 ms.
 #define SCAN_NCLS 7
 // Points from which each class takes its own launch, several tiles per step
 // (and tiny tiles a lane each).  Mixed and own launches, scan and postscan in
@@ -1600,7 +1600,7 @@ __device__ inline int scan_class(uint32_t m, uint32_t tiny)
 __global__ void __launch_bounds__(1024) k_scan_classes(uint32_t ntiles, const uint32_t *tile_cnt,
                                                       uint32_t *la, uint32_t *lb, uint32_t *lc,
                                                       uint32_t *ld, uint32_t *ncls,
-                                                      uint32_t tiny, int want_empty, TileRec *rec)
+                                                      uint32_t tiny)
 {
   // slots are claimed per block: the waves' class counts summed in LDS, one
   // atomic per class and block (atomics on the list counters are
@@ -1609,10 +1609,6 @@ __global__ void __launch_bounds__(1024) k_scan_classes(uint32_t ntiles, const ui
   __shared__ uint32_t bbase[SCAN_NCLS];
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t m = t < ntiles ? tile_cnt[t] : 0u;
-  if (want_empty && t < ntiles && m == 0) {
-    TileRec r = {0, 0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    rec[t] = r;
-  }
   const int c = scan_class(m, tiny);
   const uint32_t lane = __lane_id(), w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
   uint64_t mk[SCAN_NCLS];
@@ -2220,6 +2216,42 @@ __global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey,
   } while (ring && !nontree);
   double w = count * g.spacing / 6;
   rec[t].hs = sqrt(me.hs_scan * me.hs_scan + w * w);
+}
+
+// The tiles' records in the caller's layout, empty tiles zero but for their
+// address; a block's 256 records pass through LDS and leave in whole lines.
+__global__ void __launch_bounds__(256) k_tile_out(uint32_t ntiles, const uint32_t *tile_cnt,
+                                                  const TileRec *rec, const int32_t *tex,
+                                                  const int32_t *tey, const int32_t *nground,
+                                                  wb_tile *out)
+{
+  constexpr uint32_t W = sizeof(wb_tile) / 4;
+  __shared__ __align__(16) wb_tile s[256];
+  const uint32_t t0 = blockIdx.x * 256, t = t0 + threadIdx.x;
+  if (t < ntiles) {
+    wb_tile o = {};
+    o.flowsnake_x = tex[t];
+    o.flowsnake_y = tey[t];
+    if (tile_cnt[t]) {
+      const TileRec r = rec[t];
+      o.npoints = r.npoints;
+      o.nground = nground ? nground[t] : r.nground;
+      o.tree_flags = r.tree_flags;
+      o.fit_fp64 = r.fit_fp64;
+      o.density = r.density;
+      o.hs_scan = r.hs_scan;
+      o.hs = r.hs;
+      o.height = r.height;
+      o.tilt_x = r.tilt_x;
+      o.tilt_y = r.tilt_y;
+    }
+    s[threadIdx.x] = o;
+  }
+  __syncthreads();
+  const uint32_t n = min(256u, ntiles - t0) * W;
+  const uint32_t *src = (const uint32_t *)s;
+  uint32_t *dst = (uint32_t *)(out + t0);
+  for (uint32_t k = threadIdx.x; k < n; k += 256) dst[k] = src[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -3798,7 +3830,8 @@ struct ClassifyRun {
   hipStream_t st;
   const wb_classify_params *p;
   uint8_t *d_class_out;
-  bool want_tiles, scan_only;
+  wb_tile *tiles_out;  // host, or null
+  bool scan_only;
   ClassifyOut *out;
   uint64_t n;
   TileGeo g;
@@ -3902,10 +3935,11 @@ static void open_release(wb_ctx *c, OpenBuffers &B)
 
 static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double *corners,
                              int ncorners, const wb_classify_params *p, uint8_t *d_class_out,
-                             bool want_tiles, bool scan_only, uint64_t nbatch, ClassifyOut *out)
+                             wb_tile *tiles_out, bool scan_only, uint64_t nbatch,
+                             ClassifyOut *out)
 {
   R.t = t; R.c = c; R.st = c->stream; R.p = p; R.d_class_out = d_class_out;
-  R.want_tiles = want_tiles; R.scan_only = scan_only; R.out = out;
+  R.tiles_out = tiles_out; R.scan_only = scan_only; R.out = out;
   R.cls = nullptr; R.heavy = nullptr; R.h_nheavy = 0; R.h_nslow = 0;
   hipStream_t st = R.st;
   const uint64_t n = R.n = t->n;
@@ -3980,8 +4014,7 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
     const bool many = n >= SCAN_MANY && prec == WB_FIT_FP64;
     if (g.ntiles) {
       hipLaunchKernelGGL(k_scan_classes, dim3(wb_blocks(g.ntiles, 1024)), dim3(1024), 0, st,
-                         g.ntiles, tile_cnt, la, lb, lc, ld, ncls, many ? 8u : 0u, want_tiles ? 1 : 0,
-                         rec);
+                         g.ntiles, tile_cnt, la, lb, lc, ld, ncls, many ? 8u : 0u);
       const uint32_t e = g.ntiles - 1;
       const ClassList c8 = {la, 1, ncls}, c16 = {lb, 1, ncls + 1}, c32 = {lc, 1, ncls + 2};
       const ClassList c64 = {ld, 1, ncls + 3}, c128 = {lc + e, -1, ncls + 4};
@@ -4115,7 +4148,7 @@ static void classify_finish(ClassifyRun &R)
   const TileGeo &g = R.g;
   hipEvent_t *ev = R.ev;
   ClassifyOut *out = R.out;
-  const bool want_tiles = R.want_tiles, scan_only = R.scan_only;
+  const bool want_tiles = R.tiles_out != nullptr, scan_only = R.scan_only;
   int32_t *memb = R.memb;
   uint32_t *nmemb = R.nmemb, *nslow = R.nslow, *err = R.err;
   TileRec *rec = R.rec;
@@ -4189,25 +4222,22 @@ static void classify_finish(ClassifyRun &R)
   WB_CHECK(hipEventRecord(ev[3], st));
   uint32_t *herr = c->hbox + WB_HBOX_ERR;
   WB_CHECK(hipMemcpyAsync(herr, err, 128, hipMemcpyDeviceToHost, st));
-  if (want_tiles) {
-    out->tiles.resize(g.ntiles);
-    out->tex.resize(g.ntiles);
-    out->tey.resize(g.ntiles);
-    std::vector<int32_t> ng(g.ntiles, 0);
-    WB_CHECK(hipMemcpyAsync(out->tiles.data(), rec, sizeof(TileRec) * (size_t)g.ntiles, hipMemcpyDeviceToHost, st));
-    WB_CHECK(hipMemcpyAsync(out->tex.data(), R.tex, 4ull * g.ntiles, hipMemcpyDeviceToHost, st));
-    WB_CHECK(hipMemcpyAsync(out->tey.data(), R.tey, 4ull * g.ntiles, hipMemcpyDeviceToHost, st));
-    if (!scan_only)
-      WB_CHECK(hipMemcpyAsync(ng.data(), nground, 4ull * g.ntiles, hipMemcpyDeviceToHost, st));
-    WB_CHECK(hipStreamSynchronize(st));
-    for (uint32_t k = 0; k < g.ntiles; k++) out->tiles[k].nground = ng[k];
-  }
   WB_CHECK(hipStreamSynchronize(st));
   uint32_t h_err[32];
   std::copy(herr, herr + 32, h_err);
   // the exact-gap and heavy point counts (nslow[0], nslow[1])
   R.h_nslow = h_err[14];
   R.h_nheavy = h_err[15];
+  if (want_tiles && g.ntiles && !(h_err[0] & 3u)) {
+    // the records as the caller holds them, in one copy
+    wb_tile *tiles = (wb_tile *)wb_alloc(c, sizeof(wb_tile) * (size_t)g.ntiles);
+    hipLaunchKernelGGL(k_tile_out, dim3(wb_blocks(g.ntiles, 256)), dim3(256), 0, st, g.ntiles,
+                       R.tile_cnt, rec, R.tex, R.tey, scan_only ? nullptr : nground, tiles);
+    WB_CHECK(hipMemcpyAsync(R.tiles_out, tiles, sizeof(wb_tile) * (size_t)g.ntiles,
+                            hipMemcpyDeviceToHost, st));
+    WB_CHECK(hipStreamSynchronize(st));
+    wb_free(c, tiles, sizeof(wb_tile) * (size_t)g.ntiles);
+  }
   float ms1 = 0, ms2 = 0, ms3 = 0;
   hipEventElapsedTime(&ms1, ev[0], ev[1]);
   hipEventElapsedTime(&ms2, ev[1], ev[2]);
@@ -4246,11 +4276,11 @@ static void classify_finish(ClassifyRun &R)
 }
 
 void wb_run_classify(wb_tree *t, const double *corners, int ncorners,
-                     const wb_classify_params *p, uint8_t *d_class_out, bool want_tiles,
+                     const wb_classify_params *p, uint8_t *d_class_out, wb_tile *tiles_out,
                      bool scan_only, ClassifyOut *out)
 {
   ClassifyRun R;
-  classify_prepare(R, t, t->ctx, corners, ncorners, p, d_class_out, want_tiles, scan_only, 0, out);
+  classify_prepare(R, t, t->ctx, corners, ncorners, p, d_class_out, tiles_out, scan_only, 0, out);
   if (!scan_only) classify_ground_single(R);
   classify_finish(R);
 }
@@ -4264,7 +4294,7 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
   uint64_t nbatch = 0;
   for (int k = 0; k < ntrees; k++) nbatch += trees[k]->n;
   for (int k = 0; k < ntrees; k++)
-    classify_prepare(R[k], trees[k], c, corners + 6 * k, 2, p, d_class_out[k], false, false,
+    classify_prepare(R[k], trees[k], c, corners + 6 * k, 2, p, d_class_out[k], nullptr, false,
                      nbatch, &outs[k]);
   // one launch of walk A over every tree's points, one of walk B and one of
   // the heavy kernel over what the trees' walks left; the counts stay on the

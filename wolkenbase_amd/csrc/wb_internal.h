@@ -177,8 +177,6 @@ struct TileRec {
 };
 
 struct ClassifyOut {
-  std::vector<TileRec> tiles;
-  std::vector<int32_t> tex, tey;
   uint64_t borderline, atan_exact, nslow, hist[3], nonempty, nheavy, fallbacks;
   double ms_tiles, ms_scan, ms_classify, ms_classify_kernel, ms_heavy_kernel;
 };
@@ -195,7 +193,8 @@ void wb_run_points(wb_tree *t, int kind, const double *dparams, uint64_t ns, con
 // context: wb_free(c, order, 4 * ns))
 uint32_t *wb_query_order(wb_tree *t, int kind, const double *dparams, uint64_t ns);
 // the classification pass (tile geometry, membership, SCAN, POSTSCAN and,
-// unless scan_only, CLASSIFY); class bytes to d_class_out in input order
+// unless scan_only, CLASSIFY); class bytes to d_class_out in input order, the
+// tiles' records to tiles_out (host memory) unless it is null
 // several trees of one context classified together, their ground tests in
 // one launch (tiles as wb_classify with each tree's two header corners,
 // corners + 6k); d_class_out[k]: device class bytes of tree k, input order
@@ -203,7 +202,7 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
                            const wb_classify_params *p, uint8_t *const *d_class_out,
                            ClassifyOut *outs);
 void wb_run_classify(wb_tree *t, const double *corners, int ncorners,
-                     const wb_classify_params *p, uint8_t *d_class_out, bool want_tiles,
+                     const wb_classify_params *p, uint8_t *d_class_out, wb_tile *tiles_out,
                      bool scan_only, ClassifyOut *out);
 
 // ---- building blocks implemented in wb_build.hip ----

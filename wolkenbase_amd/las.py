@@ -7,8 +7,8 @@ import ctypes as C
 import numpy as np
 
 from . import (LasHeader, LasWriteParams, LasWriteStats, Octree, Stats, TileRecord, WbError,
-               WB_DEVICE_INPUT, WB_WRITE_DRY, WB_ZEROS_KEEP, WB_ZEROS_READ, _vp, default_params,
-               lib)
+               WB_DEVICE_INPUT, WB_WRITE_DRY, WB_ZEROS_KEEP, WB_ZEROS_READ, _tiles_ptr, _vp,
+               default_params, lib)
 
 ZEROS = {"read": WB_ZEROS_READ, "keep": WB_ZEROS_KEEP}
 
@@ -157,7 +157,7 @@ class Cloud:
         from . import tile_count_corners
         params = params or default_params()
         ntiles = tile_count_corners(self.corners, params.tile_size) if want_tiles else 0
-        tiles = (TileRecord * max(ntiles, 1))() if want_tiles else None
+        tiles = np.empty(ntiles, dtype=np.dtype(TileRecord)) if want_tiles else None
         st = Stats()
         if out is not None:
             cls, ptr, flags = out, out.data_ptr(), WB_DEVICE_INPUT
@@ -165,10 +165,9 @@ class Cloud:
             cls = np.zeros(self.n, dtype=np.uint8)
             ptr, flags = cls.ctypes.data, 0
         rc = lib().wb_cloud_classify(self.h, tree.h, C.byref(params), ptr, flags,
-                                     tiles if want_tiles else None, ntiles, C.byref(st))
+                                     _tiles_ptr(tiles) if want_tiles else None, ntiles, C.byref(st))
         self.ctx.check(rc, "wb_cloud_classify")
-        tarr = np.ctypeslib.as_array(tiles)[:ntiles].copy() if want_tiles else None
-        return cls, tarr, st.as_dict()
+        return cls, tiles, st.as_dict()
 
     def write(self, tree, cls, name, separate_classes=True, points_per_file=10000000,
               point_format=-1, creation=(0, 0), dry=False):
