@@ -95,11 +95,12 @@ __global__ void __launch_bounds__(256) k_scan_reduce(const uint32_t *in, uint64_
 
 // boff: the tiles' sums, or with scanned their exclusive scan; total (null or
 // two host words): the sum of all values, written by the last block
-__global__ void __launch_bounds__(256) k_scan_down(uint32_t *data, uint64_t n, const uint32_t *boff,
-                                                   int scanned, uint32_t *total)
+__global__ void __launch_bounds__(256) k_scan_down(const uint32_t *in, uint32_t *data, uint64_t n,
+                                                   const uint32_t *boff, int scanned,
+                                                   uint32_t *total)
 {
   uint32_t v[16], s = 0, tot, off = 0;
-  scan_load(data, n, v);
+  scan_load(in, n, v);
 #pragma unroll
   for (int k = 0; k < 16; k++) s += v[k];
   if (scanned) {
@@ -142,16 +143,16 @@ __global__ void __launch_bounds__(256) k_scan_down(uint32_t *data, uint64_t n, c
   }
 }
 
-static void scan_rec(wb_ctx *c, uint32_t *data, uint64_t n, uint32_t *total)
+static void scan_rec(wb_ctx *c, const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *total)
 {
   const unsigned nb = wb_blocks(n, SCAN_TILE);
   uint32_t *bs = nullptr;
   if (nb > 1) {
     bs = (uint32_t *)wb_alloc(c, sizeof(uint32_t) * nb);
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, c->stream, data, n, bs);
-    if (nb > SCAN_FLAT) scan_rec(c, bs, nb, nullptr);
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, c->stream, in, n, bs);
+    if (nb > SCAN_FLAT) scan_rec(c, bs, bs, nb, nullptr);
   }
-  hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(256), 0, c->stream, data, n, bs,
+  hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(256), 0, c->stream, in, out, n, bs,
                      nb > SCAN_FLAT ? 1 : 0, total);
   wb_free(c, bs, sizeof(uint32_t) * nb);
 }
@@ -160,9 +161,14 @@ uint64_t wb_exclusive_scan_u32(wb_ctx *c, uint32_t *data, uint64_t n)
 {
   if (n == 0) return 0;
   uint32_t *h = c->hbox + WB_HBOX_SCAN;
-  scan_rec(c, data, n, h);
+  scan_rec(c, data, data, n, h);
   WB_CHECK(hipStreamSynchronize(c->stream));
   return (uint64_t)h[0] | ((uint64_t)h[1] << 32);
+}
+
+void wb_exclusive_scan_u32_to(wb_ctx *c, const uint32_t *in, uint32_t *out, uint64_t n)
+{
+  if (n) scan_rec(c, in, out, n, c->hbox + WB_HBOX_SCAN);
 }
 
 // ---------------------------------------------------------------------------
@@ -622,20 +628,31 @@ __global__ void k_split_level_t(const K *key, const Active *act, const uint32_t 
 // node's sorted keys: 64 evenly spaced samples place every boundary between
 // two neighbouring samples, then lanes 8(c-1)..8(c-1)+7 narrow boundary c by
 // a 9-way search (8 probes per round).  Lanes 0..7 then make child c = lane.
+// The children's numbers are claimed once per block of eight nodes: atomics
+// on one counter are serialised (about 10 ns each), and claimed by wave they
+// were the kernel (1500 nodes 24 us, now 8).
+#define SPLIT_WAVES 8
 template <typename K>
-__global__ void __launch_bounds__(256) k_split_level(
+__global__ void __launch_bounds__(64 * SPLIT_WAVES) k_split_level(
     const K *key, const Active *act, const uint32_t *act_cnt, uint32_t act_cap, int level,
     int max_level, Active *next, uint32_t *next_cnt, uint32_t next_cap, LeafTmp *leaves,
     uint32_t leaf_cap, double *node_cube, int32_t *node_child, int32_t *node_parent,
     uint32_t node_cap, SplitOut *out, uint32_t *bits)
 {
-  if (out->overflow) return;
+  // (the same answer for the whole block: the waves meet at barriers below)
+  __shared__ uint32_t failed;
+  if (threadIdx.x == 0) failed = out->overflow;
+  __syncthreads();
+  if (failed) return;
   const uint32_t nact = min(*act_cnt, act_cap);
   if (nact > SPLIT_WAVE_MAX) return;  // k_split_level_t takes this level
-  const uint32_t lane = threadIdx.x & 63;
+  __shared__ uint32_t wn[SPLIT_WAVES], wl[SPLIT_WAVES], base[3];
+  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x / 64;
   const int lv = level + 1;
-  for (uint32_t a = blockIdx.x * 4 + threadIdx.x / 64; a < nact; a += gridDim.x * 4) {
-    const Active A = act[a];
+  for (uint32_t a0 = blockIdx.x * SPLIT_WAVES; a0 < nact; a0 += gridDim.x * SPLIT_WAVES) {
+    // (a wave past the last node takes part with no children)
+    const bool have = a0 + w < nact;
+    const Active A = act[have ? a0 + w : a0];
     const int node = A.node;
     const uint32_t len = A.end - A.start;  // > 537: an active node
     // samples l = 0..63 (sorted, so their digits are too)
@@ -682,28 +699,40 @@ __global__ void __launch_bounds__(256) k_split_level(
     const uint32_t b_lo = lane == 0 ? A.start : s_lo;
     const uint32_t b_hi = lane == 7 ? A.end : s_hi;
     const uint32_t cnt = b_hi - b_lo;
-    const bool valid = lane < 8 && cnt > 0;
+    const bool valid = have && lane < 8 && cnt > 0;
     const bool big = valid && cnt > WB_RECORDS;
     const bool is_node = big && lv < max_level, is_leaf = valid && !big;
     if (big && lv >= max_level) atomicOr(&out->overflow, 1u);
-    // one counter update per wave and kind; children numbered in child order
+    // one counter update per block and kind; children numbered in child order
     const uint64_t mnode = __ballot(is_node), mleaf = __ballot(is_leaf);
-    uint32_t nbase = 0, sbase = 0, lbase = 0;
     if (lane == 0) {
-      if (mnode) {
-        nbase = atomicAdd(&out->n_node, (uint32_t)__popcll(mnode));
-        sbase = atomicAdd(next_cnt, (uint32_t)__popcll(mnode));
+      wn[w] = (uint32_t)__popcll(mnode);
+      wl[w] = (uint32_t)__popcll(mleaf);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t nn = 0, nf = 0;
+      for (int k = 0; k < SPLIT_WAVES; k++) {
+        const uint32_t p = wn[k], q = wl[k];
+        wn[k] = nn;
+        wl[k] = nf;
+        nn += p;
+        nf += q;
       }
-      if (mleaf) {
-        lbase = atomicAdd(&out->n_leaf, (uint32_t)__popcll(mleaf));
+      if (nn) {
+        base[0] = atomicAdd(&out->n_node, nn);
+        base[1] = atomicAdd(next_cnt, nn);
+      }
+      if (nf) {
+        base[2] = atomicAdd(&out->n_leaf, nf);
         atomicMax(&out->maxdepth, (uint32_t)lv);
       }
     }
-    nbase = (uint32_t)__shfl((int)nbase, 0, 64);
-    sbase = (uint32_t)__shfl((int)sbase, 0, 64);
-    lbase = (uint32_t)__shfl((int)lbase, 0, 64);
+    __syncthreads();
+    const uint32_t nbase = base[0] + wn[w], sbase = base[1] + wn[w], lbase = base[2] + wl[w];
+    __syncthreads();  // before the next round's counts
     const uint64_t below = (1ull << lane) - 1;
-    if (lane < 8) {
+    if (have && lane < 8) {
       const int cch = (int)lane;
       int32_t code = -1;
       if (valid) {
@@ -999,6 +1028,21 @@ __device__ inline void lower_to(double *z, double v)
   else atomicMax((unsigned long long *)z, (unsigned long long)b);
 }
 
+#define CANON_PT 3  // 256 * 3 >= WB_RECORDS
+template <int NE>
+__device__ inline void count_below(const uint32_t *id, uint32_t m, const uint32_t (&my)[CANON_PT],
+                                   uint32_t (&rank)[CANON_PT])
+{
+  const uint4 *q = (const uint4 *)id;
+#pragma unroll 4
+  for (uint32_t j = 0; j < (m + 3) / 4; j++) {
+    const uint4 v = q[j];
+#pragma unroll
+    for (int k = 0; k < NE; k++)
+      rank[k] += (v.x < my[k]) + (v.y < my[k]) + (v.z < my[k]) + (v.w < my[k]);
+  }
+}
+
 // A block per leaf.
 // The canonical order (input order inside each leaf): a point's place is the
 // number of smaller input indices in the leaf, counted by a thread per point
@@ -1011,7 +1055,6 @@ __device__ inline void lower_to(double *z, double v)
 // internal node (the ground test raises a child cube's bottom face to it,
 // wb::hyp_intersect_low): up the parents until one is as low already (then so
 // are those above it, or its own block is on the way to them).
-#define CANON_PT 3  // 256 * 3 >= WB_RECORDS
 __global__ void __launch_bounds__(256) k_leaf_finish(const uint32_t *leaf_start,
                                                      const uint32_t *sidx, const double *pz,
                                                      const int32_t *leaf_parent,
@@ -1040,21 +1083,9 @@ __global__ void __launch_bounds__(256) k_leaf_finish(const uint32_t *leaf_start,
   __syncthreads();
   const uint32_t w0 = t & ~(WAVE - 1u);  // the wave's first element
   if (w0 < m) {
-    const uint4 *q = (const uint4 *)id;
-    const uint32_t nq = (m + 3) / 4;
-    if (w0 + 256 >= m) {
-      for (uint32_t j = 0; j < nq; j++) {
-        const uint4 v = q[j];
-        rank[0] += (v.x < my[0]) + (v.y < my[0]) + (v.z < my[0]) + (v.w < my[0]);
-      }
-    } else {
-      for (uint32_t j = 0; j < nq; j++) {
-        const uint4 v = q[j];
-#pragma unroll
-        for (int k = 0; k < CANON_PT; k++)
-          rank[k] += (v.x < my[k]) + (v.y < my[k]) + (v.z < my[k]) + (v.w < my[k]);
-      }
-    }
+    if (w0 + 256 >= m) count_below<1>(id, m, my, rank);
+    else if (w0 + 512 >= m) count_below<2>(id, m, my, rank);
+    else count_below<3>(id, m, my, rank);
 #pragma unroll
     for (int k = 0; k < CANON_PT; k++) {
       const uint32_t e = t + 256u * k;
@@ -1242,9 +1273,9 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
       WB_CHECK(hipMemcpyAsync(act, &r0, sizeof r0, hipMemcpyHostToDevice, c->stream));
     }
     for (int level = 0; n > 0 && level < max_level; level++) {
-      const dim3 gw(std::min<uint32_t>(wb_blocks(act_ub, 4), 512)), gt(wb_blocks(act_ub, 128));
+      const dim3 gw(std::min<uint32_t>(wb_blocks(act_ub, SPLIT_WAVES), 256)), gt(wb_blocks(act_ub, 128));
       if (narrow) {
-        hipLaunchKernelGGL(k_split_level<uint32_t>, gw, dim3(256), 0, c->stream, key32, act,
+        hipLaunchKernelGGL(k_split_level<uint32_t>, gw, dim3(64 * SPLIT_WAVES), 0, c->stream, key32, act,
                            d_cnt + level, node_cap, level, max_level, nxt, d_cnt + level + 1,
                            node_cap, lt, leaf_cap, t->node_cube, t->node_child, t->node_parent,
                            node_cap, d_out, bits);
@@ -1254,7 +1285,7 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
                              node_cap, lt, leaf_cap, t->node_cube, t->node_child,
                              t->node_parent, node_cap, d_out, bits);
       } else {
-        hipLaunchKernelGGL(k_split_level<uint64_t>, gw, dim3(256), 0, c->stream, t->key, act,
+        hipLaunchKernelGGL(k_split_level<uint64_t>, gw, dim3(64 * SPLIT_WAVES), 0, c->stream, t->key, act,
                            d_cnt + level, node_cap, level, max_level, nxt, d_cnt + level + 1,
                            node_cap, lt, leaf_cap, t->node_cube, t->node_child, t->node_parent,
                            node_cap, d_out, bits);

@@ -747,6 +747,24 @@ __global__ void k_tile_geo(TileGeo g, int32_t *tex, int32_t *tey, int *bounds)
   }
 }
 
+// clears a pass's counters: per tile the points, the list places taken and the
+// state (0 empty, 1 scanned, 2 a tree tile), and the 64 words of err (one launch: a memset of an odd size is two)
+__global__ void __launch_bounds__(256) k_pass_init(uint32_t ntiles, uint32_t *tile_cnt,
+                                                   uint32_t *tile_fill, uint32_t *state,
+                                                   uint32_t *err)
+{
+  const uint32_t b = blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++)
+    if (b + 256 * k < ntiles) {
+      tile_cnt[b + 256 * k] = 0;
+      tile_fill[b + 256 * k] = 0;
+    }
+  const uint32_t w = blockIdx.x * 256 + threadIdx.x;
+  if (w < ntiles / 4 + 1) state[w] = 0;
+  if (b < 64) err[b] = 0;
+}
+
 __global__ void k_fill_i32(int32_t *p, uint64_t n, int32_t v)
 {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1353,7 +1371,7 @@ __device__ __attribute__((always_inline)) inline void fit_solve(TileFit &F)
 
 __device__ __attribute__((always_inline)) inline void fit_record(const TileFit &F, double r,
                                                                  double min_hs, int fit_fp64,
-                                                                 TileRec *out)
+                                                                 TileRec *out, uint8_t *state)
 {
   double density = 0;
   int tree = 0;
@@ -1374,6 +1392,7 @@ __device__ __attribute__((always_inline)) inline void fit_record(const TileFit &
   rr.tilt_x = F.sx;
   rr.tilt_y = F.sy;
   *out = rr;
+  *state = (uint8_t)(1 + tree);
 }
 
 // The scan of up to T tiles of at most 64*K points each by one wave, K points
@@ -1388,7 +1407,7 @@ template <int K, bool F32, int T>
 __device__ __attribute__((always_inline)) inline void scan_reg(
     const TreeView &V, const TileGeo &g, const uint32_t (&t)[T], const uint32_t (&m)[T],
     const int32_t *tex, const int32_t *tey, const uint32_t *tile_off, const uint32_t *lists,
-    double min_hs, int prec, TileRec *rec, unsigned long long *ctr)
+    double min_hs, int prec, TileRec *rec, uint8_t *state, unsigned long long *ctr)
 {
   const uint32_t lane = __lane_id();
   uint32_t c[T][K];
@@ -1563,7 +1582,7 @@ __device__ __attribute__((always_inline)) inline void scan_reg(
   for (int j = 0; j < T; j++)
     if (lane == (uint32_t)j) tl = t[j];
   if (lane < T && F.m) {
-    fit_record(F, r, min_hs, fell_back, rec + tl);
+    fit_record(F, r, min_hs, fell_back, rec + tl, state + tl);
     if (fell_back) atomicAdd(&ctr[7], 1ull);
   }
 }
@@ -1662,7 +1681,7 @@ __global__ void __launch_bounds__(64, MINW) k_scan_reg(TreeView V, TileGeo g, co
                                                  const int32_t *tey, const uint32_t *tile_off,
                                                  const uint32_t *tile_cnt, const uint32_t *lists,
                                                  ClassList cl, double min_hs, int prec,
-                                                 TileRec *rec, unsigned long long *ctr)
+                                                 TileRec *rec, uint8_t *state, unsigned long long *ctr)
 {
   const uint32_t n = (uint32_t)rfl((int)*cl.n);
   uint32_t i = blockIdx.x * T;
@@ -1680,7 +1699,7 @@ __global__ void __launch_bounds__(64, MINW) k_scan_reg(TreeView V, TileGeo g, co
       const uint32_t k = i + gridDim.x * T + j;
       next[j] = k < n ? cl.at(k) : 0xffffffffu;
     }
-    scan_reg<K, F32, T>(V, g, t, m, tex, tey, tile_off, lists, min_hs, prec, rec, ctr);
+    scan_reg<K, F32, T>(V, g, t, m, tex, tey, tile_off, lists, min_hs, prec, rec, state, ctr);
   }
 }
 
@@ -1749,7 +1768,7 @@ template <int GS, int R>
 __device__ __attribute__((always_inline)) inline void scan_rows(
     const TreeView &V, const TileGeo &g, const int32_t *tex, const int32_t *tey,
     const uint32_t *tile_off, const uint32_t *tile_cnt, const uint32_t *lists, const ClassList &cl,
-    uint32_t n, uint32_t i0, double min_hs, TileRec *rec, unsigned long long *ctr)
+    uint32_t n, uint32_t i0, double min_hs, TileRec *rec, uint8_t *state, unsigned long long *ctr)
 {
   constexpr uint32_t NG = WAVE / GS;
   const uint32_t lane = __lane_id(), grp = lane / GS, gl = lane % GS, gbase = lane - gl;
@@ -1872,7 +1891,7 @@ __device__ __attribute__((always_inline)) inline void scan_rows(
     }
     if (nedge && lane == 0) atomicAdd(&ctr[0], (unsigned long long)nedge);
   }
-  if (lane < NG * R && F.m) fit_record(F, r, min_hs, 0, rec + tl);
+  if (lane < NG * R && F.m) fit_record(F, r, min_hs, 0, rec + tl, state + tl);
 }
 
 template <int GS, int R, int MINW>
@@ -1880,13 +1899,13 @@ __global__ void __launch_bounds__(64, MINW) k_scan_row(TreeView V, TileGeo g, co
                                                        const int32_t *tey, const uint32_t *tile_off,
                                                        const uint32_t *tile_cnt,
                                                        const uint32_t *lists, ClassList cl,
-                                                       double min_hs, TileRec *rec,
+                                                       double min_hs, TileRec *rec, uint8_t *state,
                                                        unsigned long long *ctr)
 {
   constexpr uint32_t per = WAVE / GS * R;
   const uint32_t n = (uint32_t)rfl((int)*cl.n);
   for (uint32_t i0 = blockIdx.x * per; i0 < n; i0 += gridDim.x * per)
-    scan_rows<GS, R>(V, g, tex, tey, tile_off, tile_cnt, lists, cl, n, i0, min_hs, rec, ctr);
+    scan_rows<GS, R>(V, g, tex, tey, tile_off, tile_cnt, lists, cl, n, i0, min_hs, rec, state, ctr);
 }
 
 // The classes of 1 to 256 points in one launch, for the clouds whose classes
@@ -1899,7 +1918,7 @@ __global__ void __launch_bounds__(64, 4) k_scan_mixed(TreeView V, TileGeo g, con
                                                       const uint32_t *tile_cnt,
                                                       const uint32_t *lists, ClassList c16,
                                                       ClassList c32, ClassList c64, ClassList c128,
-                                                      ClassList c256, double min_hs, TileRec *rec,
+                                                      ClassList c256, double min_hs, TileRec *rec, uint8_t *state,
                                                       unsigned long long *ctr)
 {
   const uint32_t n16 = (uint32_t)rfl((int)*c16.n), n32 = (uint32_t)rfl((int)*c32.n);
@@ -1911,19 +1930,19 @@ __global__ void __launch_bounds__(64, 4) k_scan_mixed(TreeView V, TileGeo g, con
   for (uint32_t u = blockIdx.x; u < end; u += gridDim.x) {
     if (u >= e32) {
       scan_rows<16, 1>(V, g, tex, tey, tile_off, tile_cnt, lists, c16, n16, 4 * (u - e32), min_hs,
-                       rec, ctr);
+                       rec, state, ctr);
     } else if (u >= e64) {
       scan_rows<32, 1>(V, g, tex, tey, tile_off, tile_cnt, lists, c32, n32, 2 * (u - e64), min_hs,
-                       rec, ctr);
+                       rec, state, ctr);
     } else {
       const uint32_t t[1] = {u >= e128 ? c64.at(u - e128) : u >= e256 ? c128.at(u - e256) : c256.at(u)};
       const uint32_t m[1] = {tile_cnt[t[0]]};
       if (u >= e128)
-        scan_reg<1, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, ctr);
+        scan_reg<1, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, state, ctr);
       else if (u >= e256)
-        scan_reg<2, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, ctr);
+        scan_reg<2, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, state, ctr);
       else
-        scan_reg<4, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, ctr);
+        scan_reg<4, false, 1>(V, g, t, m, tex, tey, tile_off, lists, min_hs, WB_FIT_FP64, rec, state, ctr);
     }
   }
 }
@@ -1950,7 +1969,7 @@ __device__ inline double lane_pairwise(const double (&v)[8], uint32_t m)
 __global__ void __launch_bounds__(64) k_scan_lane(TreeView V, TileGeo g, const int32_t *tex,
                                                   const int32_t *tey, const uint32_t *tile_off,
                                                   const uint32_t *tile_cnt, const uint32_t *lists,
-                                                  ClassList cl, double min_hs, TileRec *rec,
+                                                  ClassList cl, double min_hs, TileRec *rec, uint8_t *state,
                                                   unsigned long long *ctr)
 {
   const uint32_t n = *cl.n;
@@ -2050,14 +2069,15 @@ __global__ void __launch_bounds__(64) k_scan_lane(TreeView V, TileGeo g, const i
     }
 #pragma unroll
     for (int k = 0; k < 7; k++) F.hist[k] = (h >> (4 * k)) & 15u;
-    fit_record(F, r, min_hs, 0, rec + t);
+    fit_record(F, r, min_hs, 0, rec + t, state + t);
   }
 }
 
 // the scan of one tile of up to SCAN_CAP points by one wave (LDS sort)
 __device__ void scan_big(const TreeView &T, const TileGeo &g, int ex, int ey, uint32_t off,
                          uint32_t m, const uint32_t *lists, double min_hs, int prec,
-                         TileRec *out, unsigned long long *ctr, uint32_t *cp, int *histo)
+                         TileRec *out, uint8_t *state, unsigned long long *ctr, uint32_t *cp,
+                         int *histo)
 {
   const int lane = threadIdx.x;
   uint32_t P = 1;
@@ -2152,6 +2172,7 @@ __device__ void scan_big(const TreeView &T, const TileGeo &g, int ex, int ey, ui
     rr.tilt_x = sx;
     rr.tilt_y = sy;
     *out = rr;
+    *state = (uint8_t)(1 + tree);
     if (prec != WB_FIT_FP64) atomicAdd(&ctr[7], 1ull);
   }
   __syncthreads();
@@ -2163,7 +2184,8 @@ __global__ void __launch_bounds__(64) k_scan(TreeView T, TileGeo g, const int32_
                                              const int32_t *tey, const uint32_t *tile_off,
                                              const uint32_t *tile_cnt, const uint32_t *lists,
                                              ClassList cl, double min_hs, int prec, TileRec *rec,
-                                             uint32_t *err, unsigned long long *ctr)
+                                             uint8_t *state, uint32_t *err,
+                                             unsigned long long *ctr)
 {
   __shared__ uint32_t cp[SCAN_CAP];
   __shared__ int histo[7];
@@ -2175,7 +2197,8 @@ __global__ void __launch_bounds__(64) k_scan(TreeView T, TileGeo g, const int32_
       if (threadIdx.x == 0) atomicOr(err, 2u);
       continue;
     }
-    scan_big(T, g, tex[t], tey[t], tile_off[t], m, lists, min_hs, prec, rec + t, ctr, cp, histo);
+    scan_big(T, g, tex[t], tey[t], tile_off[t], m, lists, min_hs, prec, rec + t, state + t,
+             ctr, cp, histo);
   }
 }
 
@@ -2183,7 +2206,7 @@ __global__ void __launch_bounds__(64) k_scan(TreeView T, TileGeo g, const int32_
 // number of tree tiles met along six rays before an empty ring or a
 // non-tree tile.
 __global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey,
-                           const uint32_t *tile_cnt, TileRec *rec,
+                           const uint8_t *state, TileRec *rec, int32_t *nground,
                            unsigned long long *nonempty)
 {
   // the non-empty tiles counted per block (one atomic on the counter per
@@ -2192,30 +2215,44 @@ __global__ void k_postscan(TileGeo g, const int32_t *tex, const int32_t *tey,
   if (threadIdx.x == 0) bcount = 0;
   __syncthreads();
   uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = t < g.ntiles && tile_cnt[t];
+  if (t < g.ntiles) nground[t] = 0;
+  const uint8_t mine = t < g.ntiles ? state[t] : 0;
+  const bool live = mine != 0;
   const uint64_t lv = __ballot(live);
   if (__lane_id() == 0 && lv) atomicAdd(&bcount, (uint32_t)__popcll(lv));
   __syncthreads();
   if (threadIdx.x == 0 && bcount) atomicAdd(nonempty, (unsigned long long)bcount);
   if (!live) return;
-  TileRec me = rec[t];
+  const double hs_scan = rec[t].hs_scan;
   const int r1x[6] = {1, 1, 0, -1, -1, 0}, r1y[6] = {0, 1, 1, 0, -1, -1};  // root1, eisenstein.cpp:51
   int i = 1, ring, nontree, count = 0;
-  do {
-    ring = nontree = 0;
-    for (int j = 0; j < 6 && (me.tree_flags & 1); j++) {
-      int o;
-      if (!tile_at(g, tex[t] + r1x[j] * i, tey[t] + r1y[j] * i, &o)) continue;
-      if (tile_cnt[o - g.lo]) {
-        ring++;
-        if (rec[o - g.lo].tree_flags & 1) count++;
-        else nontree++;
+  if (mine == 2) {
+    // a ring's six tiles are read together, each by its place and its state:
+    // the longest chain of rings is the kernel (18.5k points 22 us with the
+    // count and the record read tile by tile, 10 so; 1.17M 41 and 22)
+    const int ex = tex[t], ey = tey[t];
+    do {
+      ring = nontree = 0;
+      int o[6];
+      uint8_t q[6];
+#pragma unroll
+      for (int j = 0; j < 6; j++) {
+        int cnt;
+        o[j] = tile_at(g, ex + r1x[j] * i, ey + r1y[j] * i, &cnt) ? cnt - g.lo : -1;
       }
-    }
-    ++i;
-  } while (ring && !nontree);
+#pragma unroll
+      for (int j = 0; j < 6; j++) q[j] = o[j] >= 0 ? state[o[j]] : 0;
+#pragma unroll
+      for (int j = 0; j < 6; j++) {
+        ring += q[j] != 0;
+        count += q[j] == 2;
+        nontree += q[j] == 1;
+      }
+      ++i;
+    } while (ring && !nontree);
+  }
   double w = count * g.spacing / 6;
-  rec[t].hs = sqrt(me.hs_scan * me.hs_scan + w * w);
+  rec[t].hs = sqrt(hs_scan * hs_scan + w * w);
 }
 
 // The tiles' records in the caller's layout, empty tiles zero but for their
@@ -3839,6 +3876,7 @@ struct ClassifyRun {
   int32_t *tex, *tey, *memb, *grid;
   uint32_t *tile_cnt, *tile_fill, *nmemb, *err, *nslow, *tile_off, *lists;
   TileRec *rec;
+  uint8_t *state;
   unsigned long long *ctr;
   uint64_t gcells, total;
   uint8_t *cls;
@@ -3956,6 +3994,7 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
   int32_t *tey = R.tey = geo.tey;
   uint32_t *tile_cnt = R.tile_cnt = (uint32_t *)wb_alloc(c, 4ull * g.ntiles + 4);
   uint32_t *tile_fill = R.tile_fill = (uint32_t *)wb_alloc(c, 4ull * g.ntiles + 4);
+  uint8_t *state = R.state = (uint8_t *)wb_alloc(c, (size_t)g.ntiles + 4);
   TileRec *rec = R.rec = (TileRec *)wb_alloc(c, sizeof(TileRec) * (size_t)g.ntiles);
   int32_t *memb = R.memb = (int32_t *)wb_alloc(c, 4ull * MAX_MEMB * n + 16);
   uint32_t *nmemb = R.nmemb = (uint32_t *)wb_alloc(c, 4ull * n + 4);
@@ -3969,9 +4008,8 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
   unsigned long long *ctr = R.ctr = (unsigned long long *)err + 1;
   uint32_t *nslow = R.nslow = (uint32_t *)(ctr + 6);
   R.heavy_next = err + 18;
-  WB_CHECK(hipMemsetAsync(err, 0, 256, st));
-  WB_CHECK(hipMemsetAsync(tile_cnt, 0, 4ull * g.ntiles, st));
-  WB_CHECK(hipMemsetAsync(tile_fill, 0, 4ull * g.ntiles, st));
+  hipLaunchKernelGGL(k_pass_init, dim3(wb_blocks(std::max<uint64_t>(g.ntiles, 256), 1024)),
+                     dim3(256), 0, st, g.ntiles, tile_cnt, tile_fill, (uint32_t *)state, err);
   TreeView T = view(t);
   g.gx0 = geo.gx0;
   g.gy0 = geo.gy0;
@@ -3989,8 +4027,17 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
   wb_free(c, lflags, (size_t)LEAF_WIN * t->nleaves + 16);
   // tile lists in canonical order
   uint32_t *tile_off = R.tile_off = (uint32_t *)wb_alloc(c, 4ull * g.ntiles + 4);
-  WB_CHECK(hipMemcpyAsync(tile_off, tile_cnt, 4ull * g.ntiles, hipMemcpyDeviceToDevice, st));
-  const uint64_t total = R.total = wb_exclusive_scan_u32(c, tile_off, g.ntiles);
+  wb_exclusive_scan_u32_to(c, tile_cnt, tile_off, g.ntiles);
+  // room for the most list entries there can be, so that the host need not
+  // wait for their number (about 40 us); from 16M points, where the wait is
+  // lost in the pass and the room is not, the number itself
+  uint64_t total = MAX_MEMB * n;
+  if (n > (16u << 20)) {
+    WB_CHECK(hipStreamSynchronize(st));
+    const uint32_t *h = c->hbox + WB_HBOX_SCAN;
+    total = (uint64_t)h[0] | ((uint64_t)h[1] << 32);
+  }
+  R.total = total;
   uint32_t *lists = R.lists = (uint32_t *)wb_alloc(c, 4 * total + 4);
   if (n > 0)
     hipLaunchKernelGGL(k_tile_lists, dim3(wb_blocks(n, 256)), dim3(256), 0, st, n, memb, nmemb,
@@ -4021,14 +4068,14 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
       const ClassList c256 = {lb + e, -1, ncls + 5}, cbig = {la + e, -1, ncls + 6};
 #define WB_SCAN_REG(K, F32, T, W, least, CL)                                                      \
   hipLaunchKernelGGL((k_scan_reg<K, F32, T, W>), nb(least, T), dim3(64), 0, st, T_, g, tex, tey,  \
-                     tile_off, tile_cnt, lists, CL, p->min_hs, prec, rec, ctr)
+                     tile_off, tile_cnt, lists, CL, p->min_hs, prec, rec, state, ctr)
       const TreeView &T_ = T;
       if (many) {
         hipLaunchKernelGGL(k_scan_lane, nb(1, WAVE), dim3(64), 0, st, T, g, tex, tey, tile_off,
-                           tile_cnt, lists, c8, p->min_hs, rec, ctr);
+                           tile_cnt, lists, c8, p->min_hs, rec, state, ctr);
 #define WB_SCAN_ROW(GS, R, W, least, CL)                                                          \
   hipLaunchKernelGGL((k_scan_row<GS, R, W>), nb(least, WAVE / GS * R), dim3(64), 0, st, T, g, tex, \
-                     tey, tile_off, tile_cnt, lists, CL, p->min_hs, rec, ctr)
+                     tey, tile_off, tile_cnt, lists, CL, p->min_hs, rec, state, ctr)
         WB_SCAN_ROW(16, 4, 3, 9, c16);
         WB_SCAN_ROW(32, 4, 3, 17, c32);
         WB_SCAN_REG(1, false, 4, 4, 33, c64);
@@ -4037,7 +4084,7 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
         WB_SCAN_REG(4, false, 1, 4, 129, c256);
       } else if (prec == WB_FIT_FP64) {
         hipLaunchKernelGGL(k_scan_mixed, nb(1, 1), dim3(64), 0, st, T, g, tex, tey, tile_off, tile_cnt,
-                           lists, c16, c32, c64, c128, c256, p->min_hs, rec, ctr);
+                           lists, c16, c32, c64, c128, c256, p->min_hs, rec, state, ctr);
       } else {
         WB_SCAN_REG(1, true, 1, 4, 1, c16);
         WB_SCAN_REG(1, true, 1, 4, 17, c32);
@@ -4047,14 +4094,14 @@ static void classify_prepare(ClassifyRun &R, wb_tree *t, wb_ctx *c, const double
       }
 #undef WB_SCAN_REG
       hipLaunchKernelGGL(k_scan, dim3(std::min(nb(257, 1).x, 4096u)), dim3(64), 0, st, T, g, tex,
-                         tey, tile_off, tile_cnt, lists, cbig, p->min_hs, prec, rec, err, ctr);
+                         tey, tile_off, tile_cnt, lists, cbig, p->min_hs, prec, rec, state, err, ctr);
     }
     wb_free(c, lb, 4ull * g.ntiles + 4);
     wb_free(c, lc, 4ull * g.ntiles + 4);
     wb_free(c, ld, 4ull * g.ntiles + 4);
   }
   hipLaunchKernelGGL(k_postscan, dim3(wb_blocks(g.ntiles, 256)), dim3(256), 0, st, g, tex, tey,
-                     tile_cnt, rec, ctr + 5);
+                     state, rec, (int32_t *)tile_fill, ctr + 5);
   WB_CHECK(hipEventRecord(ev[2], st));
   for (int k = 4; k < 8; k++) WB_CHECK(hipEventRecord(ev[k], st));
   if (scan_only) return;
@@ -4155,9 +4202,8 @@ static void classify_finish(ClassifyRun &R)
   unsigned long long *ctr = R.ctr;
   uint8_t *cls = R.cls, *d_class_out = R.d_class_out;
   const ClassifyArgs &A = R.A;
-  int32_t *nground = (int32_t *)R.tile_fill;  // reused once the lists are built
+  int32_t *nground = (int32_t *)R.tile_fill;  // (k_postscan cleared it)
   if (!scan_only) {
-    WB_CHECK(hipMemsetAsync(nground, 0, 4ull * g.ntiles, st));
     if (n > 0) {
       const unsigned nbk = wb_blocks(n, 256);
       uint32_t *partial = (uint32_t *)wb_alloc(c, 12ull * nbk);
@@ -4260,6 +4306,7 @@ static void classify_finish(ClassifyRun &R)
   wb_free(c, R.tile_cnt, 4ull * g.ntiles + 4);
   wb_free(c, R.tile_fill, 4ull * g.ntiles + 4);
   wb_free(c, rec, sizeof(TileRec) * (size_t)g.ntiles);
+  wb_free(c, R.state, (size_t)g.ntiles + 4);
   wb_free(c, memb, 4ull * MAX_MEMB * n + 16);
   wb_free(c, nmemb, 4ull * n + 4);
   wb_free(c, R.tile_off, 4ull * g.ntiles + 4);

@@ -208,6 +208,9 @@ void wb_run_classify(wb_tree *t, const double *corners, int ncorners,
 // ---- building blocks implemented in wb_build.hip ----
 // exclusive scan of u32 in place, returns the total (synchronous read-back)
 uint64_t wb_exclusive_scan_u32(wb_ctx *c, uint32_t *data, uint64_t n);
+// the same out of place and without waiting; the total (two words) is at
+// c->hbox + WB_HBOX_SCAN once the stream has passed
+void wb_exclusive_scan_u32_to(wb_ctx *c, const uint32_t *in, uint32_t *out, uint64_t n);
 // LSD radix sort of (u64 key, u32 val) pairs on bits [64-8*passes, 64)
 void wb_radix_sort_pairs(wb_ctx *c, uint64_t *key, uint32_t *val, uint64_t n, int passes);
 // LSD radix sort of (u32 key, u32 val) pairs on bits [32-8*passes, 32)
