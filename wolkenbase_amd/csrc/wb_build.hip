@@ -1114,6 +1114,25 @@ __global__ void __launch_bounds__(256) k_leaf_finish(const uint32_t *leaf_start,
   }
 }
 
+// A wave per leaf: whether it holds a point outside its cube (only leaves
+// with an extreme cell can, and only where a point lies outside the root).
+__global__ void __launch_bounds__(256) k_leaf_out(const uint32_t *leaf_start, uint32_t nl,
+                                                  const double *px, const double *py,
+                                                  const double *pz, const double *leaf_cube,
+                                                  uint8_t *out)
+{
+  const uint32_t l = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  if (l >= nl) return;
+  const double *c = leaf_cube + 4 * (size_t)l;
+  const double h = c[3] / 2;
+  bool o = false;
+  for (uint32_t j = leaf_start[l] + lane; j < leaf_start[l + 1]; j += WAVE)
+    o = o || !(px[j] >= c[0] - h && px[j] <= c[0] + h && py[j] >= c[1] - h && py[j] <= c[1] + h &&
+               pz[j] >= c[2] - h && pz[j] <= c[2] + h);
+  const uint64_t any = __ballot(o);
+  if (lane == 0) out[l] = any != 0;
+}
+
 // ---------------------------------------------------------------------------
 // host driver
 // ---------------------------------------------------------------------------
@@ -1396,6 +1415,12 @@ void wb_build_tree(wb_tree *t, const int32_t *dx, const int32_t *dy, const int32
     hipLaunchKernelGGL(k_leaf_finish, dim3(nl), dim3(256), 0, c->stream, t->leaf_start, t->sidx,
                        t->pz, t->leaf_parent, t->node_child, t->node_parent, t->canon,
                        t->crank, t->leaf_low, t->child_zlow);
+    t->leaf_out = nullptr;
+    if (t->outside_root) {
+      t->leaf_out = wb_talloc<uint8_t>(t, nl);
+      hipLaunchKernelGGL(k_leaf_out, dim3(wb_blocks(nl, 4)), dim3(256), 0, c->stream, t->leaf_start,
+                         nl, t->px, t->py, t->pz, t->leaf_cube, t->leaf_out);
+    }
     WB_CHECK(hipEventRecord(evb[3], c->stream));
   } else {
     t->evb_read = true;

@@ -81,6 +81,7 @@ struct TreeView {
   double ox, oy, oz, side;  // the root cube
   const uint2 *node_crange;
   const double *child_zlow;
+  const uint8_t *leaf_out;
   const uint32_t *pt_leaf, *canon, *crank, *sidx;
   uint32_t nleaves, nnodes;
   uint64_t n;
@@ -97,6 +98,7 @@ static TreeView view(const wb_tree *t)
   v.ox = t->center[0]; v.oy = t->center[1]; v.oz = t->center[2]; v.side = t->side;
   v.chunk_sx = t->chunk_sx; v.chunk_sy = t->chunk_sy; v.chunk_sz = t->chunk_sz; v.node_crange = t->node_crange;
   v.child_zlow = t->child_zlow;
+  v.leaf_out = t->leaf_out;
   v.pt_leaf = t->pt_leaf; v.canon = t->canon; v.crank = t->crank;
   v.sidx = t->sidx; v.nleaves = t->nleaves; v.nnodes = t->nnodes; v.n = t->n;
   return v;
@@ -2385,6 +2387,7 @@ struct ClassifyArgs {
   uint32_t *pool;
   uint64_t pool_shared, pool_cap;
   uint32_t unit_cap, open_per;
+  uint32_t walk_per;  // points of a wave of walk A (at least open_per)
   int open_classes;
   uint32_t *nopen, *open_next;
   unsigned long long *npool;
@@ -2526,6 +2529,16 @@ struct WaveStack {
 __device__ inline double uload(const double *p, size_t i)
 {
   return ((const __attribute__((address_space(4))) double *)p)[i];
+}
+
+// a value every lane reads from the same address, as uload
+__device__ inline float uloadf(const float *p, size_t i)
+{
+  return ((const __attribute__((address_space(4))) float *)p)[i];
+}
+__device__ inline uint32_t uloadu(const uint32_t *p, size_t i)
+{
+  return ((const __attribute__((address_space(4))) uint32_t *)p)[i];
 }
 
 // A lane's hyperboloid as hyp_near reads it
@@ -2702,8 +2715,8 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
   const TreeView &T = A.T;
   const uint32_t lane = __lane_id();
   // work index: a sorted slot, or a work item
-  const uint64_t i = unit * WAVE + lane;
-  const bool inrange = i < (A.items ? A.n_items : T.n);
+  const uint64_t i = unit * A.walk_per + lane;
+  const bool inrange = lane < A.walk_per && i < (A.items ? A.n_items : T.n);
   // lane state: 0 undecided, 1 not ground, 3 no tile; handed on: 5 to the
   // heavy kernel, walk A cut short
   int state = 3;
@@ -2748,9 +2761,11 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
       // the lanes' own tests: whether the cube, its bottom face raised, may
       // meet the lane's hyperboloid and care wedges
       bool on = (m >> lane) & 1;
-      const bool anyw = IN && __ballot(on && W.n >= 0) != 0;
+      // a leaf whose points lie in its cube, also where not every leaf's do
+      const bool lin = IN || (code < 0 && rfl((int)T.leaf_out[-2 - code]) == 0);
+      const bool anyw = lin && __ballot(on && W.n >= 0) != 0;
       const double hh = side / 2, x0 = cx - hh, x1 = cx + hh, y0 = cy - hh, y1 = cy + hh;
-      if (!IN) {
+      if (!lin) {
         // a point may lie outside its leaf's cube, so reaching the leaf does
         // not follow from the point: findBlocks' own test, cube by cube
         wb::Shape H = wb::make_cylinder(x, y, 0);
@@ -2761,7 +2776,8 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
         on = on && wb::hyp_intersect(H, cx, cy, cz, side);
         m = __ballot(on);
       } else if (code < 0 || anyw) {
-        const double zb = fmax(cz - hh, (double)__uint_as_float((uint32_t)rfl((int)en.w)));
+        const double zb = fmax(cz - hh, IN ? (double)__uint_as_float((uint32_t)rfl((int)en.w))
+                                           : (double)uloadf(T.leaf_low, (uint32_t)(-2 - code)));
         on = on && near_t(P, s2, fmin(fmax(x, x0), x1), fmin(fmax(y, y0), y1), zb) >= P.thr;
         if (anyw) on = on && wb::lane_hit(W, x, y, x0, x1, y0, y1);
         m = __ballot(on);
@@ -2815,7 +2831,7 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
       if (state == 0 && occ != checked) {
         checked = occ;
         if (gap_verdict(occ) == 1) state = 1;
-        else if (IN) wb::lane_wedges_update(occ, edges, W);
+        else wb::lane_wedges_update(occ, edges, W);
       }
       alive = __ballot(state == 0);
       if (alive == 0) break;
@@ -2910,16 +2926,6 @@ struct OpenPoint {
   int hi[2], lo[2];
 };
 
-// a value every lane reads from the same address, as uload
-__device__ inline float uloadf(const float *p, size_t i)
-{
-  return ((const __attribute__((address_space(4))) float *)p)[i];
-}
-__device__ inline uint32_t uloadu(const uint32_t *p, size_t i)
-{
-  return ((const __attribute__((address_space(4))) uint32_t *)p)[i];
-}
-
 template <bool IN, bool GAP>
 __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t *pool, uint32_t nleaf,
                                           const Near &P, OpenPoint &O, const float *edges,
@@ -2944,7 +2950,8 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
       const double *c = T.leaf_cube + 4 * (size_t)leaf_l;
       const double h = c[3] / 2;
       lh = union_hits(U, s2, c[0] - h, c[0] + h, c[1] - h, c[1] + h,
-                      IN ? fmax(c[2] - h, (double)T.leaf_low[leaf_l]) : c[2] - h);
+                      IN || !T.leaf_out[leaf_l] ? fmax(c[2] - h, (double)T.leaf_low[leaf_l])
+                                                : c[2] - h);
     }
     uint64_t ltodo = __ballot(lh);
     while (ltodo) {
@@ -2953,11 +2960,11 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
       const uint32_t leaf = (uint32_t)__builtin_amdgcn_readlane((int)leaf_l, (int)ls);
       const uint32_t b = uloadu(T.leaf_start, leaf), e = uloadu(T.leaf_start, leaf + 1);
       bool on = O.state == want, all = false;
-      bool anyw = IN && __ballot(on && O.W.n >= 0) != 0;
+      bool anyw = __ballot(on && O.W.n >= 0) != 0;
       {
         const double *c = T.leaf_cube + 4 * (size_t)leaf;
         const double cx = uload(c, 0), cy = uload(c, 1), cz = uload(c, 2), hh = uload(c, 3) / 2;
-        if (IN) {
+        if (IN || rfl((int)T.leaf_out[leaf]) == 0) {
           const double x0 = cx - hh, x1 = cx + hh, y0 = cy - hh, y1 = cy + hh;
           on = on && near_t(P, s2, fmin(fmax(x, x0), x1), fmin(fmax(y, y0), y1),
                             fmax(cz - hh, (double)uloadf(T.leaf_low, leaf))) >= P.thr;
@@ -2982,10 +2989,12 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
         }
       }
       if (!__ballot(on)) continue;
+      const bool anyall = !IN && __ballot(all) != 0;
       const uint32_t q0 = b / WB_OCT, nq = (e - 1) / WB_OCT - q0 + 1;
       for (uint32_t qb = 0; qb < nq; qb += WAVE) {
         bool h = qb + lane < nq;
-        if (IN && h) {
+        // (a lane that takes the whole leaf takes points outside its box's reach)
+        if (h && (IN || !anyall)) {
           const Union R = {U.x0 - T.ox, U.x1 - T.ox, U.y0 - T.oy, U.y1 - T.oy, U.cz - T.oz, U.thr};
           const float4 bx = T.oct_xy[q0 + qb + lane];
           h = union_hits(R, s2, bx.x, bx.y, bx.z, bx.w, T.oct_z[q0 + qb + lane]);
@@ -3032,6 +3041,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
               const double dx = gx - (up ? qx : ox), dy = gy - (up ? qy : oy);
               const double dz = (up ? qz : oz) - gz;
               bool c = wb::hyp_near(s2, dx, dy, dz) >= (up ? qt : ot);
+              if (!IN) c = c | (__shfl((int)all, (int)(up ? o2 : o1), WAVE) != 0);
               if (anyw && __ballot(c)) {
                 wb::LaneWedges V;
                 const int o = (int)(up ? o2 : o1);
@@ -3045,7 +3055,6 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
               if (lane == o1) cand = (uint32_t)cm;
               if (lane == o2 && o2 != o1) cand = (uint32_t)(cm >> 32);
             }
-            if (!IN && all) cand = 0xffffffffu;
             // the group's slots inside the leaf
             const uint32_t s0 = chk * WB_CHUNK;
             if (b > s0) cand &= ~0u << (b - s0);
@@ -3064,7 +3073,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
             for (uint32_t k = 0; k < WB_OCT; k++) {
               const uint32_t j = WB_OCT * (q % (WB_CHUNK / WB_OCT)) + k;
               const double dx = rdl(gx, j) - x, dy = rdl(gy, j) - y, dz = P.cz - rdl(gz, j);
-              bool c = hit & (wb::hyp_near(s2, dx, dy, dz) >= P.thr);
+              bool c = hit & (all | (wb::hyp_near(s2, dx, dy, dz) >= P.thr));
               if (!__ballot(c)) continue;
               if (anyw) c = c & wb::lane_dir(O.W, (float)dx, (float)dy);
               c8 |= c ? 1u << k : 0u;
@@ -3073,7 +3082,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
             const uint32_t k0 = b > q * WB_OCT ? b - q * WB_OCT : 0;
             const uint32_t k1 = e < (q + 1) * WB_OCT ? e - q * WB_OCT : WB_OCT;
             const uint32_t in8 = ((1u << k1) - 1) & ~((1u << k0) - 1);
-            cand |= ((!IN && all ? 0xffu : c8) & in8) << (WB_OCT * (q % (WB_CHUNK / WB_OCT)));
+            cand |= (c8 & in8) << (WB_OCT * (q % (WB_CHUNK / WB_OCT)));
           }
           if (!hit) cand = 0;
           uint32_t taken = 0;
@@ -3132,7 +3141,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
           }
           // many candidates: the directions just found may leave out the next
           // group's
-          if (IN && !GAP && taken >= OPEN_REFRESH && O.occ != checked && O.state == 0) {
+          if (!GAP && taken >= OPEN_REFRESH && O.occ != checked && O.state == 0) {
             checked = O.occ;
             if (gap_verdict(O.occ) == 1) {
               O.state = 1;
@@ -3141,7 +3150,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
               wb::lane_wedges_update(O.occ, edges, O.W);
             }
           }
-          if (IN && !GAP && taken >= OPEN_REFRESH) anyw = __ballot(on && O.W.n >= 0) != 0;
+          if (!GAP && taken >= OPEN_REFRESH) anyw = __ballot(on && O.W.n >= 0) != 0;
         }
       }
       if (!GAP) {
@@ -3156,7 +3165,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
         if (O.state == 0 && O.occ != checked) {
           checked = O.occ;
           if (gap_verdict(O.occ) == 1) O.state = 1;
-          else if (IN) wb::lane_wedges_update(O.occ, edges, O.W);
+          else wb::lane_wedges_update(O.occ, edges, O.W);
         }
       }
       alive = __ballot(O.state == want);
@@ -3198,7 +3207,6 @@ __device__ __forceinline__ void open_body(const ClassifyArgs &A, uint32_t u, con
   const Near P = make_near(A, x, y, z, hs);
   int nexact = 0;
   wb::lane_wedges_update(O.occ, edges, O.W);
-  if (!IN) O.W.n = -1;
   open_pass<IN, false>(A, pool, nleaf, P, O, edges, edge, nexact);
   if (O.state == 0) {
     O.state = gap_verdict(O.occ);
@@ -3224,7 +3232,7 @@ __device__ __forceinline__ void open_body(const ClassifyArgs &A, uint32_t u, con
       wb::border_wedges(before, after, nr, w, edges);
       O.W.ax[0] = w.ax[0]; O.W.ay[0] = w.ay[0]; O.W.bx[0] = w.bx[0]; O.W.by[0] = w.by[0];
       O.W.ax[1] = w.ax[2]; O.W.ay[1] = w.ay[2]; O.W.bx[1] = w.bx[2]; O.W.by[1] = w.by[2];
-      O.W.n = IN && nr ? nr == 2 ? 3 : 1 : -1;
+      O.W.n = nr ? nr == 2 ? 3 : 1 : -1;
     }
     O.border = (uint32_t)before[0] | (uint32_t)after[0] << 8 | (uint32_t)before[1] << 16 |
                (uint32_t)after[1] << 24;
@@ -3279,7 +3287,7 @@ __global__ void __launch_bounds__(WAVE, MINW) k_ground_resident(ClassifyArgs A, 
   __shared__ WaveStack S;
   __shared__ float edges[3 * 128];
   ground_setup(A, edges);
-  const uint64_t nunits = ((A.items ? A.n_items : A.T.n) + WAVE - 1) / WAVE;
+  const uint64_t nunits = ((A.items ? A.n_items : A.T.n) + A.walk_per - 1) / A.walk_per;
   uint64_t unit = blockIdx.x;
   while (unit < nunits) {
     walk_body<IN>(A, unit, S, edges);
@@ -3984,27 +3992,32 @@ static const wb_ctx::TileGeoCache &tile_geometry(wb_ctx *c, const TileGeo &g0)
 
 static void open_buffers(wb_ctx *c, ClassifyArgs &A, uint64_t n, uint64_t nbatch, OpenBuffers &B)
 {
-  const uint64_t waves = (n + WAVE - 1) / WAVE;
+  const uint64_t resident = 20 * (uint64_t)c->ncu;
+  // Points of a wave of walk A and of a unit of walk B.  A wave of 16 takes
+  // more than a quarter of the time of one of 64 (lanes that need the same
+  // nodes and points share their tests), but with few waves the longest one is
+  // the kernel (ground test of 18.5k points 0.27 ms with waves of 64, 0.25
+  // with 16; 150k with outliers above 1.60 and 1.31; 300k, waves of 32, 1.77
+  // and 1.65).
+  const uint64_t all = (nbatch ? nbatch : n) / WAVE;
+  A.walk_per = 2 * all < resident ? 16 : all < resident ? 32 : WAVE;
+  A.open_per = WAVE;
+  const uint64_t waves = (n + A.walk_per - 1) / A.walk_per;
   B.nrec = (size_t)waves * WAVE;
   const uint32_t ucap = (uint32_t)std::min<uint64_t>(waves * 4, 0x3fffffffull);
   A.pool_shared = waves * OPEN_LIST;
   B.npool = (size_t)(waves * (OPEN_LIST + 16) + 65536);
   A.pool_cap = B.npool;
   A.unit_cap = (uint32_t)waves;
-  A.open_per = WAVE;
   // The longest first while a long one is a large part of the whole (1.17M
   // points 3.07 to 2.49 ms); with more points neighbours in space stay
   // neighbours in time, which the caches gain from, and no place in a class is
   // claimed (23.7M points, mostly ground: 31.8 to 29.8 ms).
-  const uint64_t resident = 20 * (uint64_t)c->ncu;
   A.open_classes = nbatch || c->sharing || waves < 20 * resident;
   if (A.open_classes) {
     A.unit_cap = ucap;
-    // Lanes of a unit.  A unit of 16 takes more than a quarter of the time of
-    // one of 64 (lanes that need the same points share their tests), but with
-    // few units the longest one is the kernel.
-    const uint64_t all = nbatch ? nbatch / WAVE : waves;
     A.open_per = 2 * all < resident ? OPEN_P1 : 3 * all < 4 * resident ? OPEN_P2 : WAVE;
+    A.open_per = std::min(A.open_per, A.walk_per);
   }
   B.nunit = (size_t)A.unit_cap * (A.open_classes ? OPEN_CLASSES : 1);
   A.open = B.open = (HeavyRec *)wb_alloc(c, sizeof(HeavyRec) * B.nrec + 16);
@@ -4183,7 +4196,7 @@ static void launch_ground(wb_ctx *c, const ClassifyArgs &A, uint64_t n, uint32_t
   const uint32_t ncu = (uint32_t)c->ncu;
   if (ev) WB_CHECK(hipEventRecord(ev[0], st));
   if (n > 0) {
-    const uint32_t nb = wb_blocks(n, WAVE);
+    const uint32_t nb = wb_blocks(n, A.walk_per);
     const dim3 one(WAVE);
     // sharing: 16 of the 20 waves a CU holds: a wave slot and LDS stay free on
     // every SIMD for other contexts' kernels
@@ -4207,7 +4220,7 @@ static void launch_ground(wb_ctx *c, const ClassifyArgs &A, uint64_t n, uint32_t
       if (A.cube_wedges) hipLaunchKernelGGL(k_ground_open_resident<true>, ogrid, one, 0, st, A);
       else hipLaunchKernelGGL(k_ground_open_resident<false>, ogrid, one, 0, st, A);
     } else {
-      const dim3 ogrid(nb * (WAVE / A.open_per));
+      const dim3 ogrid(nb * (A.walk_per / A.open_per));
       if (A.cube_wedges) hipLaunchKernelGGL(k_ground_open<true>, ogrid, one, 0, st, A);
       else hipLaunchKernelGGL(k_ground_open<false>, ogrid, one, 0, st, A);
     }
@@ -4400,7 +4413,7 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
   for (int k = 0; k < ntrees; k++) {
     AA[k] = R[k].A;
     inside = inside && AA[k].cube_wedges;
-    const uint64_t nb = boff[k] + (uint64_t)wb_blocks(R[k].n, WAVE);
+    const uint64_t nb = boff[k] + (uint64_t)wb_blocks(R[k].n, AA[k].walk_per);
     if (nb > 0xffffffffull) throw std::string("too many points in one batch");
     boff[k + 1] = (uint32_t)nb;
   }
@@ -4412,7 +4425,7 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
   WB_CHECK(hipMemcpyAsync(doff, boff.data(), 4 * (ntrees + 1), hipMemcpyHostToDevice, st));
   for (int k = 0; k < ntrees; k++) WB_CHECK(hipEventRecord(R[k].ev[4], st));
   if (boff[ntrees]) {
-    const dim3 one(WAVE), ogrid(boff[ntrees] * (WAVE / AA[0].open_per));
+    const dim3 one(WAVE), ogrid(boff[ntrees] * (AA[0].walk_per / AA[0].open_per));
     if (inside) {
       hipLaunchKernelGGL((k_ground_batch<true, WB_GROUND_MINW>), dim3(boff[ntrees]), one, 0, st, dAA,
                          doff, ntrees);

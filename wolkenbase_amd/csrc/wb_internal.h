@@ -127,6 +127,7 @@ struct wb_tree {
   float4 *oct_xy;
   float *oct_z;
   float *leaf_low;  // per leaf, at most the lowest z stored in it
+  uint8_t *leaf_out;  // with outside_root: leaves with a point outside their cube
   uint32_t *leaf_start;
   double *leaf_cube;
   int32_t *leaf_parent;
