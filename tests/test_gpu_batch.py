@@ -69,3 +69,26 @@ def test_batch_refuses_trees_of_two_contexts(ctx):
         t1.free()
         t2.free()
         other.close()
+
+
+@pytest.mark.parametrize("order", [(0, 1), (1, 0), (0, 0, 1)])
+def test_batch_with_points_outside_one_root(ctx, order):
+    # a tree with points outside its root cube (a header box smaller than the
+    # cloud) in one launch with trees that have none
+    inside = synth.generate(seed=77, extent=20.0, density=25.0, outliers=0.02, outlier_low=0.0)
+    outside = synth.generate(seed=31, extent=40.0, density=20.0, embankments=1, outliers=0.01)
+    lo, hi = np.array(outside["bbmin"], float), np.array(outside["bbmax"], float)
+    z = outside["offset"][2] + outside["scale"][2] * outside["zi"]
+    outside = dict(outside, bbmin=[*(lo + 0.05 * (hi - lo))[:2], float(np.percentile(z, 20))],
+                   bbmax=[*(lo + 0.95 * (hi - lo))[:2], float(np.percentile(z, 90))])
+    clouds = [(inside, outside)[k] for k in order]
+    trees = [build(ctx, c) for c in clouds]
+    try:
+        got, _ = W.classify_batch(trees, [c["bbmin"] for c in clouds],
+                                  [c["bbmax"] for c in clouds])
+        for g, c in zip(got, clouds):
+            want, _, _ = O.run(c)
+            assert np.array_equal(g, want)
+    finally:
+        for t in trees:
+            t.free()

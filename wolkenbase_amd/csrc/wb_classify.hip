@@ -98,10 +98,17 @@ static TreeView view(const wb_tree *t)
   v.ox = t->center[0]; v.oy = t->center[1]; v.oz = t->center[2]; v.side = t->side;
   v.chunk_sx = t->chunk_sx; v.chunk_sy = t->chunk_sy; v.chunk_sz = t->chunk_sz; v.node_crange = t->node_crange;
   v.child_zlow = t->child_zlow;
-  v.leaf_out = t->leaf_out;
+  v.leaf_out = t->leaf_out;  // (null without a point outside the root)
   v.pt_leaf = t->pt_leaf; v.canon = t->canon; v.crank = t->crank;
   v.sidx = t->sidx; v.nleaves = t->nleaves; v.nnodes = t->nnodes; v.n = t->n;
   return v;
+}
+
+// every point of the leaf lies in its cube (a tree of a batch may have no
+// leaf_out where another one has)
+__device__ inline bool leaf_inside(const TreeView &T, uint32_t leaf)
+{
+  return !T.leaf_out || T.leaf_out[leaf] == 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -2762,7 +2769,7 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
       // meet the lane's hyperboloid and care wedges
       bool on = (m >> lane) & 1;
       // a leaf whose points lie in its cube, also where not every leaf's do
-      const bool lin = IN || (code < 0 && rfl((int)T.leaf_out[-2 - code]) == 0);
+      const bool lin = IN || (code < 0 && leaf_inside(T, (uint32_t)(-2 - code)));
       const bool anyw = lin && __ballot(on && W.n >= 0) != 0;
       const double hh = side / 2, x0 = cx - hh, x1 = cx + hh, y0 = cy - hh, y1 = cy + hh;
       if (!lin) {
@@ -2950,7 +2957,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
       const double *c = T.leaf_cube + 4 * (size_t)leaf_l;
       const double h = c[3] / 2;
       lh = union_hits(U, s2, c[0] - h, c[0] + h, c[1] - h, c[1] + h,
-                      IN || !T.leaf_out[leaf_l] ? fmax(c[2] - h, (double)T.leaf_low[leaf_l])
+                      IN || leaf_inside(T, leaf_l) ? fmax(c[2] - h, (double)T.leaf_low[leaf_l])
                                                 : c[2] - h);
     }
     uint64_t ltodo = __ballot(lh);
@@ -2964,7 +2971,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
       {
         const double *c = T.leaf_cube + 4 * (size_t)leaf;
         const double cx = uload(c, 0), cy = uload(c, 1), cz = uload(c, 2), hh = uload(c, 3) / 2;
-        if (IN || rfl((int)T.leaf_out[leaf]) == 0) {
+        if (IN || leaf_inside(T, leaf)) {
           const double x0 = cx - hh, x1 = cx + hh, y0 = cy - hh, y1 = cy + hh;
           on = on && near_t(P, s2, fmin(fmax(x, x0), x1), fmin(fmax(y, y0), y1),
                             fmax(cz - hh, (double)uloadf(T.leaf_low, leaf))) >= P.thr;
