@@ -602,3 +602,42 @@ def test_scan_of_every_tile_size(ctx, height):
         want = tile_record(px[ids] - cx, py[ids] - cy, pz[ids], r, prm.min_hs)
         for f, v in want.items():
             assert tiles[f][k] == v, (k, f, len(ids))
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_gap_borders_far_from_the_point_match_oracle(ctx, seed):
+    # points high above the apex of an empty sector of 144 degrees: whether
+    # they are ground rests on the extreme directions in the two bins beside a
+    # run of 24 or 25, which points of any leaf along the sector's edges give,
+    # also after nearer ones have taken those bins
+    rng = np.random.default_rng(seed)
+    t0 = rng.random() * 2 * np.pi
+    # two dense strips from 10 to 60 m along a sector of 138 degrees, thin in
+    # the six degrees next to it (a few points), and some in the other directions
+    n = 80000
+    th = np.radians(rng.random(n) * 14)
+    keep = (th > math.radians(6)) | (rng.random(n) < 1e-4)
+    side = rng.random(n) < 0.5
+    a = t0 + np.where(side, math.radians(138) + th, -th)
+    r = 10 + 50 * np.sqrt(rng.random(n))
+    a, r = a[keep], r[keep]
+    ao = t0 + math.radians(152) + rng.random(3000) * math.radians(194)
+    ro = 5 + 55 * rng.random(3000)
+    a, r = np.concatenate([a, ao]), np.concatenate([r, ro])
+    m = 300
+    x = np.concatenate([r * np.cos(a), rng.normal(0, 0.7, m)])
+    y = np.concatenate([r * np.sin(a), rng.normal(0, 0.7, m)])
+    z = np.concatenate([rng.random(len(a)) * 0.2, np.full(m, 62.0)])
+    xi, yi, zi = (np.round(v * 1000).astype(np.int32) for v in (x + 100, y + 100, z))
+    sc, off = np.array([0.001] * 3), np.array([5e5, 4.4e6, 0.0])
+    raw = np.stack([xi, yi, zi])
+    cloud = dict(xi=xi, yi=yi, zi=zi, scale=sc, offset=off, bbmin=off + sc * raw.min(1),
+                 bbmax=off + sc * raw.max(1))
+    tree, _, _ = build_both(ctx, cloud)
+    got, _, st = W.classify(tree, cloud["bbmin"], cloud["bbmax"], want_tiles=False)
+    want, _, _ = O.run(cloud)
+    high = np.arange(len(x)) >= len(x) - m
+    print("gap points", st["exact_gap_points"], "differ", int((got != want).sum()),
+          "of the high ones ground", int((want[high] == 2).sum()))
+    assert st["exact_gap_points"] > 0 and (want[high] > 0).all()
+    assert np.array_equal(got, want)

@@ -595,3 +595,21 @@ def test_octet_bounds_round_outwards(hm):
         assert hm.wbh_rel_down(v, o, side) <= d - slack
         assert hm.wbh_rel_up(v, o, side) >= d + slack
     assert hm.wbh_rel_down(1e300, 0.0, 1.0) <= 3.1e38 and hm.wbh_rel_up(-1e300, 0.0, 1.0) >= -3.1e38
+
+
+def test_borders_open_clears_the_bins_beside_care_runs(hm):
+    hm.wbh_borders_open.restype = C.c_uint64
+    hm.wbh_borders_open.argtypes = [C.c_uint64]
+    rng = np.random.default_rng(35)
+    runs = 0
+    for it in range(20000):
+        occ, base = 0, int(rng.integers(0, 64))
+        for _ in range(int(rng.integers(1, 12))):
+            occ |= 1 << ((base + int(rng.integers(0, 41))) % 64)
+        care = care_bins(occ)
+        want = occ
+        for b in care:
+            want &= ~((1 << ((b + 1) % 64)) | (1 << ((b - 1) % 64)))
+        runs += len(care) > 0
+        assert hm.wbh_borders_open(occ) == want, hex(occ)
+    assert runs > 5000

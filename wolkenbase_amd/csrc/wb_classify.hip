@@ -2838,7 +2838,7 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
       if (state == 0 && occ != checked) {
         checked = occ;
         if (gap_verdict(occ) == 1) state = 1;
-        else wb::lane_wedges_update(occ, edges, W);
+        else wb::lane_wedges_update(wb::borders_open(occ), edges, W);
       }
       alive = __ballot(state == 0);
       if (alive == 0) break;
@@ -2918,9 +2918,9 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
 // the 23.7M-point tile with all outliers above the surface).  Walks A and B
 // and the gap pass in one kernel, with every lane testing every child, sample
 // and box by hyp_in and the gap pass left to the heavy kernel, took 41.5 and
-// 12.7 ms on that tile against 9 + 20 and 0.25 ms now, 4.9 and 0.32 against
-// 3.7 and 0.08 ms on the one with low outliers, 2.7 and 0.67 against 2.0 and
-// 0.08 ms on 1.17M points, 0.46 and 0.04 against 0.28 and 0.01 ms on 18.5k.
+// 12.7 ms on that tile against 9 + 19 and 0.3 ms now, 4.9 and 0.32 against
+// 4.3 and 0.08 ms on the one with low outliers, 2.7 and 0.67 against 2.0 and
+// 0.08 ms on 1.17M points, 0.46 and 0.04 against 0.25 and 0.01 ms on 18.5k.
 struct OpenPoint {
   int state;  // 0 undecided, 1 not ground, 2 ground, 3 none, 4 the exact gap
               // decides; to the heavy kernel: 6 walk B, 7 the exact gap

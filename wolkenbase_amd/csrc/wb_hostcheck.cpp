@@ -80,6 +80,8 @@ int wbh_lane_wedges(uint64_t occ, double px, double py, double x0, double x1, do
          (wb::lane_dir(w, (float)(x0 - px), (float)(y0 - py)) ? 2 : 0);
 }
 
+uint64_t wbh_borders_open(uint64_t occ) { return wb::borders_open(occ); }
+
 // bit 0: hyp_in; bit 1: hyp_near reaches its threshold
 int wbh_hyp_near(const double *p, const double *q)
 {

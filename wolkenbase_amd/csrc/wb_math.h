@@ -937,6 +937,21 @@ WB_HD bool wedge_hit2(int n, const float ax[2], const float ay[2], const float b
 // A lane's care wedges: those of care_wedges, at most two; a lane with
 // more (two runs, one of them 32 bins or more) is not pruned (n < 0).  n: 0
 // none, 1 one run, 2 one run split in two, 3 two runs (two wedges).
+// occ without the bins that border its care runs.  Where a run of 24 or 25
+// empty bins is what remains, the extreme directions in its two border bins
+// decide, so a walk whose leaves are to serve that question too must keep the
+// leaves of the border bins, also once these are occupied: its wedges are those
+// of this mask.
+WB_HD uint64_t borders_open(uint64_t occ)
+{
+  int rs[2], rl[2];
+  const int nr = care_runs(occ, rs, rl);
+  uint64_t m = occ;
+  for (int r = 0; r < 2; r++)
+    if (r < nr) m &= ~((1ull << ((rs[r] + 63) & 63)) | (1ull << ((rs[r] + rl[r]) & 63)));
+  return m;
+}
+
 struct LaneWedges {
   float ax[2], ay[2], bx[2], by[2];
   int n;
