@@ -476,13 +476,15 @@ static int check_kind(int kind) { return kind == WB_SHAPE_CYLINDER || kind == WB
 // Batches of fewer shapes take a wave per shape in the caller's order; the
 // others a lane per shape, sorted so that the 64 of a wave share one walk.
 // The sort and the longest of those walks (each as long as 64 shapes') cost
-// about 0.4 to 1 ms whatever the number, a wave per shape 2.4 to 3.6 ns a
-// shape counted and 4 to 7 ns listed.  1 m spheres at points of 1.15M and 20M
-// points, wave and lane per shape, ms: counted, 65k 0.17 and 0.42, 0.22 and
-// 1.09; 262k 0.64 and 0.69, 0.84 and 1.06; 1M 2.4 and 1.1, 3.2 and 1.5.
-// Counted and listed: 65k 0.46 and 0.91, 0.59 and 2.3; 262k 1.7 and 1.3, 2.3
-// and 2.0.  Small batches gain most: 4096 cylinders of 0.877 m 0.035 and 1.5.
-#define WB_QUERY_SORT_MIN 393216
+// 0.25 to 1.2 ms whatever the number, a wave per shape 2.4 to 3.6 ns a shape
+// counted and 4 to 7 ns listed.  1 m spheres and cylinders at points of 1.15M
+// and 20M points, wave and lane per shape, ms: counted, 262k 0.64 and 0.48,
+// 0.76 and 0.87, 0.85 and 0.84, 0.96 and 1.18; 524k 1.25 and 0.70, 1.49 and
+// 1.29, 1.69 and 1.11, 1.90 and 1.70.  Counted and listed, 131k 0.88 and 0.90,
+// 1.11 and 1.57, 1.16 and 1.87, 1.46 and 2.60; 262k 1.72 and 1.08, 2.16 and
+// 1.90, 2.29 and 1.79, 2.85 and 2.67.  Small batches gain most: 4096 cylinders
+// of 0.877 m 0.035 and 1.5.
+#define WB_QUERY_SORT_MIN 327680
 #define WB_QUERY_SORT_MIN_LIST 196608
 
 // Events around a query's kernels on the context stream; ms() after the

@@ -3346,8 +3346,8 @@ __device__ __forceinline__ bool open_unit(const ClassifyArgs &A, uint32_t u, con
 // classes block u takes unit u of their order, else wave u's.  (A resident
 // grid that takes the units by a counter was 3 to 7% slower on 40k to 300k
 // points: every claim waits for the counter's word.)
-template <bool IN>
-__global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open(ClassifyArgs A)
+template <bool IN, int MINW>
+__global__ void __launch_bounds__(WAVE, MINW) k_ground_open(ClassifyArgs A)
 {
   __shared__ float edges[3 * 128];
   __shared__ double2 edge[WAVE];
@@ -4228,8 +4228,16 @@ static void launch_ground(wb_ctx *c, const ClassifyArgs &A, uint64_t n, uint32_t
       else hipLaunchKernelGGL(k_ground_open_resident<false>, ogrid, one, 0, st, A);
     } else {
       const dim3 ogrid(nb * (A.walk_per / A.open_per));
-      if (A.cube_wedges) hipLaunchKernelGGL(k_ground_open<true>, ogrid, one, 0, st, A);
-      else hipLaunchKernelGGL(k_ground_open<false>, ogrid, one, 0, st, A);
+      // with many units six waves per SIMD hide more than the registers they
+      // give up cost (23.7M points, mostly ground: about 1 ms of 29 less than
+      // with five); with few the longest unit is the kernel (1.17M: 1.95 ms
+      // with five, 2.09 with six)
+      if (A.cube_wedges && A.open_classes)
+        hipLaunchKernelGGL((k_ground_open<true, WB_OPEN_MINW>), ogrid, one, 0, st, A);
+      else if (A.cube_wedges)
+        hipLaunchKernelGGL((k_ground_open<true, 6>), ogrid, one, 0, st, A);
+      else
+        hipLaunchKernelGGL((k_ground_open<false, WB_OPEN_MINW>), ogrid, one, 0, st, A);
     }
   }
   if (ev) {
