@@ -508,10 +508,12 @@ def test_membership_candidates_cover_every_tile_within_reach():
                     assert (a, b) in seven, (x, y, a, b)
 
 
-def test_lane_wedges_keep_every_care_direction(hm):
+@pytest.mark.parametrize("grow", [0, 1])
+def test_lane_wedges_keep_every_care_direction(hm, grow):
     # a lane's two-wedge forms: a box, or a direction, they refuse holds no
-    # direction in an empty run of 24 bins or more
-    hm.wbh_lane_wedges.argtypes = [C.c_uint64] + [C.c_double] * 6
+    # direction in an empty run of 24 bins or more, nor, grown, in the bins
+    # beside it
+    hm.wbh_lane_wedges.argtypes = [C.c_uint64, C.c_int] + [C.c_double] * 6
     hm.wbh_dir_bin.argtypes = [C.c_double, C.c_double]
     rng = np.random.default_rng(31)
     refused = [0, 0]
@@ -522,13 +524,15 @@ def test_lane_wedges_keep_every_care_direction(hm):
         for _ in range(nb):
             occ |= 1 << ((base + int(rng.integers(0, 40))) % 64)
         care = care_bins(occ)
+        if grow:
+            care = care | {(b + 1) % 64 for b in care} | {(b - 1) % 64 for b in care}
         w, h = rng.uniform(0, 3, 2) if it % 3 else (0.0, 0.0)
         x0, y0 = rng.normal(size=2) * 3
         if it % 2:  # a corner within 0.01 rad of a bin's edge
             th = -math.pi + int(rng.integers(0, 64)) * math.pi / 32 + rng.uniform(-0.01, 0.01)
             d = rng.uniform(0.1, 20)
             x0, y0 = d * math.cos(th), d * math.sin(th)
-        got = hm.wbh_lane_wedges(occ, 0.0, 0.0, x0, x0 + w, y0, y0 + h)
+        got = hm.wbh_lane_wedges(occ, grow, 0.0, 0.0, x0, x0 + w, y0, y0 + h)
         first = hm.wbh_dir_bin(y0, x0)
         if not got & 2:
             refused[1] += 1
@@ -595,21 +599,3 @@ def test_octet_bounds_round_outwards(hm):
         assert hm.wbh_rel_down(v, o, side) <= d - slack
         assert hm.wbh_rel_up(v, o, side) >= d + slack
     assert hm.wbh_rel_down(1e300, 0.0, 1.0) <= 3.1e38 and hm.wbh_rel_up(-1e300, 0.0, 1.0) >= -3.1e38
-
-
-def test_borders_open_clears_the_bins_beside_care_runs(hm):
-    hm.wbh_borders_open.restype = C.c_uint64
-    hm.wbh_borders_open.argtypes = [C.c_uint64]
-    rng = np.random.default_rng(35)
-    runs = 0
-    for it in range(20000):
-        occ, base = 0, int(rng.integers(0, 64))
-        for _ in range(int(rng.integers(1, 12))):
-            occ |= 1 << ((base + int(rng.integers(0, 41))) % 64)
-        care = care_bins(occ)
-        want = occ
-        for b in care:
-            want &= ~((1 << ((b + 1) % 64)) | (1 << ((b - 1) % 64)))
-        runs += len(care) > 0
-        assert hm.wbh_borders_open(occ) == want, hex(occ)
-    assert runs > 5000

@@ -2838,7 +2838,7 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
       if (state == 0 && occ != checked) {
         checked = occ;
         if (gap_verdict(occ) == 1) state = 1;
-        else wb::lane_wedges_update(wb::borders_open(occ), edges, W);
+        else wb::lane_wedges_update(occ, edges, W, 1);
       }
       alive = __ballot(state == 0);
       if (alive == 0) break;

@@ -66,7 +66,8 @@ int wbh_wedge_hit(uint64_t occ, double px, double py, double x0, double x1, doub
 
 // a lane's wedges (at most two) of a direction mask: bit 0 the box test, bit 1
 // the test of the direction of the box's first corner
-int wbh_lane_wedges(uint64_t occ, double px, double py, double x0, double x1, double y0, double y1)
+int wbh_lane_wedges(uint64_t occ, int grow, double px, double py, double x0, double x1, double y0,
+                    double y1)
 {
   static float tab[3 * 128];
   static int filled;
@@ -75,12 +76,10 @@ int wbh_lane_wedges(uint64_t occ, double px, double py, double x0, double x1, do
     filled = 1;
   }
   wb::LaneWedges w;
-  wb::lane_wedges_update(occ, tab, w);
+  wb::lane_wedges_update(occ, tab, w, grow);
   return (wb::lane_hit(w, px, py, x0, x1, y0, y1) ? 1 : 0) |
          (wb::lane_dir(w, (float)(x0 - px), (float)(y0 - py)) ? 2 : 0);
 }
-
-uint64_t wbh_borders_open(uint64_t occ) { return wb::borders_open(occ); }
 
 // bit 0: hyp_in; bit 1: hyp_near reaches its threshold
 int wbh_hyp_near(const double *p, const double *q)
