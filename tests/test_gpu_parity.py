@@ -641,3 +641,56 @@ def test_gap_borders_far_from_the_point_match_oracle(ctx, seed):
           "of the high ones ground", int((want[high] == 2).sum()))
     assert st["exact_gap_points"] > 0 and (want[high] > 0).all()
     assert np.array_equal(got, want)
+
+
+def test_neighbour_at_the_corner_of_a_wide_group_matches_oracle(ctx):
+    # sparse leaves of 512 m.  At each inner corner of four of them a point
+    # high up sits two units from a neighbour that is the topmost and leftmost
+    # point of its leaf, so also of its 32-point group, whose box of up to
+    # 512 m spreads to the lower right; the neighbour's direction is the first
+    # edge of an empty run of 24 bins (45 to 180 degrees) that it makes one of
+    # 23.  Without it the gap is above 144 degrees.  (The points that bound the
+    # run are the lowest of their groups, so the first walk finds them.)
+    unit, cell, half = 2.0 ** -10, 512.0, 4
+    ext = 2 * half * cell
+    lo, hi = np.array([1.0, 1.0, 1.0]), np.array([ext - 1, ext - 1, cell - 1])
+    center, side = W.Octree.size_fit(lo, hi)
+    org = np.asarray(center) - side / 2
+    zc = org[2] + cell * np.ceil(-org[2] / cell)  # one layer of cells holds every point
+    rng = np.random.default_rng(41)
+    px, py, pz = [], [], []
+    th = np.radians(180 + 5.625 * (np.arange(40) + 0.5))  # the bins 0 to 39
+    th[0], th[39] = np.radians(184.9), np.radians(360 + 39.5)
+    corners = [org[0] + cell * np.arange(round((0 - org[0]) / cell) + 1, round((ext - org[0]) / cell)),
+               org[1] + cell * np.arange(round((0 - org[1]) / cell) + 1, round((ext - org[1]) / cell))]
+    eyes = []
+    n = 0
+    for cx in corners[0]:
+        for cy in corners[1]:
+            r = rng.uniform(10.0, 20.0, 40)
+            eyes.append(n)
+            px += [cx - unit, cx, *(cx - unit + r * np.cos(th))]
+            py += [cy - 2 * unit, cy - unit, *(cy - 2 * unit + r * np.sin(th))]
+            pz += [zc + 31.0, zc + 6.0, zc + 2.0, *(zc + rng.uniform(2.5, 4.0, 38)), zc + 2.0]
+            n = len(px)
+    for x0 in [org[0] + cell * k for k in range(round((ext - org[0]) / cell))]:
+        for y0 in [org[1] + cell * k for k in range(round((ext - org[1]) / cell))]:
+            px += list(x0 + rng.uniform(0.01, 0.99, 300) * cell)
+            py += list(y0 + rng.uniform(0.01, 0.99, 300) * cell)
+            pz += list(zc + rng.uniform(70, 110, 300))
+    xi, yi, zi = (np.round(np.array(v) / unit).astype(np.int32) for v in (px, py, pz))
+    keep = (xi * unit >= lo[0]) & (xi * unit <= hi[0]) & (yi * unit >= lo[1]) & (yi * unit <= hi[1])
+    eyes = (np.cumsum(keep) - 1)[np.array(eyes)]
+    xi, yi, zi = xi[keep], yi[keep], zi[keep]
+    cloud = dict(xi=xi, yi=yi, zi=zi, scale=np.full(3, unit), offset=np.zeros(3), bbmin=lo, bbmax=hi)
+    op, prm = O.default_params(), W.default_params(tile_size=4.0)
+    op.tile_size = 4.0
+    tree, _, _ = build_both(ctx, cloud)
+    assert (tree.leaves()["side"] == cell).all()
+    got, _, _ = W.classify(tree, lo, hi, prm, want_tiles=False)
+    want, _, _ = O.run(cloud, op)
+    tree.free()
+    print("eyes", len(eyes), "not ground", int((want[eyes] == 1).sum()), "differ",
+          int((got != want).sum()))
+    assert (want[eyes] == 1).all()
+    assert np.array_equal(got, want)

@@ -545,6 +545,51 @@ def test_lane_wedges_keep_every_care_direction(hm, grow):
     assert min(refused) > 500
 
 
+@pytest.mark.parametrize("grow", [0, 1])
+def test_lane_wedges_keep_near_corners_of_large_boxes(hm, grow):
+    # boxes from as large as the point's distance to a million times that, at
+    # map coordinates on a millimetre grid and at finer FP64 ones, a corner on
+    # or near an edge of a run of 24 to 40 empty bins (due north, on a
+    # diagonal, or anywhere): refused only if no corner, nor the point of the
+    # box nearest to the eye, is a care direction
+    hm.wbh_lane_wedges.argtypes = [C.c_uint64, C.c_int] + [C.c_double] * 6
+    hm.wbh_dir_bin.argtypes = [C.c_double, C.c_double]
+    rng = np.random.default_rng(35)
+    refused, kept = 0, 0
+    for it in range(60000):
+        px, py = (5e5, 4.4e6) if it % 2 else (0.0, 0.0)
+        unit = 0.001 if it % 2 else 10.0 ** rng.uniform(-6, -2)
+        if it % 5 < 3:  # on an axis or a diagonal, both of which are bin edges
+            dx, dy = unit * rng.integers(1, 4) * rng.permutation(
+                [(1, 0), (-1, 0), (0, 1), (0, -1), (1, 1), (1, -1), (-1, 1), (-1, -1)])[0]
+        else:
+            dx, dy = unit * rng.integers(-3, 4, 2)
+        cx, cy = px + dx, py + dy
+        if cx == px and cy == py:
+            continue
+        b = hm.wbh_dir_bin(cy - py, cx - px)
+        length = int(rng.integers(24, 41))
+        # in the (grown) run's first or last bin, or beside it
+        first = (b + grow, b - length + 1 - grow, b + 1 + grow, b - length - grow)[it % 4]
+        occ = (1 << 64) - 1
+        for k in range(length):
+            occ &= ~(1 << ((first + k) % 64))
+        care = care_bins(occ)
+        if grow:
+            care = care | {(k + 1) % 64 for k in care} | {(k - 1) % 64 for k in care}
+        w, h = unit * 10.0 ** rng.uniform(0, 6, 2) * rng.choice([-1.0, 1.0], 2)
+        x0, x1, y0, y1 = min(cx, cx + w), max(cx, cx + w), min(cy, cy + h), max(cy, cy + h)
+        if hm.wbh_lane_wedges(occ, grow, px, py, x0, x1, y0, y1) & 1:
+            kept += 1
+            continue
+        refused += 1
+        near = min(max(px, x0), x1), min(max(py, y0), y1)
+        for x, y in ((cx, cy), (x0, y0), (x0, y1), (x1, y0), (x1, y1), near):
+            assert (x, y) != (px, py)
+            assert hm.wbh_dir_bin(y - py, x - px) not in care, (occ, px, py, x0, x1, y0, y1, x, y)
+    assert refused > 1000 and kept > 20000, (refused, kept)
+
+
 def test_hyp_near_covers_hyp_in(hm):
     # every point hyp_in takes reaches hyp_near's threshold: random points, and
     # points within a few roundings of the surface at map coordinates

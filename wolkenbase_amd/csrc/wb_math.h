@@ -914,21 +914,32 @@ WB_HD bool wedge_hit(const Wedges &w, double px, double py, double x0, double x1
 
 // wedge_hit for at most two wedges (n of them, n <= 2; n < 0 is no pruning)
 // on a box given by its corners' offsets from the point, u0 <= u1 in x and
-// v0 <= v1 in y, already rounded to float: the same test per wedge.
+// v0 <= v1 in y, already rounded to float: false, as wedge_hit's, only if the
+// box lies outside every wedge.
 WB_HD bool wedge_hit2(int n, const float ax[2], const float ay[2], const float bx[2],
                       const float by[2], float u0, float u1, float v0, float v1)
 {
   if (n < 0) return true;
   bool hit = false;
-  // the largest value of each cross product over the box: at its middle, plus
-  // the half widths times the edge's components (rounding within 10^-6 of
-  // the offsets, against the wedges' 10^-3 rad)
+  // The largest value of each cross product over the box: at its middle, plus
+  // the half widths times the edge's components.  A corner close to the point
+  // comes out of that by cancellation, with an error that goes with the box
+  // and not with the corner's distance: the conversions to float and the sums
+  // uc, uh, vc and vh leave at most 3 * 2^-24 of S = |uc| + uh + |vc| + vh in a
+  // product, its four roundings at most 4 * 2^-24.  eps, 2^-20 of S, is part of
+  // every product and covers both twice over, so a box with a direction of a
+  // care bin (10^-3 rad inside a widened edge) is kept.  (At the corner the
+  // edge's signs pick, as wedge_hit takes it, a product needs no eps but two
+  // selects.)
   const float uc = 0.5f * (u0 + u1), vc = 0.5f * (v0 + v1), uh = 0.5f * (u1 - u0),
               vh = 0.5f * (v1 - v0);
+  const float eps = 0x1p-20f * ((fabsf(uc) + uh) + (fabsf(vc) + vh));
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const float ra = fmaf(ax[k], vc, fmaf(-ay[k], uc, fmaf(fabsf(ax[k]), vh, fabsf(ay[k]) * uh)));
-    const float lb = fmaf(uc, by[k], fmaf(-vc, bx[k], fmaf(fabsf(by[k]), uh, fabsf(bx[k]) * vh)));
+    const float ra =
+        fmaf(ax[k], vc, fmaf(-ay[k], uc, fmaf(fabsf(ax[k]), vh, fmaf(fabsf(ay[k]), uh, eps))));
+    const float lb =
+        fmaf(uc, by[k], fmaf(-vc, bx[k], fmaf(fabsf(by[k]), uh, fmaf(fabsf(bx[k]), vh, eps))));
     const bool in_k = !(ra < 0) & !(lb < 0);
     hit |= k < n ? in_k : false;
   }
