@@ -694,3 +694,55 @@ def test_neighbour_at_the_corner_of_a_wide_group_matches_oracle(ctx):
           int((got != want).sum()))
     assert (want[eyes] == 1).all()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("kind", [W.WB_SHAPE_CYLINDER, W.WB_SHAPE_SPHERE, W.WB_SHAPE_HYPERBOLOID])
+def test_queries_either_side_of_the_sort_line_match_oracle(ctx, kind):
+    """Batches of one shape less than a lane per shape is taken from, and of
+    just as many (the batches of test_batched_queries_large_batch take a wave
+    per shape).  Few of many small shapes are far outside the cloud, of radius
+    zero, hold every point or hold whole leaves and cut others; every distinct
+    shape's count and list are the oracle's, each copy's are the same."""
+    cloud = synth.generate(seed=31, extent=80.0, density=25.0, outliers=0.01)
+    tree, ref, (x, y, z) = build_both(ctx, cloud)
+    rng = np.random.default_rng(300 + kind)
+    at = 2 if kind == W.WB_SHAPE_CYLINDER else 3
+    small = random_shapes(rng, x, y, z, kind, 4000)
+    if kind == W.WB_SHAPE_HYPERBOLOID:  # lowered, so that few points are under them
+        small[:, 2] -= np.sign(small[:, 4]) * rng.uniform(0.0, 15.0, len(small))
+    else:
+        small[:, at] = rng.uniform(0.05, 0.5, len(small))
+    small = small[tree.count_points_in((kind, small)) < 40][:300]
+    far, zero, wide = small[:3].copy(), small[3:6].copy(), random_shapes(rng, x, y, z, kind, 30)
+    far[:, 0] += 1e4
+    zero[:, at] = 0.0
+    if kind == W.WB_SHAPE_HYPERBOLOID:
+        big = np.array([[x.mean(), y.mean(), z.max() + 1e4, 1.0, 1.0]])
+    elif kind == W.WB_SHAPE_SPHERE:
+        wide[:, at] = np.linspace(5.0, 40.0, 30)
+        big = np.array([[x.mean(), y.mean(), z.mean(), 1e5, 0.0]])
+    else:
+        wide[:, at] = np.linspace(5.0, 40.0, 30)
+        big = np.array([[x.mean(), y.mean(), 1e5, 0.0, 0.0]])
+    P = np.concatenate([far, zero, wide, big, small])
+    ns = len(P) - len(small)
+    want = [ref.points_in(kind, p) for p in P]
+    count = np.array([len(w) for w in want], dtype=np.uint64)
+    assert count[ns - 1] == len(x) and (count[:3] == 0).all() and len(small) == 300
+    half = tree.info()["nleaves"] // 2
+    lines = {W.WB_SHAPE_SPHERE: (163840 + half, 131072 + half),
+             W.WB_SHAPE_CYLINDER: (327680, 172032 + half),
+             W.WB_SHAPE_HYPERBOLOID: (327680, 196608)}[kind]
+    for line in lines:
+        for n in (line - 1, line):
+            # the special shapes once each among the small ones, in random order
+            pick = np.concatenate([np.arange(ns), ns + np.arange(n - ns) % len(small)])
+            rng.shuffle(pick)
+            got = tree.count_points_in((kind, P[pick]))
+            assert np.array_equal(got, count[pick]), n
+            if line != lines[1]:
+                continue
+            lists = tree.points_in((kind, P[pick]))
+            for k, s in enumerate(pick):
+                assert np.array_equal(lists[k], want[s]), (n, s)
+    tree.free()

@@ -474,18 +474,36 @@ int wb_tree_order(wb_tree *t, uint32_t *order)
 static int check_kind(int kind) { return kind == WB_SHAPE_CYLINDER || kind == WB_SHAPE_SPHERE || kind == WB_SHAPE_HYPERBOLOID; }
 
 // Batches of fewer shapes take a wave per shape in the caller's order; the
-// others a lane per shape, sorted so that the 64 of a wave share one walk.
-// The sort and the longest of those walks (each as long as 64 shapes') cost
-// 0.25 to 1.2 ms whatever the number, a wave per shape 2.4 to 3.6 ns a shape
-// counted and 4 to 7 ns listed.  1 m spheres and cylinders at points of 1.15M
-// and 20M points, wave and lane per shape, ms: counted, 262k 0.64 and 0.48,
-// 0.76 and 0.87, 0.85 and 0.84, 0.96 and 1.18; 524k 1.25 and 0.70, 1.49 and
-// 1.29, 1.69 and 1.11, 1.90 and 1.70.  Counted and listed, 131k 0.88 and 0.90,
-// 1.11 and 1.57, 1.16 and 1.87, 1.46 and 2.60; 262k 1.72 and 1.08, 2.16 and
-// 1.90, 2.29 and 1.79, 2.85 and 2.67.  Small batches gain most: 4096 cylinders
-// of 0.877 m 0.035 and 1.5.
-#define WB_QUERY_SORT_MIN 327680
-#define WB_QUERY_SORT_MIN_LIST 196608
+// others a lane per shape, sorted so that the 64 of a wave share one walk.  A
+// wave per shape costs 1.6 to 3.2 ns a shape counted and 4 to 8 listed, a little
+// more in a large cloud; a lane per shape a sort (0.1 to 0.2 ms) and walks that
+// take as long as the longest wave's, more in a cloud of many leaves, over which
+// the same shapes lie apart.  So the lines of spheres and cylinders rise with
+// the leaves, and they are where the small shapes (0.3 m, 2 to 10 points each)
+// meet: shapes of 1 m meet at 1.1 to 1.5 times as many, of 3 m at twice.
+// Kernels, wave and lane per shape, ms, in clouds of 0.1M points, 1.15M, 6M at
+// 5 per m2, and 24M, either side of the lines:
+//   spheres of 0.3 m counted, 131k 0.21 0.19, 0.27 0.27, 0.32 0.34, 0.36 0.61;
+//   180k 0.29 0.22, 0.37 0.28, 0.43 0.32, 0.49 0.60; 262k 0.42 0.24, 0.54 0.29,
+//   0.62 0.30, 0.71 0.56; of 1 m, 164k 0.32 0.34, 0.41 0.41, 0.42 0.44, 0.54 0.91
+//   spheres of 0.3 m listed, 115k 0.47 0.46, 0.60 0.54, 0.64 0.67, 0.79 1.39;
+//   164k 0.64 0.47, 0.83 0.61, 0.89 0.62, 1.10 1.31; of 1 m, 131k 0.68 0.78,
+//   0.90 0.87, 0.81 0.92, 1.17 2.09
+//   cylinders of 0.3 m listed, 131k 0.66 0.95, 0.82 1.02, 0.82 0.89, 1.12 1.95;
+//   262k 1.30 1.30, 1.57 1.31, 1.59 0.99, 2.16 1.86
+//   cylinders of 0.3 m counted, 295k 0.55 0.63, 0.66 0.64, 0.70 0.48, 0.87 0.94;
+//   524k 0.97 0.87, 1.16 0.84, 1.24 0.66, 1.54 1.15; of 1 m, 327k 0.78 1.02,
+//   0.94 0.94, 0.85 0.63, 1.20 1.35
+// Hyperboloids with nothing below them meet at 524k listed (0.93 0.76, 1.16 0.96,
+// 1.86 2.81, 1.73 4.66); above a thousand points each a wave per shape is the
+// faster one at any number measured (24M, 524k counted 10.0 and 27.8).
+static uint64_t query_sort_min(const wb_tree *t, int kind, bool list)
+{
+  const uint64_t leaves = t->nleaves;
+  if (kind == WB_SHAPE_SPHERE) return (list ? 131072 : 163840) + leaves / 2;
+  if (kind == WB_SHAPE_CYLINDER && list) return 172032 + leaves / 2;
+  return list ? 196608 : 327680;
+}
 
 // Events around a query's kernels on the context stream; ms() after the
 // stream has passed the second one.
@@ -535,7 +553,7 @@ int wb_count_points_in(wb_tree *t, int kind, const double *params, uint64_t ns, 
   WB_CHECK(hipMemcpyAsync(dp, params, pb, hipMemcpyHostToDevice, c->stream));
   QueryTimer qt(c);
   qt.start();
-  uint32_t *order = ns >= WB_QUERY_SORT_MIN ? wb_query_order(t, kind, dp, ns) : nullptr;
+  uint32_t *order = ns >= query_sort_min(t, kind, false) ? wb_query_order(t, kind, dp, ns) : nullptr;
   wb_run_count(t, kind, dp, ns, dc, order);
   qt.stop();
   WB_CHECK(hipMemcpyAsync(counts, dc, 8 * ns, hipMemcpyDeviceToHost, c->stream));
@@ -593,7 +611,8 @@ int wb_points_in(wb_tree *t, int kind, const double *params, uint64_t ns, uint64
   WB_CHECK(hipMemcpyAsync(dp, params, pb, hipMemcpyHostToDevice, c->stream));
   QueryTimer qt(c);
   qt.start();
-  uint32_t *order = ns >= (idx ? WB_QUERY_SORT_MIN_LIST : WB_QUERY_SORT_MIN) ? wb_query_order(t, kind, dp, ns) : nullptr;
+  uint32_t *order =
+      ns >= query_sort_min(t, kind, idx != nullptr) ? wb_query_order(t, kind, dp, ns) : nullptr;
   wb_run_count(t, kind, dp, ns, dc, order);
   qt.stop();
   std::vector<uint64_t> cnt(ns);
