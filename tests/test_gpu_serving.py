@@ -75,6 +75,29 @@ def test_admission_waits_for_memory():
     ctx.close()
 
 
+@pytest.mark.parametrize("extent,density,trees", [(1000.0, 0.3, 1), (330.0, 9.0, 1), (100.0, 15.0, 1),
+                                                  (15.0, 25.0, 1), (100.0, 15.0, 4)])
+def test_memory_stays_within_the_estimate(extent, density, trees):
+    # what a context holds after its first request (its pool keeps every
+    # buffer) is no more than the request was admitted with
+    tiles = [synth.generate(seed=700 + k, extent=extent, density=density) for k in range(trees)]
+    need = sum(serve.Request(t).need for t in tiles)
+    ctx = W.Context(0)
+    try:
+        ctx.sync()
+        free = W.device_memory(0)[0]
+        if trees == 1:
+            serve.classify_tile(ctx, tiles[0], W.default_params())
+        else:
+            serve.classify_tiles(ctx, tiles, W.default_params())
+        ctx.sync()
+        used = free - W.device_memory(0)[0]
+    finally:
+        ctx.close()
+    print("points", sum(len(t["xi"]) for t in tiles), "used", used >> 20, "MiB of", need >> 20)
+    assert used <= need
+
+
 def test_pinned_buffers():
     a = W.pinned_empty(1000, np.int32)
     assert a.dtype == np.int32 and a.shape == (1000,) and a.flags.writeable

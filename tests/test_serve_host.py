@@ -237,3 +237,15 @@ def test_stream_strata_follow_the_lognormal():
     specs = serve.stream_specs(10000, seed=1, max_points=1e7)
     n = np.array([s["extent"] ** 2 * s["density"] for s in specs])
     assert n.min() == pytest.approx(5e4, rel=1e-9) and n.max() == pytest.approx(1e7, rel=1e-9)
+
+
+def test_memory_estimate_counts_tiles():
+    # 27.8M tile numbers over 1 km x 1 km, whatever the points; a box that is
+    # missing or no box adds none (the request fails by itself)
+    box = dict(bbmin=[0.0, 0.0, 0.0], bbmax=[1000.0, 1000.0, 30.0])
+    base = serve.BYTES_PER_POINT * 10 + serve.BYTES_FIXED
+    assert serve.Request(dict(_tile(10), **box)).need == base + serve.BYTES_PER_TILE * 27845425
+    few = serve.Request(dict(_tile(10), **box), tile_size=10.0).need
+    assert base < few < base + serve.BYTES_PER_TILE * 10 ** 6
+    for bad in (dict(), dict(bbmin=None, bbmax=None), dict(box, bbmax=["a", 0, 0])):
+        assert serve.Request(dict(_tile(10), **bad)).need == base

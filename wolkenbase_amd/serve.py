@@ -42,9 +42,16 @@ import numpy as np
 import wolkenbase_amd as W
 from wolkenbase_amd import synth
 
-# device bytes per point at the peak of build + classify: sort buffers,
-# coordinates, per-point tile membership, classify scratch (an upper estimate)
+# device bytes at the peak of build + classify (upper estimates): per point
+# sort buffers, coordinates, tile membership and the ground test's scratch,
+# per tile number the records, counts and address grid (a tile number holds no
+# point where the cloud is sparse or its box wide: 1 km x 1 km has 27.8M), and
+# what does not go with either.  A context that classified one tile of 0.3M to
+# 20M points at 25 per m2 holds 150 to 231 per point, of 5M points on
+# 1 km x 1 km 4.0 GB, about 110 per tile number.
 BYTES_PER_POINT = 240
+BYTES_PER_TILE = 140
+BYTES_FIXED = 64 << 20
 # service-time model for the response ratio: a fixed cost per tile (launches,
 # host waits, the slowest wave of the ground kernel) plus a cost per point
 SERVICE_FIXED_S = 2.0e-3
@@ -55,12 +62,26 @@ def service_estimate(n):
     return SERVICE_FIXED_S + SERVICE_PER_POINT_S * n
 
 
+def memory_estimate(tile, tile_size=1.0):
+    """Device bytes that building and classifying a tile takes at most."""
+    ntiles = 0
+    try:
+        box = np.array([tile["bbmin"], tile["bbmax"]], dtype=np.float64)
+        if box.shape == (2, 3) and np.isfinite(box).all():
+            ntiles = W.tile_count(box[0], box[1], tile_size)
+    except (KeyError, TypeError, ValueError, W.WbError):
+        pass  # the pass fails on such a box, with the reason
+    return BYTES_PER_POINT * len(tile["xi"]) + BYTES_PER_TILE * ntiles + BYTES_FIXED
+
+
 class Request:
-    def __init__(self, tile, tag=None):
+    """tile_size: the server's parameters' (the number of tiles goes with it)."""
+
+    def __init__(self, tile, tag=None, tile_size=1.0):
         self.tile = tile
         self.tag = tag
         self.n = len(tile["xi"])
-        self.need = BYTES_PER_POINT * self.n + (64 << 20)
+        self.need = memory_estimate(tile, tile_size)
         self.est = service_estimate(self.n)
         self.done = threading.Event()
         self.t_arrive = self.t_start = self.t_end = None
@@ -380,7 +401,7 @@ def load_test(pool, slots, load, nreq, seed, device=0, policy="ratio", small_slo
     try:
         # capacity: every pool tile submitted at once
         t0 = time.perf_counter()
-        reqs = [srv.submit(Request(t, k)) for k, t in enumerate(pool)]
+        reqs = [srv.submit(Request(t, k, params.tile_size)) for k, t in enumerate(pool)]
         for r in reqs:
             r.done.wait()
         capacity = npts.sum() / (time.perf_counter() - t0)
@@ -398,7 +419,7 @@ def load_test(pool, slots, load, nreq, seed, device=0, policy="ratio", small_slo
                 if d <= 0:
                     break
                 time.sleep(min(d, 0.002))
-            reqs.append(srv.submit(Request(pool[k], int(k))))
+            reqs.append(srv.submit(Request(pool[k], int(k), params.tile_size)))
         for r in reqs:
             r.done.wait()
     finally:
