@@ -121,3 +121,47 @@ def test_batch_of_large_trees_equals_single(ctx, members):
         assert np.array_equal(g, cls)
         assert st["exact_gap_points"] == one["exact_gap_points"]
         t.free()
+
+
+@pytest.mark.parametrize("slope", [0.3, 0.05])
+@pytest.mark.parametrize("n,outside", [(18_500, False), (60_000, True), (60_000, False), (240_000, False),
+                                       (400_000, True), (1_300_000, False), (7_600_000, False)])
+def test_shallow_slopes_match_oracle(ctx, n, outside, slope):
+    # hyperboloids that reach most of the cloud: lists and units that are cut
+    # short at every size, their points left to the wave-per-point kernel
+    if n < 100_000:
+        cloud = synth.generate(seed=62, extent=math.sqrt(n / 28.0), density=25.0, outliers=0.02,
+                               outlier_low=0.2, buildings=4, trees=33)
+        if outside:
+            hi = np.array(cloud["bbmax"], float)
+            hi[2] = np.percentile(cloud["offset"][2] + cloud["scale"][2] * cloud["zi"], 60)
+            cloud = dict(cloud, bbmin=np.array(cloud["bbmin"], float) + [0, 0, 40.0], bbmax=hi + [0, 0, 40.0])
+    else:
+        cloud = make(n, outside)
+    center, side = W.Octree.size_fit(cloud["bbmin"], cloud["bbmax"])
+    xyz = [cloud["offset"][a] + cloud["scale"][a] * cloud[k].astype(np.float64)
+           for a, k in enumerate(("xi", "yi", "zi"))]
+    out = np.zeros(len(xyz[0]), dtype=bool)
+    for v, c in zip(xyz, center):
+        out |= (v < c - side / 2) | (v > c + side / 2)
+    assert out.any() == outside
+    prm, op = W.default_params(max_slope=slope), O.default_params()
+    op.max_slope = slope
+    tree = W.Octree.build(ctx, cloud["xi"], cloud["yi"], cloud["zi"], cloud["scale"],
+                          cloud["offset"], center, side)
+    tiles, _ = W.scan_tiles(tree, cloud["bbmin"], cloud["bbmax"], prm)
+    cls, _, st = W.classify(tree, cloud["bbmin"], cloud["bbmax"], prm, want_tiles=False)
+    tree.free()
+    # points low above their surroundings: what lies under them is not the whole cloud
+    rng = np.random.default_rng(n)
+    m = 400
+    low = np.flatnonzero(~out & (xyz[2] < np.percentile(xyz[2], 50)))
+    pick = np.concatenate([rng.choice(np.flatnonzero(~out), m // 4, replace=False),
+                           rng.choice(low, m, replace=False)])
+    hs, sure = deciding_hs(cloud, tiles, xyz[0][pick], xyz[1][pick])
+    pick, hs = pick[sure], hs[sure]
+    want = O.Tree(*xyz, center, side).classify_points(pick, hs, op)
+    want[hs == 0] = 0
+    print("n", len(cls), "gap points", st["exact_gap_points"], "heavy", st["heavy_points"],
+          "sample", np.bincount(want, minlength=3), "differ", int((want != cls[pick]).sum()))
+    assert np.array_equal(cls[pick], want)

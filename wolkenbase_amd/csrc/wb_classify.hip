@@ -2395,6 +2395,8 @@ struct ClassifyArgs {
   uint64_t pool_shared, pool_cap;
   uint32_t unit_cap, open_per;
   uint32_t walk_per;  // points of a wave of walk A (at least open_per)
+  uint32_t leaf_cap;  // leaves a wave of walk A lists at most
+  int open_budget;  // groups and rounds of candidates a unit of walk B takes at most
   int open_classes;
   uint32_t *nopen, *open_next;
   unsigned long long *npool;
@@ -2518,8 +2520,9 @@ __device__ inline void half_or(uint64_t v, uint64_t &h0, uint64_t &h1)
 // is popped, and its children are taken before its siblings), so the lanes
 // that reach them are kept per level.
 #define WB_STK (7 * (WB_MAX_LEVEL + 1) + 8 + 2)
-// leaves walk A takes before it hands its open lanes to k_ground_heavy,
-// or, of all entries it takes from its stack
+// leaves walk A takes at most before it hands its open lanes to
+// k_ground_heavy (ClassifyArgs::leaf_cap is the number), or, of all entries it
+// takes from its stack
 #define GROUND_LEAVES 256
 #define GROUND_STEPS 1024
 struct WaveStack {
@@ -2794,7 +2797,7 @@ __device__ __forceinline__ void walk_body(const ClassifyArgs &A, uint64_t unit, 
         sp = push_children<IN>(T, S, sp, code, lvl, cx, cy, cz, side, m, U, s2, rx, ry);
         continue;
       }
-      if (nleaf == GROUND_LEAVES) {
+      if (nleaf == A.leaf_cap) {
         if (state == 0) state = 5;
         break;
       }
@@ -2944,6 +2947,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
   const double slack = sure_slack(A);
   const int want = GAP ? 4 : 0;
   bool pend = false;
+  uint32_t work = 0;  // groups, and rounds of candidates
   uint64_t checked = O.occ;
   uint64_t alive = __ballot(O.state == want);
   if (alive == 0) return;
@@ -3146,6 +3150,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
               }
             }
           }
+          work += taken + 1;
           // many candidates: the directions just found may leave out the next
           // group's
           if (!GAP && taken >= OPEN_REFRESH && O.occ != checked && O.state == 0) {
@@ -3175,6 +3180,9 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
           else wb::lane_wedges_update(O.occ, edges, O.W);
         }
       }
+      // a long unit's open lanes go to the heavy kernel, a wave to the point
+      if (__builtin_expect(rfl((int)work) > A.open_budget, 0))
+        O.state = O.state == want ? (GAP ? 7 : 6) : O.state;
       alive = __ballot(O.state == want);
       if (alive == 0) break;
       const int na = __popcll(alive);
@@ -4009,6 +4017,30 @@ static void open_buffers(wb_ctx *c, ClassifyArgs &A, uint64_t n, uint64_t nbatch
   const uint64_t all = (nbatch ? nbatch : n) / WAVE;
   A.walk_per = 2 * all < resident ? 16 : all < resident ? 32 : WAVE;
   A.open_per = WAVE;
+  // How long a wave may go on before its open lanes go to the wave-per-point
+  // kernel: the leaves walk A lists, and the groups and rounds of candidates
+  // walk B takes.  Hyperboloids of a shallow slope reach many leaves and hold
+  // most of their points, and points outside the root lie in leaves that no
+  // cube bounds; the longest waves are then the kernels of all but the largest
+  // clouds, and the heavy kernel, 30 to 60 ns a point, has the chip to itself.
+  // The three kernels in ms with 256 leaves and no budget, and so: slope 0.1,
+  // high outliers, 35k points 0.99 0.78, 60k 3.12 1.7, 150k 2.6 1.6, 400k 4.1 2.2,
+  // 1.17M 5.4 3.8, 2.4M 7.2 5.2, 7M 16.4 13.4, 23.7M 34.3 35.6; low ones, 150k 1.4
+  // 1.0, 1.17M 3.2 1.9, 7M 4.4 3.6, 23.7M 9.3 7.5; slope 1 with points outside the
+  // root, 60k 1.66 1.14, 70k 1.65 1.33.  At slope 1 in a root that holds all, the
+  // walks' longest waves cost less than the heavy kernel's start in some clouds
+  // and more in others (150k points, low outliers, 0.66 0.62; none 0.91 0.98).
+  // (Slope 0.3, 7M and more, is as slope 1: 16.1 and, handing over, 17.3.)
+  const bool shallow = A.max_slope < (all < 12 * resident ? 0.5 : 0.2);
+  A.leaf_cap = GROUND_LEAVES;
+  A.open_budget = INT32_MAX;
+  if (shallow || !A.cube_wedges) {
+    if (16 * all < resident) A.leaf_cap = 96;
+    else if (3 * all < resident) A.leaf_cap = shallow ? 32 : 64;
+    else if (all < 3 * resident) A.leaf_cap = 96;
+    else if (shallow) A.leaf_cap = all < 12 * resident ? 128 : 160;
+    A.open_budget = all < (shallow ? 12 : 3) * resident ? 512 : shallow ? 1024 : 2048;
+  }
   const uint64_t waves = (n + A.walk_per - 1) / A.walk_per;
   B.nrec = (size_t)waves * WAVE;
   const uint32_t ucap = (uint32_t)std::min<uint64_t>(waves * 4, 0x3fffffffull);
