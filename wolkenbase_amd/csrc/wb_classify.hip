@@ -2479,23 +2479,6 @@ __device__ inline uint64_t wave_or(uint64_t v)
 {
   return ((uint64_t)wave_or32((uint32_t)(v >> 32)) << 32) | wave_or32((uint32_t)v);
 }
-// OR over lanes 0-31 (h0) and over lanes 32-63 (h1): the row steps of
-// wave_or32, then row 0 folded into row 1 and row 2 into row 3, so lanes 31
-// and 63 hold the two halves' ORs.  Every lane active.
-__device__ inline void half_or(uint64_t v, uint64_t &h0, uint64_t &h1)
-{
-  uint32_t a = (uint32_t)v, b = (uint32_t)(v >> 32);
-  a = dpp_or<0xb1, 0xf>(a);   b = dpp_or<0xb1, 0xf>(b);   // quad_perm 1,0,3,2
-  a = dpp_or<0x4e, 0xf>(a);   b = dpp_or<0x4e, 0xf>(b);   // quad_perm 2,3,0,1
-  a = dpp_or<0x124, 0xf>(a);  b = dpp_or<0x124, 0xf>(b);  // row_ror 4
-  a = dpp_or<0x128, 0xf>(a);  b = dpp_or<0x128, 0xf>(b);  // row_ror 8
-  a = dpp_or<0x142, 0xa>(a);  b = dpp_or<0x142, 0xa>(b);  // row_bcast 15 into rows 1, 3
-  h0 = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)b, 31) << 32) |
-       (uint32_t)__builtin_amdgcn_readlane((int)a, 31);
-  h1 = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)b, 63) << 32) |
-       (uint32_t)__builtin_amdgcn_readlane((int)a, 63);
-}
-
 
 // ---------------------------------------------------------------------------
 // Ground-test walk: findBlocks (octree.cpp:234-251) for 64 hyperboloids at
@@ -2601,9 +2584,9 @@ __device__ inline uint32_t xor_bits8(uint32_t m, int r)
   return m;
 }
 
-// visiting order: child k has rank k ^ o (o: the xy quadrant taken first;
-// for a downward hyperboloid the lower half, bit 2 clear, comes first)
-__device__ inline int child_rank(int k, int o, int zf) { return ((k ^ o) & 3) | ((k ^ zf) & 4); }
+// visiting order: child k has rank k ^ o (o: the xy quadrant taken first; the
+// lower half, bit 2 clear, comes first, since the hyperboloids open downwards)
+__device__ inline int child_rank(int k, int o) { return k ^ o; }
 
 // Pushes the children of node `code` (cube cx, cy, cz, side at level lvl)
 // that may meet the hyperboloid of an open lane, in reverse visiting order:
@@ -3482,7 +3465,6 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
   work_point(A, i, slot, hs);
   const double x = T.px[slot], y = T.py[slot], z = T.pz[slot];
   const wb::Shape H = wb::make_hyperboloid(x - 0, y - 0, z - A.thickness, hs, A.max_slope);
-  const int zf = A.max_slope > 0 ? 0 : 4;
   int nexact = 0;
   // the directions k_ground found are a subset of D; the walks it completed
   // did not pass and are not repeated
@@ -3541,7 +3523,7 @@ __device__ __forceinline__ void heavy_body(const ClassifyArgs &A, const HeavyRec
           const double cx = nc[0], cy = nc[1], cz = nc[2], side = nc[3];
           const int o = (x >= cx ? 1 : 0) | (y >= cy ? 2 : 0);
           ck = T.node_child[8 * (size_t)code + k];
-          t = child_rank(k, o, zf);
+          t = child_rank(k, o);
           if (ck != -1) {
             const double ncx = cx + (double)(2 * (k & 1) - 1) * side / 4;
             const double ncy = cy + (double)(2 * ((k & 2) / 2) - 1) * side / 4;

@@ -772,8 +772,8 @@ WB_HD bool hyp_may_hit_box(const Shape &s, double x0, double x1, double y0, doub
 // (bins are pi/32 wide and the bin of a direction is that of atan2i, within
 // 2^-31 turn of the true angle), split in two where wider than pi so that
 // each is convex; at most two runs of >= 24 bins fit in 64 bins.  The exact
-// border pass never uses them: it needs the directions in the occupied bins
-// next to a run.
+// border pass needs the directions in the occupied bins next to a run too: its
+// wedges are border_wedges.
 // ---------------------------------------------------------------------------
 WB_HD uint64_t rotr64_(uint64_t x, int a) { return a ? (x >> a) | (x << (64 - a)) : x; }
 WB_HD uint64_t rotl64_(uint64_t x, int a) { return a ? (x << a) | (x >> (64 - a)) : x; }
