@@ -1553,7 +1553,8 @@ __device__ __attribute__((always_inline)) inline void scan_reg(
     WB_SUM(F.s1z, 1.0 * z)
 #undef WB_SUM
   }
-  fit_solve(F);
+  // (with the FP32 options only a tile that fell back has sums to solve)
+  if (!F32 || prec == WB_FIT_FP64 || __ballot(fell_back != 0)) fit_solve(F);
   if (F32 && !fit64) {
     F.sx = px;
     F.sy = py;
