@@ -924,22 +924,21 @@ WB_HD bool wedge_hit2(int n, const float ax[2], const float ay[2], const float b
   // The largest value of each cross product over the box: at its middle, plus
   // the half widths times the edge's components.  A corner close to the point
   // comes out of that by cancellation, with an error that goes with the box
-  // and not with the corner's distance: the conversions to float and the sums
-  // uc, uh, vc and vh leave at most 3 * 2^-24 of S = |uc| + uh + |vc| + vh in a
-  // product, its four roundings at most 4 * 2^-24.  eps, 2^-20 of S, is part of
-  // every product and covers both twice over, so a box with a direction of a
-  // care bin (10^-3 rad inside a widened edge) is kept.  (At the corner the
-  // edge's signs pick, as wedge_hit takes it, a product needs no eps but two
-  // selects.)
-  const float uc = 0.5f * (u0 + u1), vc = 0.5f * (v0 + v1), uh = 0.5f * (u1 - u0),
-              vh = 0.5f * (v1 - v0);
-  const float eps = 0x1p-20f * ((fabsf(uc) + uh) + (fabsf(vc) + vh));
+  // and not with the corner's distance: roundings (the offsets', the sums' and
+  // the product's own) leave at most 2^-24 (7 |uc| + 8 uh) of the edge's
+  // component in x, and the same in y.  So the half widths are taken 2^-17
+  // wider.  That covers an axis with |uc| <= 17 uh; on one farther off, every
+  // point of the box is at least 16/17 of |uc| away, and a direction of a care
+  // bin, 10^-3 rad inside a widened edge, makes its product thousands of times
+  // the error.  (At the corner the edge's signs pick, as wedge_hit takes it, a
+  // product needs no such care but two selects.)
+  constexpr float wide = 0.5f * (1.0f + 0x1p-17f);
+  const float uc = 0.5f * (u0 + u1), vc = 0.5f * (v0 + v1), uh = wide * (u1 - u0),
+              vh = wide * (v1 - v0);
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const float ra =
-        fmaf(ax[k], vc, fmaf(-ay[k], uc, fmaf(fabsf(ax[k]), vh, fmaf(fabsf(ay[k]), uh, eps))));
-    const float lb =
-        fmaf(uc, by[k], fmaf(-vc, bx[k], fmaf(fabsf(by[k]), uh, fmaf(fabsf(bx[k]), vh, eps))));
+    const float ra = fmaf(ax[k], vc, fmaf(-ay[k], uc, fmaf(fabsf(ax[k]), vh, fabsf(ay[k]) * uh)));
+    const float lb = fmaf(uc, by[k], fmaf(-vc, bx[k], fmaf(fabsf(by[k]), uh, fabsf(bx[k]) * vh)));
     const bool in_k = !(ra < 0) & !(lb < 0);
     hit |= k < n ? in_k : false;
   }
