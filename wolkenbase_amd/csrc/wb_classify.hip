@@ -2920,7 +2920,8 @@ struct OpenPoint {
   int hi[2], lo[2];
 };
 
-template <bool IN, bool GAP>
+// CAP: a long unit's open lanes go to the heavy kernel (A.open_budget).
+template <bool IN, bool GAP, bool CAP>
 __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t *pool, uint32_t nleaf,
                                           const Near &P, OpenPoint &O, const float *edges,
                                           double2 *edge, int &nexact)
@@ -3134,7 +3135,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
               }
             }
           }
-          work += taken + 1;
+          if (CAP) work += taken + 1;
           // many candidates: the directions just found may leave out the next
           // group's
           if (!GAP && taken >= OPEN_REFRESH && O.occ != checked && O.state == 0) {
@@ -3164,8 +3165,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
           else wb::lane_wedges_update(O.occ, edges, O.W);
         }
       }
-      // a long unit's open lanes go to the heavy kernel, a wave to the point
-      if (__builtin_expect(rfl((int)work) > A.open_budget, 0))
+      if (CAP && __builtin_expect(rfl((int)work) > A.open_budget, 0))
         O.state = O.state == want ? (GAP ? 7 : 6) : O.state;
       alive = __ballot(O.state == want);
       if (alive == 0) break;
@@ -3178,7 +3178,7 @@ __device__ __forceinline__ void open_pass(const ClassifyArgs &A, const uint32_t 
   }
 }
 
-template <bool IN>
+template <bool IN, bool CAP>
 __device__ __forceinline__ void open_body(const ClassifyArgs &A, uint32_t u, const float *edges,
                                           double2 *edge)
 {
@@ -3206,7 +3206,7 @@ __device__ __forceinline__ void open_body(const ClassifyArgs &A, uint32_t u, con
   const Near P = make_near(A, x, y, z, hs);
   int nexact = 0;
   wb::lane_wedges_update(O.occ, edges, O.W);
-  open_pass<IN, false>(A, pool, nleaf, P, O, edges, edge, nexact);
+  open_pass<IN, false, CAP>(A, pool, nleaf, P, O, edges, edge, nexact);
   if (O.state == 0) {
     O.state = gap_verdict(O.occ);
     if (O.state == 0) O.state = 4;
@@ -3237,7 +3237,7 @@ __device__ __forceinline__ void open_body(const ClassifyArgs &A, uint32_t u, con
                (uint32_t)after[1] << 24;
     O.hi[0] = O.hi[1] = -1;
     O.lo[0] = O.lo[1] = 0x7fffffff;
-    open_pass<IN, true>(A, pool, nleaf, P, O, edges, edge, nexact);
+    open_pass<IN, true, CAP>(A, pool, nleaf, P, O, edges, edge, nexact);
     if (O.state == 4) {
       const int g0 = (int)(((uint32_t)O.lo[0] - (uint32_t)O.hi[0]) & 0x7fffffffu);
       const int g1 = (int)(((uint32_t)O.lo[1] - (uint32_t)O.hi[1]) & 0x7fffffffu);
@@ -3316,7 +3316,7 @@ __global__ void __launch_bounds__(WAVE, MINW) k_ground_batch(const ClassifyArgs 
 
 // Unit u of walk B in the order of the classes (those with the longest leaf
 // lists first); false past the last.
-template <bool IN>
+template <bool IN, bool CAP>
 __device__ __forceinline__ bool open_unit(const ClassifyArgs &A, uint32_t u, const float *edges,
                                           double2 *edge)
 {
@@ -3330,7 +3330,7 @@ __device__ __forceinline__ bool open_unit(const ClassifyArgs &A, uint32_t u, con
     }
   }
   if (cls == OPEN_CLASSES) return false;
-  open_body<IN>(A, cls * A.unit_cap + u, edges, edge);
+  open_body<IN, CAP>(A, cls * A.unit_cap + u, edges, edge);
   return true;
 }
 
@@ -3338,19 +3338,19 @@ __device__ __forceinline__ bool open_unit(const ClassifyArgs &A, uint32_t u, con
 // classes block u takes unit u of their order, else wave u's.  (A resident
 // grid that takes the units by a counter was 3 to 7% slower on 40k to 300k
 // points: every claim waits for the counter's word.)
-template <bool IN, int MINW>
+template <bool IN, bool CAP, int MINW>
 __global__ void __launch_bounds__(WAVE, MINW) k_ground_open(ClassifyArgs A)
 {
   __shared__ float edges[3 * 128];
   __shared__ double2 edge[WAVE];
   ground_setup(A, edges);
-  if (A.open_classes) open_unit<IN>(A, blockIdx.x, edges, edge);
-  else if (blockIdx.x < A.unit_cap) open_body<IN>(A, blockIdx.x, edges, edge);
+  if (A.open_classes) open_unit<IN, CAP>(A, blockIdx.x, edges, edge);
+  else if (blockIdx.x < A.unit_cap) open_body<IN, CAP>(A, blockIdx.x, edges, edge);
 }
 
 // The same as a grid that stays resident and takes the units by a counter
 // (A.open_next, zero before the launch): with the context's sharing switch.
-template <bool IN>
+template <bool IN, bool CAP>
 __global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open_resident(ClassifyArgs A)
 {
   __shared__ float edges[3 * 128];
@@ -3359,7 +3359,7 @@ __global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open_resident(Cla
   for (;;) {
     uint32_t u = 0;
     if (threadIdx.x == 0) u = atomicAdd(A.open_next, 1u);
-    if (!open_unit<IN>(A, (uint32_t)rfl((int)u), edges, edge)) return;
+    if (!open_unit<IN, CAP>(A, (uint32_t)rfl((int)u), edges, edge)) return;
   }
 }
 
@@ -3401,7 +3401,7 @@ __global__ void __launch_bounds__(WAVE) k_batch_sums(const ClassifyArgs *AA, int
 // the longest lists of every tree first (uoff: k_batch_sums).  A grid of as
 // many blocks as there can be units needs no counter: taking the units tree by
 // tree, each wave by each tree's counter, took 12 trees of 150k points 4.4 ms.
-template <bool IN>
+template <bool IN, bool CAP>
 __global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open_batch(const ClassifyArgs *AA,
                                                                           const uint32_t *uoff,
                                                                           int ntrees)
@@ -3412,7 +3412,7 @@ __global__ void __launch_bounds__(WAVE, WB_OPEN_MINW) k_ground_open_batch(const 
   if (e == ntrees * OPEN_CLASSES) return;
   const ClassifyArgs &A = AA[e % ntrees];
   ground_setup(A, edges);
-  open_body<IN>(A, (uint32_t)(e / ntrees) * A.unit_cap + blockIdx.x - uoff[e], edges, edge);
+  open_body<IN, CAP>(A, (uint32_t)(e / ntrees) * A.unit_cap + blockIdx.x - uoff[e], edges, edge);
 }
 
 // One heavy point per 64-lane block.  The shape is the same in every lane,
@@ -4237,22 +4237,31 @@ static void launch_ground(wb_ctx *c, const ClassifyArgs &A, uint64_t n, uint32_t
       else
         hipLaunchKernelGGL((k_ground<false, WB_GROUND_MINW>), dim3(nb), one, 0, st, A);
     }
+    const bool cap = A.open_budget != INT32_MAX;
     if (c->sharing) {  // 12 of the 20 waves a CU holds
       const dim3 ogrid(std::min<uint32_t>(nb, 12u * ncu));
-      if (A.cube_wedges) hipLaunchKernelGGL(k_ground_open_resident<true>, ogrid, one, 0, st, A);
-      else hipLaunchKernelGGL(k_ground_open_resident<false>, ogrid, one, 0, st, A);
+      if (!A.cube_wedges)
+        hipLaunchKernelGGL((k_ground_open_resident<false, true>), ogrid, one, 0, st, A);
+      else if (cap)
+        hipLaunchKernelGGL((k_ground_open_resident<true, true>), ogrid, one, 0, st, A);
+      else
+        hipLaunchKernelGGL((k_ground_open_resident<true, false>), ogrid, one, 0, st, A);
     } else {
       const dim3 ogrid(nb * (A.walk_per / A.open_per));
       // with many units six waves per SIMD hide more than the registers they
       // give up cost (23.7M points, mostly ground: about 1 ms of 29 less than
       // with five); with few the longest unit is the kernel (1.17M: 1.95 ms
       // with five, 2.09 with six)
-      if (A.cube_wedges && A.open_classes)
-        hipLaunchKernelGGL((k_ground_open<true, WB_OPEN_MINW>), ogrid, one, 0, st, A);
-      else if (A.cube_wedges)
-        hipLaunchKernelGGL((k_ground_open<true, 6>), ogrid, one, 0, st, A);
+      if (!A.cube_wedges)
+        hipLaunchKernelGGL((k_ground_open<false, true, WB_OPEN_MINW>), ogrid, one, 0, st, A);
+      else if (cap && A.open_classes)
+        hipLaunchKernelGGL((k_ground_open<true, true, WB_OPEN_MINW>), ogrid, one, 0, st, A);
+      else if (cap)
+        hipLaunchKernelGGL((k_ground_open<true, true, 6>), ogrid, one, 0, st, A);
+      else if (A.open_classes)
+        hipLaunchKernelGGL((k_ground_open<true, false, WB_OPEN_MINW>), ogrid, one, 0, st, A);
       else
-        hipLaunchKernelGGL((k_ground_open<false, WB_OPEN_MINW>), ogrid, one, 0, st, A);
+        hipLaunchKernelGGL((k_ground_open<true, false, 6>), ogrid, one, 0, st, A);
     }
   }
   if (ev) {
@@ -4440,9 +4449,11 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
   std::vector<ClassifyArgs> AA(ntrees);
   std::vector<uint32_t> boff(ntrees + 1, 0);
   bool inside = true;  // every tree's points lie in their leaves' cubes
+  bool cap = false;    // a tree's units are cut short
   for (int k = 0; k < ntrees; k++) {
     AA[k] = R[k].A;
     inside = inside && AA[k].cube_wedges;
+    cap = cap || AA[k].open_budget != INT32_MAX;
     const uint64_t nb = boff[k] + (uint64_t)wb_blocks(R[k].n, AA[k].walk_per);
     if (nb > 0xffffffffull) throw std::string("too many points in one batch");
     boff[k + 1] = (uint32_t)nb;
@@ -4460,12 +4471,13 @@ void wb_run_classify_batch(wb_ctx *c, wb_tree *const *trees, int ntrees, const d
       hipLaunchKernelGGL((k_ground_batch<true, WB_GROUND_MINW>), dim3(boff[ntrees]), one, 0, st, dAA,
                          doff, ntrees);
       hipLaunchKernelGGL(k_batch_sums, dim3(1), one, 0, st, dAA, ntrees, 1, dsum);
-      hipLaunchKernelGGL(k_ground_open_batch<true>, ogrid, one, 0, st, dAA, dsum, ntrees);
+      if (cap) hipLaunchKernelGGL((k_ground_open_batch<true, true>), ogrid, one, 0, st, dAA, dsum, ntrees);
+      else hipLaunchKernelGGL((k_ground_open_batch<true, false>), ogrid, one, 0, st, dAA, dsum, ntrees);
     } else {
       hipLaunchKernelGGL((k_ground_batch<false, WB_GROUND_MINW>), dim3(boff[ntrees]), one, 0, st,
                          dAA, doff, ntrees);
       hipLaunchKernelGGL(k_batch_sums, dim3(1), one, 0, st, dAA, ntrees, 1, dsum);
-      hipLaunchKernelGGL(k_ground_open_batch<false>, ogrid, one, 0, st, dAA, dsum, ntrees);
+      hipLaunchKernelGGL((k_ground_open_batch<false, true>), ogrid, one, 0, st, dAA, dsum, ntrees);
     }
   }
   for (int k = 0; k < ntrees; k++) {
